@@ -69,6 +69,7 @@ __global__ __launch_bounds__(VAL_THREADS) void k_validate(const int4 *__restrict
                                                           int64_t V, int32_t *__restrict__ err) {
     __shared__ int32_t red[2][VAL_THREADS / 64];
     const int64_t ntiles = (T + VAL_TILE - 1) / VAL_TILE;
+    int32_t wide7 = 0, wide8 = 0;  // thread 0: this block's wide tiles
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         int32_t lo = INT32_MAX, hi = -1;
         bool bad = false;
@@ -101,12 +102,14 @@ __global__ __launch_bounds__(VAL_THREADS) void k_validate(const int4 *__restrict
                 hi = max(hi, red[1][w]);
             }
             if (lo >= 0 && hi >= lo) {
-                if ((hi >> 7) - (lo >> 7) >= 1024) atomicAdd(err + 1, 1);
-                if ((hi >> 8) - (lo >> 8) >= 1024) atomicAdd(err + 2, 1);
+                wide7 += (hi >> 7) - (lo >> 7) >= 1024;
+                wide8 += (hi >> 8) - (lo >> 8) >= 1024;
             }
         }
         __syncthreads();  // red is reused by the next tile
     }
+    if (wide7) atomicAdd(err + 1, wide7);
+    if (wide8) atomicAdd(err + 2, wide8);
 }
 
 __global__ void k_label6(const uint32_t *__restrict__ classes, int64_t V,
@@ -220,7 +223,7 @@ int tg_mesh_create(tg_mesh **out, const int32_t *cells, int64_t n_cells,
         int32_t *err = m->counters.as<int32_t>();
         if ((rc = tg::fill_i32(err, 0, 3, m->stream))) return bail(rc);
         const int64_t tiles = (n_cells + VAL_TILE - 1) / VAL_TILE;
-        const unsigned g = (unsigned)std::min<int64_t>(tiles, 16384);
+        const unsigned g = (unsigned)std::min<int64_t>(tiles, 1024);
         hipLaunchKernelGGL(k_validate, dim3(g), dim3(VAL_THREADS), 0, m->stream,
                            (const int4 *)m->tv.p, n_cells, n_points, err);
         if (hipGetLastError() != hipSuccess) return bail(fail(TG_ERR_HIP, "k_validate launch"));

@@ -30,7 +30,6 @@ using tg::C_ERR;
 using tg::C_FIX;
 using tg::C_FIXBIG;
 using tg::C_HEAVY;
-using tg::C_MAXDEG;
 using tg::HEAVY_CAP;
 
 // critPoints.cu:136-140: equal scalars fall back to the id comparison.
@@ -229,10 +228,6 @@ __global__ __launch_bounds__(BLOCK) void k_vv_cp_lane(
     wave_append(heavy, counters + C_HEAVY, v, active && over);
     wave_append(fix, counters + C_FIX, v,
                 active && !over && classify && (nl >= 2 || nu >= 2));
-    int wmax = (active && !over) ? m : 0;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) wmax = max(wmax, __shfl_xor(wmax, d, 64));
-    if (__lane_id() == 0 && wmax > 0) atomicMax(counters + C_MAXDEG, wmax);
 }
 
 // Serial fallback for vertices whose neighbour list overflows the lane list:
@@ -319,7 +314,6 @@ __global__ __launch_bounds__(64) void k_vv_cp_heavy(
             classes[3 * (int64_t)v + 2] = verdict(nl, nu);
         }
         deg[v] = m;
-        atomicMax(counters + C_MAXDEG, m);
         // ascending row via insertion sort in LDS
         for (int i = 1; i < m; i++) {
             const int32_t x = list[i];

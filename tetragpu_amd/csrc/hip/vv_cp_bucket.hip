@@ -35,7 +35,6 @@ using tg::C_ERR;
 using tg::C_FIX;
 using tg::C_FIXBIG;
 using tg::C_HEAVY;
-using tg::C_MAXDEG;
 using tg::HEAVY_CAP;
 
 constexpr int SLOTS = 32;
@@ -941,10 +940,6 @@ __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_vv_cp(
     if (act) rowsrc[v0 + vl] = 3 * cbeg + loff;
     wave_append(heavy, counters + C_HEAVY, v0 + vl, hv);
     wave_append(fixd, counters + tg::C_FIXD, v0 + vl, ok && classify && (nl >= 2 || nu >= 2));
-    int dm = ok ? d : 0;
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) dm = max(dm, __shfl_xor(dm, s, 64));
-    if (lane == 0 && dm > 0) atomicMax(counters + C_MAXDEG, dm);
     __syncthreads();
 
     // phase 4: coalesced store of the bucket's rows and row descriptors
@@ -1174,10 +1169,6 @@ __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_own(
     if (act) rowsrc[v0 + vl] = 3 * cbeg + loff;
     wave_append(heavy, counters + C_HEAVY, v0 + vl, hv);
     wave_append(fixd, counters + tg::C_FIXD, v0 + vl, ok && classify && (nl >= 2 || nu >= 2));
-    int dm = ok ? d : 0;
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) dm = max(dm, __shfl_xor(dm, s, 64));
-    if (lane == 0 && dm > 0) atomicMax(counters + C_MAXDEG, dm);
     __syncthreads();
 
     int32_t *dst = scratch + 3 * (int64_t)cbeg;
@@ -1356,7 +1347,6 @@ __global__ __launch_bounds__(HV_THREADS) void k_bkt_heavy(
         if (tid == 0) {
             const uint32_t nl = (uint32_t)misc[2], nu = (uint32_t)misc[3];
             deg[v] = m;
-            atomicMax(counters + C_MAXDEG, m);
             if (classify) {
                 classes[3 * (int64_t)v] = nl;
                 classes[3 * (int64_t)v + 1] = nu;
