@@ -97,6 +97,57 @@ __device__ __forceinline__ T wave_inclusive_sum(T x) {
     return x;
 }
 
+// Hides a value from the compiler's analyses, which walk nested minima and
+// maxima in a time that is exponential in the depth of a sorting network.
+template <typename T>
+__device__ __forceinline__ T opaque(T x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(x));
+#endif
+    return x;
+}
+
+// Keeps the compiler's scheduler from moving instructions across (long
+// unrolled walks would otherwise start many elements early and spill).
+__device__ __forceinline__ void sched_fence() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// Words that workgroups of one launch hand to each other (one word carries
+// flag and value, so no order with other memory is needed).
+__device__ __forceinline__ uint64_t load_agent(const uint64_t *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+    return __atomic_load_n(p, __ATOMIC_RELAXED);
+#endif
+}
+__device__ __forceinline__ void store_agent(uint64_t *p, uint64_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+    __atomic_store_n(p, v, __ATOMIC_RELAXED);
+#endif
+}
+__device__ __forceinline__ void pause() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_s_sleep(1);
+#endif
+}
+
+// Orders the LDS accesses of one wave's lanes (its LDS instructions execute
+// in order, so the compiler alone has to be held).
+__device__ __forceinline__ void wave_sync() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#else
+    (void)__ballot(1);
+#endif
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T x) {
 #pragma unroll

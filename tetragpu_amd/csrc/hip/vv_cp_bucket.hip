@@ -530,49 +530,9 @@ __global__ __launch_bounds__(S1_THREADS) void k_s1_scatter(const int4 *__restric
 }
 
 // ---- B: per-bucket neighbour sets, link components, sorted rows --------------
-// Probe order of key u in a 32-slot table: 8 groups of 4 slots (one 16-byte
-// LDS read per group), starting at the home group from a multiplicative
-// hash; inside a group a key claims the first empty slot at or after its
-// hint slot (cyclic), so two new keys of one group seldom race for a slot.
+// Home slot of key u in a 32-slot table.
 __device__ __forceinline__ uint32_t key_hash(int32_t u) {
-    return ((uint32_t)u * 2654435769u) >> 27;  // 5 bits: group (3) | slot hint (2)
-}
-
-// First empty slot of a group snapshot at or after slot p (cyclic), or -1.
-__device__ __forceinline__ int first_empty_from(const int4 q, int p) {
-    const uint32_t m = (uint32_t)(q.x == -1) | ((uint32_t)(q.y == -1) << 1) |
-                       ((uint32_t)(q.z == -1) << 2) | ((uint32_t)(q.w == -1) << 3);
-    const uint32_t r = ((m | (m << 4)) >> p) & 15u;  // rotate so slot p is bit 0
-    return r ? (int)((__ffs(r) - 1 + p) & 3) : -1;
-}
-
-// Insert u into a vertex's table (lock-free: slots only go from empty (-1)
-// to a key by CAS, and every thread inserting u follows the same probe
-// order, so u lands in exactly one slot).  Returns the slot or -1 if full.
-// HINT: start each group at the key's hint slot (else at slot 0); every
-// insert into one table must use the same setting.
-template <bool HINT>
-__device__ __forceinline__ int hash_insert(int32_t *tab, int32_t u) {
-    const uint32_t h = key_hash(u);
-#pragma unroll 1
-    for (int step = 0; step < SLOTS / 4; step++) {
-        const int g = (int)(((h >> 2) + (uint32_t)step) & (SLOTS / 4 - 1));
-        int32_t *grp = tab + 4 * g;
-        int4 q = *reinterpret_cast<const int4 *>(grp);
-#pragma unroll 1
-        for (int tries = 0; tries < 4; tries++) {
-            if (q.x == u) return 4 * g;
-            if (q.y == u) return 4 * g + 1;
-            if (q.z == u) return 4 * g + 2;
-            if (q.w == u) return 4 * g + 3;
-            const int e = first_empty_from(q, HINT ? (int)(h & 3u) : 0);
-            if (e < 0) break;
-            const int32_t old = atomicCAS(&grp[e], -1, u);
-            if (old == -1 || old == u) return 4 * g + e;
-            q = *reinterpret_cast<const int4 *>(grp);  // lost to another key
-        }
-    }
-    return -1;
+    return ((uint32_t)u * 2654435769u) >> 27;
 }
 
 // Components of `mask` under the slot adjacency, numbered 0.. in order of
@@ -654,12 +614,10 @@ __device__ __forceinline__ void lean_insert3(int32_t *tab, int32_t x, int32_t y,
     sz = dz ? pz : -1;
 }
 
-// INS selects phase 1: 0 batches of four records per thread with group
-// snapshots; 1 record by record with lean_insert3, four records per thread
-// in flight, the wave in lock-step per record (about 40 % fewer VALU
-// instructions per key; same time on MI355X, where the insert is bound by the
-// dependent LDS round trips of the probe chains, not by instruction count).
-template <int BV_LOG, typename S, int INS>
+// B, shared-table form (lean insert): record by record with lean_insert3, four
+// records per thread in flight, the wave in lock-step per record.  Bound by
+// the dependent LDS round trips of the probe chains, not by instruction count.
+template <int BV_LOG, typename S>
 __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_vv_cp(
     const Rec rec, const int32_t *__restrict__ h2s, int32_t nslice,
     const S *__restrict__ scal, int32_t V, int classify, int32_t *__restrict__ scratch,
@@ -668,15 +626,11 @@ __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_vv_cp(
     int32_t *__restrict__ counters) {
     constexpr int BV = 1 << BV_LOG;
     constexpr int NT = 2 * BV;
-    constexpr int BATCH = 4;
     constexpr int PER_T = BV * SLOTS / NT;  // slots per thread in phase 2 (16)
     // table strides: a vertex's slots start 36 (keys, 16-byte groups) or 33
     // (adjacency) words after the previous vertex's, so accesses of many
     // vertices at one slot index spread over the LDS banks
     constexpr int KS = SLOTS + 4, AS = SLOTS + 1;
-    // hint slots cut CAS conflicts but cost registers: at 512 threads they
-    // would halve the resident blocks (measured on MI355X, Kuhn 128^3)
-    constexpr bool HINT = BV_LOG == 7;
     __shared__ __align__(16) int32_t key[BV * KS];
     __shared__ uint32_t adj[BV * AS];
     __shared__ uint32_t occ[BV], lowm[BV];
@@ -702,137 +656,41 @@ __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_vv_cp(
     }
     __syncthreads();
 
-    if constexpr (INS == 1) {
-        // four records per thread in flight: record i + k * NT sits in ring
-        // slot k; a slot is refilled with the record four strides ahead as
-        // soon as its record is taken
-        constexpr int DEPTH = 4;
-        uint32_t q[DEPTH][3];
+    // phase 1: neighbour sets and shared-tet link adjacency
+    // four records per thread in flight: record i + k * NT sits in ring
+    // slot k; a slot is refilled with the record four strides ahead as
+    // soon as its record is taken
+    constexpr int DEPTH = 4;
+    uint32_t q[DEPTH][3];
+#pragma unroll
+    for (int k = 0; k < DEPTH; k++) {
+        const int32_t i = cbeg + tid + k * NT;
+        q[k][0] = 0xFFFFFFFFu;
+        if (i < cend) {
+            q[k][0] = rec.w0[i];
+            q[k][1] = rec.w1[i];
+            q[k][2] = rec.w2[i];
+        }
+    }
+#pragma unroll 1
+    for (int32_t i0 = cbeg + tid; i0 < cend; i0 += DEPTH * NT) {
 #pragma unroll
         for (int k = 0; k < DEPTH; k++) {
-            const int32_t i = cbeg + tid + k * NT;
+            const uint32_t w0 = q[k][0], w1 = q[k][1], w2 = q[k][2];
+            const int32_t nx = i0 + (k + DEPTH) * NT;
             q[k][0] = 0xFFFFFFFFu;
-            if (i < cend) {
-                q[k][0] = rec.w0[i];
-                q[k][1] = rec.w1[i];
-                q[k][2] = rec.w2[i];
+            if (nx < cend) {
+                q[k][0] = rec.w0[nx];
+                q[k][1] = rec.w1[nx];
+                q[k][2] = rec.w2[nx];
             }
-        }
-#pragma unroll 1
-        for (int32_t i0 = cbeg + tid; i0 < cend; i0 += DEPTH * NT) {
-#pragma unroll
-            for (int k = 0; k < DEPTH; k++) {
-                const uint32_t w0 = q[k][0], w1 = q[k][1], w2 = q[k][2];
-                const int32_t nx = i0 + (k + DEPTH) * NT;
-                q[k][0] = 0xFFFFFFFFu;
-                if (nx < cend) {
-                    q[k][0] = rec.w0[nx];
-                    q[k][1] = rec.w1[nx];
-                    q[k][2] = rec.w2[nx];
-                }
-                if (w0 == 0xFFFFFFFFu) continue;
-                uint32_t v, x, y, z;
-                rec_unpack(w0, w1, w2, v, x, y, z);
-                const int vl = (int)(v & (BV - 1));
-                int a, b2, c;
-                lean_insert3(key + vl * KS, (int32_t)x, (int32_t)y, (int32_t)z, a, b2, c);
-                atomicAdd(&ccount[vl], 1);
-                if ((a | b2 | c) < 0) {
-                    ovf[vl] = 1;
-                } else {
-                    uint32_t *av = adj + vl * AS;
-                    atomicOr(&av[a], (1u << b2) | (1u << c));
-                    atomicOr(&av[b2], (1u << a) | (1u << c));
-                    atomicOr(&av[c], (1u << a) | (1u << b2));
-                }
-            }
-        }
-    } else
-    // phase 1: neighbour sets and shared-tet link adjacency.  For a batch of
-    // keys: all group reads are issued together; a key found in its group
-    // snapshot is placed, otherwise it claims the snapshot's first empty
-    // slot by CAS, and all those CAS are issued before any result is used,
-    // so a batch costs about two LDS round trips.  Keys whose CAS lost to a
-    // different key (or whose group was full) are queued in a per-lane mask
-    // and resolved by one shared probing loop.
-    for (int32_t i0 = cbeg + tid; i0 < cend; i0 += BATCH * NT) {
-        constexpr int NK = 3 * BATCH;
-        uint32_t w[BATCH][3];
-#pragma unroll
-        for (int k = 0; k < BATCH; k++) {
-            const int32_t i = i0 + k * NT;
-            w[k][0] = 0xFFFFFFFFu;
-            if (i < cend) {
-                w[k][0] = rec.w0[i];
-                w[k][1] = rec.w1[i];
-                w[k][2] = rec.w2[i];
-            }
-        }
-        int32_t u[NK];
-        int vls[BATCH];
-#pragma unroll
-        for (int k = 0; k < BATCH; k++) {
-            uint32_t v = 0, x = 0, y = 0, z = 0;
-            if (w[k][0] != 0xFFFFFFFFu) rec_unpack(w[k][0], w[k][1], w[k][2], v, x, y, z);
-            vls[k] = (int)(v & (BV - 1));
-            u[3 * k] = (int32_t)x;
-            u[3 * k + 1] = (int32_t)y;
-            u[3 * k + 2] = (int32_t)z;
-        }
-        int4 grp[NK];
-#pragma unroll
-        for (int j = 0; j < NK; j++) {
-            const uint32_t g = key_hash(u[j]) >> 2;
-            grp[j] = *reinterpret_cast<const int4 *>(key + vls[j / 3] * KS + 4 * g);
-        }
-        int sl[NK], cs[NK];
-#pragma unroll
-        for (int j = 0; j < NK; j++) {
-            const int32_t x = u[j];
-            const uint32_t h = key_hash(x);
-            const int g = (int)(h >> 2);
-            const int4 q = grp[j];
-            const int f = q.x == x ? 0 : q.y == x ? 1 : q.z == x ? 2 : q.w == x ? 3 : -1;
-            const int e = first_empty_from(q, HINT ? (int)(h & 3u) : 0);
-            const bool valid = w[j / 3][0] != 0xFFFFFFFFu;
-            sl[j] = f >= 0 ? 4 * g + f : -1;
-            cs[j] = (valid && f < 0 && e >= 0) ? 4 * g + e : -1;  // slot to claim
-            if (valid && f < 0 && e < 0) sl[j] = -2;            // group full
-        }
-        int32_t old[NK];
-#pragma unroll
-        for (int j = 0; j < NK; j++)
-            old[j] = cs[j] >= 0 ? atomicCAS(key + vls[j / 3] * KS + cs[j], -1, u[j]) : 0;
-        uint32_t pending = 0;
-#pragma unroll
-        for (int j = 0; j < NK; j++) {
-            if (cs[j] >= 0) sl[j] = (old[j] == -1 || old[j] == u[j]) ? cs[j] : -2;
-            if (sl[j] == -2) pending |= 1u << j;
-        }
-        while (__any(pending != 0)) {
-            if (pending) {
-                const int j = __ffs(pending) - 1;
-                pending &= pending - 1u;
-                int32_t x = 0;
-                int vl = 0;
-#pragma unroll
-                for (int t = 0; t < NK; t++)
-                    if (t == j) {
-                        x = u[t];
-                        vl = vls[t / 3];
-                    }
-                const int r = hash_insert<HINT>(key + vl * KS, x);
-#pragma unroll
-                for (int t = 0; t < NK; t++)
-                    if (t == j) sl[t] = r;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < BATCH; k++) {
-            if (w[k][0] == 0xFFFFFFFFu) continue;
-            const int vl = vls[k];
+            if (w0 == 0xFFFFFFFFu) continue;
+            uint32_t v, x, y, z;
+            rec_unpack(w0, w1, w2, v, x, y, z);
+            const int vl = (int)(v & (BV - 1));
+            int a, b2, c;
+            lean_insert3(key + vl * KS, (int32_t)x, (int32_t)y, (int32_t)z, a, b2, c);
             atomicAdd(&ccount[vl], 1);
-            const int a = sl[3 * k], b2 = sl[3 * k + 1], c = sl[3 * k + 2];
             if ((a | b2 | c) < 0) {
                 ovf[vl] = 1;
             } else {
@@ -953,6 +811,397 @@ __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_vv_cp(
         }
     } else {
         for (int i = tid; i < xt; i += NT) dst[i] = key[i];
+    }
+}
+
+// ---- B, sorting form: one lane per vertex, rows from a register network ---------
+// The default bucket kernel.  A bucket's records are first counted per vertex
+// and placed, vertex by vertex, in LDS (one returning LDS atomic per record);
+// then each lane takes one vertex: it loads its records' 3 x c keys into
+// registers, sorts them with a compile-time network, and reads the distinct
+// neighbours off in order.  A key carries its record's number in its low
+// byte, so the same walk notes which slots each record joins (the link
+// triangles).  Scalars, components and rows follow per lane; every LDS access
+// after the placement is to the lane's own column (word slot * 64 + lane: no
+// bank conflicts, no atomics between lanes, no retries).  Where record counts
+// are uneven, lanes take the vertices by falling count, so that a wave's
+// network is no longer than its own vertices need.
+//
+// What bounds it: VALU issue of the sort (671 compare-exchanges for the 24
+// records of an interior Kuhn vertex) at two waves per SIMD.  The shared hash
+// tables it replaced waited on chains of dependent LDS round trips.  LDS is
+// what limits the waves: 20 KB a wave, records of nine bytes, for 64 vertices
+// of 33 records each.
+constexpr int SK_MAXREC = 48;       // records per vertex; more go to the heavy kernel
+constexpr int SK_PRE = 24;          // records per thread held in registers while counting
+constexpr int SK_ROWS = SLOTS + 1;  // row slots per vertex, the last one for what does not fit
+template <int BV>
+constexpr int sk_slab = BV * 275 / 8;  // record slots of a block of BV vertices
+template <int BV>
+constexpr int sk_span = sk_slab<BV> - SK_MAXREC - BV;  // offsets of one round
+
+// Knuth's merge exchange (The Art of Computer Programming 3, 5.2.2 M) for any
+// N: for p = 2^(t-1) .. 1, compare (i, i + p) where i & p == 0, then
+// (i, i + q - p) where i & p for q = 2^(t-1) .. 2p.
+template <int N, int D, int P, int R>
+__device__ __forceinline__ void sort_stage(uint32_t (&k)[N]) {
+#pragma unroll
+    for (int i = 0; i < N - D; i++)
+        if ((i & P) == R) {
+            const uint32_t a = k[i], b = k[i + D];
+            k[i] = tgd::opaque(min(a, b));
+            k[i + D] = tgd::opaque(max(a, b));
+        }
+}
+template <int N, int P, int Q>
+__device__ __forceinline__ void sort_merges(uint32_t (&k)[N]) {
+    if constexpr (Q > P) {
+        sort_stage<N, Q - P, P, P>(k);
+        sort_merges<N, P, Q / 2>(k);
+    }
+}
+template <int N, int P, int TOP>
+__device__ __forceinline__ void sort_phases(uint32_t (&k)[N]) {
+    if constexpr (P > 0) {
+        sort_stage<N, P, P, 0>(k);
+        sort_merges<N, P, TOP>(k);
+        sort_phases<N, P / 2, TOP>(k);
+    }
+}
+constexpr int top_power(int n) { return n <= 2 ? 1 : 2 * top_power((n + 1) / 2); }  // 2^(ceil(log2 n) - 1)
+template <int N>
+__device__ __forceinline__ void sort_keys(uint32_t (&k)[N]) {
+    sort_phases<N, top_power(N), top_power(N)>(k);
+}
+
+// Components of `mask` as label_components, over a lane's column of the
+// adjacency and of the row (slot f at word f * 64).
+__device__ __forceinline__ uint32_t label_columns(const uint32_t *adj, uint32_t *row,
+                                                  uint32_t mask, uint32_t tag) {
+    uint32_t cnt = 0, rem = mask;
+    while (rem) {
+        uint32_t comp = rem & (0u - rem);
+        uint32_t front = comp;
+        while (front) {
+            const int f = __ffs(front) - 1;
+            front &= front - 1u;
+            const uint32_t nb = adj[f * 64] & mask & ~comp;
+            row[f * 64] = (row[f * 64] << 6) | tag | cnt;
+            comp |= nb;
+            front |= nb;
+        }
+        rem &= ~comp;
+        cnt++;
+    }
+    return cnt;
+}
+
+// Records in LDS: three 24-bit keys as two words and a byte.
+struct Slab {
+    uint32_t *w0, *w1;
+    uint8_t *b2;
+};
+
+// Rows of a wave's vertices, at most R records each: sorts the lane's c
+// records (at slots pos, pos + 1, ..) and leaves the distinct neighbours in
+// the lane's row column, ascending; with CP, the link adjacency in its
+// adjacency column.  Returns their number (over SLOTS: the columns are not
+// usable).  Contains one workgroup barrier, between the reads of the records
+// and the columns that overlay them; every wave of the block makes one call
+// (of some R), so all waves meet at it.
+//
+// A key is neighbour << 8 | code.  R <= 32: the code is the record's number
+// and the walk collects each record's slots as a 32-bit mask.  R > 32: the
+// code is (record / 2) << 3 | 3 * (record & 1) + corner and the walk collects
+// six 5-bit slot numbers per word, so that 48 records fit the same columns.
+template <int R, bool CP>
+__device__ __forceinline__ int sort_rows(const Slab &rec, int pos, int c, uint32_t *row,
+                                         uint32_t *adj) {
+    constexpr int N = 3 * R;
+    constexpr bool MASKS = R <= 32;
+    constexpr int NCOL = MASKS ? R : R / 2;  // words of collected slots
+    constexpr uint32_t NOKEY = 0xFFFFFF00u | (MASKS ? (uint32_t)R : 8u * NCOL + 5u);
+    uint32_t k[N];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint32_t code = MASKS ? (uint32_t)r : (uint32_t)(8 * (r / 2) + 3 * (r & 1));
+        const bool on = r < c;
+        const uint32_t a = rec.w0[pos + r], b = rec.w1[pos + r], z = rec.b2[pos + r];
+        k[3 * r] = on ? (a << 8) | code : NOKEY;
+        k[3 * r + 1] = on ? (b << 8) | (MASKS ? code : code + 1) : NOKEY;
+        k[3 * r + 2] = on ? (z << 24) | ((b >> 24) << 16) | ((a >> 24) << 8) |
+                                (MASKS ? code : code + 2)
+                          : NOKEY;
+        if (r % 8 == 7) tgd::sched_fence();
+    }
+    __syncthreads();
+    sort_keys(k);
+    if (CP) {
+#pragma unroll
+        for (int r = 0; r < NCOL; r++) adj[r * 64] = 0u;
+    }
+    int slot = -1;
+    uint32_t prev = ~k[0];
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        slot += (k[j] ^ prev) > 255u;
+        prev = k[j];
+        row[min(slot, SLOTS) * 64] = k[j] >> 8;
+        if (CP) {
+            if constexpr (MASKS)
+                atomicOr(&adj[(k[j] & 63u) * 64], 1u << (slot & 31));
+            else
+                atomicOr(&adj[((k[j] >> 3) & 31u) * 64],
+                         (uint32_t)(slot & 31) << (5u * (k[j] & 7u)));
+        }
+        if (j % 8 == 7) tgd::sched_fence();
+    }
+    const int d = slot + 1 - (3 * c < N);  // the padding counts once
+    if (CP) {
+        uint32_t m[NCOL];
+#pragma unroll
+        for (int r = 0; r < NCOL; r++) m[r] = adj[r * 64];
+#pragma unroll
+        for (int s = 0; s < SLOTS; s++) adj[s * 64] = 0u;
+        if constexpr (MASKS) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                uint32_t q = m[r];
+#pragma unroll
+                for (int j = 0; j < 3; j++) {  // row SLOTS takes what records beyond c would set
+                    const uint32_t s = min((uint32_t)(__ffs(q) - 1), (uint32_t)SLOTS);
+                    q &= q - 1u;
+                    atomicOr(&adj[s * 64], m[r]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const uint32_t q = m[r / 2] >> (15 * (r & 1));
+                const uint32_t s0 = q & 31u, s1 = (q >> 5) & 31u, s2 = (q >> 10) & 31u;
+                const uint32_t b = r < c ? (1u << s0) | (1u << s1) | (1u << s2) : 0u;
+                atomicOr(&adj[s0 * 64], b);
+                atomicOr(&adj[s1 * 64], b);
+                atomicOr(&adj[s2 * 64], b);
+            }
+        }
+    }
+    return d;
+}
+
+// CP: classes as well as rows.
+template <int BV_LOG, typename S, bool CP>
+__global__ __launch_bounds__(1 << BV_LOG, 2) void k_bkt_sort(
+    const Rec rec, const int32_t *__restrict__ h2s, int32_t nslice,
+    const S *__restrict__ scal, int32_t V, int32_t *__restrict__ scratch,
+    int32_t *__restrict__ deg, int32_t *__restrict__ rowsrc, uint32_t *__restrict__ classes,
+    int32_t *__restrict__ heavy, int32_t *__restrict__ fixd, uint8_t *__restrict__ rowdesc,
+    int32_t *__restrict__ counters) {
+    constexpr int BV = 1 << BV_LOG, NT = BV, NW = NT / 64;
+    constexpr int SLAB = sk_slab<BV>, SPAN = sk_span<BV>;
+    constexpr int32_t ELSEWHERE = -(1 << 30);  // cursor of a vertex without slots this round
+    constexpr int COLS = NW * SK_ROWS * 64;    // row columns, then as many adjacency words
+    constexpr int WORDS = (9 * SLAB + 3) / 4;
+    static_assert(WORDS >= 2 * COLS, "the columns overlay the records");
+    static_assert(COLS >= BV * SLOTS, "the adjacency columns become the row staging");
+    __shared__ uint32_t slab[WORDS];
+    __shared__ int32_t cur[BV];     // by vertex: count, cursor, results, row offset
+    __shared__ uint16_t vert[BV];   // lane -> vertex
+    __shared__ int32_t hist[64];
+    __shared__ int32_t wsum[NW][4];
+    __shared__ int32_t base[2];
+    const int tid = threadIdx.x, lane = __lane_id(), wid = tid / 64;
+    const int32_t b = blockIdx.x, v0 = b << BV_LOG;
+    const int nv = min(BV, V - v0);
+    const int32_t cbeg = h2s[(int64_t)b * nslice], n = h2s[(int64_t)(b + 1) * nslice] - cbeg;
+    const Slab sl{slab, slab + SLAB, (uint8_t *)(slab + 2 * SLAB)};
+    cur[tid] = 0;
+    if (tid < 64) hist[tid] = 0;
+    __syncthreads();
+
+    // records in register chunks of SK_PRE per thread, all loads in flight;
+    // a bucket of one chunk is read once
+    uint32_t w[SK_PRE][3];
+    auto load = [&](int32_t c0) {
+#pragma unroll
+        for (int k = 0; k < SK_PRE; k++) {
+            const int32_t i = c0 + k * NT + tid;
+            w[k][0] = i < n ? rec.w0[cbeg + i] : 0u;
+            w[k][1] = i < n ? rec.w1[cbeg + i] : 0u;
+            w[k][2] = i < n ? rec.w2[cbeg + i] : 0u;
+        }
+    };
+    const bool one_chunk = n <= SK_PRE * NT;
+    for (int32_t c0 = 0; c0 < n; c0 += SK_PRE * NT) {
+        load(c0);
+#pragma unroll
+        for (int k = 0; k < SK_PRE; k++)
+            if (c0 + k * NT + tid < n) atomicAdd(&cur[w[k][0] & (uint32_t)(BV - 1)], 1);
+    }
+    __syncthreads();
+
+    // lanes by falling record count where that saves a wave a longer network:
+    // counting sort over the counts (heavy vertices last, with none)
+    const int32_t vcnt = cur[tid];
+    int mv = tid;  // my vertex
+    {
+        const int32_t c0 = vcnt <= SK_MAXREC ? vcnt : 0;
+        const int rank = atomicAdd(&hist[SK_MAXREC - c0], 1);
+        __syncthreads();
+        // block-uniform: the same words read by every thread
+        const int h = hist[lane];
+        const int most = SK_MAXREC - (__ffsll((unsigned long long)__ballot(h > 0)) - 1);
+        const int inc = tgd::wave_inclusive_sum(h);
+        const int few = __shfl(inc, SK_MAXREC, 64) - __shfl(inc, SK_MAXREC - 16, 64);  // count < 16
+        if (most > 24 || few >= 64) {
+            vert[__shfl(inc - h, SK_MAXREC - c0, 64) + rank] = (uint16_t)tid;
+            __syncthreads();
+            mv = vert[tid];
+        }
+    }
+    const int32_t cnt = cur[mv];
+    // vertices in rounds: those whose first record falls in the k-th span of
+    // SPAN; one vertex's run may reach past the span's end
+    const int32_t c = cnt <= SK_MAXREC ? cnt : 0;
+    const int32_t ci = tgd::wave_inclusive_sum(c);
+    if (lane == 63) wsum[wid][0] = ci;
+    __syncthreads();
+    int32_t cb = 0, ct = 0;
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+        if (i == wid) cb = ct;
+        ct += wsum[i][0];
+    }
+    const int32_t rounds = max(1, (ct + SPAN - 1) / SPAN);
+    const int32_t at = cb + ci - c;
+    const int32_t round = min(at / SPAN, rounds - 1);
+    // first record slot; one slot of skew per lane spreads equal-length runs over the banks
+    const int32_t pos = at - round * SPAN + tid;
+
+    uint32_t *row = slab + wid * SK_ROWS * 64 + lane, *adj = row + COLS;
+    uint32_t *stage = slab + COLS;  // the adjacency columns, once they are done with
+    int32_t out = 0;  // words of the bucket's scratch range used by earlier rounds
+    for (int32_t rd = 0; rd < rounds; rd++) {
+        const bool mine = mv < nv && round == rd;
+        const int32_t cr = mine ? c : 0;
+        cur[mv] = cr > 0 ? pos : ELSEWHERE;
+        __syncthreads();
+        for (int32_t c0 = 0; c0 < n; c0 += SK_PRE * NT) {
+            if (!one_chunk || rd > 0) load(c0);
+#pragma unroll
+            for (int k = 0; k < SK_PRE; k++)
+                if (c0 + k * NT + tid < n) {
+                    uint32_t rv, x, y, z;
+                    rec_unpack(w[k][0], w[k][1], w[k][2], rv, x, y, z);
+                    const int32_t p = atomicAdd(&cur[rv & (uint32_t)(BV - 1)], 1);
+                    if (p >= 0) {
+                        sl.w0[p] = x | (z << 24);
+                        sl.w1[p] = y | ((z >> 8) << 24);
+                        sl.b2[p] = (uint8_t)(z >> 16);
+                    }
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < SK_PRE; k++)  // loaded again if needed: frees the registers
+            w[k][0] = w[k][1] = w[k][2] = 0u;
+        __syncthreads();
+        const int at_ = mine ? pos : 0;
+        int d;
+        if (__any(cr > 40)) d = sort_rows<SK_MAXREC, CP>(sl, at_, cr, row, adj);
+        else if (__any(cr > 32)) d = sort_rows<40, CP>(sl, at_, cr, row, adj);
+        else if (__any(cr > 24)) d = sort_rows<32, CP>(sl, at_, cr, row, adj);
+        else if (__any(cr > 8)) d = sort_rows<24, CP>(sl, at_, cr, row, adj);
+        else d = sort_rows<8, CP>(sl, at_, cr, row, adj);
+        const bool hv = mine && (cnt > SK_MAXREC || d > SLOTS);
+        const bool ok = mine && !hv;
+        uint32_t nl = 0, nu = 0;
+        if (CP && ok) {
+            const int32_t v = v0 + mv;
+            const S sv = scal[v];
+            uint32_t lm = 0;
+            constexpr int G = 16;  // scalar gathers in flight
+            for (int s0 = 0; s0 < d; s0 += G) {
+                int32_t u[G];
+                S su[G];
+#pragma unroll
+                for (int i = 0; i < G; i++) u[i] = s0 + i < d ? (int32_t)row[(s0 + i) * 64] : v;
+#pragma unroll
+                for (int i = 0; i < G; i++) su[i] = s0 + i < d ? scal[u[i]] : sv;
+#pragma unroll
+                for (int i = 0; i < G; i++)
+                    lm |= (uint32_t)is_lower(su[i], sv, u[i], v) << ((s0 + i) & 31);
+            }
+            const uint32_t om = d >= 32 ? ~0u : (1u << d) - 1u;
+            lm &= om;
+            nl = label_columns(adj, row, lm, 32u);
+            nu = label_columns(adj, row, om & ~lm, 0u);
+        }
+        // results by vertex: row length, components, heavy, of this round
+        cur[mv] = (int32_t)((uint32_t)(ok ? d : 0) | nl << 8 | nu << 16 | (uint32_t)hv << 24 |
+                            (uint32_t)mine << 25);
+        __syncthreads();
+        // thread tid takes vertex tid: offsets of the rows and of the heavy
+        // vertices' room (3 words per record), places in the lists, results
+        const uint32_t res = (uint32_t)cur[tid];
+        const bool vh = (res >> 24) & 1u, vm = (res >> 25) & 1u;
+        const uint32_t vl = (res >> 8) & 255u, vu = (res >> 16) & 255u;
+        const int32_t x = (int32_t)(res & 255u), y = vh ? 3 * vcnt : 0;
+        const bool fx = vl >= 2 || vu >= 2;
+        const int32_t xi = tgd::wave_inclusive_sum(x), yi = tgd::wave_inclusive_sum(y);
+        const uint64_t hm = __ballot(vh), fm = __ballot(fx);
+        if (lane == 63) {
+            wsum[wid][0] = xi;
+            wsum[wid][1] = yi;
+            wsum[wid][2] = (int32_t)__popcll(hm);
+            wsum[wid][3] = (int32_t)__popcll(fm);
+        }
+        __syncthreads();
+        int32_t xb = 0, yb = 0, hb = 0, fb = 0, xt = 0, yt = 0, ht = 0, ft = 0;
+#pragma unroll
+        for (int i = 0; i < NW; i++) {
+            if (i == wid) xb = xt, yb = yt, hb = ht, fb = ft;
+            xt += wsum[i][0];
+            yt += wsum[i][1];
+            ht += wsum[i][2];
+            ft += wsum[i][3];
+        }
+        // one list atomic per block and round: same-address atomics of every
+        // wave (10 ns each) would take longer than the kernel
+        if (tid == 0) {
+            base[0] = ht ? atomicAdd(counters + C_HEAVY, ht) : 0;
+            base[1] = ft ? atomicAdd(counters + tg::C_FIXD, ft) : 0;
+        }
+        const int32_t v = v0 + tid;
+        if (vm) {
+            rowsrc[v] = 3 * cbeg + out + (vh ? xt + yb + yi - y : xb + xi - x);
+            if (!vh) {
+                deg[v] = x;
+                if (CP) {
+                    classes[3 * (int64_t)v] = vl;
+                    classes[3 * (int64_t)v + 1] = vu;
+                    classes[3 * (int64_t)v + 2] = verdict(vl, vu);
+                }
+            }
+        }
+        cur[tid] = xb + xi - x;
+        __syncthreads();
+        const uint64_t below = (1ull << lane) - 1ull;
+        if (vh) heavy[base[0] + hb + (int32_t)__popcll(hm & below)] = v;
+        if (fx) fixd[base[1] + fb + (int32_t)__popcll(fm & below)] = v;
+        if (ok) {
+            uint32_t *to = stage + cur[mv];
+            for (int s = 0; s < d; s++) to[s] = row[s * 64];
+        }
+        __syncthreads();
+        int32_t *dst = scratch + 3 * (int64_t)cbeg + out;
+        uint8_t *ddst = rowdesc + 3 * (int64_t)cbeg + out;
+        for (int i = tid; i < xt; i += NT) {
+            const uint32_t pk = stage[i];
+            dst[i] = (int32_t)(CP ? pk >> 6 : pk);
+            if (CP) ddst[i] = (uint8_t)(pk & 63u);
+        }
+        out += xt + yt;
+        if (rd + 1 < rounds) __syncthreads();  // the slab and the cursors are reused
     }
 }
 
@@ -1567,22 +1816,32 @@ int launch_bucketed_typed(tg::BucketBuffers &k, bool classify, hipStream_t s) {
     int32_t nsl = 1;
     int rc = route_records<false>(k, s, ranges, nsl);
     if (rc) return rc;
-#define TG_BKT(KERNEL)                                                                       \
-    hipLaunchKernelGGL(KERNEL, dim3(p.nb), dim3(p.bv_log == 7 ? 256 : 512), 0, s, r2, ranges, nsl, \
+#define TG_BKT(KERNEL, THREADS)                                                              \
+    hipLaunchKernelGGL(KERNEL, dim3(p.nb), dim3(THREADS), 0, s, r2, ranges, nsl,                \
                        scal, V, cls, b.scratch, b.deg, k.rowsrc, b.classes, b.heavy, b.fixd,   \
                        b.rowdesc, b.counters)
     if (p.owner) {
-        if (p.bv_log == 7) TG_BKT((k_bkt_own<7, S>));
-        else TG_BKT((k_bkt_own<8, S>));
-    } else if (p.ins == 1) {
-        if (p.bv_log == 7) TG_BKT((k_bkt_vv_cp<7, S, 1>));
-        else TG_BKT((k_bkt_vv_cp<8, S, 1>));
+        if (p.bv_log == 7) TG_BKT((k_bkt_own<7, S>), 256);
+        else TG_BKT((k_bkt_own<8, S>), 512);
+    } else if (p.ins == 1 || V > (int32_t)M24) {  // the sorting form keeps key 2^24 - 1 for padding
+        if (p.bv_log == 7) TG_BKT((k_bkt_vv_cp<7, S>), 256);
+        else TG_BKT((k_bkt_vv_cp<8, S>), 512);
     } else {
-        if (p.bv_log == 7) TG_BKT((k_bkt_vv_cp<7, S, 0>));
-        else TG_BKT((k_bkt_vv_cp<8, S, 0>));
+#define TG_SORT(BVL, SC, CLS)                                                                   \
+    hipLaunchKernelGGL((k_bkt_sort<BVL, SC, CLS>), dim3(p.nb), dim3(1 << BVL), 0, s, r2, ranges,  \
+                       nsl, (const SC *)scal, V, b.scratch, b.deg, k.rowsrc, b.classes, b.heavy,  \
+                       b.fixd, b.rowdesc, b.counters)
+        if (p.bv_log == 7) {
+            if (classify) TG_SORT(7, S, true);
+            else TG_SORT(7, float, false);
+        } else {
+            if (classify) TG_SORT(8, S, true);
+            else TG_SORT(8, float, false);
+        }
+#undef TG_SORT
     }
 #undef TG_BKT
-    TG_LAUNCH_CHECK("k_bkt_vv_cp");
+    TG_LAUNCH_CHECK("bucket kernel");
     if (mk) mk->mark("bkt_vv_cp", s);
     if (p.bv_log == 7)
         hipLaunchKernelGGL((k_bkt_heavy<7, S>), dim3(256), dim3(HV_THREADS), 0, s, r2, ranges, nsl,
