@@ -775,150 +775,239 @@ __global__ void k_ef_copy(const int64_t *__restrict__ et_off, int64_t E,
 constexpr int ROW_THREADS = 64;
 constexpr int ROW_CAP = 100;  // 26 KB per 64 threads (with three spare slots): six waves per CU
 
-// Cells in the order of their corner-0 entries in VT (rows by vertex, cells
-// ascending within a row), for k_tt on meshes with rows beyond its LDS
-// column: neighbouring lanes then take cells around one vertex and share
-// its VT row, where the mesh's own cell order may scatter them (on a mesh
-// of uniform short rows the pass costs more than the sharing saves).  One pass counts the corner-0 codes per chunk, a scan of
-// the chunk counts gives each chunk's start, a second pass fills the order
-// stably (block-wide ballot scans, one per round of 256 codes).
-constexpr int C0_THREADS = 256, C0_PER = 16, C0_CHUNK = C0_THREADS * C0_PER;
+// ---- TT: union of the VT rows of a cell's corners, minus the cell -----------------
+// One lane per cell, one kernel: the four rows are loaded whole (16-byte
+// quads, independent) into registers, merged by a compile-time bitonic
+// network, and the distinct cells other than the lane's own counted; the
+// block's total joins a chained scan over tiles of TT_THREADS cells, which
+// gives every row its exact place; then the rows go through an LDS window per
+// wave to contiguous 16-byte stores.  A wave takes the smallest network that
+// holds its rows; a lane with a row beyond the largest one merges serially
+// from global memory.
+//
+// What bounds it: VALU issue of the network (560 compare-exchanges for rows of
+// up to 24) and the loads of 4 x 64 different rows per wave.  It replaced a
+// merge of LDS columns by one lane each (100 words a lane, six waves per CU,
+// waiting on dependent LDS reads; longer rows from global memory), which wrote
+// padded rows, scanned their lengths and packed them.
+constexpr int TT_THREADS = 256;
+constexpr int TT_WIN = 2240;  // words of a wave's output window: two windows for 64 x 69 words
+constexpr int TT_ROW = 48;    // longest row of the largest network
 
-__global__ __launch_bounds__(C0_THREADS) void k_c0_count(const int32_t *__restrict__ vtc,
-                                                         int64_t n, int64_t *__restrict__ bcnt) {
-    __shared__ int32_t total;
-    if (threadIdx.x == 0) total = 0;
-    __syncthreads();
-    const int64_t b0 = (int64_t)blockIdx.x * C0_CHUNK;
-    int32_t c = 0;
-    for (int i = 0; i < C0_PER; i++) {
-        const int64_t k = b0 + (int64_t)i * C0_THREADS + threadIdx.x;
-        c += k < n && (vtc[k] & 3) == 0;
+// Tiles' totals as they become known: bits 62-63 hold 0 (nothing yet), 1 (the
+// tile's own sum) or 2 (the sum of all tiles up to it).
+constexpr uint64_t TILE_SUM = 1ull << 62, TILE_PREFIX = 2ull << 62, TILE_VALUE = TILE_SUM - 1;
+
+// Sum of the tiles before `tile`, by one whole wave.  Every tile with a lower
+// number was started earlier (numbers are handed out by a counter) and
+// publishes its sum without waiting for anything, so the wait ends.
+__device__ __forceinline__ int64_t tiles_before(const uint64_t *state, int32_t tile) {
+    const int lane = __lane_id();
+    int64_t sum = 0;
+    for (int32_t top = tile - 1;;) {
+        const int32_t i = top - lane;
+        const uint64_t s = i >= 0 ? tgd::load_agent(state + i) : TILE_PREFIX;
+        const uint64_t full = __ballot((s >> 62) == 2), none = __ballot((s >> 62) == 0);
+        const int stop = full ? __ffsll((unsigned long long)full) - 1 : 63;
+        if (none & ((2ull << stop) - 1ull)) {
+            tgd::pause();
+            continue;
+        }
+        sum += tgd::wave_sum(lane <= stop ? (int64_t)(s & TILE_VALUE) : (int64_t)0);
+        if (full) return sum;
+        top -= 64;
     }
-    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-    if ((threadIdx.x & 63) == 0) atomicAdd(&total, c);
-    __syncthreads();
-    if (threadIdx.x == 0) bcnt[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(C0_THREADS) void k_c0_fill(const int32_t *__restrict__ vtc, int64_t n,
-                                                        const int64_t *__restrict__ bbase,
-                                                        int32_t *__restrict__ order) {
-    __shared__ int32_t wsum[C0_THREADS / 64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t b0 = (int64_t)blockIdx.x * C0_CHUNK;
-    int64_t base = bbase[blockIdx.x];
-    for (int i = 0; i < C0_PER; i++) {
-        const int64_t k = b0 + (int64_t)i * C0_THREADS + threadIdx.x;
-        const int32_t code = k < n ? vtc[k] : 1;
-        const bool f = (code & 3) == 0;
-        const unsigned long long m = __ballot(f);
-        const int before = __popcll(m & ((1ull << lane) - 1));
-        if (lane == 0) wsum[w] = __popcll(m);
-        __syncthreads();
-        int32_t off = 0, tot = 0;
+// Bitonic merge of k[B .. B + n), any n: the first part sorted against the
+// direction, the second along it (H. W. Lang's form for arbitrary n: compare
+// at the largest power of two below n, then both parts).
+constexpr int pow2_below(int n) { return n <= 2 ? 1 : 2 * pow2_below((n + 1) / 2); }
+template <int B, int n, bool UP, int N>
+__device__ __forceinline__ void bitonic_merge(int32_t (&k)[N]) {
+    if constexpr (n > 1) {
+        constexpr int m = pow2_below(n);
 #pragma unroll
-        for (int j = 0; j < C0_THREADS / 64; j++) {
-            const int32_t x = wsum[j];
-            off += j < w ? x : 0;
-            tot += x;
+        for (int i = B; i < B + n - m; i++) {
+            const int32_t a = k[i], b = k[i + m];
+            k[i] = tgd::opaque(UP ? min(a, b) : max(a, b));
+            k[i + m] = tgd::opaque(UP ? max(a, b) : min(a, b));
         }
-        if (f) order[base + off + before] = code >> 2;
-        base += tot;
-        __syncthreads();  // wsum is rewritten next round
+        bitonic_merge<B, m, UP>(k);
+        bitonic_merge<B + m, n - m, UP>(k);
     }
 }
 
-// TT(t): union of VT rows of t's corners, minus t (4-way merge), written in
-// one pass to a padded slot at pad[t] of |VT rows| - 4 words rounded up to a
-// multiple of four, with its length in cnt[t]; the rows are packed after
-// the scan of cnt.
-__global__ void k_tt_bound(const int4 *__restrict__ tv4, int64_t T,
-                           const int32_t *__restrict__ vt_off, int64_t *__restrict__ ub,
-                           int32_t *__restrict__ long_rows) {
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < T;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const int4 q = tv4[t];
-        const i32x2u r0 = *reinterpret_cast<const i32x2u *>(vt_off + q.x);
-        const i32x2u r1 = *reinterpret_cast<const i32x2u *>(vt_off + q.y);
-        const i32x2u r2 = *reinterpret_cast<const i32x2u *>(vt_off + q.z);
-        const i32x2u r3 = *reinterpret_cast<const i32x2u *>(vt_off + q.w);
-        const int64_t n = (int64_t)(r0.y - r0.x) + (r1.y - r1.x) + (r2.y - r2.x) + (r3.y - r3.x) - 4;
-        ub[t] = (n + 3) & ~(int64_t)3;
-        if (n + 4 > ROW_CAP) *long_rows = 1;  // every writer stores the same value
+// Row of n <= R corner codes as cells, INF after them; DOWN: in reverse.
+// Whole quads are read, up to three words past the row (vtc carries them).
+template <int B, int R, bool DOWN, int N>
+__device__ __forceinline__ void load_row(int32_t (&k)[N], const int32_t *__restrict__ src, int n) {
+#pragma unroll
+    for (int i = 0; i < R; i += 4) {
+        i32x4u q = {0, 0, 0, 0};
+        if (i < n) q = *reinterpret_cast<const i32x4u *>(src + i);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            k[B + (DOWN ? R - 1 - i - j : i + j)] = i + j < n ? q[j] >> 2 : INF;
     }
 }
 
-__global__ __launch_bounds__(ROW_THREADS) void k_tt(const int4 *__restrict__ tv4, int64_t T,
-                                                    const int32_t *__restrict__ vt_off,
-                                                    const int32_t *__restrict__ vtc,
-                                                    const int32_t *__restrict__ order,
-                                                    const int64_t *__restrict__ pad,
-                                                    int64_t *__restrict__ cnt,
-                                                    int32_t *__restrict__ out) {
-    __shared__ int32_t buf[ROW_CAP + 3][ROW_THREADS];  // three spare slots for stage_quads
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < T;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t t = order ? order[i] : i;  // cells in VT order when given
-        const int4 q = tv4[t];
-        const i32x2u r0 = *reinterpret_cast<const i32x2u *>(vt_off + q.x);
-        const i32x2u r1 = *reinterpret_cast<const i32x2u *>(vt_off + q.y);
-        const i32x2u r2 = *reinterpret_cast<const i32x2u *>(vt_off + q.z);
-        const i32x2u r3 = *reinterpret_cast<const i32x2u *>(vt_off + q.w);
-        int32_t p0 = r0.x, e0 = r0.y, p1 = r1.x, e1 = r1.y;
-        int32_t p2 = r2.x, e2 = r2.y, p3 = r3.x, e3 = r3.y;
-        QuadOut o;
-        o.row = out + pad[t];
-        const int32_t n0 = e0 - p0, n1 = e1 - p1, n2 = e2 - p2, n3 = e3 - p3;
-        if (n0 + n1 + n2 + n3 <= ROW_CAP) {
-            // heads as LDS positions
-            int32_t a0 = 0, a1 = n0, a2 = n0 + n1, a3 = n0 + n1 + n2;
-            const int32_t z0 = n0, z1 = n0 + n1, z2 = n0 + n1 + n2, z3 = n0 + n1 + n2 + n3;
-            stage_quads(buf, 0, vtc + p0, n0, 2);
-            stage_quads(buf, z0, vtc + p1, n1, 2);
-            stage_quads(buf, z1, vtc + p2, n2, 2);
-            stage_quads(buf, z2, vtc + p3, n3, 2);
-            int32_t h0 = a0 < z0 ? buf[a0][threadIdx.x] : INF;
-            int32_t h1 = a1 < z1 ? buf[a1][threadIdx.x] : INF;
-            int32_t h2 = a2 < z2 ? buf[a2][threadIdx.x] : INF;
-            int32_t h3 = a3 < z3 ? buf[a3][threadIdx.x] : INF;
-            // branch-free advance: every head re-reads its (clamped) position,
-            // so the four LDS reads of an iteration issue together
-            const int32_t last = max(z3 - 1, 0);
-            while (true) {
-                const int32_t mn = min(min(h0, h1), min(h2, h3));
-                if (mn == INF) break;
-                a0 += h0 == mn;
-                a1 += h1 == mn;
-                a2 += h2 == mn;
-                a3 += h3 == mn;
-                const int32_t y0 = buf[min(a0, last)][threadIdx.x];
-                const int32_t y1 = buf[min(a1, last)][threadIdx.x];
-                const int32_t y2 = buf[min(a2, last)][threadIdx.x];
-                const int32_t y3 = buf[min(a3, last)][threadIdx.x];
-                h0 = a0 < z0 ? y0 : INF;
-                h1 = a1 < z1 ? y1 : INF;
-                h2 = a2 < z2 ? y2 : INF;
-                h3 = a3 < z3 ? y3 : INF;
-                if (mn == (int32_t)t) continue;
-                o.put(mn);
-            }
+struct TtRows {  // the lane's four VT rows
+    int32_t p[4], n[4];
+};
+
+// Serial four-way merge from global memory: f(i, x) for the i-th distinct
+// cell x other than t, ascending; returns their number.
+template <typename F>
+__device__ __forceinline__ int32_t tt_serial(const int32_t *vtc, const TtRows &r, int32_t t, F f) {
+    int32_t i[4] = {0, 0, 0, 0}, h[4], m = 0;
+#pragma unroll
+    for (int c = 0; c < 4; c++) h[c] = r.n[c] > 0 ? vtc[r.p[c]] >> 2 : INF;
+    while (true) {
+        const int32_t x = min(min(h[0], h[1]), min(h[2], h[3]));
+        if (x == INF) return m;
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (h[c] == x) h[c] = ++i[c] < r.n[c] ? vtc[r.p[c] + i[c]] >> 2 : INF;
+        if (x != t) f(m++, x);
+    }
+}
+
+// One wave's share of a tile with a network for rows of up to R entries.
+// Contains two workgroup barriers; every wave of the block makes one call
+// (of some R), so all waves meet at both.
+template <int R>
+__device__ __forceinline__ void tt_wave(const int32_t *__restrict__ vtc, const TtRows &r, bool act,
+                                        int32_t t, int32_t last, int32_t tile, uint64_t *state,
+                                        int64_t *__restrict__ off, int32_t *__restrict__ out,
+                                        int32_t *win, int32_t (&wtot)[TT_THREADS / 64],
+                                        int64_t &tbase) {
+    constexpr int N = 4 * R;
+    const int lane = __lane_id(), wid = threadIdx.x / 64;
+    int32_t k[N];
+    load_row<0, R, false>(k, vtc + r.p[0], r.n[0]);
+    load_row<R, R, true>(k, vtc + r.p[1], r.n[1]);
+    load_row<2 * R, R, true>(k, vtc + r.p[2], r.n[2]);
+    load_row<3 * R, R, false>(k, vtc + r.p[3], r.n[3]);
+    bitonic_merge<0, 2 * R, false>(k);
+    bitonic_merge<2 * R, 2 * R, true>(k);
+    bitonic_merge<0, N, true>(k);
+    const int nv = r.n[0] + r.n[1] + r.n[2] + r.n[3];
+    const bool serial = max(max(r.n[0], r.n[1]), max(r.n[2], r.n[3])) > TT_ROW;
+    int32_t m = 0;  // distinct values, less the cell itself and the padding
+#pragma unroll
+    for (int j = 1; j < N; j++) m += k[j] != k[j - 1];
+    m = act ? m - (nv < N) : 0;
+    if (serial) m = tt_serial(vtc, r, t, [](int32_t, int32_t) {});
+    const int32_t inc = tgd::wave_inclusive_sum(m);
+    if (lane == 63) wtot[wid] = inc;
+    __syncthreads();
+    int32_t before = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < TT_THREADS / 64; i++) {
+        if (i < wid) before += wtot[i];
+        total += wtot[i];
+    }
+    if (threadIdx.x == 0) tgd::store_agent(state + tile, TILE_SUM | (uint64_t)total);
+    const int32_t first = inc - m, wn = __shfl(inc, 63, 64);
+    // the wave's rows, one window after the other; the first one is filled
+    // while the tile's place is being found
+    for (int32_t w0 = 0;; w0 += TT_WIN) {
+        int32_t pos = first - w0 - 1;
+        if (serial) {
+            tt_serial(vtc, r, t, [&](int32_t i, int32_t x) {
+                if ((uint32_t)(first - w0 + i) < (uint32_t)TT_WIN) win[first - w0 + i] = x;
+            });
         } else {
-            int32_t h0 = p0 < e0 ? vtc[p0] >> 2 : INF, h1 = p1 < e1 ? vtc[p1] >> 2 : INF;
-            int32_t h2 = p2 < e2 ? vtc[p2] >> 2 : INF, h3 = p3 < e3 ? vtc[p3] >> 2 : INF;
-            while (true) {
-                const int32_t mn = min(min(h0, h1), min(h2, h3));
-                if (mn == INF) break;
-                if (h0 == mn) h0 = ++p0 < e0 ? vtc[p0] >> 2 : INF;
-                if (h1 == mn) h1 = ++p1 < e1 ? vtc[p1] >> 2 : INF;
-                if (h2 == mn) h2 = ++p2 < e2 ? vtc[p2] >> 2 : INF;
-                if (h3 == mn) h3 = ++p3 < e3 ? vtc[p3] >> 2 : INF;
-                if (mn == (int32_t)t) continue;
-                o.put(mn);
+            // compared afresh in every window: masks kept from the count
+            // above, one per key, would not fit the scalar registers
+            const int32_t mv = tgd::opaque(nv);
+            int32_t prev = -1;
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                k[j] = tgd::opaque(k[j]);
+                const bool keep = k[j] != prev && k[j] != t && j < mv;
+                prev = k[j];
+                pos += keep;
+                if (keep && (uint32_t)pos < (uint32_t)TT_WIN) win[pos] = k[j];
             }
         }
-        o.flush();
-        cnt[t] = o.n;
+        if (w0 == 0) {
+            if (wid == 0) {
+                const int64_t b = tiles_before(state, tile);
+                if (lane == 0) {
+                    tgd::store_agent(state + tile, TILE_PREFIX | (uint64_t)(b + total));
+                    tbase = b;
+                }
+            }
+            __syncthreads();
+            if (act) off[t] = tbase + before + first;
+            if (t == last) off[t + 1] = tbase + total;
+        }
+        tgd::wave_sync();  // the window is whole
+        int32_t *dst = out + (tbase + before + w0);
+        const int32_t cnt = min(wn - w0, TT_WIN);
+        for (int32_t i = 4 * lane; i + 3 < cnt; i += 256)
+            *reinterpret_cast<i32x4u *>(dst + i) = *reinterpret_cast<const i32x4u *>(win + i);
+        const int32_t tail = cnt & ~3;
+        if (cnt > 0 && tail + lane < cnt) dst[tail + lane] = win[tail + lane];
+        if (w0 + TT_WIN >= wn) return;
+        tgd::wave_sync();  // and has been read
+    }
+}
+
+__global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const int4 *__restrict__ tv4, int64_t T,
+                                                   const int32_t *__restrict__ vt_off,
+                                                   const int32_t *__restrict__ vtc,
+                                                   int32_t *ticket, uint64_t *state,
+                                                   int64_t *__restrict__ off,
+                                                   int32_t *__restrict__ out) {
+    __shared__ __align__(16) int32_t win[TT_THREADS / 64][TT_WIN];
+    __shared__ int32_t wtot[TT_THREADS / 64];
+    __shared__ int64_t tbase;
+    __shared__ int32_t next;
+    if (threadIdx.x == 0) next = atomicAdd(ticket, 1);
+    __syncthreads();
+    const int32_t tile = next;
+    const int64_t t = (int64_t)tile * TT_THREADS + threadIdx.x;
+    const bool act = t < T;
+    const int32_t last = (int32_t)(T - 1);
+    TtRows r;
+    const int4 q = act ? tv4[t] : make_int4(0, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const i32x2u o = *reinterpret_cast<const i32x2u *>(vt_off + corner(q, c));
+        r.p[c] = o.x;
+        r.n[c] = act ? o.y - o.x : 0;
+    }
+    int32_t *w = win[threadIdx.x / 64];
+    const int longest = max(max(r.n[0], r.n[1]), max(r.n[2], r.n[3]));
+    const int need = longest > TT_ROW ? 0 : longest;  // serial lanes need no network
+    if (__any(need > 40)) tt_wave<TT_ROW>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
+    else if (__any(need > 32)) tt_wave<40>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
+    else if (__any(need > 24)) tt_wave<32>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
+    else tt_wave<24>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
+}
+
+// Sum of squared row lengths (VT: the lengths of all cells' four rows
+// together); one atomic per block of few.
+constexpr int SQ_THREADS = 1024, SQ_BLOCKS = 64;
+__global__ __launch_bounds__(SQ_THREADS) void k_row_squares(const int32_t *__restrict__ row_off,
+                                                            int64_t rows,
+                                                            unsigned long long *__restrict__ sum) {
+    __shared__ int64_t ws[SQ_THREADS / 64];
+    int64_t s = 0;
+    for (int64_t v = (int64_t)blockIdx.x * SQ_THREADS + threadIdx.x; v < rows;
+         v += (int64_t)gridDim.x * SQ_THREADS) {
+        const int64_t n = row_off[v + 1] - row_off[v];
+        s += n * n;
+    }
+    s = tgd::wave_sum(s);
+    if (__lane_id() == 0) ws[threadIdx.x / 64] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < SQ_THREADS / 64; w++) s += ws[w];
+        if (s) atomicAdd(sum, (unsigned long long)s);
     }
 }
 
@@ -947,45 +1036,6 @@ __global__ __launch_bounds__(256) void k_pack_rows(const int64_t *__restrict__ p
             else hi = mid - 1;
         }
         dst[o] = src[s_pad[lo] + (o - s_off[lo])];
-    }
-}
-
-// Pack of long padded rows with a lane per output word: one wave per 64
-// consecutive rows copies their contiguous output range 64 words at a time
-// (full, aligned stores; reads nearly contiguous, the slots being
-// consecutive), each word finding its row by a six-step search of the
-// rows' output starts held in LDS.  Four chunks per lane are in flight.
-__global__ __launch_bounds__(256) void k_pack_rows_wave(const int64_t *__restrict__ pad,
-                                                        const int64_t *__restrict__ off,
-                                                        int64_t rows,
-                                                        const int32_t *__restrict__ src,
-                                                        int32_t *__restrict__ dst) {
-    __shared__ int32_t s_start[4][65];  // output start of each row, relative to the wave's
-    __shared__ int64_t s_pad[4][64];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t r0 = ((int64_t)blockIdx.x * 4 + w) * 64;
-    const int nr = r0 < rows ? (int)min<int64_t>(64, rows - r0) : 0;
-    const int64_t o0 = nr > 0 ? off[r0] : 0;
-    // rows past the end start at INT32_MAX and are never chosen
-    s_start[w][lane] = lane < nr ? (int32_t)(off[r0 + lane] - o0) : INT32_MAX;
-    if (lane == 0) s_start[w][64] = nr > 0 ? (int32_t)(off[r0 + nr] - o0) : 0;
-    s_pad[w][lane] = lane < nr ? pad[r0 + lane] : 0;
-    __syncthreads();
-    const int32_t total = s_start[w][64];
-    for (int32_t k0 = 0; k0 < total; k0 += 4 * 64) {
-        int32_t v[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int32_t k = min(k0 + 64 * u + lane, total - 1);
-            int lo = 0;
-#pragma unroll
-            for (int step = 32; step >= 1; step >>= 1)
-                if (s_start[w][lo + step] <= k) lo += step;
-            v[u] = src[s_pad[w][lo] + (k - s_start[w][lo])];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-            if (k0 + 64 * u + lane < total) dst[o0 + k0 + 64 * u + lane] = v[u];
     }
 }
 
@@ -1382,58 +1432,35 @@ int ensure_tt(tg_mesh &m) {
     if (m.tt_built) return OK;
     int rc;
     if ((rc = ensure_vt_sorted(m))) return rc;
-    const int64_t T = m.n_cells;
+    const int64_t T = m.n_cells, V = m.n_points;
+    const int64_t tiles = (T + TT_THREADS - 1) / TT_THREADS;
+    // tmp_b: sum of the rows' lengths, tile counter, tile sums
     if ((rc = m.tt_off.ensure(sizeof(int64_t) * (size_t)(T + 1))) ||
-        (rc = m.tmp_b.ensure(sizeof(int64_t) * (size_t)(T + 2))))
+        (rc = m.tmp_b.ensure(sizeof(int64_t) * (size_t)(tiles + 2))))
         return rc;
-    int64_t *off = m.tt_off.as<int64_t>(), *pad = m.tmp_b.as<int64_t>();
-    // pad[T + 1]: set when a cell's rows exceed the LDS column (they merge
-    // from global memory, where lanes that share rows gain most)
-    int32_t *long_rows = reinterpret_cast<int32_t *>(pad + T + 1);
-    if (T > 0) {
-        hipLaunchKernelGGL(k_fill_i32v, dim3(1), dim3(64), 0, m.stream, long_rows, 0, (int64_t)2);
-        hipLaunchKernelGGL(k_tt_bound, dim3(grid(T)), dim3(256), 0, m.stream,
-                           m.tv.as<const int4>(), T, m.vt_off.as<int32_t>(), pad, long_rows);
-        TG_LAUNCH_CHECK("k_tt_bound");
+    int64_t *off = m.tt_off.as<int64_t>(), *words = m.tmp_b.as<int64_t>();
+    int32_t *ticket = reinterpret_cast<int32_t *>(words + 1);
+    uint64_t *state = reinterpret_cast<uint64_t *>(words + 2);
+    if (T == 0) {
+        if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) return rc;
+    } else {
+        if ((rc = fill_i32((int32_t *)words, 0, 2 * (tiles + 2), m.stream))) return rc;
+        hipLaunchKernelGGL(k_row_squares, dim3(std::min(grid(V, SQ_THREADS), (unsigned)SQ_BLOCKS)),
+                           dim3(SQ_THREADS), 0, m.stream, m.vt_off.as<int32_t>(), V,
+                           (unsigned long long *)words);
+        TG_LAUNCH_CHECK("k_row_squares");
     }
-    int64_t padded = 0, has_long = 0;
-    if ((rc = scan_counts64(m, pad, T, padded))) return rc;
-    if (T > 0 && (rc = read_i64(m, pad, T + 1, has_long))) return rc;
-    // tmp_c: the padded rows, then the cell order and its chunk counts
-    const int64_t nchunk = (4 * T + C0_CHUNK - 1) / C0_CHUNK;
-    const int64_t at_order = (padded + 1) & ~(int64_t)1;  // 8-byte aligned chunk counts
-    const int64_t at_cnt = at_order + ((T + 1) & ~(int64_t)1);
-    if ((rc = m.tmp_c.ensure(sizeof(int32_t) * (size_t)(at_cnt + 2 * (nchunk + 1))))) return rc;
-    const int32_t *order = nullptr;
-    if (T > 0 && has_long) {
-        int32_t *ord = m.tmp_c.as<int32_t>() + at_order;
-        int64_t *bcnt = reinterpret_cast<int64_t *>(m.tmp_c.as<int32_t>() + at_cnt);
-        hipLaunchKernelGGL(k_c0_count, dim3((unsigned)nchunk), dim3(C0_THREADS), 0, m.stream,
-                           m.vtc.as<int32_t>(), 4 * T, bcnt);
-        TG_LAUNCH_CHECK("k_c0_count");
-        int64_t found = 0;
-        if ((rc = scan_counts64(m, bcnt, nchunk, found))) return rc;
-        if (found == T) {  // one corner-0 code per cell
-            hipLaunchKernelGGL(k_c0_fill, dim3((unsigned)nchunk), dim3(C0_THREADS), 0, m.stream,
-                               m.vtc.as<int32_t>(), 4 * T, bcnt, ord);
-            TG_LAUNCH_CHECK("k_c0_fill");
-            order = ord;
-        }
-    }
+    int64_t rows = 0, nnz = 0;
+    if (T > 0 && (rc = read_i64(m, words, 0, rows))) return rc;
+    // a cell's four rows hold the cell itself four times
+    if ((rc = m.tt_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(rows - 4 * T, 1))))
+        return rc;
     if (T > 0) {
-        hipLaunchKernelGGL(k_tt, dim3(grid(T, ROW_THREADS)), dim3(ROW_THREADS), 0, m.stream,
+        hipLaunchKernelGGL(k_tt, dim3((unsigned)tiles), dim3(TT_THREADS), 0, m.stream,
                            m.tv.as<const int4>(), T, m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(),
-                           order, pad, off, m.tmp_c.as<int32_t>());
+                           ticket, state, off, m.tt_vals.as<int32_t>());
         TG_LAUNCH_CHECK("k_tt");
-    }
-    int64_t nnz = 0;
-    if ((rc = scan_counts64(m, off, T, nnz))) return rc;
-    if ((rc = m.tt_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)))) return rc;
-    if (T > 0) {
-        hipLaunchKernelGGL(k_pack_rows_wave, dim3((unsigned)((T + 255) / 256)), dim3(256), 0,
-                           m.stream, pad, off, T, m.tmp_c.as<int32_t>(),
-                           m.tt_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_pack_rows_wave");
+        if ((rc = read_i64(m, off, T, nnz))) return rc;
     }
     m.tt_nnz = nnz;
     m.tt_built = true;
