@@ -1,5 +1,9 @@
-// Device-wide exclusive scan (reduce -> scan partials -> downsweep) and fill
-// kernels.  Tiles of 4096 items per 256-thread workgroup; every tile is read
+// Device-wide exclusive scan and fill kernels.  Up to 16384 items: one
+// workgroup, one launch.  Up to SCAN_SUMMED tiles of 4096 items: two launches,
+// per-tile sums, then the downsweep, in which every workgroup adds up the sums
+// before its tile itself (at most 8 a thread; launches are what a scan of this
+// size costs: Kuhn 24^3's three scans took 20 us in nine launches).  More
+// tiles: the sums are scanned by a launch in between.  Every tile is read
 // twice and written once.
 #include "common.h"
 
@@ -8,6 +12,11 @@ namespace {
 constexpr int SCAN_BLOCK = 256;
 constexpr int SCAN_ITEMS = 16;
 constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
+constexpr int SCAN_ONE = 1024;       // threads of the single-workgroup scan
+constexpr int64_t SCAN_SUMMED = 2048;  // tiles whose sums each workgroup adds up itself
+// What k_scan_down finds in partials: nothing (one workgroup), the tiles'
+// sums, or their exclusive scan.
+enum Partials { ALONE, SUMS, PREFIXES };
 
 template <typename TIn, typename TAcc>
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(
@@ -61,18 +70,25 @@ __global__ __launch_bounds__(1024) void k_scan_partials(
 
 __device__ __forceinline__ int pad(int i) { return i + (i >> 5); }
 
-template <typename TIn, typename TOut, typename TAcc>
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(
+template <typename TIn, typename TOut, typename TAcc, int BLOCK, Partials HAVE>
+__global__ __launch_bounds__(BLOCK) void k_scan_down(
     const TIn *in, TOut *out, int64_t n, const TAcc *__restrict__ partials) {
-    __shared__ TAcc lds[SCAN_TILE + SCAN_TILE / 32];
-    __shared__ TAcc wsum[SCAN_BLOCK / 64];
-    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
+    constexpr int TILE = BLOCK * SCAN_ITEMS;
+    __shared__ TAcc lds[TILE + TILE / 32];
+    __shared__ TAcc wsum[BLOCK / 64], wbase[BLOCK / 64];
+    const int64_t base = (int64_t)blockIdx.x * TILE;
     const int t = threadIdx.x, lane = __lane_id(), wid = t / 64;
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
-        const int i = k * SCAN_BLOCK + t;
+        const int i = k * BLOCK + t;
         const int64_t g = base + i;
         lds[pad(i)] = g < n ? (TAcc)in[g] : (TAcc)0;
+    }
+    if (HAVE == SUMS) {
+        TAcc before = 0;
+        for (int64_t i = t; i < (int64_t)blockIdx.x; i += BLOCK) before += partials[i];
+        before = tgd::wave_sum(before);
+        if (lane == 0) wbase[wid] = before;
     }
     __syncthreads();
     TAcc v[SCAN_ITEMS];
@@ -85,17 +101,23 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_down(
     const TAcc inc = tgd::wave_inclusive_sum(s);
     if (lane == 63) wsum[wid] = inc;
     __syncthreads();
-    TAcc run = partials[blockIdx.x] + inc - s;
-    for (int w = 0; w < wid; w++) run += wsum[w];
+    TAcc run = inc - s;
+    if (HAVE == PREFIXES) run += partials[blockIdx.x];
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; w++) {
+        if (HAVE == SUMS) run += wbase[w];
+        if (w < wid) run += wsum[w];
+    }
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
         lds[pad(t * SCAN_ITEMS + k)] = run;
         run += v[k];
     }
+    if (HAVE != PREFIXES && blockIdx.x == gridDim.x - 1 && t == BLOCK - 1) out[n] = (TOut)run;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
-        const int i = k * SCAN_BLOCK + t;
+        const int i = k * BLOCK + t;
         const int64_t g = base + i;
         if (g < n) out[g] = (TOut)lds[pad(i)];
     }
@@ -118,14 +140,25 @@ int scan_impl(const TIn *in, TOut *out, int64_t n, void *tmp, hipStream_t s) {
     }
     const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
     TAcc *partials = (TAcc *)tmp;
+    if (n <= SCAN_ONE * SCAN_ITEMS) {
+        hipLaunchKernelGGL((k_scan_down<TIn, TOut, TAcc, SCAN_ONE, ALONE>), dim3(1),
+                           dim3(SCAN_ONE), 0, s, in, out, n, partials);
+        TG_LAUNCH_CHECK("k_scan_down");
+        return tg::OK;
+    }
     hipLaunchKernelGGL((k_scan_reduce<TIn, TAcc>), dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s,
                        in, n, partials);
     TG_LAUNCH_CHECK("k_scan_reduce");
-    hipLaunchKernelGGL((k_scan_partials<TAcc, TOut>), dim3(1), dim3(1024), 0, s, partials, nb,
-                       out + n);
-    TG_LAUNCH_CHECK("k_scan_partials");
-    hipLaunchKernelGGL((k_scan_down<TIn, TOut, TAcc>), dim3((unsigned)nb), dim3(SCAN_BLOCK), 0,
-                       s, in, out, n, partials);
+    if (nb <= SCAN_SUMMED) {
+        hipLaunchKernelGGL((k_scan_down<TIn, TOut, TAcc, SCAN_BLOCK, SUMS>), dim3((unsigned)nb),
+                           dim3(SCAN_BLOCK), 0, s, in, out, n, partials);
+    } else {
+        hipLaunchKernelGGL((k_scan_partials<TAcc, TOut>), dim3(1), dim3(1024), 0, s, partials, nb,
+                           out + n);
+        TG_LAUNCH_CHECK("k_scan_partials");
+        hipLaunchKernelGGL((k_scan_down<TIn, TOut, TAcc, SCAN_BLOCK, PREFIXES>),
+                           dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, out, n, partials);
+    }
     TG_LAUNCH_CHECK("k_scan_down");
     return tg::OK;
 }
