@@ -76,6 +76,8 @@ void pinned_slot_free(void *p);
 // captured into graphs).
 int fill_i32(int32_t *p, int32_t value, int64_t n, hipStream_t s);
 int fill_u8(uint8_t *p, uint8_t value, int64_t n, hipStream_t s);
+// Zeros in up to three arrays with one launch (NULL or 0: none).
+int zero_i32(int32_t *a, int64_t na, int32_t *b, int64_t nb, int32_t *c, int64_t nc, hipStream_t s);
 
 }  // namespace tg
 

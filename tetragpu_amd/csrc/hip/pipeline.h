@@ -89,7 +89,7 @@ int launch_vv_cp(VvCpBuffers &b, const VvCpConfig &cfg, bool classify,
                  hipStream_t s);
 // Gather rows from padded scratch (row of v starts at rowsrc[v]) into the CSR.
 int launch_rows_compact(const int32_t *rowsrc, const int32_t *vv_off, const int32_t *scratch,
-                        int32_t V, int32_t *cols, hipStream_t s);
+                        int32_t V, int bv_log, int32_t *cols, hipStream_t s);
 // Row-membership link components for the vertices queued in fix/fixbig.
 int launch_cp_fix(VvCpBuffers &b, hipStream_t s);
 // Whole pipeline: counters reset, VT corners, VV, critical points.

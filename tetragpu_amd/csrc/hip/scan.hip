@@ -130,6 +130,15 @@ __global__ void k_fill(T *__restrict__ p, T value, int64_t n) {
         p[i] = value;
 }
 
+__global__ void k_zero3(int32_t *a, int64_t na, int32_t *b, int64_t nb, int32_t *c, int64_t nc) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < na + nb + nc;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        if (i < na) a[i] = 0;
+        else if (i < na + nb) b[i - na] = 0;
+        else c[i - na - nb] = 0;
+    }
+}
+
 template <typename TIn, typename TOut, typename TAcc>
 int scan_impl(const TIn *in, TOut *out, int64_t n, void *tmp, hipStream_t s) {
     if (n < 0) return tg::ERR_ARG;
@@ -191,6 +200,18 @@ int fill_i32(int32_t *p, int32_t value, int64_t n, hipStream_t s) {
     if (g > 4096) g = 4096;
     hipLaunchKernelGGL((k_fill<int32_t>), dim3(g), dim3(256), 0, s, p, value, n);
     TG_LAUNCH_CHECK("k_fill<i32>");
+    return OK;
+}
+int zero_i32(int32_t *a, int64_t na, int32_t *b, int64_t nb, int32_t *c, int64_t nc,
+             hipStream_t s) {
+    if (!a) na = 0;
+    if (!b) nb = 0;
+    if (!c) nc = 0;
+    if (na + nb + nc <= 0) return OK;
+    unsigned g = grid_for(na + nb + nc, 256);
+    if (g > 4096) g = 4096;
+    hipLaunchKernelGGL(k_zero3, dim3(g), dim3(256), 0, s, a, na, b, nb, c, nc);
+    TG_LAUNCH_CHECK("k_zero3");
     return OK;
 }
 int fill_u8(uint8_t *p, uint8_t value, int64_t n, hipStream_t s) {

@@ -358,26 +358,38 @@ __global__ __launch_bounds__(256) void k_vv_compact(
     }
 }
 
+// A block takes the R vertices of one bucket: without a heavy vertex or a
+// second placement round their rows sit back to back in scratch and move as
+// one run (R was 256 for buckets of 128 too, which made every block search:
+// Kuhn 24^3 15 -> 5 us).
+template <int R>
 __global__ __launch_bounds__(256) void k_rows_compact(
     const int32_t *__restrict__ rowsrc, const int32_t *__restrict__ vv_off,
     const int32_t *__restrict__ scratch, int32_t V, int32_t *__restrict__ cols) {
-    __shared__ int32_t s_off[257];
-    __shared__ int32_t s_src[256];
-    const int32_t v0 = (int32_t)blockIdx.x * 256;
-    const int nv = min(256, V - v0);
+    __shared__ int32_t s_off[R + 1];
+    __shared__ int32_t s_src[R];
+    const int32_t v0 = (int32_t)blockIdx.x * R;
+    const int nv = min(R, V - v0);
     for (int i = threadIdx.x; i <= nv; i += 256) {
         s_off[i] = vv_off[v0 + i];
         if (i < nv) s_src[i] = rowsrc[v0 + i];
     }
     __syncthreads();
     const int32_t ob = s_off[0], oe = s_off[nv];
-    // rows that sit back to back in scratch (a bucket of 256 vertices with
-    // no heavy vertex) move as one run
     const int32_t shift = s_src[0] - ob;
     bool run = true;
     for (int i = threadIdx.x; i < nv; i += 256) run = run && s_src[i] - s_off[i] == shift;
     if (__syncthreads_and(run)) {
-        for (int32_t o = ob + threadIdx.x; o < oe; o += 256) cols[o] = scratch[(int64_t)o + shift];
+        constexpr int U = 4;
+        for (int32_t o = ob + threadIdx.x; o < oe; o += U * 256) {
+            int32_t x[U];
+#pragma unroll
+            for (int k = 0; k < U; k++)
+                x[k] = o + k * 256 < oe ? scratch[(int64_t)o + k * 256 + shift] : 0;
+#pragma unroll
+            for (int k = 0; k < U; k++)
+                if (o + k * 256 < oe) cols[o + k * 256] = x[k];
+        }
         return;
     }
     for (int32_t o = ob + threadIdx.x; o < oe; o += 256) {
@@ -435,18 +447,17 @@ __device__ __forceinline__ uint32_t n_components64(const uint64_t *adj, uint64_t
 // One wave per queued vertex v (degree <= 64): lane i holds neighbour
 // a = VV(v)[i], walks VV(a) and marks each member of VV(v) it meets, giving
 // a 64-bit adjacency row of the link graph under the row-membership rule;
-// lane 0 then counts lower and upper components by bit-parallel BFS.
+// lane 0 then counts lower and upper components by bit-parallel BFS.  The
+// wave is number `w` of `nw`.
 template <typename S>
-__global__ __launch_bounds__(64) void k_cp_fix_wave(
+__device__ __forceinline__ void fix_waves(
     const int32_t *__restrict__ off, const int32_t *__restrict__ cols,
     const S *__restrict__ scal, const int32_t *__restrict__ fix,
     int32_t *__restrict__ fixbig, int32_t *__restrict__ counters,
-    uint32_t *__restrict__ classes) {
-    __shared__ int32_t nbs[64];
-    __shared__ uint64_t adjm[64];
-    const int lane = threadIdx.x;
+    uint32_t *__restrict__ classes, int32_t *nbs, uint64_t *adjm, int32_t w, int32_t nw) {
+    const int lane = __lane_id();
     const int32_t n = counters[C_FIX];
-    for (int32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    for (int32_t i = w; i < n; i += nw) {
         const int32_t v = fix[i];
         const int32_t b = off[v];
         const int d = off[v + 1] - b;
@@ -460,7 +471,7 @@ __global__ __launch_bounds__(64) void k_cp_fix_wave(
         const uint64_t lowmask = __ballot(lo);
         const uint64_t full = d == 64 ? ~0ull : ((1ull << d) - 1ull);
         nbs[lane] = a;
-        __syncthreads();
+        tgd::wave_sync();
         uint64_t row = 0;
         if (on) {
             const int32_t rb = off[a], re = off[a + 1];
@@ -481,7 +492,7 @@ __global__ __launch_bounds__(64) void k_cp_fix_wave(
             }
         }
         adjm[lane] = row;
-        __syncthreads();
+        tgd::wave_sync();
         if (lane == 0) {
             const uint32_t nl = n_components64(adjm, lowmask & full);
             const uint32_t nu = n_components64(adjm, ~lowmask & full);
@@ -489,21 +500,37 @@ __global__ __launch_bounds__(64) void k_cp_fix_wave(
             classes[3 * (int64_t)v + 1] = nu;
             classes[3 * (int64_t)v + 2] = verdict(nl, nu);
         }
-        __syncthreads();
+        tgd::wave_sync();
     }
+}
+
+template <typename S>
+__global__ __launch_bounds__(64) void k_cp_fix_wave(
+    const int32_t *__restrict__ off, const int32_t *__restrict__ cols,
+    const S *__restrict__ scal, const int32_t *__restrict__ fix,
+    int32_t *__restrict__ fixbig, int32_t *__restrict__ counters,
+    uint32_t *__restrict__ classes) {
+    __shared__ int32_t nbs[64];
+    __shared__ uint64_t adjm[64];
+    fix_waves(off, cols, scal, fix, fixbig, counters, classes, nbs, adjm, (int32_t)blockIdx.x,
+              (int32_t)gridDim.x);
 }
 
 // Link pass driven by the row descriptors of the bucketed form: for a queued
 // vertex v (degree <= 32) each neighbour carries its class and the number of
 // its shared-tet component.  Only neighbours outside the largest component of
-// a multi-component class walk their rows; every row-membership edge between
-// two components of one class joins them, and the classes' counts are the
-// components of that component graph.  Two vertices per wave, 32 lanes each.
+// a multi-component class have their rows walked; every row-membership edge
+// between two components of one class joins them, and the classes' counts are
+// the components of that component graph.  Two vertices per wave, 32 lanes
+// each.  Few neighbours walk (one to five of 32 on a noisy field), so the
+// lanes go over a row's entries, not over the neighbours: a fifth of the
+// instructions, and whole lines per load.  Bound by the chain of dependent
+// loads per vertex and the gathers of the rows.
 __global__ __launch_bounds__(64) void k_cp_fix_desc(
     const int32_t *__restrict__ off, const int32_t *__restrict__ cols,
     const int32_t *__restrict__ rowsrc, const uint8_t *__restrict__ rowdesc,
-    const int32_t *__restrict__ fixd, int32_t *__restrict__ fix,
-    int32_t *__restrict__ counters, uint32_t *__restrict__ classes) {
+    const int32_t *__restrict__ fixd, const int32_t *__restrict__ counters,
+    uint32_t *__restrict__ classes) {
     __shared__ int32_t nbs[2][32];
     __shared__ uint8_t dsc[2][32];
     __shared__ uint32_t cadj[2][2][32];
@@ -526,10 +553,7 @@ __global__ __launch_bounds__(64) void k_cp_fix_desc(
         const int32_t v = nv_, b = nb_, rs = nrs_;
         int d = live ? ne_ - b : 0;
         head(i + 2 * gridDim.x, nv_, nb_, ne_, nrs_);
-        if (d > 32) {  // not from the bucketed kernel: generic pass
-            if (lane == 0) fix[atomicAdd(counters + C_FIX, 1)] = v;
-            d = 0;
-        }
+        d = min(d, 32);  // rows with descriptors have no more
         const bool on = lane < d;
         const int32_t a = on ? cols[b + lane] : INT32_MAX;
         const uint32_t ds = on ? rowdesc[rs + lane] : 0u;
@@ -555,35 +579,55 @@ __global__ __launch_bounds__(64) void k_cp_fix_desc(
             if (j < nc0 && s0 > best0) { best0 = s0; big0 = j; }
             if (j < nc1 && s1 > best1) { best1 = s1; big1 = j; }
         }
-        __syncthreads();
+        tgd::wave_sync();
         const int nck = cls ? nc1 : nc0;
         const int big = cls ? big1 : big0;
-        if (on && nck >= 2 && comp != big) {
-            const int32_t rb = off[a], re = off[a + 1];
-            for (int32_t j0 = rb; j0 < re; j0 += 16) {
-                int32_t c[16];
+        const bool walk = on && nck >= 2 && comp != big;
+        int32_t rb = 0, rn = 0;
+        if (walk) {
+            rb = off[a];
+            rn = off[a + 1] - rb;
+        }
+        // the walking neighbours' rows one after the other, the 32 lanes over
+        // a row's entries, four rows' loads in flight
+        uint32_t left = (uint32_t)(__ballot(walk) >> (32 * half));
+        while (__any(left != 0)) {
+            constexpr int G = 4;
+            int32_t c[G], b0[G], n0[G];
+            int from[G];
 #pragma unroll
-                for (int k = 0; k < 16; k++) c[k] = j0 + k < re ? cols[j0 + k] : INT32_MAX;
+            for (int q = 0; q < G; q++) {
+                const int src = left ? __ffs(left) - 1 : 0;
+                const bool has = left != 0;
+                left &= left - 1u;
+                b0[q] = __shfl(rb, src, 32);
+                n0[q] = has ? __shfl(rn, src, 32) : 0;
+                from[q] = __shfl((int)ds, src, 32);
+                c[q] = lane < n0[q] ? cols[b0[q] + lane] : INT32_MAX;
+            }
 #pragma unroll
-                for (int k = 0; k < 16; k++) {
-                    // lower bound in the 32 sorted entries (INT32_MAX past d):
-                    // fixed steps, so the 16 searches overlap their LDS reads
+            for (int q = 0; q < G; q++) {
+                for (int32_t j = lane;;) {
+                    // lower bound in the 32 sorted entries (INT32_MAX past d)
                     int lo = 0;
 #pragma unroll
                     for (int step = 16; step >= 1; step >>= 1)
-                        if (nbs[half][lo + step - 1] < c[k]) lo += step;
-                    if (lo < d && nbs[half][lo] == c[k]) {
-                        const int dk = dsc[half][lo];
-                        const int ck = dk & 31;
-                        if ((dk >> 5) == cls && ck != comp) {
-                            atomicOr(&cadj[half][cls][comp], 1u << ck);
-                            atomicOr(&cadj[half][cls][ck], 1u << comp);
+                        if (nbs[half][lo + step - 1] < c[q]) lo += step;
+                    if (lo < d && nbs[half][lo] == c[q]) {
+                        const int dk = dsc[half][lo], ck = dk & 31, fk = from[q] & 31;
+                        const int fc = from[q] >> 5;
+                        if ((dk >> 5) == fc && ck != fk) {
+                            atomicOr(&cadj[half][fc][fk], 1u << ck);
+                            atomicOr(&cadj[half][fc][ck], 1u << fk);
                         }
                     }
+                    j += 32;  // rows of more than 32 entries
+                    if (!__any(j - lane < n0[q])) break;
+                    c[q] = j < n0[q] ? cols[b0[q] + j] : INT32_MAX;
                 }
             }
         }
-        __syncthreads();
+        tgd::wave_sync();
         if (lane == 0 && live && d > 0) {
             const uint32_t m1 = nc1 >= 32 ? ~0u : ((1u << nc1) - 1u);
             const uint32_t m0 = nc0 >= 32 ? ~0u : ((1u << nc0) - 1u);
@@ -593,7 +637,7 @@ __global__ __launch_bounds__(64) void k_cp_fix_desc(
             classes[3 * (int64_t)v + 1] = nu;
             classes[3 * (int64_t)v + 2] = verdict(nl, nu);
         }
-        __syncthreads();
+        tgd::wave_sync();
     }
 }
 
@@ -628,18 +672,22 @@ __device__ __forceinline__ void fb_unite(int32_t *par, int a, int b) {
     }
 }
 
+struct FixBig {
+    int32_t nb[HEAVY_CAP], par[HEAVY_CAP];
+    uint8_t lowf[HEAVY_CAP];
+    int32_t cnt[2];
+};
+
+// Block number `w` of `nw`.
 template <typename S>
-__global__ __launch_bounds__(FB_THREADS) void k_cp_fix_big(
+__device__ __forceinline__ void fix_blocks(
     const int32_t *__restrict__ off, const int32_t *__restrict__ cols,
     const S *__restrict__ scal, const int32_t *__restrict__ fixbig,
-    int32_t *__restrict__ counters, uint32_t *__restrict__ classes) {
-    __shared__ int32_t nb[HEAVY_CAP];
-    __shared__ int32_t par[HEAVY_CAP];
-    __shared__ uint8_t lowf[HEAVY_CAP];
-    __shared__ int32_t cnt[2];
+    int32_t *__restrict__ counters, uint32_t *__restrict__ classes, FixBig &st, int32_t w,
+    int32_t nw) {
     const int tid = threadIdx.x;
     const int32_t n = counters[C_FIXBIG];
-    for (int32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    for (int32_t i = w; i < n; i += nw) {
         const int32_t v = fixbig[i];
         const int32_t b = off[v];
         const int d = off[v + 1] - b;
@@ -650,15 +698,15 @@ __global__ __launch_bounds__(FB_THREADS) void k_cp_fix_big(
         const S sv = scal[v];
         for (int k = tid; k < d; k += FB_THREADS) {
             const int32_t a = cols[b + k];
-            nb[k] = a;
-            par[k] = k;
-            lowf[k] = (uint8_t)is_lower(scal[a], sv, a, v);
+            st.nb[k] = a;
+            st.par[k] = k;
+            st.lowf[k] = (uint8_t)is_lower(scal[a], sv, a, v);
         }
-        if (tid < 2) cnt[tid] = 0;
+        if (tid < 2) st.cnt[tid] = 0;
         __syncthreads();
         for (int ia = tid; ia < d; ia += FB_THREADS) {
-            const int32_t a = nb[ia];
-            const uint8_t la = lowf[ia];
+            const int32_t a = st.nb[ia];
+            const uint8_t la = st.lowf[ia];
             const int32_t je = off[a + 1];
             for (int32_t j = off[a]; j < je; j++) {
                 const int32_t c = cols[j];
@@ -666,23 +714,61 @@ __global__ __launch_bounds__(FB_THREADS) void k_cp_fix_big(
                 int lo = 0, hi = d;  // first entry of v's row >= c
                 while (lo < hi) {
                     const int mid = (lo + hi) >> 1;
-                    if (nb[mid] < c) lo = mid + 1;
+                    if (st.nb[mid] < c) lo = mid + 1;
                     else hi = mid;
                 }
-                if (lo < d && nb[lo] == c && lowf[lo] == la) fb_unite(par, ia, lo);
+                if (lo < d && st.nb[lo] == c && st.lowf[lo] == la) fb_unite(st.par, ia, lo);
             }
         }
         __syncthreads();
         for (int k = tid; k < d; k += FB_THREADS)
-            if (par[k] == k) atomicAdd(&cnt[lowf[k] ? 0 : 1], 1);
+            if (st.par[k] == k) atomicAdd(&st.cnt[st.lowf[k] ? 0 : 1], 1);
         __syncthreads();
         if (tid == 0) {
-            const uint32_t nl = (uint32_t)cnt[0], nu = (uint32_t)cnt[1];
+            const uint32_t nl = (uint32_t)st.cnt[0], nu = (uint32_t)st.cnt[1];
             classes[3 * (int64_t)v] = nl;
             classes[3 * (int64_t)v + 1] = nu;
             classes[3 * (int64_t)v + 2] = verdict(nl, nu);
         }
-        __syncthreads();  // nb, par, lowf and cnt are reused by the next vertex
+        __syncthreads();  // the staging is reused by the next vertex
+    }
+}
+
+template <typename S>
+__global__ __launch_bounds__(FB_THREADS) void k_cp_fix_big(
+    const int32_t *__restrict__ off, const int32_t *__restrict__ cols,
+    const S *__restrict__ scal, const int32_t *__restrict__ fixbig,
+    int32_t *__restrict__ counters, uint32_t *__restrict__ classes) {
+    __shared__ FixBig st;
+    fix_blocks(off, cols, scal, fixbig, counters, classes, st, (int32_t)blockIdx.x,
+               (int32_t)gridDim.x);
+}
+
+// Both passes in one launch, for the bucketed form, whose lists hold only what
+// the heavy kernel queued (rows over 32 entries by their length, so neither
+// pass adds to the other's list): most meshes have none, and an empty launch
+// costs 4 us.
+constexpr int REST_WAVES = 1024, REST_BIG = 256;  // blocks of each
+template <typename S>
+__global__ __launch_bounds__(FB_THREADS) void k_cp_fix_rest(
+    const int32_t *__restrict__ off, const int32_t *__restrict__ cols,
+    const S *__restrict__ scal, const int32_t *__restrict__ fix, int32_t *__restrict__ fixbig,
+    int32_t *__restrict__ counters, uint32_t *__restrict__ classes) {
+    __shared__ union {
+        FixBig big;
+        struct {
+            int32_t nbs[FB_THREADS / 64][64];
+            uint64_t adjm[FB_THREADS / 64][64];
+        } wave;
+    } st;
+    if (blockIdx.x < REST_BIG) {  // the longest ones start first
+        fix_blocks(off, cols, scal, fixbig, counters, classes, st.big, (int32_t)blockIdx.x, REST_BIG);
+    } else {
+        const int wid = threadIdx.x / 64;
+        fix_waves(off, cols, scal, fix, fixbig, counters, classes, st.wave.nbs[wid],
+                  st.wave.adjm[wid],
+                  (int32_t)(blockIdx.x - REST_BIG) * (FB_THREADS / 64) + wid,
+                  REST_WAVES * (FB_THREADS / 64));
     }
 }
 
@@ -690,19 +776,24 @@ template <typename S>
 int launch_cp_fix_typed(tg::VvCpBuffers &b, hipStream_t s) {
     const int32_t V = (int32_t)b.n_points;
     const S *scal = (const S *)b.scalars;
-    const unsigned g = std::min<unsigned>(tg::grid_for(V, 1), 16384u);
     if (b.fixd) {
-        hipLaunchKernelGGL(k_cp_fix_desc, dim3(std::max(1u, g / 2)), dim3(64), 0, s, b.vv_off,
-                           b.vv_cols, b.rowsrc,
-                           b.rowdesc, b.fixd, b.fix, b.counters, b.classes);
+        // two vertices a block; 32 blocks per CU
+        const unsigned g = std::min<unsigned>(tg::grid_for(V, 2), 8192u);
+        hipLaunchKernelGGL(k_cp_fix_desc, dim3(g), dim3(64), 0, s, b.vv_off, b.vv_cols, b.rowsrc,
+                           b.rowdesc, b.fixd, b.counters, b.classes);
         TG_LAUNCH_CHECK("k_cp_fix_desc");
+        hipLaunchKernelGGL((k_cp_fix_rest<S>), dim3(REST_WAVES + REST_BIG), dim3(FB_THREADS), 0, s,
+                           b.vv_off, b.vv_cols, scal, b.fix, b.fixbig, b.counters, b.classes);
+        TG_LAUNCH_CHECK("k_cp_fix_rest");
+    } else {
+        const unsigned g = std::min<unsigned>(tg::grid_for(V, 1), 16384u);
+        hipLaunchKernelGGL((k_cp_fix_wave<S>), dim3(g), dim3(64), 0, s, b.vv_off, b.vv_cols, scal,
+                           b.fix, b.fixbig, b.counters, b.classes);
+        TG_LAUNCH_CHECK("k_cp_fix_wave");
+        hipLaunchKernelGGL((k_cp_fix_big<S>), dim3(256), dim3(FB_THREADS), 0, s, b.vv_off, b.vv_cols,
+                           scal, b.fixbig, b.counters, b.classes);
+        TG_LAUNCH_CHECK("k_cp_fix_big");
     }
-    hipLaunchKernelGGL((k_cp_fix_wave<S>), dim3(g), dim3(64), 0, s, b.vv_off, b.vv_cols, scal,
-                       b.fix, b.fixbig, b.counters, b.classes);
-    TG_LAUNCH_CHECK("k_cp_fix_wave");
-    hipLaunchKernelGGL((k_cp_fix_big<S>), dim3(256), dim3(FB_THREADS), 0, s, b.vv_off, b.vv_cols, scal,
-                       b.fixbig, b.counters, b.classes);
-    TG_LAUNCH_CHECK("k_cp_fix_big");
     if (b.marks) b.marks->mark("cp_fix", s);
     return tg::OK;
 }
@@ -797,10 +888,14 @@ int launch_vt_corners(VvCpBuffers &b, int block, hipStream_t s) {
 }
 
 int launch_rows_compact(const int32_t *rowsrc, const int32_t *vv_off, const int32_t *scratch,
-                        int32_t V, int32_t *cols, hipStream_t s) {
+                        int32_t V, int bv_log, int32_t *cols, hipStream_t s) {
     if (V <= 0) return OK;
-    hipLaunchKernelGGL(k_rows_compact, dim3(grid_for(V, 256)), dim3(256), 0, s, rowsrc, vv_off,
-                       scratch, V, cols);
+    if (bv_log == 7)
+        hipLaunchKernelGGL(k_rows_compact<128>, dim3(grid_for(V, 128)), dim3(256), 0, s, rowsrc,
+                           vv_off, scratch, V, cols);
+    else
+        hipLaunchKernelGGL(k_rows_compact<256>, dim3(grid_for(V, 256)), dim3(256), 0, s, rowsrc,
+                           vv_off, scratch, V, cols);
     TG_LAUNCH_CHECK("k_rows_compact");
     return OK;
 }
@@ -813,13 +908,13 @@ int launch_cp_fix(VvCpBuffers &b, hipStream_t s) {
 int run_vv_cp_bucketed(BucketBuffers &k, bool classify, hipStream_t s) {
     VvCpBuffers &b = k.base;
     if (b.marks) b.marks->begin(s);
-    int rc = fill_i32(b.counters, 0, N_COUNTERS, s);
-    if (rc) return rc;
+    int rc = OK;
     const int32_t V = (int32_t)b.n_points;
-    if (V > 0 && (rc = launch_bucketed_vv_cp(k, classify, s))) return rc;
+    if (V == 0 && (rc = fill_i32(b.counters, 0, N_COUNTERS, s))) return rc;
+    if (V > 0 && (rc = launch_bucketed_vv_cp(k, classify, s))) return rc;  // clears the counters
     if ((rc = scan_exclusive_i32(b.deg, b.vv_off, V, b.scan_tmp, s))) return rc;
     if (b.marks) b.marks->mark("vv_scan", s);
-    if ((rc = launch_rows_compact(k.rowsrc, b.vv_off, b.scratch, V, b.vv_cols, s))) return rc;
+    if ((rc = launch_rows_compact(k.rowsrc, b.vv_off, b.scratch, V, k.plan.bv_log, b.vv_cols, s))) return rc;
     if (b.marks) b.marks->mark("vv_compact", s);
     if (classify && (rc = launch_cp_fix(b, s))) return rc;
     return OK;

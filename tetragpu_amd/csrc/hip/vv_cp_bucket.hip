@@ -28,6 +28,7 @@
 #include <algorithm>
 
 #include "bucket.h"
+#include "networks.h"
 
 namespace {
 
@@ -840,40 +841,6 @@ constexpr int sk_slab = BV * 275 / 8;  // record slots of a block of BV vertices
 template <int BV>
 constexpr int sk_span = sk_slab<BV> - SK_MAXREC - BV;  // offsets of one round
 
-// Knuth's merge exchange (The Art of Computer Programming 3, 5.2.2 M) for any
-// N: for p = 2^(t-1) .. 1, compare (i, i + p) where i & p == 0, then
-// (i, i + q - p) where i & p for q = 2^(t-1) .. 2p.
-template <int N, int D, int P, int R>
-__device__ __forceinline__ void sort_stage(uint32_t (&k)[N]) {
-#pragma unroll
-    for (int i = 0; i < N - D; i++)
-        if ((i & P) == R) {
-            const uint32_t a = k[i], b = k[i + D];
-            k[i] = tgd::opaque(min(a, b));
-            k[i + D] = tgd::opaque(max(a, b));
-        }
-}
-template <int N, int P, int Q>
-__device__ __forceinline__ void sort_merges(uint32_t (&k)[N]) {
-    if constexpr (Q > P) {
-        sort_stage<N, Q - P, P, P>(k);
-        sort_merges<N, P, Q / 2>(k);
-    }
-}
-template <int N, int P, int TOP>
-__device__ __forceinline__ void sort_phases(uint32_t (&k)[N]) {
-    if constexpr (P > 0) {
-        sort_stage<N, P, P, 0>(k);
-        sort_merges<N, P, TOP>(k);
-        sort_phases<N, P / 2, TOP>(k);
-    }
-}
-constexpr int top_power(int n) { return n <= 2 ? 1 : 2 * top_power((n + 1) / 2); }  // 2^(ceil(log2 n) - 1)
-template <int N>
-__device__ __forceinline__ void sort_keys(uint32_t (&k)[N]) {
-    sort_phases<N, top_power(N), top_power(N)>(k);
-}
-
 // Components of `mask` as label_components, over a lane's column of the
 // adjacency and of the row (slot f at word f * 64).
 __device__ __forceinline__ uint32_t label_columns(const uint32_t *adj, uint32_t *row,
@@ -935,7 +902,7 @@ __device__ __forceinline__ int sort_rows(const Slab &rec, int pos, int c, uint32
         if (r % 8 == 7) tgd::sched_fence();
     }
     __syncthreads();
-    sort_keys(k);
+    tgn::sort_keys(k);
     if (CP) {
 #pragma unroll
         for (int r = 0; r < NCOL; r++) adj[r * 64] = 0u;
@@ -1725,8 +1692,10 @@ __global__ __launch_bounds__(VT_THREADS) void k_bkt_vt(const Rec rec,
 // [bucket][slice]); the choice is made on the mesh's first run.  VTREC:
 // records carry the corner code 4t + j (low 24 bits, high bits) instead of
 // the other three corners.
+// reset: zero the first `reset` run counters as well.
 template <bool VTREC>
-int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, int32_t &nsl) {
+int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, int32_t &nsl,
+                  int reset) {
     const tg::BucketPlan &p = k.plan;
     tg::VvCpBuffers &b = k.base;
     const int64_t T = b.n_cells;
@@ -1740,11 +1709,17 @@ int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, i
     int route = k.route ? *k.route : tg::ROUTE_TWO;
     ranges = k.h2;
     nsl = p.slices;
+    const bool routed_two = route == tg::ROUTE_TWO;  // else the counters are zeroed already
     if (route != tg::ROUTE_TWO) {
         int32_t *bstart = k.h2, *bused = k.h1;
-        if ((rc = tg::fill_i32(bstart, 0, p.nb, s)) || (rc = tg::fill_i32(bused, 0, p.nb, s)))
-            return rc;
-        hipLaunchKernelGGL(k_s1_count, dim3(p.nchunks), dim3(S1_THREADS), 0, s, tv4, T, p.tpc,
+        // chunks of at most tpc tets, and shorter ones (whole tiles) while
+        // they would leave the chip's 256 CUs short of blocks: Kuhn 24^3 in
+        // chunks of 4096 took 9 + 21 us with 21 blocks, in tiles of 1024 6 + 9
+        const int64_t tpc = std::max<int64_t>(
+            S1_TILE, std::min<int64_t>(p.tpc, (T / 512 + S1_TILE - 1) / S1_TILE * S1_TILE));
+        const int64_t nch = std::max<int64_t>(1, (T + tpc - 1) / tpc);
+        if ((rc = tg::zero_i32(bstart, p.nb, bused, p.nb, b.counters, reset, s))) return rc;
+        hipLaunchKernelGGL(k_s1_count, dim3((unsigned)nch), dim3(S1_THREADS), 0, s, tv4, T, tpc,
                            p.bv_log, bstart, b.counters);
         TG_LAUNCH_CHECK("k_s1_count");
         if (route == tg::ROUTE_AUTO) {
@@ -1757,9 +1732,9 @@ int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, i
                 TG_HIP(hipMemcpyAsync(&wide, b.counters + tg::C_WIDE, sizeof wide,
                                       hipMemcpyDeviceToHost, s));
                 TG_HIP(hipStreamSynchronize(s));
-                const int64_t per = (p.tpc + S1_TILE - 1) / S1_TILE;
-                const int64_t last = T - (int64_t)(p.nchunks - 1) * p.tpc;
-                const int64_t tiles = (int64_t)(p.nchunks - 1) * per + (last + S1_TILE - 1) / S1_TILE;
+                const int64_t per = (tpc + S1_TILE - 1) / S1_TILE;
+                const int64_t last = T - (nch - 1) * tpc;
+                const int64_t tiles = (nch - 1) * per + (last + S1_TILE - 1) / S1_TILE;
                 route = (int64_t)wide * 64 <= tiles ? tg::ROUTE_ONE : tg::ROUTE_TWO;
                 *k.route = route;
             }
@@ -1767,8 +1742,8 @@ int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, i
         if (route == tg::ROUTE_ONE) {
             if ((rc = tg::scan_exclusive_i32(bstart, bstart, p.nb, b.scan_tmp, s))) return rc;
             if (mk) mk->mark("s1_count", s);
-            hipLaunchKernelGGL(k_s1_scatter<VTREC>, dim3(p.nchunks), dim3(S1_THREADS), 0, s, tv4, T,
-                               p.tpc, p.bv_log, bstart, bused, r2);
+            hipLaunchKernelGGL(k_s1_scatter<VTREC>, dim3((unsigned)nch), dim3(S1_THREADS), 0, s, tv4, T,
+                               tpc, p.bv_log, bstart, bused, r2);
             TG_LAUNCH_CHECK("k_s1_scatter");
             if (mk) mk->mark("s1_scatter", s);
             ranges = bstart;
@@ -1776,6 +1751,8 @@ int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, i
         }
     }
     if (route == tg::ROUTE_TWO) {
+        if (routed_two && (rc = tg::zero_i32(b.counters, reset, nullptr, 0, nullptr, 0, s)))
+            return rc;
         hipLaunchKernelGGL(k_l1_count, dim3(p.nchunks), dim3(L1_THREADS), 0, s, tv4, T, p.tpc,
                            cshift, p.nc, p.nchunks, k.h1);
         TG_LAUNCH_CHECK("k_l1_count");
@@ -1814,7 +1791,7 @@ int launch_bucketed_typed(tg::BucketBuffers &k, bool classify, hipStream_t s) {
     const Rec r2{k.rec2, k.rec2 + n, k.rec2 + 2 * n};
     const int32_t *ranges = nullptr;
     int32_t nsl = 1;
-    int rc = route_records<false>(k, s, ranges, nsl);
+    int rc = route_records<false>(k, s, ranges, nsl, tg::N_COUNTERS);
     if (rc) return rc;
 #define TG_BKT(KERNEL, THREADS)                                                              \
     hipLaunchKernelGGL(KERNEL, dim3(p.nb), dim3(THREADS), 0, s, r2, ranges, nsl,                \
@@ -1894,11 +1871,13 @@ int run_vt_bucketed(BucketBuffers &k, int32_t *vt_off, int32_t *vtc, int32_t *vt
     const int32_t V = (int32_t)b.n_points;
     if (V <= 0) return fill_i32(vt_off, 0, 1, s);
     if (4 * b.n_cells > (int64_t)INT32_MAX) return ERR_CAPACITY;
-    int rc = fill_i32(b.counters + C_WIDE, 0, 1, s);  // the routing choice counts wide tiles
+    int rc = OK;
+    if (!k.route || *k.route == ROUTE_AUTO)  // the routing choice counts wide tiles
+        rc = fill_i32(b.counters + C_WIDE, 0, 1, s);
     if (rc) return rc;
     const int32_t *ranges = nullptr;
     int32_t nsl = 1;
-    if ((rc = route_records<true>(k, s, ranges, nsl))) return rc;
+    if ((rc = route_records<true>(k, s, ranges, nsl, 0))) return rc;
     const int64_t n = 4 * b.n_cells;
     const Rec r2{k.rec2, k.rec2 + n, k.rec2 + 2 * n};
     int32_t *stage = (int32_t *)k.rec1;
