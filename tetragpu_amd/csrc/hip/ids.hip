@@ -18,11 +18,13 @@
 // positional triple, and face ids are ranks of first occurrences.
 //
 // The remaining relations are two-pass CSR builds (count, scan, fill) over
-// sorted rows: ET(e) = VT(lo) n VT(hi); EF, TT, FF, EE by merging sorted
+// sorted rows, or joins with a chained scan (ET(e) = VT(lo) n VT(hi), TT, EE);
+// EF, FF by merging sorted
 // lists; FT from the face matches.
 #include <algorithm>
 
 #include "ids.h"
+#include "networks.h"
 #include "tetra_c.h"
 
 namespace {
@@ -72,8 +74,7 @@ __device__ __forceinline__ int32_t bsearch_i32(const int32_t *a, int32_t n, int3
 typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef int32_t i32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// Merges of a few short sorted rows (ET, TT, EE) stage the rows in LDS
-// first: one column per thread (consecutive threads in consecutive banks),
+// k_edge_first stages its row in LDS: one column per thread (consecutive threads in consecutive banks),
 // filled by independent 16-byte loads, so a row costs one memory latency
 // instead of one per element; the merge then reads LDS.  Whole quads are
 // read, up to three words past the row (the source array carries that
@@ -95,32 +96,11 @@ __device__ __forceinline__ void stage_quads(int32_t (*buf)[W], int at,
     }
 }
 
-// A thread's output row written in 16-byte stores: words gather in a
-// register quad, stored when full; the last, partial quad is stored whole,
-// so the row's slot must start 16-byte aligned and span a multiple of four
-// words.  One store per four words instead of one per word: scattered
-// per-thread rows cost the vector memory path per store instruction.
-struct QuadOut {
-    int32_t *row;
-    int64_t n = 0;
-    int4 q = make_int4(0, 0, 0, 0);
-    __device__ __forceinline__ void put(int32_t v) {
-        const int k = (int)(n & 3);
-        q.x = k == 0 ? v : q.x;
-        q.y = k == 1 ? v : q.y;
-        q.z = k == 2 ? v : q.z;
-        q.w = k == 3 ? v : q.w;
-        if (k == 3) *reinterpret_cast<int4 *>(row + n - 3) = q;
-        n++;
-    }
-    __device__ __forceinline__ void flush() {
-        if (n & 3) *reinterpret_cast<int4 *>(row + (n & ~(int64_t)3)) = q;
-    }
-};
-
-// QuadOut for a row at its final, exact position: full quads in unaligned
-// 16-byte stores, the last one to three words one by one (the words after
-// the row belong to the next row).
+// A thread's output row at its exact position: words gather in a register
+// quad, full quads leave in unaligned 16-byte stores, the last one to three
+// words one by one (the words after the row belong to the next row).  One
+// store per four words instead of one per word: scattered per-thread rows cost
+// the vector memory path per store instruction.
 struct QuadOutExact {
     int32_t *row;
     int64_t n = 0;
@@ -144,20 +124,23 @@ struct QuadOutExact {
 };
 
 // ---- edges --------------------------------------------------------------------
-// Lane per vertex v: first position of every upper edge (v, u>v), flag it.
-// Every pair of v's cells whose low vertex is v also records the VV index of
-// its edge in te (replaced by the edge id once ids exist): the row search is
-// done here, on v's own row, instead of once per cell on random rows.
+// Lane per vertex v: first position of every edge (v, u) of its row; upper
+// ones (u > v) are flagged.
+// Every pair of v's cells whose low vertex is v also records its edge's first
+// position in te (replaced by the edge id, its rank, once ranks exist): the
+// row search is done here, on v's own row, instead of once per cell on random
+// rows, and the ranks (8 bytes per 32 positions) are a sixth of the VV-aligned
+// ids that te could index instead.
 // Rows up to EDGE_CAP entries are staged in LDS (one column per thread: the
 // VV row and the first positions), and the vertex's cells are fetched eight
 // at a time with independent loads; longer rows work in global memory.
-constexpr int EDGE_THREADS = 64, EDGE_CAP = 48;
+constexpr int EDGE_THREADS = 64, EDGE_CAP = 32;  // 17 KB a wave: nine waves per CU
 
 __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
     const int4 *__restrict__ tv4, const int32_t *__restrict__ vt_off,
     const int32_t *__restrict__ vtc, const int32_t *__restrict__ vv_off,
     const int32_t *__restrict__ vv, int64_t V, int32_t *__restrict__ efirst,
-    uint8_t *__restrict__ flags, int32_t *__restrict__ te_idx) {
+    uint8_t *__restrict__ flags, int32_t *__restrict__ te_first) {
     __shared__ int32_t srow[EDGE_CAP + 3][EDGE_THREADS];  // three spare slots for stage_quads
     __shared__ int32_t sef[EDGE_CAP][EDGE_THREADS];
     const int tid = threadIdx.x;
@@ -185,15 +168,18 @@ __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
                     for (int j = 0; j < 4; j++) {
                         if (j == jv) continue;
                         const int32_t u = corner(q[c], j);
-                        if (u < v) continue;
-                        int32_t lo = 0;  // lower bound of u in the staged row (rn < 64)
+                        int32_t lo = 0;  // place of u in the staged row (rn <= 32)
 #pragma unroll
-                        for (int step = 32; step >= 1; step >>= 1)
+                        for (int step = 16; step >= 1; step >>= 1)
                             if (lo + step - 1 < rn && srow[lo + step - 1][tid] < u) lo += step;
                         const int32_t idx = lo < rn && srow[lo][tid] == u ? lo : -1;
                         const int32_t pos = 6 * t + pair_index(min(j, (int)jv), max(j, (int)jv));
-                        te_idx[pos] = idx >= 0 ? rb + idx : -1;
-                        if (idx >= 0 && sef[idx][tid] == INF) sef[idx][tid] = pos;
+                        int32_t p1 = INF;  // first position of the edge
+                        if (idx >= 0) {
+                            p1 = min(sef[idx][tid], pos);  // cells ascend
+                            sef[idx][tid] = p1;
+                        }
+                        if (u > v) te_first[pos] = p1;
                     }
                 }
             }
@@ -214,11 +200,10 @@ __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
             for (int j = 0; j < 4; j++) {
                 if (j == jv) continue;
                 const int32_t u = corner(q, j);
-                if (u < v) continue;
                 const int32_t idx = bsearch_i32(row, rn, u);
                 const int32_t pos = 6 * t + pair_index(min(j, jv), max(j, jv));
-                te_idx[pos] = idx >= 0 ? rb + idx : -1;
                 if (idx >= 0 && ef[idx] == INF) ef[idx] = pos;
+                if (u > v) te_first[pos] = idx >= 0 ? ef[idx] : INF;
             }
         }
         for (int32_t i = 0; i < rn; i++)
@@ -226,7 +211,9 @@ __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
     }
 }
 
-// bytes -> bitmap words and their popcounts
+// bytes (0 or 1) -> bitmap words and their popcounts.  32 bytes per lane in
+// two 16-byte loads; the multiplication gathers the low bits of four bytes
+// (bit 8 i moves to bit 28 + i; no other product bit reaches 28).
 __global__ void k_pack_flags(const uint8_t *__restrict__ flags, int64_t n,
                              uint32_t *__restrict__ bits, int32_t *__restrict__ pop) {
     const int64_t nw = (n + 31) / 32;
@@ -234,22 +221,39 @@ __global__ void k_pack_flags(const uint8_t *__restrict__ flags, int64_t n,
          w += (int64_t)gridDim.x * blockDim.x) {
         uint32_t m = 0;
         const int64_t b = 32 * w;
-        for (int i = 0; i < 32 && b + i < n; i++) m |= (uint32_t)(flags[b + i] != 0) << i;
+        if (b + 32 <= n) {
+            const uint4 *p = reinterpret_cast<const uint4 *>(flags + b);
+            const uint4 q0 = p[0], q1 = p[1];
+            const uint32_t x[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) m |= ((x[i] * 0x10204080u) >> 28) << (4 * i);
+        } else {
+            for (int i = 0; i < 32 && b + i < n; i++) m |= (uint32_t)(flags[b + i] != 0) << i;
+        }
         bits[w] = m;
         pop[w] = __popc(m);
     }
 }
 
-__device__ __forceinline__ int32_t rank_of(const uint32_t *bits, const int32_t *wpre, int32_t p) {
-    const int32_t w = p >> 5;
-    return wpre[w] + __popc(bits[w] & ((1u << (p & 31)) - 1u));
+// A bitmap word and the number of set bits before it, side by side: a random
+// rank lookup touches one line instead of two.
+__global__ void k_rank_words(const uint32_t *__restrict__ bits, const int32_t *__restrict__ wpre,
+                             int64_t nw, uint2 *__restrict__ rank) {
+    for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w < nw;
+         w += (int64_t)gridDim.x * blockDim.x)
+        rank[w] = make_uint2(bits[w], (uint32_t)wpre[w]);
+}
+
+__device__ __forceinline__ int32_t rank_of(const uint2 *__restrict__ rank, int32_t p) {
+    const uint2 w = rank[p >> 5];
+    return (int32_t)w.y + __popc(w.x & ((1u << (p & 31)) - 1u));
 }
 
 // Lane per vertex v: ids of v's upper edges (VV-aligned) and EV.
 __global__ void k_edge_ids(const int32_t *__restrict__ vv_off, const int32_t *__restrict__ vv,
                            int64_t V, const int32_t *__restrict__ efirst,
-                           const uint32_t *__restrict__ bits, const int32_t *__restrict__ wpre,
-                           int32_t *__restrict__ vv_eid, int32_t *__restrict__ ev) {
+                           const uint2 *__restrict__ rank, int32_t *__restrict__ vv_eid,
+                           int32_t *__restrict__ ev) {
     for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V;
          v += (int64_t)gridDim.x * blockDim.x) {
         const int32_t rb = vv_off[v], re = vv_off[v + 1];
@@ -268,9 +272,8 @@ __global__ void k_edge_ids(const int32_t *__restrict__ vv_off, const int32_t *__
             for (int c = 0; c < 8; c++) {
                 const int on = (int)(i0 + c < re) & (int)(u[c] > v) & (int)(p[c] != INF);
                 const int32_t q = on ? p[c] : 0;
-                const uint32_t w = bits[q >> 5];
-                const int32_t pre = wpre[q >> 5];
-                id[c] = on ? pre + __popc(w & ((1u << (q & 31)) - 1u)) : -1;
+                const int32_t r = rank_of(rank, q);
+                id[c] = on ? r : -1;
             }
 #pragma unroll
             for (int c = 0; c < 8; c++) {
@@ -348,90 +351,49 @@ __global__ __launch_bounds__(VE_THREADS) void k_ve_fill(const int32_t *__restric
     }
 }
 
-// lower entries (u < v) take the id stored in u's row
-__global__ void k_edge_lower(const int32_t *__restrict__ vv_off, const int32_t *__restrict__ vv,
-                             int64_t V, int32_t *__restrict__ vv_eid) {
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        for (int32_t i = vv_off[v]; i < vv_off[v + 1]; i++) {
-            const int32_t u = vv[i];
-            if (u > v) continue;
-            const int32_t ub = vv_off[u];
-            const int32_t j = bsearch_i32(vv + ub, vv_off[u + 1] - ub, (int32_t)v);
-            vv_eid[i] = j >= 0 ? vv_eid[ub + j] : -1;
+// Each vertex's edge ids, ascending (for EE): the upper entries' ids are in
+// vv_eid, a lower entry's is the rank of its first position, which
+// k_edge_first noted for both ends of an edge.  (Searching v in each lower
+// neighbour's row took 0.63 ms at 5.3 M cells, and sorting the rows in memory
+// 0.28; this pass 0.19.)  Rows of up to 32 entries are sorted in registers,
+// longer ones in memory.
+__global__ __launch_bounds__(256) void k_vertex_edges(const int32_t *__restrict__ vv_off,
+                                                      const int32_t *__restrict__ vv, int64_t V,
+                                                      const int32_t *__restrict__ efirst,
+                                                      const uint2 *__restrict__ rank,
+                                                      const int32_t *__restrict__ vv_eid,
+                                                      int32_t *__restrict__ out) {
+    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= V) return;
+    const int32_t rb = vv_off[v], rn = vv_off[v + 1] - rb;
+    auto id_of = [&](int32_t i) {
+        const int32_t p = efirst[i];
+        return vv[i] > (int32_t)v ? vv_eid[i] : p != INF ? rank_of(rank, p) : -1;
+    };
+    if (rn <= 32) {
+        int32_t k[32];
+#pragma unroll
+        for (int i = 0; i < 32; i++) k[i] = i < rn ? id_of(rb + i) : INF;
+        tgn::sort_keys(k);
+#pragma unroll
+        for (int i = 0; i < 32; i++)
+            if (i < rn) out[rb + i] = k[i];
+    } else {
+        for (int32_t i = 0; i < rn; i++) {
+            const int32_t x = id_of(rb + i);
+            int32_t j = i;
+            for (; j > 0 && out[rb + j - 1] > x; j--) out[rb + j] = out[rb + j - 1];
+            out[rb + j] = x;
         }
     }
 }
 
-// TE: the VV indices recorded by k_edge_first become edge ids
-__global__ void k_te(int32_t *__restrict__ te, int64_t n, const int32_t *__restrict__ vv_eid) {
+// TE: the first positions recorded by k_edge_first become edge ids
+__global__ void k_te(int32_t *__restrict__ te, int64_t n, const uint2 *__restrict__ rank) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t k = te[i];
-        te[i] = k >= 0 ? vv_eid[k] : -1;
-    }
-}
-
-// ---- ET = VT(lo) n VT(hi) -------------------------------------------------------
-// Both rows are staged in LDS when they fit (stage_quads), then merged in
-// one pass into a padded slot at pad[e] of min(|VT(lo)|, |VT(hi)|) words
-// rounded up to a multiple of four (QuadOut), with the row length in
-// cnt[e]; k_pack_rows packs the rows afterwards.
-constexpr int ET_THREADS = 64, ET_CAP = 125;  // with stage_quads' three spare slots: 32 KB
-
-__global__ void k_et_bound(const int32_t *__restrict__ ev, int64_t E, int64_t V,
-                           const int32_t *__restrict__ vt_off, int64_t *__restrict__ ub) {
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t a = ev[2 * e], b = ev[2 * e + 1];
-        const bool ok = a >= 0 && a < V && b >= 0 && b < V;  // always, for a built EV
-        const int64_t n = ok ? min(vt_off[a + 1] - vt_off[a], vt_off[b + 1] - vt_off[b]) : 0;
-        ub[e] = (n + 3) & ~(int64_t)3;
-    }
-}
-
-__global__ __launch_bounds__(ET_THREADS) void k_et(const int32_t *__restrict__ ev, int64_t E,
-                                                   int64_t V, const int32_t *__restrict__ vt_off,
-                                                   const int32_t *__restrict__ vtc,
-                                                   const int64_t *__restrict__ pad,
-                                                   int64_t *__restrict__ cnt,
-                                                   int32_t *__restrict__ out) {
-    __shared__ int32_t buf[ET_CAP + 3][ET_THREADS];
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t a = ev[2 * e], b = ev[2 * e + 1];
-        const bool ok = a >= 0 && a < V && b >= 0 && b < V;  // always, for a built EV
-        int32_t i = ok ? vt_off[a] : 0, ie = ok ? vt_off[a + 1] : 0;
-        int32_t j = ok ? vt_off[b] : 0, je = ok ? vt_off[b + 1] : 0;
-        QuadOut o;
-        o.row = out + pad[e];
-        const int32_t na = ie - i, nb = je - j;
-        if (na + nb <= ET_CAP) {
-            stage_quads(buf, 0, vtc + i, na, 2);
-            stage_quads(buf, na, vtc + j, nb, 2);
-            i = 0, ie = na, j = na, je = na + nb;
-            int32_t x = i < ie ? buf[i][threadIdx.x] : INF, y = j < je ? buf[j][threadIdx.x] : INF;
-            const int32_t last = max(je - 1, 0);
-            while (x != INF && y != INF) {  // branch-free advance (two reads per step)
-                if (x == y) o.put(x);
-                const int32_t m = min(x, y);
-                i += x == m;
-                j += y == m;
-                const int32_t xa = buf[min(i, last)][threadIdx.x], yb = buf[min(j, last)][threadIdx.x];
-                x = i < ie ? xa : INF;
-                y = j < je ? yb : INF;
-            }
-        } else {
-            int32_t x = i < ie ? vtc[i] >> 2 : INF, y = j < je ? vtc[j] >> 2 : INF;
-            while (x != INF && y != INF) {
-                if (x == y) o.put(x);
-                const int32_t m = min(x, y);
-                if (x == m) x = ++i < ie ? vtc[i] >> 2 : INF;
-                if (y == m) y = ++j < je ? vtc[j] >> 2 : INF;
-            }
-        }
-        o.flush();
-        cnt[e] = o.n;
+        const int32_t p = te[i];
+        te[i] = p != INF ? rank_of(rank, p) : -1;
     }
 }
 
@@ -548,13 +510,12 @@ __global__ void k_face_first(const int4 *__restrict__ tv4, int64_t T, const int3
 // FT (<= 2 tets, ascending, -1 pad)
 __global__ void k_face_ids(const int4 *__restrict__ tv4, int64_t T,
                            const int32_t *__restrict__ ffirst, const int32_t *__restrict__ other,
-                           const uint32_t *__restrict__ bits,
-                           const int32_t *__restrict__ wpre, int32_t *__restrict__ tf,
+                           const uint2 *__restrict__ rank, int32_t *__restrict__ tf,
                            int32_t *__restrict__ fv, int32_t *__restrict__ ft) {
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < 4 * T;
          p += (int64_t)gridDim.x * blockDim.x) {
         const int32_t f = ffirst[p];
-        const int32_t id = rank_of(bits, wpre, f);
+        const int32_t id = rank_of(rank, f);
         tf[p] = id;
         if (f != (int32_t)p) continue;
         const int32_t t = (int32_t)(p >> 2);
@@ -674,125 +635,25 @@ __device__ __forceinline__ void insert_sorted(int32_t *row, int64_t &m, int32_t 
     m++;
 }
 
-// EF(e): faces holding e, from the two faces of e in each cell of ET(e).
-// One pass builds each sorted, duplicate-free row in a padded slot of
-// 2|ET(e)| words (tmp + 2 et_off[e]; in an LDS column while it fits) and
-// counts it; k_ef_copy then packs the rows after the scan of the counts.
-constexpr int EF_CAP = 64;
-
-__global__ __launch_bounds__(ET_THREADS) void k_ef(const int64_t *__restrict__ et_off,
-                                                   int64_t E, const int32_t *__restrict__ et,
-                                                   const int32_t *__restrict__ te,
-                                                   const int32_t *__restrict__ tf,
-                                                   int64_t *__restrict__ cnt,
-                                                   int32_t *__restrict__ tmp) {
-    __shared__ int32_t col[EF_CAP][ET_THREADS];
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t b0 = et_off[e], b1 = et_off[e + 1];
-        const bool lds = 2 * (b1 - b0) <= EF_CAP;
-        int32_t *grow = tmp + 2 * b0;
-        int64_t m = 0;
-        // four cells at a time: their TE and TF rows are loaded together
-        // (unconditional loads from a clamped cell index)
-        for (int64_t i0 = b0; i0 < b1; i0 += 4) {
-            int32_t tc[4];
-            int2 r01[4], r23[4], r45[4];
-            int4 fr[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) tc[c] = et[min(i0 + c, b1 - 1)];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int2 *tr = reinterpret_cast<const int2 *>(te + 6 * (int64_t)tc[c]);
-                r01[c] = tr[0];
-                r23[c] = tr[1];
-                r45[c] = tr[2];
-                fr[c] = reinterpret_cast<const int4 *>(tf)[tc[c]];
-            }
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                if (i0 + c >= b1) break;
-                const int32_t ee = (int32_t)e;
-                const int k = r01[c].x == ee ? 0 : r01[c].y == ee ? 1 : r23[c].x == ee ? 2
-                            : r23[c].y == ee ? 3 : r45[c].x == ee ? 4 : r45[c].y == ee ? 5 : 6;
-                if (k == 6) continue;  // TE and ET disagree: no face of this cell
-                // corner pair of edge slot k; faces holding both corners
-                const int pi[6] = {0, 0, 0, 1, 1, 2}, pj[6] = {1, 2, 3, 2, 3, 3};
-                for (int s = 0; s < 4; s++) {
-                    int lo, mid, hi;
-                    face_pos(s, lo, mid, hi);
-                    const bool has_i = lo == pi[k] || mid == pi[k] || hi == pi[k];
-                    const bool has_j = lo == pj[k] || mid == pj[k] || hi == pj[k];
-                    if (!(has_i && has_j)) continue;
-                    const int32_t x = s == 0 ? fr[c].x : s == 1 ? fr[c].y : s == 2 ? fr[c].z : fr[c].w;
-                    if (lds) {  // insert into the ascending column unless present
-                        int64_t p = m;
-                        while (p > 0 && col[p - 1][threadIdx.x] > x) p--;
-                        if (p > 0 && col[p - 1][threadIdx.x] == x) continue;
-                        for (int64_t q = m; q > p; q--) col[q][threadIdx.x] = col[q - 1][threadIdx.x];
-                        col[p][threadIdx.x] = x;
-                        m++;
-                    } else {
-                        insert_sorted(grow, m, x);
-                    }
-                }
-            }
-        }
-        if (lds) {
-            QuadOutExact o;
-            o.row = grow;
-            for (int64_t q = 0; q < m; q++) o.put(col[q][threadIdx.x]);
-            o.flush();
-        }
-        cnt[e] = m;
-    }
-}
-
-// packed rows from the padded ones (off: exclusive scan of the counts)
-__global__ void k_ef_copy(const int64_t *__restrict__ et_off, int64_t E,
-                          const int64_t *__restrict__ off, const int32_t *__restrict__ tmp,
-                          int32_t *__restrict__ out) {
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        // 16-byte loads (the padded buffer carries four words of slack) and
-        // stores, the last one to three words one by one
-        const int32_t *src = tmp + 2 * et_off[e];
-        const int64_t o = off[e], n = off[e + 1] - o;
-        QuadOutExact w;
-        w.row = out + o;
-        for (int64_t q = 0; q < n; q += 4) {
-            const i32x4u v = *reinterpret_cast<const i32x4u *>(src + q);
-            w.put(v.x);
-            if (q + 1 < n) w.put(v.y);
-            if (q + 2 < n) w.put(v.z);
-            if (q + 3 < n) w.put(v.w);
-        }
-        w.flush();
-    }
-}
-
-// TT and EE merge columns (stage_quads): ROW_CAP words per thread.
-constexpr int ROW_THREADS = 64;
-constexpr int ROW_CAP = 100;  // 26 KB per 64 threads (with three spare slots): six waves per CU
-
-// ---- TT: union of the VT rows of a cell's corners, minus the cell -----------------
-// One lane per cell, one kernel: the four rows are loaded whole (16-byte
-// quads, independent) into registers, merged by a compile-time bitonic
-// network, and the distinct cells other than the lane's own counted; the
-// block's total joins a chained scan over tiles of TT_THREADS cells, which
-// gives every row its exact place; then the rows go through an LDS window per
-// wave to contiguous 16-byte stores.  A wave takes the smallest network that
-// holds its rows; a lane with a row beyond the largest one merges serially
-// from global memory.
+// ---- joins of a few short sorted rows: TT, ET and EE -------------------------------
+// TT(t): union of the VT rows of t's corners, minus t.  ET(e): intersection of
+// the VT rows of e's ends.  EE(e): union of its ends' edge-id rows, minus e.
+// One lane per output row, one kernel: the lane's rows are loaded whole
+// (16-byte quads, independent) into registers, merged by a compile-time
+// bitonic network, and what the join keeps is counted; the block's total joins
+// a chained scan over tiles of rows, which gives every row its exact place;
+// then the rows go through an LDS window per wave to contiguous 16-byte stores.
+// A wave takes the smallest network that holds its rows; a lane with a row
+// beyond the largest one merges serially from global memory.
 //
-// What bounds it: VALU issue of the network (560 compare-exchanges for rows of
-// up to 24) and the loads of 4 x 64 different rows per wave.  It replaced a
-// merge of LDS columns by one lane each (100 words a lane, six waves per CU,
-// waiting on dependent LDS reads; longer rows from global memory), which wrote
-// padded rows, scanned their lengths and packed them.
-constexpr int TT_THREADS = 256;
-constexpr int TT_WIN = 2240;  // words of a wave's output window: two windows for 64 x 69 words
-constexpr int TT_ROW = 48;    // longest row of the largest network
+// What bounds it: the gathers of NR x 64 different rows per wave (TT: 4 rows of
+// 96 bytes a cell, 2.0 M cells in random order 0.76 ms) and VALU issue of the
+// network (560 compare-exchanges for four rows of 24).  It replaced a merge of
+// LDS columns by one lane each (26-32 KB a wave, waiting on dependent LDS
+// reads; longer rows from global memory), which wrote padded rows, scanned
+// their lengths and packed them (TT 2.71 ms).
+constexpr int JOIN_ROW = 48;  // longest row of the largest network
+enum Join { UNION_LESS_SELF, INTERSECT };
 
 // Tiles' totals as they become known: bits 62-63 hold 0 (nothing yet), 1 (the
 // tile's own sum) or 2 (the sum of all tiles up to it).
@@ -819,28 +680,10 @@ __device__ __forceinline__ int64_t tiles_before(const uint64_t *state, int32_t t
     }
 }
 
-// Bitonic merge of k[B .. B + n), any n: the first part sorted against the
-// direction, the second along it (H. W. Lang's form for arbitrary n: compare
-// at the largest power of two below n, then both parts).
-constexpr int pow2_below(int n) { return n <= 2 ? 1 : 2 * pow2_below((n + 1) / 2); }
-template <int B, int n, bool UP, int N>
-__device__ __forceinline__ void bitonic_merge(int32_t (&k)[N]) {
-    if constexpr (n > 1) {
-        constexpr int m = pow2_below(n);
-#pragma unroll
-        for (int i = B; i < B + n - m; i++) {
-            const int32_t a = k[i], b = k[i + m];
-            k[i] = tgd::opaque(UP ? min(a, b) : max(a, b));
-            k[i + m] = tgd::opaque(UP ? max(a, b) : min(a, b));
-        }
-        bitonic_merge<B, m, UP>(k);
-        bitonic_merge<B + m, n - m, UP>(k);
-    }
-}
-
-// Row of n <= R corner codes as cells, INF after them; DOWN: in reverse.
-// Whole quads are read, up to three words past the row (vtc carries them).
-template <int B, int R, bool DOWN, int N>
+// Row of n <= R words, shifted right by SH, INF after them; DOWN: in reverse.
+// Whole quads are read, up to three words past the row (the source arrays
+// carry them).
+template <int B, int R, bool DOWN, int SH, int N>
 __device__ __forceinline__ void load_row(int32_t (&k)[N], const int32_t *__restrict__ src, int n) {
 #pragma unroll
     for (int i = 0; i < R; i += 4) {
@@ -848,75 +691,112 @@ __device__ __forceinline__ void load_row(int32_t (&k)[N], const int32_t *__restr
         if (i < n) q = *reinterpret_cast<const i32x4u *>(src + i);
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            k[B + (DOWN ? R - 1 - i - j : i + j)] = i + j < n ? q[j] >> 2 : INF;
+            k[B + (DOWN ? R - 1 - i - j : i + j)] = i + j < n ? q[j] >> SH : INF;
     }
 }
 
-struct TtRows {  // the lane's four VT rows
-    int32_t p[4], n[4];
+template <int NR>
+struct Rows {  // the lane's rows
+    int32_t p[NR], n[NR];
+    __device__ __forceinline__ int longest() const {
+        int m = 0;
+#pragma unroll
+        for (int c = 0; c < NR; c++) m = max(m, n[c]);
+        return m;
+    }
 };
 
-// Serial four-way merge from global memory: f(i, x) for the i-th distinct
-// cell x other than t, ascending; returns their number.
-template <typename F>
-__device__ __forceinline__ int32_t tt_serial(const int32_t *vtc, const TtRows &r, int32_t t, F f) {
-    int32_t i[4] = {0, 0, 0, 0}, h[4], m = 0;
+// Serial merge from global memory: f(i, x) for the i-th value x that the join
+// keeps, ascending; returns their number.
+template <int NR, Join J, int SH, typename F>
+__device__ __forceinline__ int32_t join_serial(const int32_t *src, const Rows<NR> &r, int32_t self,
+                                               F f) {
+    int32_t i[NR], h[NR], m = 0;
 #pragma unroll
-    for (int c = 0; c < 4; c++) h[c] = r.n[c] > 0 ? vtc[r.p[c]] >> 2 : INF;
+    for (int c = 0; c < NR; c++) {
+        i[c] = 0;
+        h[c] = r.n[c] > 0 ? src[r.p[c]] >> SH : INF;
+    }
     while (true) {
-        const int32_t x = min(min(h[0], h[1]), min(h[2], h[3]));
-        if (x == INF) return m;
+        int32_t x = h[0];
 #pragma unroll
-        for (int c = 0; c < 4; c++)
-            if (h[c] == x) h[c] = ++i[c] < r.n[c] ? vtc[r.p[c] + i[c]] >> 2 : INF;
-        if (x != t) f(m++, x);
+        for (int c = 1; c < NR; c++) x = min(x, h[c]);
+        if (x == INF) return m;
+        int in = 0;
+#pragma unroll
+        for (int c = 0; c < NR; c++)
+            if (h[c] == x) {
+                in++;
+                h[c] = ++i[c] < r.n[c] ? src[r.p[c] + i[c]] >> SH : INF;
+            }
+        if (J == INTERSECT ? in == NR : x != self) f(m++, x);
     }
 }
+
+// Block of one kernel: its threads and the words of a wave's output window.
+template <int THREADS, int WIN>
+struct JoinBlock {
+    int32_t win[THREADS / 64][WIN];
+    int32_t wtot[THREADS / 64];
+    int64_t base;
+    int32_t tile;
+};
 
 // One wave's share of a tile with a network for rows of up to R entries.
 // Contains two workgroup barriers; every wave of the block makes one call
 // (of some R), so all waves meet at both.
-template <int R>
-__device__ __forceinline__ void tt_wave(const int32_t *__restrict__ vtc, const TtRows &r, bool act,
-                                        int32_t t, int32_t last, int32_t tile, uint64_t *state,
-                                        int64_t *__restrict__ off, int32_t *__restrict__ out,
-                                        int32_t *win, int32_t (&wtot)[TT_THREADS / 64],
-                                        int64_t &tbase) {
-    constexpr int N = 4 * R;
+template <int NR, Join J, int SH, int R, int THREADS, int WIN>
+__device__ __forceinline__ void join_wave(JoinBlock<THREADS, WIN> &blk,
+                                          const int32_t *__restrict__ src, const Rows<NR> &r,
+                                          bool act, int32_t self, int64_t row, int64_t rows,
+                                          uint64_t *state, int64_t *__restrict__ off,
+                                          int32_t *__restrict__ out) {
+    static_assert(NR == 2 || NR == 4, "merge tree");
+    constexpr int N = NR * R;
     const int lane = __lane_id(), wid = threadIdx.x / 64;
+    const int32_t tile = blk.tile;
+    int32_t *win = blk.win[wid];
     int32_t k[N];
-    load_row<0, R, false>(k, vtc + r.p[0], r.n[0]);
-    load_row<R, R, true>(k, vtc + r.p[1], r.n[1]);
-    load_row<2 * R, R, true>(k, vtc + r.p[2], r.n[2]);
-    load_row<3 * R, R, false>(k, vtc + r.p[3], r.n[3]);
-    bitonic_merge<0, 2 * R, false>(k);
-    bitonic_merge<2 * R, 2 * R, true>(k);
-    bitonic_merge<0, N, true>(k);
-    const int nv = r.n[0] + r.n[1] + r.n[2] + r.n[3];
-    const bool serial = max(max(r.n[0], r.n[1]), max(r.n[2], r.n[3])) > TT_ROW;
-    int32_t m = 0;  // distinct values, less the cell itself and the padding
+    int nv = 0;
 #pragma unroll
-    for (int j = 1; j < N; j++) m += k[j] != k[j - 1];
-    m = act ? m - (nv < N) : 0;
-    if (serial) m = tt_serial(vtc, r, t, [](int32_t, int32_t) {});
+    for (int c = 0; c < NR; c++) nv += r.n[c];
+    if constexpr (NR == 4) {
+        load_row<0, R, false, SH>(k, src + r.p[0], r.n[0]);
+        load_row<R, R, true, SH>(k, src + r.p[1], r.n[1]);
+        load_row<2 * R, R, true, SH>(k, src + r.p[2], r.n[2]);
+        load_row<3 * R, R, false, SH>(k, src + r.p[3], r.n[3]);
+        tgn::bitonic_merge<0, 2 * R, false>(k);
+        tgn::bitonic_merge<2 * R, 2 * R, true>(k);
+    } else {
+        load_row<0, R, true, SH>(k, src + r.p[0], r.n[0]);
+        load_row<R, R, false, SH>(k, src + r.p[1], r.n[1]);
+    }
+    tgn::bitonic_merge<0, N, true>(k);
+    const bool serial = r.longest() > JOIN_ROW;
+    int32_t m = 0;  // distinct values, less the lane's own and the padding; or equal pairs
+#pragma unroll
+    for (int j = 1; j < N; j++) m += J == INTERSECT ? k[j] == k[j - 1] : k[j] != k[j - 1];
+    m -= J == INTERSECT ? max(N - nv - 1, 0) : (int)(nv < N);
+    if (!act) m = 0;
+    if (serial) m = join_serial<NR, J, SH>(src, r, self, [](int32_t, int32_t) {});
     const int32_t inc = tgd::wave_inclusive_sum(m);
-    if (lane == 63) wtot[wid] = inc;
+    if (lane == 63) blk.wtot[wid] = inc;
     __syncthreads();
     int32_t before = 0, total = 0;
 #pragma unroll
-    for (int i = 0; i < TT_THREADS / 64; i++) {
-        if (i < wid) before += wtot[i];
-        total += wtot[i];
+    for (int i = 0; i < THREADS / 64; i++) {
+        if (i < wid) before += blk.wtot[i];
+        total += blk.wtot[i];
     }
     if (threadIdx.x == 0) tgd::store_agent(state + tile, TILE_SUM | (uint64_t)total);
     const int32_t first = inc - m, wn = __shfl(inc, 63, 64);
     // the wave's rows, one window after the other; the first one is filled
     // while the tile's place is being found
-    for (int32_t w0 = 0;; w0 += TT_WIN) {
+    for (int32_t w0 = 0;; w0 += WIN) {
         int32_t pos = first - w0 - 1;
         if (serial) {
-            tt_serial(vtc, r, t, [&](int32_t i, int32_t x) {
-                if ((uint32_t)(first - w0 + i) < (uint32_t)TT_WIN) win[first - w0 + i] = x;
+            join_serial<NR, J, SH>(src, r, self, [&](int32_t i, int32_t x) {
+                if ((uint32_t)(first - w0 + i) < (uint32_t)WIN) win[first - w0 + i] = x;
             });
         } else {
             // compared afresh in every window: masks kept from the count
@@ -926,10 +806,10 @@ __device__ __forceinline__ void tt_wave(const int32_t *__restrict__ vtc, const T
 #pragma unroll
             for (int j = 0; j < N; j++) {
                 k[j] = tgd::opaque(k[j]);
-                const bool keep = k[j] != prev && k[j] != t && j < mv;
+                const bool keep = (J == INTERSECT ? k[j] == prev : k[j] != prev && k[j] != self) && j < mv;
                 prev = k[j];
                 pos += keep;
-                if (keep && (uint32_t)pos < (uint32_t)TT_WIN) win[pos] = k[j];
+                if (keep && (uint32_t)pos < (uint32_t)WIN) win[pos] = k[j];
             }
         }
         if (w0 == 0) {
@@ -937,42 +817,44 @@ __device__ __forceinline__ void tt_wave(const int32_t *__restrict__ vtc, const T
                 const int64_t b = tiles_before(state, tile);
                 if (lane == 0) {
                     tgd::store_agent(state + tile, TILE_PREFIX | (uint64_t)(b + total));
-                    tbase = b;
+                    blk.base = b;
                 }
             }
             __syncthreads();
-            if (act) off[t] = tbase + before + first;
-            if (t == last) off[t + 1] = tbase + total;
+            if (act) off[row] = blk.base + before + first;
+            if (row == rows - 1) off[rows] = blk.base + total;
         }
         tgd::wave_sync();  // the window is whole
-        int32_t *dst = out + (tbase + before + w0);
-        const int32_t cnt = min(wn - w0, TT_WIN);
+        int32_t *dst = out + (blk.base + before + w0);
+        const int32_t cnt = min(wn - w0, WIN);
         for (int32_t i = 4 * lane; i + 3 < cnt; i += 256)
             *reinterpret_cast<i32x4u *>(dst + i) = *reinterpret_cast<const i32x4u *>(win + i);
         const int32_t tail = cnt & ~3;
         if (cnt > 0 && tail + lane < cnt) dst[tail + lane] = win[tail + lane];
-        if (w0 + TT_WIN >= wn) return;
+        if (w0 + WIN >= wn) return;
         tgd::wave_sync();  // and has been read
     }
 }
 
-__global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const int4 *__restrict__ tv4, int64_t T,
-                                                   const int32_t *__restrict__ vt_off,
-                                                   const int32_t *__restrict__ vtc,
-                                                   int32_t *ticket, uint64_t *state,
-                                                   int64_t *__restrict__ off,
-                                                   int32_t *__restrict__ out) {
-    __shared__ __align__(16) int32_t win[TT_THREADS / 64][TT_WIN];
-    __shared__ int32_t wtot[TT_THREADS / 64];
-    __shared__ int64_t tbase;
-    __shared__ int32_t next;
-    if (threadIdx.x == 0) next = atomicAdd(ticket, 1);
+// This block's tile number, handed out in the order blocks start.
+__device__ __forceinline__ int32_t take_tile(int32_t *ticket, int32_t &shared) {
+    if (threadIdx.x == 0) shared = atomicAdd(ticket, 1);
     __syncthreads();
-    const int32_t tile = next;
-    const int64_t t = (int64_t)tile * TT_THREADS + threadIdx.x;
+    return shared;
+}
+
+// Windows: two for 64 x 69 words.
+constexpr int TT_THREADS = 256, TT_WIN = 2240;
+__global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const int4 *__restrict__ tv4, int64_t T,
+                                                      const int32_t *__restrict__ vt_off,
+                                                      const int32_t *__restrict__ vtc,
+                                                      int32_t *ticket, uint64_t *state,
+                                                      int64_t *__restrict__ off,
+                                                      int32_t *__restrict__ out) {
+    __shared__ __align__(16) JoinBlock<TT_THREADS, TT_WIN> blk;
+    const int64_t t = (int64_t)take_tile(ticket, blk.tile) * TT_THREADS + threadIdx.x;
     const bool act = t < T;
-    const int32_t last = (int32_t)(T - 1);
-    TtRows r;
+    Rows<4> r;
     const int4 q = act ? tv4[t] : make_int4(0, 0, 0, 0);
 #pragma unroll
     for (int c = 0; c < 4; c++) {
@@ -980,13 +862,145 @@ __global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const int4 *__restrict__ t
         r.p[c] = o.x;
         r.n[c] = act ? o.y - o.x : 0;
     }
-    int32_t *w = win[threadIdx.x / 64];
-    const int longest = max(max(r.n[0], r.n[1]), max(r.n[2], r.n[3]));
-    const int need = longest > TT_ROW ? 0 : longest;  // serial lanes need no network
-    if (__any(need > 40)) tt_wave<TT_ROW>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
-    else if (__any(need > 32)) tt_wave<40>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
-    else if (__any(need > 24)) tt_wave<32>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
-    else tt_wave<24>(vtc, r, act, (int32_t)t, last, tile, state, off, out, w, wtot, tbase);
+    const int need = r.longest() > JOIN_ROW ? 0 : r.longest();  // serial lanes need no network
+#define TG_JOIN(R) join_wave<4, UNION_LESS_SELF, 2, R>(blk, vtc, r, act, (int32_t)t, t, T, state, off, out)
+    if (__any(need > 40)) TG_JOIN(JOIN_ROW);
+    else if (__any(need > 32)) TG_JOIN(40);
+    else if (__any(need > 24)) TG_JOIN(32);
+    else TG_JOIN(24);
+#undef TG_JOIN
+}
+
+// ET and EE: the rows of edge e's two ends in src (corner codes by vt_off, or
+// edge ids by vv_off).  512 edges a tile: tile numbers cost 10 ns each.
+// Windows: one for ET (64 x 5 words), one for EE (64 x 26).
+constexpr int EJ_THREADS = 512;
+template <Join J, int SH, int WIN>
+__global__ __launch_bounds__(EJ_THREADS, 4) void k_edge_join(const int32_t *__restrict__ ev, int64_t E,
+                                                             int64_t V,
+                                                             const int32_t *__restrict__ row_off,
+                                                             const int32_t *__restrict__ src,
+                                                             int32_t *ticket, uint64_t *state,
+                                                             int64_t *__restrict__ off,
+                                                             int32_t *__restrict__ out) {
+    __shared__ __align__(16) JoinBlock<EJ_THREADS, WIN> blk;
+    const int64_t e = (int64_t)take_tile(ticket, blk.tile) * EJ_THREADS + threadIdx.x;
+    const bool act = e < E;
+    Rows<2> r;
+    const int2 ends = act ? reinterpret_cast<const int2 *>(ev)[e] : make_int2(0, 0);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int32_t v = c ? ends.y : ends.x;
+        const bool ok = v >= 0 && v < V;  // always, for a built EV
+        const i32x2u o = *reinterpret_cast<const i32x2u *>(row_off + (ok ? v : 0));
+        r.p[c] = o.x;
+        r.n[c] = act && ok ? o.y - o.x : 0;
+    }
+    const int need = r.longest() > JOIN_ROW ? 0 : r.longest();  // serial lanes need no network
+#define TG_JOIN(R) join_wave<2, J, SH, R>(blk, src, r, act, (int32_t)e, e, E, state, off, out)
+    if (__any(need > 32)) TG_JOIN(JOIN_ROW);
+    else if (__any(need > 24)) TG_JOIN(32);
+    else if (__any(need > 16)) TG_JOIN(24);
+    else TG_JOIN(16);
+#undef TG_JOIN
+}
+constexpr int ET_WIN = 448, EE_WIN = 1728;
+
+// EF(e): faces holding e, from the two faces of e in each cell of ET(e).  One
+// lane per edge builds its sorted, duplicate-free row in an LDS column (in a
+// padded slot of 2|ET(e)| words of tmp while the column is too short), the
+// block's total joins the chained scan, and the row goes to its place.  Bound
+// by the gathers of two rows (TE, TF) per cell of ET.
+constexpr int EF_THREADS = 256, EF_CAP = 32;  // 32 KB a block
+
+__global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ et_off,
+                                                   int64_t E, const int32_t *__restrict__ et,
+                                                   const int32_t *__restrict__ te,
+                                                   const int32_t *__restrict__ tf,
+                                                   int32_t *ticket, uint64_t *state,
+                                                   int64_t *__restrict__ off,
+                                                   int32_t *__restrict__ out,
+                                                   int32_t *__restrict__ tmp) {
+    __shared__ int32_t col[EF_CAP][EF_THREADS];
+    __shared__ int32_t wtot[EF_THREADS / 64];
+    __shared__ int32_t shared_tile;
+    __shared__ int64_t base;
+    const int tid = threadIdx.x, lane = __lane_id(), wid = tid / 64;
+    const int32_t tile = take_tile(ticket, shared_tile);
+    const int64_t e = (int64_t)tile * EF_THREADS + tid;
+    const bool act = e < E;
+    const int64_t b0 = act ? et_off[e] : 0, b1 = act ? et_off[e + 1] : 0;
+    const bool lds = 2 * (b1 - b0) <= EF_CAP;
+    int32_t *grow = tmp + 2 * b0;
+    int64_t m = 0;
+    // four cells at a time: their TE and TF rows are loaded together
+    // (unconditional loads from a clamped cell index)
+    for (int64_t i0 = b0; i0 < b1; i0 += 4) {
+        int32_t tc[4];
+        int2 r01[4], r23[4], r45[4];
+        int4 fr[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) tc[c] = et[min(i0 + c, b1 - 1)];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const int2 *tr = reinterpret_cast<const int2 *>(te + 6 * (int64_t)tc[c]);
+            r01[c] = tr[0];
+            r23[c] = tr[1];
+            r45[c] = tr[2];
+            fr[c] = reinterpret_cast<const int4 *>(tf)[tc[c]];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (i0 + c >= b1) break;
+            const int32_t ee = (int32_t)e;
+            const int k = r01[c].x == ee ? 0 : r01[c].y == ee ? 1 : r23[c].x == ee ? 2
+                        : r23[c].y == ee ? 3 : r45[c].x == ee ? 4 : r45[c].y == ee ? 5 : 6;
+            if (k == 6) continue;  // TE and ET disagree: no face of this cell
+            // the two face slots holding both corners of edge slot k
+            const int s0[6] = {0, 0, 1, 0, 1, 2}, s1[6] = {1, 2, 2, 3, 3, 3};
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int s = h ? s1[k] : s0[k];
+                const int32_t x = s == 0 ? fr[c].x : s == 1 ? fr[c].y : s == 2 ? fr[c].z : fr[c].w;
+                if (lds) {  // insert into the ascending column unless present
+                    int p = (int)m;
+                    while (p > 0 && col[p - 1][tid] > x) p--;
+                    if (p > 0 && col[p - 1][tid] == x) continue;
+                    for (int q = (int)m; q > p; q--) col[q][tid] = col[q - 1][tid];
+                    col[p][tid] = x;
+                    m++;
+                } else {
+                    insert_sorted(grow, m, x);
+                }
+            }
+        }
+    }
+    const int32_t inc = tgd::wave_inclusive_sum((int32_t)m);
+    if (lane == 63) wtot[wid] = inc;
+    __syncthreads();
+    int32_t before = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < EF_THREADS / 64; i++) {
+        if (i < wid) before += wtot[i];
+        total += wtot[i];
+    }
+    if (wid == 0) {
+        if (lane == 0) tgd::store_agent(state + tile, TILE_SUM | (uint64_t)total);
+        const int64_t b = tiles_before(state, tile);
+        if (lane == 0) {
+            tgd::store_agent(state + tile, TILE_PREFIX | (uint64_t)(b + total));
+            base = b;
+        }
+    }
+    __syncthreads();
+    if (!act) return;
+    QuadOutExact o;
+    const int64_t at = base + before + inc - m;
+    o.row = out + at;
+    for (int64_t q = 0; q < m; q++) o.put(lds ? col[q][tid] : grow[q]);
+    o.flush();
+    off[e] = at;
+    if (e == E - 1) off[E] = base + total;
 }
 
 // Sum of squared row lengths (VT: the lengths of all cells' four rows
@@ -1011,132 +1025,62 @@ __global__ __launch_bounds__(SQ_THREADS) void k_row_squares(const int32_t *__res
     }
 }
 
-// Pack padded rows: row r of length off[r+1] - off[r] moves from src +
-// pad[r] to dst + off[r].  A block takes 256 consecutive rows and copies its
-// contiguous output range element by element (a row found by bisection of
-// the block's row starts in LDS), so reads and writes are coalesced.
-__global__ __launch_bounds__(256) void k_pack_rows(const int64_t *__restrict__ pad,
-                                                   const int64_t *__restrict__ off, int64_t rows,
-                                                   const int32_t *__restrict__ src,
-                                                   int32_t *__restrict__ dst) {
-    __shared__ int64_t s_off[257], s_pad[256];
-    const int64_t r0 = (int64_t)blockIdx.x * 256;
-    const int nr = (int)min<int64_t>(256, rows - r0);
-    for (int i = threadIdx.x; i <= nr; i += 256) {
-        s_off[i] = off[r0 + i];
-        if (i < nr) s_pad[i] = pad[r0 + i];
+// FF(f): faces of the (at most two) cells holding f, minus f.  One lane per
+// face: both TF rows are loaded at once, the six candidates sorted by a
+// network and the distinct ones written at the place that the chained scan
+// gives.
+constexpr int FF_THREADS = 512;
+__global__ __launch_bounds__(FF_THREADS) void k_ff(const int32_t *__restrict__ ft, int64_t F,
+                                                   const int32_t *__restrict__ tf,
+                                                   int32_t *ticket, uint64_t *state,
+                                                   int64_t *__restrict__ off,
+                                                   int32_t *__restrict__ out) {
+    __shared__ int32_t rows[FF_THREADS * 6];
+    __shared__ int32_t wtot[FF_THREADS / 64];
+    __shared__ int32_t shared_tile;
+    __shared__ int64_t base;
+    const int tid = threadIdx.x, lane = __lane_id(), wid = tid / 64;
+    const int32_t tile = take_tile(ticket, shared_tile);
+    const int64_t f = (int64_t)tile * FF_THREADS + tid;
+    const bool act = f < F;
+    const int2 cells = act ? reinterpret_cast<const int2 *>(ft)[f] : make_int2(-1, -1);
+    const int4 r0 = reinterpret_cast<const int4 *>(tf)[cells.x >= 0 ? cells.x : 0];
+    const int4 r1 = reinterpret_cast<const int4 *>(tf)[cells.y >= 0 ? cells.y : 0];
+    int32_t c[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const bool on = i < 4 ? cells.x >= 0 : cells.y >= 0;
+        if (!on || c[i] == (int32_t)f) c[i] = INF;
+    }
+    tgn::sort_keys(c);
+    int m = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) m += c[i] != INF && (i == 0 || c[i] != c[i > 0 ? i - 1 : 0]);
+    const int32_t inc = tgd::wave_inclusive_sum(m);
+    if (lane == 63) wtot[wid] = inc;
+    __syncthreads();
+    int32_t before = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < FF_THREADS / 64; i++) {
+        if (i < wid) before += wtot[i];
+        total += wtot[i];
+    }
+    if (tid == 0) tgd::store_agent(state + tile, TILE_SUM | (uint64_t)total);
+    int p = before + inc - m;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        if (c[i] != INF && (i == 0 || c[i] != c[i > 0 ? i - 1 : 0])) rows[p++] = c[i];
+    if (wid == 0) {
+        const int64_t b = tiles_before(state, tile);
+        if (lane == 0) {
+            tgd::store_agent(state + tile, TILE_PREFIX | (uint64_t)(b + total));
+            base = b;
+        }
     }
     __syncthreads();
-    const int64_t ob = s_off[0], oe = s_off[nr];
-    for (int64_t o = ob + threadIdx.x; o < oe; o += 256) {
-        int lo = 0, hi = nr - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (s_off[mid] <= o) lo = mid;
-            else hi = mid - 1;
-        }
-        dst[o] = src[s_pad[lo] + (o - s_off[lo])];
-    }
-}
-
-// FF(f): faces of the cells holding f, minus f
-template <bool FILL>
-__global__ void k_ff(const int32_t *__restrict__ ft, int64_t F, const int32_t *__restrict__ tf,
-                     int64_t *__restrict__ cnt_or_off, int32_t *__restrict__ out) {
-    for (int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; f < F;
-         f += (int64_t)gridDim.x * blockDim.x) {
-        // the faces of f's (at most two) cells other than f: both TF rows are
-        // loaded at once, the six candidates sorted by a network, then the
-        // distinct ones counted or written in order
-        const int2 cells = reinterpret_cast<const int2 *>(ft)[f];
-        const int4 r0 = reinterpret_cast<const int4 *>(tf)[cells.x >= 0 ? cells.x : 0];
-        const int4 r1 = reinterpret_cast<const int4 *>(tf)[cells.y >= 0 ? cells.y : 0];
-        const int32_t me = (int32_t)f;
-        int32_t c[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const bool on = i < 4 ? cells.x >= 0 : cells.y >= 0;
-            if (!on || c[i] == me) c[i] = INT32_MAX;
-        }
-        // bitonic network over eight registers (ascending)
-#pragma unroll
-        for (int k = 2; k <= 8; k <<= 1)
-#pragma unroll
-            for (int j = k >> 1; j > 0; j >>= 1)
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const int l = i ^ j;
-                    if (l > i) {
-                        const int32_t a = c[i], b = c[l];
-                        const bool up = (i & k) == 0;
-                        c[i] = up ? min(a, b) : max(a, b);
-                        c[l] = up ? max(a, b) : min(a, b);
-                    }
-                }
-        int64_t o = FILL ? cnt_or_off[f] : 0;
-        int n = 0;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const bool keep = c[i] != INT32_MAX && (i == 0 || c[i] != c[i - 1]);
-            if (FILL && keep) out[o + n] = c[i];
-            n += keep;
-        }
-        if (!FILL) cnt_or_off[f] = n;
-    }
-}
-
-// EE(e): edges at lo or hi, minus e, ascending: merge of the two vertices'
-// edge-id lists (vv_eid rows sorted by id, in eids).  The lists share only
-// e itself, so the row length is deg(lo) + deg(hi) - 2.
-__global__ __launch_bounds__(ROW_THREADS) void k_ee(const int32_t *__restrict__ ev, int64_t E,
-                                                    const int32_t *__restrict__ vv_off,
-                                                    const int32_t *__restrict__ eids,
-                                                    const int64_t *__restrict__ off,
-                                                    int32_t *__restrict__ out) {
-    __shared__ int32_t buf[ROW_CAP + 3][ROW_THREADS];  // three spare slots for stage_quads
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t a = ev[2 * e], b = ev[2 * e + 1];
-        int32_t i = vv_off[a], ie = vv_off[a + 1], j = vv_off[b], je = vv_off[b + 1];
-        QuadOutExact o;
-        o.row = out + off[e];
-        const int32_t na = ie - i, nb = je - j;
-        if (na + nb <= ROW_CAP) {
-            stage_quads(buf, 0, eids + i, na, 0);
-            stage_quads(buf, na, eids + j, nb, 0);
-            i = 0, ie = na, j = na, je = na + nb;
-            int32_t x = i < ie ? buf[i][threadIdx.x] : INF, y = j < je ? buf[j][threadIdx.x] : INF;
-            const int32_t last = max(je - 1, 0);
-            while (x != INF || y != INF) {  // branch-free advance (two reads per step)
-                const int32_t mn = min(x, y);
-                i += x == mn;
-                j += y == mn;
-                const int32_t xa = buf[min(i, last)][threadIdx.x], yb = buf[min(j, last)][threadIdx.x];
-                x = i < ie ? xa : INF;
-                y = j < je ? yb : INF;
-                if (mn != (int32_t)e) o.put(mn);
-            }
-        } else {
-            int32_t x = i < ie ? eids[i] : INF, y = j < je ? eids[j] : INF;
-            while (x != INF || y != INF) {
-                const int32_t mn = min(x, y);
-                if (x == mn) x = ++i < ie ? eids[i] : INF;
-                if (y == mn) y = ++j < je ? eids[j] : INF;
-                if (mn != (int32_t)e) o.put(mn);
-            }
-        }
-        o.flush();
-    }
-}
-
-// row lengths of EE: deg(lo) + deg(hi) - 2
-__global__ void k_ee_count(const int32_t *__restrict__ ev, int64_t E,
-                           const int32_t *__restrict__ vv_off, int64_t *__restrict__ cnt) {
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t a = ev[2 * e], b = ev[2 * e + 1];
-        cnt[e] = (int64_t)(vv_off[a + 1] - vv_off[a]) + (vv_off[b + 1] - vv_off[b]) - 2;
-    }
+    if (act) off[f] = base + before + inc - m;
+    if (f == F - 1) off[F] = base + total;
+    for (int32_t i = tid; i < total; i += FF_THREADS) out[base + i] = rows[i];
 }
 
 __global__ void k_fill_i32v(int32_t *p, int32_t v, int64_t n) {
@@ -1178,35 +1122,57 @@ int read_i64(tg_mesh &m, const void *src, int64_t index, int64_t &out) {
     return tg::OK;
 }
 
-// rank structure over n flags: bits + exclusive prefix of word popcounts
-int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, int32_t *&bits, int32_t *&wpre,
-                int64_t &total) {
+// rank structure over n flags (0 or 1): rank_of(rank, p) is the number of
+// flags set before position p
+int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank, int64_t &total) {
     const int64_t nw = (n + 31) / 32;
     int rc;
     if ((rc = m.bitmap.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(nw, 1))) ||
         (rc = m.rank_tmp.ensure(sizeof(int32_t) * (size_t)(nw + 1))) ||
+        (rc = rank.ensure(sizeof(uint2) * (size_t)std::max<int64_t>(nw, 1))) ||
         (rc = m.scan_tmp.ensure(tg::scan_tmp_bytes(nw))))
         return rc;
-    bits = m.bitmap.as<int32_t>();
-    wpre = m.rank_tmp.as<int32_t>();
+    uint32_t *bits = m.bitmap.as<uint32_t>();
+    int32_t *wpre = m.rank_tmp.as<int32_t>();
     if (nw > 0) {
-        hipLaunchKernelGGL(k_pack_flags, dim3(grid(nw)), dim3(256), 0, m.stream, flags, n,
-                           (uint32_t *)bits, wpre);
+        hipLaunchKernelGGL(k_pack_flags, dim3(grid(nw)), dim3(256), 0, m.stream, flags, n, bits,
+                           wpre);
         TG_LAUNCH_CHECK("k_pack_flags");
     }
     if ((rc = tg::scan_exclusive_i32(wpre, wpre, nw, m.scan_tmp.p, m.stream))) return rc;
+    if (nw > 0) {
+        hipLaunchKernelGGL(k_rank_words, dim3(grid(nw)), dim3(256), 0, m.stream, bits, wpre, nw,
+                           rank.as<uint2>());
+        TG_LAUNCH_CHECK("k_rank_words");
+    }
     int32_t t32 = 0;
     if ((rc = read_i32(m, wpre, nw, t32))) return rc;
     total = t32;
     return tg::OK;
 }
 
-// count -> exclusive scan (int64) -> offsets; returns nnz
-int scan_counts64(tg_mesh &m, int64_t *cnt_off, int64_t n, int64_t &nnz) {
-    int rc = m.scan_tmp.ensure(tg::scan_tmp_bytes(n));
+// Zeroed state of a chained scan over `tiles` tiles, in tmp_b: a sum, the tile
+// counter, the tiles' sums.
+struct Chain {
+    int64_t *sum;
+    int32_t *ticket;
+    uint64_t *state;
+};
+int chain_state(tg_mesh &m, int64_t tiles, Chain &c) {
+    int rc = m.tmp_b.ensure(sizeof(int64_t) * (size_t)(tiles + 2));
     if (rc) return rc;
-    if ((rc = tg::scan_exclusive_i64(cnt_off, cnt_off, n, m.scan_tmp.p, m.stream))) return rc;
-    return read_i64(m, cnt_off, n, nnz);
+    c.sum = m.tmp_b.as<int64_t>();
+    c.ticket = reinterpret_cast<int32_t *>(c.sum + 1);
+    c.state = reinterpret_cast<uint64_t *>(c.sum + 2);
+    return tg::fill_i32((int32_t *)c.sum, 0, 2 * (tiles + 2), m.stream);
+}
+
+// Sum of squared row lengths, read back (synchronises).
+int row_squares(tg_mesh &m, const int32_t *row_off, int64_t rows, const Chain &c, int64_t &sum) {
+    hipLaunchKernelGGL(k_row_squares, dim3(std::min(grid(rows, SQ_THREADS), (unsigned)SQ_BLOCKS)),
+                       dim3(SQ_THREADS), 0, m.stream, row_off, rows, (unsigned long long *)c.sum);
+    TG_LAUNCH_CHECK("k_row_squares");
+    return read_i64(m, c.sum, 0, sum);
 }
 
 }  // namespace
@@ -1239,9 +1205,8 @@ int ensure_edges(tg_mesh &m) {
                            m.edge_first.as<int32_t>(), flags, m.te.as<int32_t>());
         TG_LAUNCH_CHECK("k_edge_first");
     }
-    int32_t *bits, *wpre;
     int64_t E = 0;
-    if ((rc = build_ranks(m, flags, 6 * T, bits, wpre, E))) return rc;
+    if ((rc = build_ranks(m, flags, 6 * T, m.edge_rank, E))) return rc;
     m.n_edges = E;
     if ((rc = m.ev.ensure(I * 2 * (size_t)std::max<int64_t>(E, 1))) ||
         (rc = m.ve_vals.ensure(I * 2 * (size_t)std::max<int64_t>(E, 1))))
@@ -1256,21 +1221,17 @@ int ensure_edges(tg_mesh &m) {
     if (V > 0) {
         hipLaunchKernelGGL(k_edge_ids, dim3(grid(V)), dim3(256), 0, m.stream,
                            m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
-                           m.edge_first.as<int32_t>(), (const uint32_t *)bits, wpre,
+                           m.edge_first.as<int32_t>(), m.edge_rank.as<uint2>(),
                            m.vv_eid.as<int32_t>(), m.ev.as<int32_t>());
         TG_LAUNCH_CHECK("k_edge_ids");
         hipLaunchKernelGGL(k_ve_fill, dim3(grid(V, VE_THREADS)), dim3(VE_THREADS), 0, m.stream,
                            m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(),
                            m.vv_eid.as<int32_t>(), V, voff, m.ve_vals.as<int32_t>());
         TG_LAUNCH_CHECK("k_ve_fill");
-        hipLaunchKernelGGL(k_edge_lower, dim3(grid(V)), dim3(256), 0, m.stream,
-                           m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
-                           m.vv_eid.as<int32_t>());
-        TG_LAUNCH_CHECK("k_edge_lower");
     }
     if (T > 0) {
         hipLaunchKernelGGL(k_te, dim3(grid(6 * T)), dim3(256), 0, m.stream, m.te.as<int32_t>(),
-                           6 * T, m.vv_eid.as<int32_t>());
+                           6 * T, m.edge_rank.as<uint2>());
         TG_LAUNCH_CHECK("k_te");
     }
     m.edges_built = true;
@@ -1283,31 +1244,22 @@ int ensure_et(tg_mesh &m) {
     // the vertex-lane VV form rewrites the corner lists unsorted: sort again
     if ((rc = ensure_edges(m)) || (rc = ensure_vt_sorted(m))) return rc;
     const int64_t E = m.n_edges;
+    const int64_t nnz = 6 * m.n_cells;  // each cell holds six edges
+    const int64_t tiles = (E + EJ_THREADS - 1) / EJ_THREADS;
+    Chain c;
     if ((rc = m.et_off.ensure(sizeof(int64_t) * (size_t)(E + 1))) ||
-        (rc = m.tmp_b.ensure(sizeof(int64_t) * (size_t)(E + 1))))
+        (rc = m.et_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1))) ||
+        (rc = chain_state(m, tiles, c)))
         return rc;
-    int64_t *off = m.et_off.as<int64_t>(), *pad = m.tmp_b.as<int64_t>();
+    int64_t *off = m.et_off.as<int64_t>();
     if (E > 0) {
-        hipLaunchKernelGGL(k_et_bound, dim3(grid(E)), dim3(256), 0, m.stream, m.ev.as<int32_t>(),
-                           E, m.n_points, m.vt_off.as<int32_t>(), pad);
-        TG_LAUNCH_CHECK("k_et_bound");
-    }
-    int64_t padded = 0;
-    if ((rc = scan_counts64(m, pad, E, padded))) return rc;
-    if ((rc = m.tmp_c.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(padded, 1)))) return rc;
-    if (E > 0) {
-        hipLaunchKernelGGL(k_et, dim3(grid(E, ET_THREADS)), dim3(ET_THREADS), 0, m.stream,
-                           m.ev.as<int32_t>(), E, m.n_points, m.vt_off.as<int32_t>(),
-                           m.vtc.as<int32_t>(), pad, off, m.tmp_c.as<int32_t>());
-        TG_LAUNCH_CHECK("k_et");
-    }
-    int64_t nnz = 0;
-    if ((rc = scan_counts64(m, off, E, nnz))) return rc;
-    if ((rc = m.et_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)))) return rc;
-    if (E > 0) {
-        hipLaunchKernelGGL(k_pack_rows, dim3((unsigned)((E + 255) / 256)), dim3(256), 0,
-                           m.stream, pad, off, E, m.tmp_c.as<int32_t>(), m.et_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_pack_rows");
+        hipLaunchKernelGGL((k_edge_join<INTERSECT, 2, ET_WIN>), dim3((unsigned)tiles),
+                           dim3(EJ_THREADS), 0, m.stream, m.ev.as<int32_t>(), E, m.n_points,
+                           m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(), c.ticket, c.state, off,
+                           m.et_vals.as<int32_t>());
+        TG_LAUNCH_CHECK("k_edge_join<ET>");
+    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
+        return rc;
     }
     m.et_built = true;
     return OK;
@@ -1337,9 +1289,8 @@ int ensure_faces(tg_mesh &m) {
                            iderr, err);
         TG_LAUNCH_CHECK("k_face_first");
     }
-    int32_t *bits, *wpre;
     int64_t F = 0;
-    if ((rc = build_ranks(m, flags, 4 * T, bits, wpre, F))) return rc;
+    if ((rc = build_ranks(m, flags, 4 * T, m.face_rank, F))) return rc;
     m.n_faces = F;
     if ((rc = m.fv.ensure(I * 3 * (size_t)std::max<int64_t>(F, 1))) ||
         (rc = m.ft.ensure(I * 2 * (size_t)std::max<int64_t>(F, 1))) ||
@@ -1347,7 +1298,7 @@ int ensure_faces(tg_mesh &m) {
         return rc;
     if (T > 0) {
         hipLaunchKernelGGL(k_face_ids, dim3(grid(4 * T)), dim3(256), 0, m.stream,
-                           m.tv.as<const int4>(), T, ffirst, other, (const uint32_t *)bits, wpre,
+                           m.tv.as<const int4>(), T, ffirst, other, m.face_rank.as<uint2>(),
                            m.tf.as<int32_t>(), m.fv.as<int32_t>(), m.ft.as<int32_t>());
         TG_LAUNCH_CHECK("k_face_ids");
     }
@@ -1370,6 +1321,7 @@ int ensure_faces(tg_mesh &m) {
                            ffirst, m.tf.as<int32_t>(), voff, m.vf_vals.as<int32_t>());
         TG_LAUNCH_CHECK("k_vf fill");
     }
+    m.face_rank.release();
     m.faces_built = true;
     return OK;
 }
@@ -1402,26 +1354,23 @@ int ensure_ef(tg_mesh &m) {
     int rc;
     if ((rc = ensure_et(m)) || (rc = ensure_faces(m))) return rc;
     const int64_t E = m.n_edges;
-    int64_t et_nnz = 0;
-    if ((rc = read_i64(m, m.et_off.p, E, et_nnz))) return rc;
+    const int64_t tiles = (E + EF_THREADS - 1) / EF_THREADS;
+    const int64_t et_nnz = 6 * m.n_cells, nnz = 3 * m.n_faces;  // a face holds three edges
+    Chain c;
     if ((rc = m.ef_off.ensure(sizeof(int64_t) * (size_t)(E + 1))) ||
-        (rc = m.tmp_c.ensure(sizeof(int32_t) * (2 * (size_t)std::max<int64_t>(et_nnz, 1) + 4))))
+        (rc = m.ef_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1))) ||
+        (rc = m.tmp_c.ensure(sizeof(int32_t) * 2 * (size_t)std::max<int64_t>(et_nnz, 1))) ||
+        (rc = chain_state(m, tiles, c)))
         return rc;
     int64_t *off = m.ef_off.as<int64_t>();
     if (E > 0) {
-        hipLaunchKernelGGL(k_ef, dim3(grid(E, ET_THREADS)), dim3(ET_THREADS), 0, m.stream,
-                           m.et_off.as<int64_t>(), E, m.et_vals.as<int32_t>(),
-                           m.te.as<int32_t>(), m.tf.as<int32_t>(), off, m.tmp_c.as<int32_t>());
+        hipLaunchKernelGGL(k_ef, dim3((unsigned)tiles), dim3(EF_THREADS), 0, m.stream,
+                           m.et_off.as<int64_t>(), E, m.et_vals.as<int32_t>(), m.te.as<int32_t>(),
+                           m.tf.as<int32_t>(), c.ticket, c.state, off, m.ef_vals.as<int32_t>(),
+                           m.tmp_c.as<int32_t>());
         TG_LAUNCH_CHECK("k_ef");
-    }
-    int64_t nnz = 0;
-    if ((rc = scan_counts64(m, off, E, nnz))) return rc;
-    if ((rc = m.ef_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)))) return rc;
-    if (E > 0) {
-        hipLaunchKernelGGL(k_ef_copy, dim3(grid(E)), dim3(256), 0, m.stream,
-                           m.et_off.as<int64_t>(), E, off, m.tmp_c.as<int32_t>(),
-                           m.ef_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_ef_copy");
+    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
+        return rc;
     }
     m.ef_nnz = nnz;
     m.ef_built = true;
@@ -1434,33 +1383,24 @@ int ensure_tt(tg_mesh &m) {
     if ((rc = ensure_vt_sorted(m))) return rc;
     const int64_t T = m.n_cells, V = m.n_points;
     const int64_t tiles = (T + TT_THREADS - 1) / TT_THREADS;
-    // tmp_b: sum of the rows' lengths, tile counter, tile sums
-    if ((rc = m.tt_off.ensure(sizeof(int64_t) * (size_t)(T + 1))) ||
-        (rc = m.tmp_b.ensure(sizeof(int64_t) * (size_t)(tiles + 2))))
+    Chain c;
+    if ((rc = m.tt_off.ensure(sizeof(int64_t) * (size_t)(T + 1))) || (rc = chain_state(m, tiles, c)))
         return rc;
-    int64_t *off = m.tt_off.as<int64_t>(), *words = m.tmp_b.as<int64_t>();
-    int32_t *ticket = reinterpret_cast<int32_t *>(words + 1);
-    uint64_t *state = reinterpret_cast<uint64_t *>(words + 2);
-    if (T == 0) {
-        if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) return rc;
-    } else {
-        if ((rc = fill_i32((int32_t *)words, 0, 2 * (tiles + 2), m.stream))) return rc;
-        hipLaunchKernelGGL(k_row_squares, dim3(std::min(grid(V, SQ_THREADS), (unsigned)SQ_BLOCKS)),
-                           dim3(SQ_THREADS), 0, m.stream, m.vt_off.as<int32_t>(), V,
-                           (unsigned long long *)words);
-        TG_LAUNCH_CHECK("k_row_squares");
-    }
+    int64_t *off = m.tt_off.as<int64_t>();
     int64_t rows = 0, nnz = 0;
-    if (T > 0 && (rc = read_i64(m, words, 0, rows))) return rc;
+    // the cells' rows together: every vertex's row once per entry
+    if (T > 0 && (rc = row_squares(m, m.vt_off.as<int32_t>(), V, c, rows))) return rc;
     // a cell's four rows hold the cell itself four times
     if ((rc = m.tt_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(rows - 4 * T, 1))))
         return rc;
     if (T > 0) {
         hipLaunchKernelGGL(k_tt, dim3((unsigned)tiles), dim3(TT_THREADS), 0, m.stream,
                            m.tv.as<const int4>(), T, m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(),
-                           ticket, state, off, m.tt_vals.as<int32_t>());
+                           c.ticket, c.state, off, m.tt_vals.as<int32_t>());
         TG_LAUNCH_CHECK("k_tt");
         if ((rc = read_i64(m, off, T, nnz))) return rc;
+    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
+        return rc;
     }
     m.tt_nnz = nnz;
     m.tt_built = true;
@@ -1472,20 +1412,23 @@ int ensure_ff(tg_mesh &m) {
     int rc;
     if ((rc = ensure_ft(m))) return rc;
     const int64_t F = m.n_faces;
-    if ((rc = m.ff_off.ensure(sizeof(int64_t) * (size_t)(F + 1)))) return rc;
+    const int64_t tiles = (F + FF_THREADS - 1) / FF_THREADS;
+    Chain c;
+    // a cell gives each of its four faces at most the three others
+    if ((rc = m.ff_off.ensure(sizeof(int64_t) * (size_t)(F + 1))) ||
+        (rc = m.ff_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(12 * m.n_cells, 1))) ||
+        (rc = chain_state(m, tiles, c)))
+        return rc;
     int64_t *off = m.ff_off.as<int64_t>();
-    if (F > 0) {
-        hipLaunchKernelGGL((k_ff<false>), dim3(grid(F)), dim3(256), 0, m.stream,
-                           m.ft.as<int32_t>(), F, m.tf.as<int32_t>(), off, nullptr);
-        TG_LAUNCH_CHECK("k_ff count");
-    }
     int64_t nnz = 0;
-    if ((rc = scan_counts64(m, off, F, nnz))) return rc;
-    if ((rc = m.ff_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)))) return rc;
     if (F > 0) {
-        hipLaunchKernelGGL((k_ff<true>), dim3(grid(F)), dim3(256), 0, m.stream,
-                           m.ft.as<int32_t>(), F, m.tf.as<int32_t>(), off, m.ff_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_ff fill");
+        hipLaunchKernelGGL(k_ff, dim3((unsigned)tiles), dim3(FF_THREADS), 0, m.stream,
+                           m.ft.as<int32_t>(), F, m.tf.as<int32_t>(), c.ticket, c.state, off,
+                           m.ff_vals.as<int32_t>());
+        TG_LAUNCH_CHECK("k_ff");
+        if ((rc = read_i64(m, off, F, nnz))) return rc;
+    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
+        return rc;
     }
     m.ff_nnz = nnz;
     m.ff_built = true;
@@ -1497,30 +1440,34 @@ int ensure_ee(tg_mesh &m) {
     int rc;
     if ((rc = ensure_edges(m))) return rc;
     const int64_t E = m.n_edges, V = m.n_points;
-    if ((rc = m.ee_off.ensure(sizeof(int64_t) * (size_t)(E + 1)))) return rc;
+    const int64_t tiles = (E + EJ_THREADS - 1) / EJ_THREADS, n2 = 2 * E;
+    Chain c;
+    // tmp_c: each vertex's edge ids, and four words of slack (rows are loaded
+    // by whole quads)
+    if ((rc = m.ee_off.ensure(sizeof(int64_t) * (size_t)(E + 1))) ||
+        (rc = m.tmp_c.ensure(sizeof(int32_t) * (size_t)(n2 + 4))) || (rc = chain_state(m, tiles, c)))
+        return rc;
     int64_t *off = m.ee_off.as<int64_t>();
-    if (E > 0) {
-        hipLaunchKernelGGL(k_ee_count, dim3(grid(E)), dim3(256), 0, m.stream, m.ev.as<int32_t>(),
-                           E, m.vv_off.as<int32_t>(), off);
-        TG_LAUNCH_CHECK("k_ee_count");
-    }
     int64_t nnz = 0;
-    if ((rc = scan_counts64(m, off, E, nnz))) return rc;
+    if (E > 0) {
+        hipLaunchKernelGGL(k_vertex_edges, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, m.stream,
+                           m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
+                           m.edge_first.as<int32_t>(), m.edge_rank.as<uint2>(),
+                           m.vv_eid.as<int32_t>(), m.tmp_c.as<int32_t>());
+        TG_LAUNCH_CHECK("k_vertex_edges");
+        // an edge's row: its ends' edges, which share only itself
+        if ((rc = row_squares(m, m.vv_off.as<int32_t>(), V, c, nnz))) return rc;
+        nnz -= n2;
+    }
     if ((rc = m.ee_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)))) return rc;
     if (E > 0) {
-        // each vertex's edge ids (the vv_eid row) sorted ascending
-        const int64_t n2 = 2 * E;
-        // four words of slack: k_ee stages rows by whole 16-byte quads
-        if ((rc = m.tmp_c.ensure(sizeof(int32_t) * (size_t)(n2 + 4)))) return rc;
-        TG_HIP(hipMemcpyAsync(m.tmp_c.p, m.vv_eid.p, sizeof(int32_t) * (size_t)n2,
-                              hipMemcpyDeviceToDevice, m.stream));
-        if ((rc = launch_sort_rows_i32(m.vv_off.as<int32_t>(), m.tmp_c.as<int32_t>(), V,
-                                       m.stream)))
-            return rc;
-        hipLaunchKernelGGL(k_ee, dim3(grid(E, ROW_THREADS)), dim3(ROW_THREADS), 0, m.stream,
-                           m.ev.as<int32_t>(), E, m.vv_off.as<int32_t>(), m.tmp_c.as<int32_t>(),
-                           off, m.ee_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_ee");
+        hipLaunchKernelGGL((k_edge_join<UNION_LESS_SELF, 0, EE_WIN>), dim3((unsigned)tiles),
+                           dim3(EJ_THREADS), 0, m.stream, m.ev.as<int32_t>(), E, V,
+                           m.vv_off.as<int32_t>(), m.tmp_c.as<int32_t>(), c.ticket, c.state, off,
+                           m.ee_vals.as<int32_t>());
+        TG_LAUNCH_CHECK("k_edge_join<EE>");
+    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
+        return rc;
     }
     m.ee_nnz = nnz;
     m.ee_built = true;

@@ -62,7 +62,7 @@ struct tg_mesh {
     tg::DevArr edge_first, ve_off, ve_vals, ev, te, vv_eid, et_off, et_vals;
     tg::DevArr face_off, vf_vals, fv, tf, fe, ft, ef_off, ef_vals;
     tg::DevArr tt_off, tt_vals, ff_off, ff_vals, ee_off, ee_vals;
-    tg::DevArr bitmap, rank_tmp, tmp_a, tmp_b, tmp_c;
+    tg::DevArr bitmap, rank_tmp, edge_rank, face_rank, tmp_a, tmp_b, tmp_c;
     bool edges_built = false, faces_built = false, vt_built = false, et_built = false,
          fe_built = false, ft_built = false, ef_built = false, tt_built = false,
          ff_built = false, ee_built = false;
