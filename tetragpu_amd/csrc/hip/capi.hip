@@ -43,8 +43,8 @@ int DevArr::ensure(size_t bytes) {
     return OK;
 }
 
-void DevArr::release() {
-    if (p) pool_free(p, cap, stream);
+void DevArr::release(bool idle) {
+    if (p) pool_free(p, cap, idle ? pool_idle() : stream);
     p = nullptr;
     cap = 0;
 }
@@ -247,8 +247,8 @@ int tg_mesh_create(tg_mesh **out, const int32_t *cells, int64_t n_cells,
 
 int tg_mesh_destroy(tg_mesh *m) {
     if (!m) return TG_OK;
-    if (m->stream) (void)hipStreamSynchronize(m->stream);
-    m->release_all();
+    const bool idle = !m->stream || hipStreamSynchronize(m->stream) == hipSuccess;
+    m->release_all(idle);
     if (m->h_pinned) tg::pinned_slot_free(m->h_pinned);
     if (m->own_stream && m->stream) (void)hipStreamDestroy(m->stream);
     delete m;

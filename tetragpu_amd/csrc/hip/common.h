@@ -60,9 +60,11 @@ int scan_exclusive_i32_to_i64(const int32_t *in, int64_t *out, int64_t n,
 
 // Stream-ordered caching allocator (pool.hip): a freed block is reused only
 // after `stream` has passed the free.  pool_alloc returns nullptr on failure
-// and the usable size in *granted.
+// and the usable size in *granted.  stream == pool_idle(): the block's stream
+// has been waited for since its last use, so it is free at once.
 void *pool_alloc(size_t bytes, size_t *granted);
 void pool_free(void *p, size_t bytes, hipStream_t stream);
+inline hipStream_t pool_idle() { return (hipStream_t)~(uintptr_t)0; }
 void pool_trim();
 size_t pool_cached_bytes();
 // Pinned host blocks from a size-classed cache (results handed to callers).

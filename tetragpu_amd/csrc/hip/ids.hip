@@ -1104,15 +1104,6 @@ int fail(int code, const char *msg) {
     return code;
 }
 
-int read_i32(tg_mesh &m, const void *src, int64_t index, int32_t &out) {
-    int32_t *h = (int32_t *)m.h_pinned;
-    TG_HIP(hipMemcpyAsync(h, (const int32_t *)src + index, sizeof(int32_t),
-                          hipMemcpyDeviceToHost, m.stream));
-    TG_HIP(hipStreamSynchronize(m.stream));
-    out = *h;
-    return tg::OK;
-}
-
 int read_i64(tg_mesh &m, const void *src, int64_t index, int64_t &out) {
     int64_t *h = (int64_t *)m.h_pinned;
     TG_HIP(hipMemcpyAsync(h, (const int64_t *)src + index, sizeof(int64_t),
@@ -1124,7 +1115,9 @@ int read_i64(tg_mesh &m, const void *src, int64_t index, int64_t &out) {
 
 // rank structure over n flags (0 or 1): rank_of(rank, p) is the number of
 // flags set before position p
-int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank, int64_t &total) {
+// (with, when given, two further words read in the same wait)
+int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank, int64_t &total,
+                const int32_t *two = nullptr, int32_t *two_out = nullptr) {
     const int64_t nw = (n + 31) / 32;
     int rc;
     if ((rc = m.bitmap.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(nw, 1))) ||
@@ -1145,9 +1138,16 @@ int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank, i
                            rank.as<uint2>());
         TG_LAUNCH_CHECK("k_rank_words");
     }
-    int32_t t32 = 0;
-    if ((rc = read_i32(m, wpre, nw, t32))) return rc;
-    total = t32;
+    int32_t *h = (int32_t *)m.h_pinned;
+    TG_HIP(hipMemcpyAsync(h, wpre + nw, sizeof(int32_t), hipMemcpyDeviceToHost, m.stream));
+    if (two)
+        TG_HIP(hipMemcpyAsync(h + 2, two, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, m.stream));
+    TG_HIP(hipStreamSynchronize(m.stream));
+    total = h[0];
+    if (two) {
+        two_out[0] = h[2];
+        two_out[1] = h[3];
+    }
     return tg::OK;
 }
 
@@ -1182,13 +1182,14 @@ namespace tg {
 int ensure_edges(tg_mesh &m) {
     if (m.edges_built) return OK;
     int rc;
-    if ((rc = ensure_vv(m)) || (rc = ensure_vt_sorted(m)) || (rc = sync_and_check(m))) return rc;
     const int64_t V = m.n_points, T = m.n_cells;
-    int32_t nnz = 0;
-    if ((rc = read_i32(m, m.vv_off.p, V, nnz))) return rc;
+    int64_t nnz = 0;
+    if ((rc = ensure_vv(m)) || (rc = ensure_vt_sorted(m)) ||
+        (rc = sync_check_read(m, m.vv_off.as<int32_t>() + V, nnz)))
+        return rc;
     const size_t I = sizeof(int32_t);
-    if ((rc = m.edge_first.ensure(I * (size_t)std::max(nnz, 1))) ||
-        (rc = m.vv_eid.ensure(I * (size_t)std::max(nnz, 1))) ||
+    if ((rc = m.edge_first.ensure(I * (size_t)std::max<int64_t>(nnz, 1))) ||
+        (rc = m.vv_eid.ensure(I * (size_t)std::max<int64_t>(nnz, 1))) ||
         (rc = m.te.ensure(I * 6 * (size_t)std::max<int64_t>(T, 1))) ||
         (rc = m.tmp_a.ensure(std::max<size_t>(6 * (size_t)T, 1))) ||  // flags
         (rc = m.ve_off.ensure(I * (size_t)(V + 1))))
@@ -1196,7 +1197,7 @@ int ensure_edges(tg_mesh &m) {
     uint8_t *flags = m.tmp_a.as<uint8_t>();
     if ((rc = fill_u8(flags, 0, 6 * T, m.stream))) return rc;
     hipLaunchKernelGGL(k_fill_i32v, dim3(grid(nnz)), dim3(256), 0, m.stream,
-                       m.edge_first.as<int32_t>(), INF, (int64_t)nnz);
+                       m.edge_first.as<int32_t>(), INF, nnz);
     TG_LAUNCH_CHECK("k_fill_i32v");
     if (V > 0) {
         hipLaunchKernelGGL(k_edge_first, dim3(grid(V, EDGE_THREADS)), dim3(EDGE_THREADS), 0, m.stream,
@@ -1290,7 +1291,11 @@ int ensure_faces(tg_mesh &m) {
         TG_LAUNCH_CHECK("k_face_first");
     }
     int64_t F = 0;
-    if ((rc = build_ranks(m, flags, 4 * T, m.face_rank, F))) return rc;
+    int32_t errs[2] = {0, 0};  // C_FTERR, C_IDERR
+    static_assert(C_IDERR == C_FTERR + 1, "read together");
+    if ((rc = build_ranks(m, flags, 4 * T, m.face_rank, F, err, errs))) return rc;
+    if (errs[1]) return fail(ERR_STATE, "face ids: TE and ET disagree (a cell is missing from ET)");
+    m.ft_ok = errs[0] == 0;
     m.n_faces = F;
     if ((rc = m.fv.ensure(I * 3 * (size_t)std::max<int64_t>(F, 1))) ||
         (rc = m.ft.ensure(I * 2 * (size_t)std::max<int64_t>(F, 1))) ||
@@ -1302,10 +1307,6 @@ int ensure_faces(tg_mesh &m) {
                            m.tf.as<int32_t>(), m.fv.as<int32_t>(), m.ft.as<int32_t>());
         TG_LAUNCH_CHECK("k_face_ids");
     }
-    int32_t ferr = 0, ierr = 0;
-    if ((rc = read_i32(m, err, 0, ferr)) || (rc = read_i32(m, iderr, 0, ierr))) return rc;
-    if (ierr) return fail(ERR_STATE, "face ids: TE and ET disagree (a cell is missing from ET)");
-    m.ft_ok = ferr == 0;
     int32_t *voff = m.face_off.as<int32_t>();
     if (V > 0) {
         hipLaunchKernelGGL((k_vf<false>), dim3(grid(V)), dim3(256), 0, m.stream,
@@ -1387,7 +1388,7 @@ int ensure_tt(tg_mesh &m) {
     if ((rc = m.tt_off.ensure(sizeof(int64_t) * (size_t)(T + 1))) || (rc = chain_state(m, tiles, c)))
         return rc;
     int64_t *off = m.tt_off.as<int64_t>();
-    int64_t rows = 0, nnz = 0;
+    int64_t rows = 0;
     // the cells' rows together: every vertex's row once per entry
     if (T > 0 && (rc = row_squares(m, m.vt_off.as<int32_t>(), V, c, rows))) return rc;
     // a cell's four rows hold the cell itself four times
@@ -1398,11 +1399,10 @@ int ensure_tt(tg_mesh &m) {
                            m.tv.as<const int4>(), T, m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(),
                            c.ticket, c.state, off, m.tt_vals.as<int32_t>());
         TG_LAUNCH_CHECK("k_tt");
-        if ((rc = read_i64(m, off, T, nnz))) return rc;
     } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
         return rc;
     }
-    m.tt_nnz = nnz;
+    m.tt_nnz = T > 0 ? -1 : 0;
     m.tt_built = true;
     return OK;
 }
@@ -1420,17 +1420,15 @@ int ensure_ff(tg_mesh &m) {
         (rc = chain_state(m, tiles, c)))
         return rc;
     int64_t *off = m.ff_off.as<int64_t>();
-    int64_t nnz = 0;
     if (F > 0) {
         hipLaunchKernelGGL(k_ff, dim3((unsigned)tiles), dim3(FF_THREADS), 0, m.stream,
                            m.ft.as<int32_t>(), F, m.tf.as<int32_t>(), c.ticket, c.state, off,
                            m.ff_vals.as<int32_t>());
         TG_LAUNCH_CHECK("k_ff");
-        if ((rc = read_i64(m, off, F, nnz))) return rc;
     } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
         return rc;
     }
-    m.ff_nnz = nnz;
+    m.ff_nnz = F > 0 ? -1 : 0;
     m.ff_built = true;
     return OK;
 }
@@ -1478,7 +1476,6 @@ int id_relation_view(tg_mesh &m, int32_t rel, RelView &r) {
     const int64_t V = m.n_points, T = m.n_cells, E = m.n_edges, F = m.n_faces;
     auto need = [&](bool ok, const char *what) { return ok ? OK : fail(ERR_STATE, what); };
     int rc;
-    int64_t nnz = 0;
     switch (rel) {
     case TG_REL_TE:
         if ((rc = need(m.edges_built, "TE not built"))) return rc;
@@ -1494,8 +1491,7 @@ int id_relation_view(tg_mesh &m, int32_t rel, RelView &r) {
         return OK;
     case TG_REL_ET:
         if ((rc = need(m.et_built, "ET not built"))) return rc;
-        if ((rc = read_i64(m, m.et_off.p, E, nnz))) return rc;
-        r = {E, nnz, 1, m.et_off.p, 8, m.et_vals.as<int32_t>()};
+        r = {E, 6 * T, 1, m.et_off.p, 8, m.et_vals.as<int32_t>()};
         return OK;
     case TG_REL_TF:
         if ((rc = need(m.faces_built, "TF not built"))) return rc;

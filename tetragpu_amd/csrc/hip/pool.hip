@@ -111,17 +111,23 @@ void *pool_alloc(size_t bytes, size_t *granted) {
 
 void pool_free(void *p, size_t bytes, hipStream_t stream) {
     if (!p) return;
+    const bool idle = stream == pool_idle();
     Pool &P = pool();
     std::lock_guard<std::mutex> g(P.mu);
     hipEvent_t ev = nullptr;
-    if (!P.events.empty()) {
+    if (idle) {
+        // the caller has waited for the stream: no event to record now and to
+        // query at every later allocation
+    } else if (!P.events.empty()) {
         ev = P.events.back();
         P.events.pop_back();
     } else if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
         ev = nullptr;
     }
-    if (ev && hipEventRecord(ev, stream) == hipSuccess) {
+    if (idle) {
+        P.free_blocks.emplace(bytes, p);
+    } else if (ev && hipEventRecord(ev, stream) == hipSuccess) {
         P.pending.push_back({p, bytes, ev});
     } else {
         // no event: wait for the stream, then the block is free now

@@ -12,7 +12,7 @@ struct DevArr {
     size_t cap = 0;
     hipStream_t stream = nullptr;  // the stream that uses it (orders its reuse)
     int ensure(size_t bytes);
-    void release();
+    void release(bool idle = false);  // idle: the stream has been waited for
     template <typename T> T *as() const { return (T *)p; }
 };
 
@@ -67,12 +67,13 @@ struct tg_mesh {
          fe_built = false, ft_built = false, ef_built = false, tt_built = false,
          ff_built = false, ee_built = false;
     bool ft_ok = true;  // every face is held by at most two cells
-    int64_t tt_nnz = 0, ff_nnz = 0, ee_nnz = 0, ef_nnz = 0;
+    // entry counts of built relations; -1: known to the device only, read when asked for
+    int64_t tt_nnz = 0, ff_nnz = 0, ee_nnz = 0, ef_nnz = 0, vv_nnz = -1;
 
     void *h_pinned = nullptr;  // small pinned staging area (64 int64)
     tg::StageMarks marks;      // per-stage events of the last pipeline run
 
-    void release_all();
+    void release_all(bool idle);
     void bind_stream(hipStream_t s);  // every DevArr of the mesh uses stream s
 };
 
@@ -96,6 +97,9 @@ int ensure_vv(tg_mesh &m);
 int build_relations(tg_mesh &m, uint32_t flags);
 // Synchronise the mesh stream and report device-side errors.
 int sync_and_check(tg_mesh &m);
+// The same, with one int32 or int64 read from device memory in the same wait.
+int sync_check_read(tg_mesh &m, const int32_t *src, int64_t &out);
+int sync_check_read(tg_mesh &m, const int64_t *src, int64_t &out);
 // Describe a built relation (synchronises to learn its size).
 int relation_view(tg_mesh &m, int32_t rel, RelView &out);
 // Fill a VvCpBuffers view over the mesh's arrays.

@@ -5,6 +5,7 @@
 #include <mutex>
 #include <vector>
 #include <cstdio>
+#include <cstring>
 
 #include "ids.h"
 #include "relations.h"
@@ -24,27 +25,17 @@ int fail(int code, const char *msg) {
     return code;
 }
 
-// Read one int32 from device memory (synchronises the stream).
-int read_i32(tg_mesh &m, const void *src, int64_t index, int32_t &out) {
-    int32_t *h = (int32_t *)m.h_pinned;
-    TG_HIP(hipMemcpyAsync(h, (const int32_t *)src + index, sizeof(int32_t),
-                          hipMemcpyDeviceToHost, m.stream));
-    TG_HIP(hipStreamSynchronize(m.stream));
-    out = *h;
-    return tg::OK;
-}
-
 }  // namespace
 
-static void release_all_impl(tg_mesh *m, hipStream_t s, bool release);
+static void release_all_impl(tg_mesh *m, hipStream_t s, bool release, bool idle);
 
 void tg_mesh::bind_stream(hipStream_t s) {
-    release_all_impl(this, s, false);
+    release_all_impl(this, s, false, false);
 }
 
-void tg_mesh::release_all() { release_all_impl(this, stream, true); }
+void tg_mesh::release_all(bool idle) { release_all_impl(this, stream, true, idle); }
 
-static void release_all_impl(tg_mesh *m, hipStream_t s, bool release) {
+static void release_all_impl(tg_mesh *m, hipStream_t s, bool release, bool idle) {
     tg_mesh &me = *m;
     tg::DevArr *all[] = {&me.tv,       &me.scal,     &me.vt_cnt,   &me.vt_off,   &me.vt_cur,   &me.vtc,
                          &me.scratch,  &me.deg,      &me.vv_off,   &me.vv_cols,  &me.classes,  &me.heavy,
@@ -57,7 +48,7 @@ static void release_all_impl(tg_mesh *m, hipStream_t s, bool release) {
                          &me.bk_fixd,  &me.bk_rowdesc, &me.bk_rec};
     for (auto *a : all) {
         a->stream = s;
-        if (release) a->release();
+        if (release) a->release(idle);
     }
     if (!release) return;
     for (auto &e : me.marks.ev)
@@ -240,6 +231,7 @@ static int run_vv(tg_mesh &m, bool classify) {
         }
     }
     m.vv_built = true;
+    m.vv_nnz = -1;
     if (classify) m.cp_built = true;
     m.counters_pending = true;
     return OK;
@@ -343,36 +335,79 @@ int build_relations(tg_mesh &m, uint32_t flags) {
     return OK;
 }
 
-int sync_and_check(tg_mesh &m) {
+namespace {
+
+int capacity_error() {
+    char buf[160];
+    std::snprintf(buf, sizeof buf,
+                  "a vertex has more than %d distinct neighbours; its row and class "
+                  "were not computed",
+                  HEAVY_CAP);
+    set_error(buf);
+    return ERR_CAPACITY;
+}
+
+// One wait for the stream's work, the run's error bits (when a run is
+// unchecked) and up to eight bytes from src: each readback on its own leaves
+// the device idle for about 30 us.
+int wait_check_read(tg_mesh &m, const void *src, size_t bytes, void *out) {
+    int64_t *h = (int64_t *)m.h_pinned;
+    const bool check = m.counters_pending;
+    if (check)
+        TG_HIP(hipMemcpyAsync(h, m.counters.as<int32_t>() + C_ERR, sizeof(int32_t),
+                              hipMemcpyDeviceToHost, m.stream));
+    if (bytes)
+        TG_HIP(hipMemcpyAsync(h + 1, src, bytes, hipMemcpyDeviceToHost, m.stream));
     TG_HIP(hipStreamSynchronize(m.stream));
-    if (!m.counters_pending) return OK;
     m.counters_pending = false;
-    int32_t err = 0;
-    int rc = read_i32(m, m.counters.p, C_ERR, err);
-    if (rc) return rc;
-    if (err & ERRBIT_CAPACITY) {
-        char buf[160];
-        std::snprintf(buf, sizeof buf,
-                      "a vertex has more than %d distinct neighbours; its row and class "
-                      "were not computed",
-                      HEAVY_CAP);
-        set_error(buf);
-        return ERR_CAPACITY;
-    }
+    if (check && (*(const int32_t *)h & ERRBIT_CAPACITY)) return capacity_error();
+    if (bytes) std::memcpy(out, h + 1, bytes);
     return OK;
 }
 
+}  // namespace
+
+int sync_and_check(tg_mesh &m) { return wait_check_read(m, nullptr, 0, nullptr); }
+
+int sync_check_read(tg_mesh &m, const int32_t *src, int64_t &out) {
+    int32_t x = 0;
+    const int rc = wait_check_read(m, src, sizeof x, &x);
+    out = x;
+    return rc;
+}
+
+int sync_check_read(tg_mesh &m, const int64_t *src, int64_t &out) {
+    return wait_check_read(m, src, sizeof out, &out);
+}
+
 int relation_view(tg_mesh &m, int32_t rel, RelView &r) {
-    int rc = sync_and_check(m);
-    if (rc) return rc;
+    int rc;
     r = RelView();
-    int32_t nnz = 0;
+    // the counts that only the device knows come with the wait
+    auto read_count = [&](int64_t &nnz, bool built, const DevArr &off, int64_t rows) {
+        if (!built || nnz >= 0) return sync_and_check(m);
+        int64_t n = 0;
+        const int e = sync_check_read(m, off.as<int64_t>() + rows, n);
+        if (!e) nnz = n;
+        return e;
+    };
+    if (rel == TG_REL_VV && m.vv_built && m.vv_nnz < 0) {
+        int64_t n = 0;
+        if ((rc = sync_check_read(m, m.vv_off.as<int32_t>() + m.n_points, n))) return rc;
+        m.vv_nnz = n;
+    } else if (rel == TG_REL_TT) {
+        rc = read_count(m.tt_nnz, m.tt_built, m.tt_off, m.n_cells);
+    } else if (rel == TG_REL_FF) {
+        rc = read_count(m.ff_nnz, m.ff_built, m.ff_off, m.n_faces);
+    } else {
+        rc = sync_and_check(m);
+    }
+    if (rc) return rc;
     switch (rel) {
     case TG_REL_VV:
         if (!m.vv_built) return fail(ERR_STATE, "VV not built");
-        if ((rc = read_i32(m, m.vv_off.p, m.n_points, nnz))) return rc;
         r.rows = m.n_points;
-        r.nnz = nnz;
+        r.nnz = m.vv_nnz;
         r.offsets = m.vv_off.p;
         r.offset_bytes = 4;
         r.values = m.vv_cols.as<int32_t>();
