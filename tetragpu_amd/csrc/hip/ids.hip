@@ -647,7 +647,7 @@ __device__ __forceinline__ void insert_sorted(int32_t *row, int64_t &m, int32_t 
 // beyond the largest one merges serially from global memory.
 //
 // What bounds it: the gathers of NR x 64 different rows per wave (TT: 4 rows of
-// 96 bytes a cell, 2.0 M cells in random order 0.76 ms) and VALU issue of the
+// 96 bytes a cell, 2.0 M cells in random order 0.65 ms) and VALU issue of the
 // network (560 compare-exchanges for four rows of 24).  It replaced a merge of
 // LDS columns by one lane each (26-32 KB a wave, waiting on dependent LDS
 // reads; longer rows from global memory), which wrote padded rows, scanned
@@ -843,8 +843,10 @@ __device__ __forceinline__ int32_t take_tile(int32_t *ticket, int32_t &shared) {
     return shared;
 }
 
-// Windows: two for 64 x 69 words.
-constexpr int TT_THREADS = 256, TT_WIN = 2240;
+// Window: what two blocks per CU (as many as the registers allow) leave of
+// the LDS; one window for 64 x 69 words (two windows of 2240: 0.76 ms at 2.0 M
+// split cells, one 0.65).
+constexpr int TT_THREADS = 256, TT_WIN = 5088;
 __global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const int4 *__restrict__ tv4, int64_t T,
                                                       const int32_t *__restrict__ vt_off,
                                                       const int32_t *__restrict__ vtc,

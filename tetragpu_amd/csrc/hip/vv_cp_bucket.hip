@@ -77,6 +77,12 @@ __device__ __forceinline__ void rec_store(const Rec &r, int64_t i, uint32_t v, u
     r.w2[i] = (b >> 16) | (c << 8);
 }
 
+// VT's records carry the corner code 4t + j (31 bits) instead: two words.
+__device__ __forceinline__ void vtrec_store(const Rec &r, int64_t i, uint32_t v, uint32_t code) {
+    r.w0[i] = v | (code << 24);
+    r.w1[i] = code >> 8;
+}
+
 __device__ __forceinline__ void rec_unpack(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t &v,
                                            uint32_t &a, uint32_t &b, uint32_t &c) {
     v = w0 & M24;
@@ -119,70 +125,80 @@ __global__ __launch_bounds__(L1_THREADS) void k_l1_count(const int4 *__restrict_
 // counting-sorted by destination bin in LDS, then each bin's run is written
 // with consecutive lanes to consecutive addresses.  A record's bin is
 // recomputed from its vertex field, so a tile costs 12 bytes of LDS per
-// record; larger tiles give longer runs per bin and fewer partial lines.
-constexpr int STAGE1 = 8192;   // level-1 records per tile (2048 tets)
-constexpr int STAGE2 = 12288;  // level-2 records per tile
+// record (VT's 8).  Larger tiles give longer runs per bin and fewer partial
+// lines; tiles of half the LDS let one block's loads and ranking run beside
+// the other's stores.  Level 2 takes the small tiles where runs stay long
+// (MI355X, 12-byte records: 16 buckets a bin 145 -> 132 us at 5.3 M cells, but
+// 32 buckets 206 -> 212 us at 7.7 M and 64 buckets 312 -> 345 us at 12.6 M).
+constexpr int STAGE1 = 8192;         // level-1 records per tile (2048 tets, a divisor of the chunks)
+constexpr int STAGE2_LARGE = 12288;  // level-2 records per tile
+constexpr int STAGE2_SMALL = 6144;
+constexpr int SMALL_BINS = 16;       // buckets per bin up to which the small tiles are taken
+constexpr int L1S_THREADS = 1024;
 
-template <int N>
+template <int N, int WORDS>
 struct Stage {
-    uint32_t w0[N], w1[N], w2[N];
+    uint32_t w[WORDS][N];
     int32_t cnt[MAX_FINE], toff[MAX_FINE], gbase[MAX_FINE];
-    int32_t total;
+    int32_t ws[MAX_FINE / 64];
 };
 
-// Exclusive scan of cnt[0..nbin) into toff, total into st.total (block-wide).
+// Exclusive scan of cnt[0..nbin) into toff (block-wide, at least MAX_FINE
+// threads, contains a barrier); returns the total.
 template <typename ST>
-__device__ __forceinline__ void stage_scan(ST &st, int nbin) {
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        int32_t carry = 0;
-        for (int b0 = 0; b0 < nbin; b0 += 64) {
-            const int i = b0 + lane;
-            const int32_t x = i < nbin ? st.cnt[i] : 0;
-            const int32_t inc = tgd::wave_inclusive_sum(x);
-            if (i < nbin) st.toff[i] = carry + inc - x;
-            carry += __shfl(inc, 63, 64);
-        }
-        if (lane == 0) st.total = carry;
+__device__ __forceinline__ int32_t stage_scan(ST &st, int nbin) {
+    const int tid = threadIdx.x, wid = tid / 64;
+    const int32_t x = tid < nbin ? st.cnt[tid] : 0;
+    const int32_t inc = tgd::wave_inclusive_sum(x);
+    if (tid < MAX_FINE && __lane_id() == 63) st.ws[wid] = inc;
+    __syncthreads();
+    int32_t before = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < MAX_FINE / 64; i++) {
+        if (i < wid) before += st.ws[i];
+        total += st.ws[i];
     }
+    if (tid < nbin) st.toff[tid] = before + inc - x;
+    return total;
 }
 
 // Write the staged tile: consecutive slots of one bin go to consecutive
 // addresses of that bin's range; the bin of a slot is (v >> shift) - base.
-template <typename ST>
-__device__ __forceinline__ void stage_flush(ST &st, Rec out, int nthreads, int shift,
-                                            int32_t base) {
-    const int32_t total = st.total;
+template <int N, int WORDS>
+__device__ __forceinline__ void stage_flush(const Stage<N, WORDS> &st, int32_t total, Rec out,
+                                            int nthreads, int shift, int32_t base) {
     for (int slot = threadIdx.x; slot < total; slot += nthreads) {
-        const uint32_t w0 = st.w0[slot];
+        const uint32_t w0 = st.w[0][slot];
         const int b = (int)((w0 & M24) >> shift) - base;
         const int64_t pos = (int64_t)st.gbase[b] + (slot - st.toff[b]);
         out.w0[pos] = w0;
-        out.w1[pos] = st.w1[slot];
-        out.w2[pos] = st.w2[slot];
+        out.w1[pos] = st.w[1][slot];
+        if constexpr (WORDS == 3) out.w2[pos] = st.w[2][slot];
     }
 }
 
 template <bool VTREC>
-__global__ __launch_bounds__(L1_THREADS) void k_l1_scatter(const int4 *__restrict__ tv4, int64_t T,
-                                                            int64_t tpc, int cshift, int32_t nc,
-                                                            int32_t nch,
-                                                            const int32_t *__restrict__ h1s,
-                                                            Rec out) {
-    constexpr int TILE = STAGE1 / 4;          // tets per tile
-    constexpr int TPT = TILE / L1_THREADS;    // tets per thread
-    __shared__ Stage<STAGE1> st;
+__global__ __launch_bounds__(L1S_THREADS) void k_l1_scatter(const int4 *__restrict__ tv4, int64_t T,
+                                                             int64_t tpc, int cshift, int32_t nc,
+                                                             int32_t nch,
+                                                             const int32_t *__restrict__ h1s,
+                                                             Rec out) {
+    constexpr int TILE = STAGE1 / 4;           // tets per tile
+    constexpr int TPT = TILE / L1S_THREADS;    // tets per thread
+    static_assert(TPT * L1S_THREADS == TILE && MAX_COARSE <= L1S_THREADS && MAX_FINE <= L1S_THREADS,
+                  "tile shape");
+    __shared__ Stage<STAGE1, VTREC ? 2 : 3> st;
     const int tid = threadIdx.x;
-    for (int i = tid; i < nc; i += L1_THREADS) st.gbase[i] = h1s[(int64_t)i * nch + blockIdx.x];
+    for (int i = tid; i < nc; i += L1S_THREADS) st.gbase[i] = h1s[(int64_t)i * nch + blockIdx.x];
     const int64_t t0 = (int64_t)blockIdx.x * tpc, t1 = min(T, t0 + tpc);
     int4 qn[TPT];
 #pragma unroll
     for (int k = 0; k < TPT; k++) {
-        const int64_t t = t0 + k * L1_THREADS + tid;
+        const int64_t t = t0 + k * L1S_THREADS + tid;
         qn[k] = t < t1 ? tv4[t] : make_int4(0, 0, 0, 0);
     }
     for (int64_t tb = t0; tb < t1; tb += TILE) {
-        for (int i = tid; i < nc; i += L1_THREADS) st.cnt[i] = 0;
+        for (int i = tid; i < nc; i += L1S_THREADS) st.cnt[i] = 0;
         __syncthreads();
         int4 q[TPT];
         bool on[TPT];
@@ -190,7 +206,7 @@ __global__ __launch_bounds__(L1_THREADS) void k_l1_scatter(const int4 *__restric
 #pragma unroll
         for (int k = 0; k < TPT; k++) {
             q[k] = qn[k];
-            on[k] = tb + k * L1_THREADS + tid < t1;
+            on[k] = tb + k * L1S_THREADS + tid < t1;
             if (on[k]) {
                 r[k][0] = atomicAdd(&st.cnt[q[k].x >> cshift], 1);
                 r[k][1] = atomicAdd(&st.cnt[q[k].y >> cshift], 1);
@@ -199,25 +215,30 @@ __global__ __launch_bounds__(L1_THREADS) void k_l1_scatter(const int4 *__restric
             }
         }
         __syncthreads();
-        stage_scan(st, nc);
+        const int32_t total = stage_scan(st, nc);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < TPT; k++) {
             if (!on[k]) continue;
             const uint32_t x = q[k].x, y = q[k].y, z = q[k].z, w = q[k].w;
-            auto put = [&](int bin, int rank, uint32_t v, uint32_t a, uint32_t b, uint32_t c) {
-                const int slot = st.toff[bin] + rank;
-                st.w0[slot] = v | (a << 24);
-                st.w1[slot] = (a >> 8) | (b << 16);
-                st.w2[slot] = (b >> 16) | (c << 8);
-            };
             if constexpr (VTREC) {
-                const uint32_t c0 = 4u * (uint32_t)(tb + k * L1_THREADS + tid);
-                put(q[k].x >> cshift, r[k][0], x, c0 & M24, c0 >> 24, 0u);
-                put(q[k].y >> cshift, r[k][1], y, (c0 + 1) & M24, (c0 + 1) >> 24, 0u);
-                put(q[k].z >> cshift, r[k][2], z, (c0 + 2) & M24, (c0 + 2) >> 24, 0u);
-                put(q[k].w >> cshift, r[k][3], w, (c0 + 3) & M24, (c0 + 3) >> 24, 0u);
+                const uint32_t c0 = 4u * (uint32_t)(tb + k * L1S_THREADS + tid);
+                auto put = [&](int bin, int rank, uint32_t v, uint32_t code) {
+                    const int slot = st.toff[bin] + rank;
+                    st.w[0][slot] = v | (code << 24);
+                    st.w[1][slot] = code >> 8;
+                };
+                put(q[k].x >> cshift, r[k][0], x, c0);
+                put(q[k].y >> cshift, r[k][1], y, c0 + 1);
+                put(q[k].z >> cshift, r[k][2], z, c0 + 2);
+                put(q[k].w >> cshift, r[k][3], w, c0 + 3);
             } else {
+                auto put = [&](int bin, int rank, uint32_t v, uint32_t a, uint32_t b, uint32_t c) {
+                    const int slot = st.toff[bin] + rank;
+                    st.w[0][slot] = v | (a << 24);
+                    st.w[1][slot] = (a >> 8) | (b << 16);
+                    st.w[2][slot] = (b >> 16) | (c << 8);
+                };
                 put(q[k].x >> cshift, r[k][0], x, y, z, w);
                 put(q[k].y >> cshift, r[k][1], y, x, z, w);
                 put(q[k].z >> cshift, r[k][2], z, x, y, w);
@@ -228,12 +249,12 @@ __global__ __launch_bounds__(L1_THREADS) void k_l1_scatter(const int4 *__restric
         // next tile's tets are in flight during the flush
 #pragma unroll
         for (int k = 0; k < TPT; k++) {
-            const int64_t t = tb + TILE + k * L1_THREADS + tid;
+            const int64_t t = tb + TILE + k * L1S_THREADS + tid;
             if (t < t1) qn[k] = tv4[t];
         }
-        stage_flush(st, out, L1_THREADS, cshift, 0);
+        stage_flush(st, total, out, L1S_THREADS, cshift, 0);
         __syncthreads();
-        for (int i = tid; i < nc; i += L1_THREADS) st.gbase[i] += st.cnt[i];
+        for (int i = tid; i < nc; i += L1S_THREADS) st.gbase[i] += st.cnt[i];
     }
 }
 
@@ -263,15 +284,13 @@ __global__ __launch_bounds__(L2_THREADS) void k_l2_count(const uint32_t *__restr
     const int32_t fb0 = c << fs;
     constexpr int U = 8;
     for (int32_t i0 = lo + threadIdx.x; i0 < hi; i0 += U * L2_THREADS) {
-        uint32_t w[U];
+        uint32_t w[U];  // all loads first, from clamped places past the end
 #pragma unroll
-        for (int k = 0; k < U; k++) {
-            const int32_t i = i0 + k * L2_THREADS;
-            w[k] = i < hi ? w0[i] : 0xFFFFFFFFu;
-        }
+        for (int k = 0; k < U; k++) w[k] = w0[min(i0 + k * L2_THREADS, hi - 1)];
 #pragma unroll
         for (int k = 0; k < U; k++)
-            if (w[k] != 0xFFFFFFFFu) atomicAdd(&hw[(int32_t)((w[k] & M24) >> bv_log) - fb0], 1);
+            if (i0 + k * L2_THREADS < hi)
+                atomicAdd(&hw[(int32_t)((w[k] & M24) >> bv_log) - fb0], 1);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < F && fb0 + i < nb; i += L2_THREADS) {
@@ -282,60 +301,61 @@ __global__ __launch_bounds__(L2_THREADS) void k_l2_count(const uint32_t *__restr
     }
 }
 
-__global__ __launch_bounds__(L2_THREADS) void k_l2_scatter(const Rec in,
+template <bool VTREC, int STAGE2, int L2S_THREADS>
+__global__ __launch_bounds__(L2S_THREADS) void k_l2_scatter(const Rec in,
                                                             const int32_t *__restrict__ h1s,
                                                             int32_t nch, int bv_log, int fs,
                                                             int32_t nb,
                                                             const int32_t *__restrict__ h2s,
                                                             Rec out) {
-    __shared__ Stage<STAGE2> st;
+    constexpr int WORDS = VTREC ? 2 : 3;
+    __shared__ Stage<STAGE2, WORDS> st;
     const int tid = threadIdx.x;
     const int32_t c = blockIdx.x, s = blockIdx.y, S = gridDim.y;
     const int32_t fb0 = c << fs;
     const int F = min(1 << fs, nb - fb0);
-    for (int i = tid; i < F; i += L2_THREADS) st.gbase[i] = h2s[(int64_t)(fb0 + i) * S + s];
+    for (int i = tid; i < F; i += L2S_THREADS) st.gbase[i] = h2s[(int64_t)(fb0 + i) * S + s];
     int32_t lo, hi;
     slice_range(h1s, nch, c, s, S, lo, hi);
-    constexpr int PER = STAGE2 / L2_THREADS;
-    uint32_t a[PER], b[PER], d[PER];
+    constexpr int PER = STAGE2 / L2S_THREADS;
+    uint32_t a[PER][WORDS];
     auto load = [&](int32_t ib) {
 #pragma unroll
         for (int k = 0; k < PER; k++) {
-            const int32_t i = ib + k * L2_THREADS + tid;
-            a[k] = 0xFFFFFFFFu;
+            const int32_t i = ib + k * L2S_THREADS + tid;
+            a[k][0] = 0xFFFFFFFFu;
             if (i < hi) {
-                a[k] = in.w0[i];
-                b[k] = in.w1[i];
-                d[k] = in.w2[i];
+                a[k][0] = in.w0[i];
+                a[k][1] = in.w1[i];
+                if constexpr (WORDS == 3) a[k][2] = in.w2[i];
             }
         }
     };
     load(lo);
     for (int32_t ib = lo; ib < hi; ib += STAGE2) {
-        for (int i = tid; i < F; i += L2_THREADS) st.cnt[i] = 0;
+        for (int i = tid; i < F; i += L2S_THREADS) st.cnt[i] = 0;
         __syncthreads();
         int f[PER], r[PER];
 #pragma unroll
         for (int k = 0; k < PER; k++) {
-            f[k] = a[k] != 0xFFFFFFFFu ? (int)((a[k] & M24) >> bv_log) - fb0 : -1;
+            f[k] = ib + k * L2S_THREADS + tid < hi ? (int)((a[k][0] & M24) >> bv_log) - fb0 : -1;
             if (f[k] >= 0) r[k] = atomicAdd(&st.cnt[f[k]], 1);
         }
         __syncthreads();
-        stage_scan(st, F);
+        const int32_t total = stage_scan(st, F);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < PER; k++)
             if (f[k] >= 0) {
                 const int slot = st.toff[f[k]] + r[k];
-                st.w0[slot] = a[k];
-                st.w1[slot] = b[k];
-                st.w2[slot] = d[k];
+#pragma unroll
+                for (int w = 0; w < WORDS; w++) st.w[w][slot] = a[k][w];
             }
         __syncthreads();
         load(ib + STAGE2);  // next tile's records are in flight during the flush
-        stage_flush(st, out, L2_THREADS, bv_log, fb0);
+        stage_flush(st, total, out, L2S_THREADS, bv_log, fb0);
         __syncthreads();
-        for (int i = tid; i < F; i += L2_THREADS) st.gbase[i] += st.cnt[i];
+        for (int i = tid; i < F; i += L2S_THREADS) st.gbase[i] += st.cnt[i];
     }
 }
 
@@ -435,7 +455,8 @@ struct S1Stage {
 
 // bstart: exclusive scan of the bucket counts; bused: zeroed fill counters.
 template <bool VTREC>
-__global__ __launch_bounds__(S1_THREADS) void k_s1_scatter(const int4 *__restrict__ tv4,
+// 64 registers: two blocks per CU
+__global__ __launch_bounds__(S1_THREADS, 8) void k_s1_scatter(const int4 *__restrict__ tv4,
                                                             int64_t T, int64_t tpc, int bv_log,
                                                             const int32_t *__restrict__ bstart,
                                                             int32_t *__restrict__ bused,
@@ -478,22 +499,21 @@ __global__ __launch_bounds__(S1_THREADS) void k_s1_scatter(const int4 *__restric
                 total += st.wsum[i];
             }
             st.toff[tid] = pre + inc - c;
-            st.gb[tid] = base;
             __syncthreads();
             if (on) {
                 auto put = [&](int j, int rank, uint32_t v, uint32_t a, uint32_t b, uint32_t cc) {
                     const int slot = st.toff[j] + rank;
                     st.w0[slot] = v | (a << 24);
                     st.w1[slot] = (a >> 8) | (b << 16);
-                    st.w2[slot] = (b >> 16) | (cc << 8);
+                    if constexpr (!VTREC) st.w2[slot] = (b >> 16) | (cc << 8);
                     st.bin[slot] = (uint16_t)j;
                 };
-                if constexpr (VTREC) {
+                if constexpr (VTREC) {  // w0 = v | code << 24, w1 = code >> 8
                     const uint32_t c0 = 4u * (uint32_t)(tb + tid);
-                    put(b0 - bmin, r0, x, c0 & M24, c0 >> 24, 0u);
-                    put(b1 - bmin, r1, y, (c0 + 1) & M24, (c0 + 1) >> 24, 0u);
-                    put(b2 - bmin, r2, z, (c0 + 2) & M24, (c0 + 2) >> 24, 0u);
-                    put(b3 - bmin, r3, w, (c0 + 3) & M24, (c0 + 3) >> 24, 0u);
+                    put(b0 - bmin, r0, x, c0, 0u, 0u);
+                    put(b1 - bmin, r1, y, c0 + 1, 0u, 0u);
+                    put(b2 - bmin, r2, z, c0 + 2, 0u, 0u);
+                    put(b3 - bmin, r3, w, c0 + 3, 0u, 0u);
                 } else {
                     put(b0 - bmin, r0, x, y, z, w);
                     put(b1 - bmin, r1, y, x, z, w);
@@ -501,24 +521,22 @@ __global__ __launch_bounds__(S1_THREADS) void k_s1_scatter(const int4 *__restric
                     put(b3 - bmin, r3, w, x, y, z);
                 }
             }
+            st.gb[tid] = base;  // the atomics' answers arrive while the records are placed
             __syncthreads();
             for (int slot = tid; slot < total; slot += S1_THREADS) {
                 const int j = st.bin[slot];
                 const int64_t pos = (int64_t)st.gb[j] + (slot - st.toff[j]);
                 out.w0[pos] = st.w0[slot];
                 out.w1[pos] = st.w1[slot];
-                out.w2[pos] = st.w2[slot];
+                if constexpr (!VTREC) out.w2[pos] = st.w2[slot];
             }
         } else if (on) {
             if constexpr (VTREC) {
                 const uint32_t c0 = 4u * (uint32_t)(tb + tid);
-                rec_store(out, (int64_t)bstart[b0] + atomicAdd(&bused[b0], 1), x, c0 & M24, c0 >> 24, 0u);
-                rec_store(out, (int64_t)bstart[b1] + atomicAdd(&bused[b1], 1), y, (c0 + 1) & M24,
-                          (c0 + 1) >> 24, 0u);
-                rec_store(out, (int64_t)bstart[b2] + atomicAdd(&bused[b2], 1), z, (c0 + 2) & M24,
-                          (c0 + 2) >> 24, 0u);
-                rec_store(out, (int64_t)bstart[b3] + atomicAdd(&bused[b3], 1), w, (c0 + 3) & M24,
-                          (c0 + 3) >> 24, 0u);
+                vtrec_store(out, (int64_t)bstart[b0] + atomicAdd(&bused[b0], 1), x, c0);
+                vtrec_store(out, (int64_t)bstart[b1] + atomicAdd(&bused[b1], 1), y, c0 + 1);
+                vtrec_store(out, (int64_t)bstart[b2] + atomicAdd(&bused[b2], 1), z, c0 + 2);
+                vtrec_store(out, (int64_t)bstart[b3] + atomicAdd(&bused[b3], 1), w, c0 + 3);
             } else {
                 rec_store(out, (int64_t)bstart[b0] + atomicAdd(&bused[b0], 1), x, y, z, w);
                 rec_store(out, (int64_t)bstart[b1] + atomicAdd(&bused[b1], 1), y, x, z, w);
@@ -1589,51 +1607,57 @@ __global__ __launch_bounds__(HV_THREADS) void k_bkt_heavy(
 // are distinct).  The bucket's rows fill the same range of the CSR that its
 // records fill in bucket order, so row offsets need no global scan.
 constexpr int VT_THREADS = 256, VT_CAP = 8192;
+constexpr int VT_PRE = 24;  // records per thread held in registers while counting
 
-template <int BV, typename P>
-__device__ __forceinline__ void vt_place_rank(const Rec &rec, int32_t cbeg, int32_t cend,
-                                              int32_t *cur, const int32_t *off, P st,
-                                              int32_t *__restrict__ vtc) {
-    const int tid = threadIdx.x;
-    for (int32_t i = cbeg + tid; i < cend; i += VT_THREADS) {
-        uint32_t v, lo, hi, unused;
-        rec_unpack(rec.w0[i], rec.w1[i], rec.w2[i], v, lo, hi, unused);
-        const int32_t pos = atomicAdd(&cur[v & (uint32_t)(BV - 1)], 1);
-        st[pos] = (int32_t)(lo | (hi << 24));
+// A row of d <= R codes (staged from st on) sorted in registers and written in
+// 16-byte stores.
+template <int R, typename P>
+__device__ __forceinline__ void vt_sort_row(P st, int d, int32_t *__restrict__ out) {
+    typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    uint32_t r[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) r[i] = i < d ? (uint32_t)st[i] : 0xFFFFFFFFu;
+    tgn::sort_keys(r);
+#pragma unroll
+    for (int i = 0; i < R; i += 4) {
+        if (i + 4 <= d) {
+            *reinterpret_cast<u32x4u *>(out + i) = u32x4u{r[i], r[i + 1], r[i + 2], r[i + 3]};
+        } else {
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                if (i + j < d) out[i + j] = (int32_t)r[i + j];
+        }
     }
-    // the workgroup barrier orders the staged writes for its own reads, LDS
-    // or global; a device-scope fence here would write back L2 per block
-    __syncthreads();
-    // rows of at most 32 entries: one thread per vertex sorts its row in
-    // registers; longer rows are listed and ranked by the whole block
+}
+
+// skew: staged words between two vertices' rows (1 in LDS: rows of equal
+// length would start in few banks).
+template <int BV, typename P>
+__device__ __forceinline__ void vt_rows(const int32_t *off, P st, int skew,
+                                        int32_t *__restrict__ vtc) {
+    const int tid = threadIdx.x;
     __shared__ int32_t nlong;
     __shared__ int32_t lng[BV];
     if (tid == 0) nlong = 0;
     __syncthreads();
-    if (tid < BV) {
-        const int32_t rb = off[tid], d = off[tid + 1] - rb;
-        if (d > 32) {
-            lng[atomicAdd(&nlong, 1)] = tid;
-        } else if (d > 0) {
-            uint32_t r[32];
-#pragma unroll
-            for (int i = 0; i < 32; i++) r[i] = i < d ? (uint32_t)st[rb + i] : 0xFFFFFFFFu;
-            sort32(r);
-#pragma unroll
-            for (int i = 0; i < 32; i++)
-                if (i < d) vtc[cbeg + rb + i] = (int32_t)r[i];
-        }
-    }
+    const int32_t rb = tid < BV ? off[tid] : 0, d = tid < BV ? off[tid + 1] - rb : 0;
+    const bool is_long = d > 32;
+    if (is_long) lng[atomicAdd(&nlong, 1)] = tid;
+    const int ds = is_long ? 0 : d;
+    if (__any(ds > 24)) vt_sort_row<32>(st + rb + skew * tid, ds, vtc + rb);
+    else vt_sort_row<24>(st + rb + skew * tid, ds, vtc + rb);
     __syncthreads();
+    // longer rows: the whole block ranks their entries
     for (int k = 0; k < nlong; k++) {
         const int vl = lng[k];
-        const int32_t rb = off[vl], re = off[vl + 1];
-        for (int32_t p = rb + tid; p < re; p += VT_THREADS) {
-            const int32_t e = st[p];
+        const int32_t lb = off[vl], le = off[vl + 1];
+        P row = st + lb + skew * vl;
+        for (int32_t p = tid; p < le - lb; p += VT_THREADS) {
+            const int32_t e = row[p];
             int32_t r = 0;
 #pragma unroll 4
-            for (int32_t q = rb; q < re; q++) r += st[q] < e;
-            vtc[cbeg + rb + r] = e;
+            for (int32_t q = 0; q < le - lb; q++) r += row[q] < e;
+            vtc[lb + r] = e;
         }
     }
 }
@@ -1648,30 +1672,48 @@ __global__ __launch_bounds__(VT_THREADS) void k_bkt_vt(const Rec rec,
                                                         int32_t *__restrict__ vt_cnt) {
     constexpr int BV = 1 << BV_LOG;
     static_assert(BV <= VT_THREADS, "one thread per vertex in the scan");
-    __shared__ int32_t cnt[BV], off[BV + 1], cur[BV];
-    __shared__ int32_t buf[VT_CAP];
+    __shared__ int32_t off[BV + 1], cur[BV];
+    __shared__ int32_t buf[VT_CAP + BV + 32];  // skewed rows; a network reads up to 32 words
     __shared__ int32_t wsum[VT_THREADS / 64];
     const int tid = threadIdx.x, lane = __lane_id(), wid = tid / 64;
     const int32_t b = blockIdx.x, v0 = b << BV_LOG;
     const int nv = min(BV, V - v0);
     const int32_t cbeg = h2s[(int64_t)b * nslice], cend = h2s[(int64_t)(b + 1) * nslice];
     const int32_t n = cend - cbeg;
-    for (int i = tid; i < BV; i += VT_THREADS) cnt[i] = 0;
+    for (int i = tid; i < BV; i += VT_THREADS) cur[i] = 0;
     __syncthreads();
-    for (int32_t i = cbeg + tid; i < cend; i += VT_THREADS)
-        atomicAdd(&cnt[rec.w0[i] & (uint32_t)(BV - 1)], 1);
+    // records in register chunks, all loads in flight; a bucket of one chunk
+    // is read once
+    uint32_t w[VT_PRE][2];
+    auto load = [&](int32_t c0) {
+#pragma unroll
+        for (int k = 0; k < VT_PRE; k++) {
+            const int32_t i = c0 + k * VT_THREADS + tid;
+            w[k][0] = i < n ? rec.w0[cbeg + i] : 0u;
+            w[k][1] = i < n ? rec.w1[cbeg + i] : 0u;
+        }
+    };
+    const bool one_chunk = n <= VT_PRE * VT_THREADS;
+    for (int32_t c0 = 0; c0 < n; c0 += VT_PRE * VT_THREADS) {
+        load(c0);
+#pragma unroll
+        for (int k = 0; k < VT_PRE; k++)
+            if (c0 + k * VT_THREADS + tid < n) atomicAdd(&cur[w[k][0] & (uint32_t)(BV - 1)], 1);
+    }
     __syncthreads();
-    const int32_t x = tid < BV ? cnt[tid] : 0;
+    const int32_t x = tid < BV ? cur[tid] : 0;
     const int32_t inc = tgd::wave_inclusive_sum(x);
     if (lane == 63) wsum[wid] = inc;
     __syncthreads();
     int32_t pre = 0;
 #pragma unroll
-    for (int w = 0; w < VT_THREADS / 64; w++)
-        if (w < wid) pre += wsum[w];
+    for (int i = 0; i < VT_THREADS / 64; i++)
+        if (i < wid) pre += wsum[i];
+    // LDS staging when the bucket fits, else the dead level-1 array
+    const bool fits = n <= VT_CAP;
     if (tid < BV) {
         off[tid] = pre + inc - x;
-        cur[tid] = pre + inc - x;
+        cur[tid] = pre + inc - x + (fits ? tid : 0);
     }
     if (tid == 0) off[BV] = n;
     __syncthreads();
@@ -1680,10 +1722,22 @@ __global__ __launch_bounds__(VT_THREADS) void k_bkt_vt(const Rec rec,
         vt_cnt[v0 + tid] = x;
     }
     if (b == nb - 1 && tid == 0) vt_off[V] = cend;
-    // LDS staging when the bucket fits, else the dead level-1 array (a
-    // separate instantiation keeps the LDS accesses on LDS instructions)
-    if (n <= VT_CAP) vt_place_rank<BV>(rec, cbeg, cend, cur, off, buf, vtc);
-    else vt_place_rank<BV>(rec, cbeg, cend, cur, off, stage + cbeg, vtc);
+    for (int32_t c0 = 0; c0 < n; c0 += VT_PRE * VT_THREADS) {
+        if (!one_chunk) load(c0);
+#pragma unroll
+        for (int k = 0; k < VT_PRE; k++)
+            if (c0 + k * VT_THREADS + tid < n) {
+                const int32_t p = atomicAdd(&cur[w[k][0] & (uint32_t)(BV - 1)], 1);
+                const int32_t code = (int32_t)((w[k][0] >> 24) | (w[k][1] << 8));
+                if (fits) buf[p] = code;
+                else stage[cbeg + p] = code;
+            }
+    }
+    // the workgroup barrier orders the staged writes for its own reads, LDS
+    // or global; a device-scope fence here would write back L2 per block
+    __syncthreads();
+    if (fits) vt_rows<BV>(off, buf, 1, vtc + cbeg);
+    else vt_rows<BV>(off, stage + cbeg, 0, vtc + cbeg);
 }
 
 // Route the corner records of every cell to the buckets of their vertex:
@@ -1759,7 +1813,7 @@ int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, i
         if ((rc = tg::scan_exclusive_i32(k.h1, k.h1, (int64_t)p.nc * p.nchunks, b.scan_tmp, s)))
             return rc;
         if (mk) mk->mark("l1_count", s);
-        hipLaunchKernelGGL(k_l1_scatter<VTREC>, dim3(p.nchunks), dim3(L1_THREADS), 0, s, tv4, T, p.tpc,
+        hipLaunchKernelGGL(k_l1_scatter<VTREC>, dim3(p.nchunks), dim3(L1S_THREADS), 0, s, tv4, T, p.tpc,
                            cshift, p.nc, p.nchunks, k.h1, r1);
         TG_LAUNCH_CHECK("k_l1_scatter");
         if (mk) mk->mark("l1_scatter", s);
@@ -1770,8 +1824,12 @@ int route_records(tg::BucketBuffers &k, hipStream_t s, const int32_t *&ranges, i
         if ((rc = tg::scan_exclusive_i32(k.h2, k.h2, (int64_t)p.nb * p.slices, b.scan_tmp, s)))
             return rc;
         if (mk) mk->mark("l2_count", s);
-        hipLaunchKernelGGL(k_l2_scatter, g2, dim3(L2_THREADS), 0, s, r1, k.h1, p.nchunks,
-                           p.bv_log, p.fs, p.nb, k.h2, r2);
+        if ((1 << p.fs) <= SMALL_BINS)
+            hipLaunchKernelGGL((k_l2_scatter<VTREC, STAGE2_SMALL, 512>), g2, dim3(512), 0, s, r1,
+                               k.h1, p.nchunks, p.bv_log, p.fs, p.nb, k.h2, r2);
+        else
+            hipLaunchKernelGGL((k_l2_scatter<VTREC, STAGE2_LARGE, 1024>), g2, dim3(1024), 0, s, r1,
+                               k.h1, p.nchunks, p.bv_log, p.fs, p.nb, k.h2, r2);
         TG_LAUNCH_CHECK("k_l2_scatter");
         if (mk) mk->mark("l2_scatter", s);
     }
