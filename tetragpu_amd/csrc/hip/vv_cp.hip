@@ -521,24 +521,120 @@ __global__ __launch_bounds__(64) void k_cp_fix_wave(
 // its shared-tet component.  Only neighbours outside the largest component of
 // a multi-component class have their rows walked; every row-membership edge
 // between two components of one class joins them, and the classes' counts are
-// the components of that component graph.  Two vertices per wave, 32 lanes
-// each.  Few neighbours walk (one to five of 32 on a noisy field), so the
-// lanes go over a row's entries, not over the neighbours: a fifth of the
-// instructions, and whole lines per load.  Bound by the chain of dependent
-// loads per vertex and the gathers of the rows.
+// the components of that component graph.  W lanes per vertex of at most W
+// neighbours: four vertices per wave where all four have 16 or fewer (most
+// of a tetrahedral mesh's), else two at a time.  Few neighbours walk (one to
+// five on a noisy field), so the lanes go over a row's entries, not over the
+// neighbours: a fifth of the instructions, and whole lines per load.  Bound by
+// instruction issue and the chain of dependent loads per vertex.  Four at a
+// time: 155 -> 133 us on the 2.1 M vertices of a noisy 12 M-cell mesh, 202 ->
+// 167 on a batch of 96; two at a time stays where most rows are longer.
+struct FixDesc {
+    int32_t nbs[64];
+    uint32_t cadj[2 * 64];
+    uint8_t dsc[64];
+};
+
+template <int W>
+__device__ __forceinline__ void fix_desc(const int32_t *__restrict__ off,
+                                         const int32_t *__restrict__ cols,
+                                         const uint8_t *__restrict__ rowdesc,
+                                         uint32_t *__restrict__ classes, FixDesc &st, int32_t v,
+                                         int32_t b, int d, int32_t rs) {
+    const int lane = __lane_id() & (W - 1), group = __lane_id() / W;
+    const uint64_t gmask = (W == 32 ? 0xFFFFFFFFull : 0xFFFFull) << (W * group);
+    int32_t *nbs = st.nbs + W * group;
+    uint32_t *cadj = st.cadj + 2 * W * group;  // [class][component]
+    uint8_t *dsc = st.dsc + W * group;
+    const bool on = lane < d;
+    const int32_t a = on ? cols[b + lane] : INT32_MAX;
+    const uint32_t ds = on ? rowdesc[rs + lane] : 0u;
+    const int cls = (int)(ds >> 5), comp = (int)(ds & 31u);
+    nbs[lane] = a;
+    dsc[lane] = (uint8_t)ds;
+    cadj[lane] = 0u;
+    cadj[W + lane] = 0u;
+    int nc1 = on && cls == 1 ? comp + 1 : 0, nc0 = on && cls == 0 ? comp + 1 : 0;
+#pragma unroll
+    for (int s = W / 2; s >= 1; s >>= 1) {
+        nc1 = max(nc1, __shfl_xor(nc1, s, W));
+        nc0 = max(nc0, __shfl_xor(nc0, s, W));
+    }
+    // largest component of each multi-component class (lowest number on
+    // ties); the ballots run over the wave, each group reads its own bits
+    int big0 = 0, big1 = 0, best0 = -1, best1 = -1;
+    for (int j = 0; __any(j < max(nc0, nc1)); j++) {
+        const uint64_t here = __ballot(on && comp == j) & gmask, one = __ballot(cls == 1);
+        const int s1 = __popcll(here & one), s0 = __popcll(here & ~one);
+        if (j < nc0 && s0 > best0) { best0 = s0; big0 = j; }
+        if (j < nc1 && s1 > best1) { best1 = s1; big1 = j; }
+    }
+    tgd::wave_sync();
+    const bool walk = on && (cls ? nc1 >= 2 && comp != big1 : nc0 >= 2 && comp != big0);
+    int32_t rb = 0, rn = 0;
+    if (walk) {
+        rb = off[a];
+        rn = off[a + 1] - rb;
+    }
+    // the walking neighbours' rows one after the other, the lanes over a row's
+    // entries, four rows' loads in flight
+    uint32_t left = (uint32_t)((__ballot(walk) & gmask) >> (W * group));
+    while (__any(left != 0)) {
+        constexpr int G = 4;
+        int32_t c[G], b0[G], n0[G];
+        int from[G];
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+            const int src = left ? __ffs(left) - 1 : 0;
+            const bool has = left != 0;
+            left &= left - 1u;
+            b0[q] = __shfl(rb, src, W);
+            n0[q] = has ? __shfl(rn, src, W) : 0;
+            from[q] = __shfl((int)ds, src, W);
+            c[q] = lane < n0[q] ? cols[b0[q] + lane] : INT32_MAX;
+        }
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+            for (int32_t j = lane; __any(j - lane < n0[q]);) {
+                // lower bound in the W sorted entries (INT32_MAX past d)
+                int lo = 0;
+#pragma unroll
+                for (int step = W / 2; step >= 1; step >>= 1)
+                    if (nbs[lo + step - 1] < c[q]) lo += step;
+                if (lo < d && nbs[lo] == c[q]) {
+                    const int dk = dsc[lo], ck = dk & 31, fk = from[q] & 31, fc = from[q] >> 5;
+                    if ((dk >> 5) == fc && ck != fk) {
+                        atomicOr(&cadj[fc * W + fk], 1u << ck);
+                        atomicOr(&cadj[fc * W + ck], 1u << fk);
+                    }
+                }
+                j += W;  // rows of more than W entries
+                c[q] = j < n0[q] ? cols[b0[q] + j] : INT32_MAX;
+            }
+        }
+    }
+    tgd::wave_sync();
+    if (lane == 0 && d > 0) {
+        const uint32_t m1 = nc1 >= 32 ? ~0u : ((1u << nc1) - 1u);
+        const uint32_t m0 = nc0 >= 32 ? ~0u : ((1u << nc0) - 1u);
+        const uint32_t nl = nc1 >= 2 ? n_components32(cadj + W, m1) : (uint32_t)nc1;
+        const uint32_t nu = nc0 >= 2 ? n_components32(cadj, m0) : (uint32_t)nc0;
+        classes[3 * (int64_t)v] = nl;
+        classes[3 * (int64_t)v + 1] = nu;
+        classes[3 * (int64_t)v + 2] = verdict(nl, nu);
+    }
+    tgd::wave_sync();
+}
+
 __global__ __launch_bounds__(64) void k_cp_fix_desc(
     const int32_t *__restrict__ off, const int32_t *__restrict__ cols,
     const int32_t *__restrict__ rowsrc, const uint8_t *__restrict__ rowdesc,
     const int32_t *__restrict__ fixd, const int32_t *__restrict__ counters,
     uint32_t *__restrict__ classes) {
-    __shared__ int32_t nbs[2][32];
-    __shared__ uint8_t dsc[2][32];
-    __shared__ uint32_t cadj[2][2][32];
-    const int lane = threadIdx.x & 31, half = threadIdx.x >> 5;
+    __shared__ FixDesc st;
+    const int quarter = __lane_id() / 16;
     const int32_t n = counters[tg::C_FIXD];
-    const uint64_t hmask = half ? 0xFFFFFFFF00000000ull : 0xFFFFFFFFull;
-    // the next vertex's id and row bounds are loaded during the current one
-    // (the pass is bound by chains of dependent loads)
+    // the next vertices' ids and row bounds are loaded during the current ones
     auto head = [&](int32_t i, int32_t &v, int32_t &b, int32_t &e, int32_t &rs) {
         v = i < n ? fixd[i] : 0;
         b = i < n ? off[v] : 0;
@@ -546,98 +642,21 @@ __global__ __launch_bounds__(64) void k_cp_fix_desc(
         rs = i < n ? rowsrc[v] : 0;
     };
     int32_t nv_, nb_, ne_, nrs_;
-    head(2 * blockIdx.x + half, nv_, nb_, ne_, nrs_);
-    for (int32_t i0 = 2 * blockIdx.x; i0 < n; i0 += 2 * gridDim.x) {
-        const int32_t i = i0 + half;
-        const bool live = i < n;
+    head(4 * blockIdx.x + quarter, nv_, nb_, ne_, nrs_);
+    for (int32_t i0 = 4 * blockIdx.x; i0 < n; i0 += 4 * gridDim.x) {
         const int32_t v = nv_, b = nb_, rs = nrs_;
-        int d = live ? ne_ - b : 0;
-        head(i + 2 * gridDim.x, nv_, nb_, ne_, nrs_);
-        d = min(d, 32);  // rows with descriptors have no more
-        const bool on = lane < d;
-        const int32_t a = on ? cols[b + lane] : INT32_MAX;
-        const uint32_t ds = on ? rowdesc[rs + lane] : 0u;
-        const int cls = (int)(ds >> 5), comp = (int)(ds & 31u);
-        nbs[half][lane] = a;
-        dsc[half][lane] = (uint8_t)ds;
-        cadj[half][0][lane] = 0u;
-        cadj[half][1][lane] = 0u;
-        int nc1 = on && cls == 1 ? comp + 1 : 0, nc0 = on && cls == 0 ? comp + 1 : 0;
-#pragma unroll
-        for (int s = 16; s >= 1; s >>= 1) {
-            nc1 = max(nc1, __shfl_xor(nc1, s, 32));
-            nc0 = max(nc0, __shfl_xor(nc0, s, 32));
-        }
-        // largest component of each multi-component class (lowest number on
-        // ties); the ballots run over the wave, each half reads its 32 bits
-        int big0 = 0, big1 = 0;
-        const int ncmax = max(__shfl(max(nc0, nc1), 0, 64), __shfl(max(nc0, nc1), 32, 64));
-        int best0 = -1, best1 = -1;
-        for (int j = 0; j < ncmax; j++) {
-            const int s0 = __popcll(__ballot(on && cls == 0 && comp == j) & hmask);
-            const int s1 = __popcll(__ballot(on && cls == 1 && comp == j) & hmask);
-            if (j < nc0 && s0 > best0) { best0 = s0; big0 = j; }
-            if (j < nc1 && s1 > best1) { best1 = s1; big1 = j; }
-        }
-        tgd::wave_sync();
-        const int nck = cls ? nc1 : nc0;
-        const int big = cls ? big1 : big0;
-        const bool walk = on && nck >= 2 && comp != big;
-        int32_t rb = 0, rn = 0;
-        if (walk) {
-            rb = off[a];
-            rn = off[a + 1] - rb;
-        }
-        // the walking neighbours' rows one after the other, the 32 lanes over
-        // a row's entries, four rows' loads in flight
-        uint32_t left = (uint32_t)(__ballot(walk) >> (32 * half));
-        while (__any(left != 0)) {
-            constexpr int G = 4;
-            int32_t c[G], b0[G], n0[G];
-            int from[G];
-#pragma unroll
-            for (int q = 0; q < G; q++) {
-                const int src = left ? __ffs(left) - 1 : 0;
-                const bool has = left != 0;
-                left &= left - 1u;
-                b0[q] = __shfl(rb, src, 32);
-                n0[q] = has ? __shfl(rn, src, 32) : 0;
-                from[q] = __shfl((int)ds, src, 32);
-                c[q] = lane < n0[q] ? cols[b0[q] + lane] : INT32_MAX;
-            }
-#pragma unroll
-            for (int q = 0; q < G; q++) {
-                for (int32_t j = lane;;) {
-                    // lower bound in the 32 sorted entries (INT32_MAX past d)
-                    int lo = 0;
-#pragma unroll
-                    for (int step = 16; step >= 1; step >>= 1)
-                        if (nbs[half][lo + step - 1] < c[q]) lo += step;
-                    if (lo < d && nbs[half][lo] == c[q]) {
-                        const int dk = dsc[half][lo], ck = dk & 31, fk = from[q] & 31;
-                        const int fc = from[q] >> 5;
-                        if ((dk >> 5) == fc && ck != fk) {
-                            atomicOr(&cadj[half][fc][fk], 1u << ck);
-                            atomicOr(&cadj[half][fc][ck], 1u << fk);
-                        }
-                    }
-                    j += 32;  // rows of more than 32 entries
-                    if (!__any(j - lane < n0[q])) break;
-                    c[q] = j < n0[q] ? cols[b0[q] + j] : INT32_MAX;
-                }
+        const int d = min(ne_ - nb_, 32);  // rows with descriptors have no more
+        head(i0 + quarter + 4 * gridDim.x, nv_, nb_, ne_, nrs_);
+        if (!__any(d > 16)) {
+            fix_desc<16>(off, cols, rowdesc, classes, st, v, b, d, rs);
+        } else {
+#pragma unroll 1
+            for (int k = 0; k < 2; k++) {
+                const int src = 16 * (2 * k + (__lane_id() >> 5));
+                fix_desc<32>(off, cols, rowdesc, classes, st, __shfl(v, src, 64),
+                             __shfl(b, src, 64), __shfl(d, src, 64), __shfl(rs, src, 64));
             }
         }
-        tgd::wave_sync();
-        if (lane == 0 && live && d > 0) {
-            const uint32_t m1 = nc1 >= 32 ? ~0u : ((1u << nc1) - 1u);
-            const uint32_t m0 = nc0 >= 32 ? ~0u : ((1u << nc0) - 1u);
-            const uint32_t nl = nc1 >= 2 ? n_components32(cadj[half][1], m1) : (uint32_t)nc1;
-            const uint32_t nu = nc0 >= 2 ? n_components32(cadj[half][0], m0) : (uint32_t)nc0;
-            classes[3 * (int64_t)v] = nl;
-            classes[3 * (int64_t)v + 1] = nu;
-            classes[3 * (int64_t)v + 2] = verdict(nl, nu);
-        }
-        tgd::wave_sync();
     }
 }
 
@@ -777,8 +796,8 @@ int launch_cp_fix_typed(tg::VvCpBuffers &b, hipStream_t s) {
     const int32_t V = (int32_t)b.n_points;
     const S *scal = (const S *)b.scalars;
     if (b.fixd) {
-        // two vertices a block; 32 blocks per CU
-        const unsigned g = std::min<unsigned>(tg::grid_for(V, 2), 8192u);
+        // four vertices a block; 32 blocks per CU
+        const unsigned g = std::min<unsigned>(tg::grid_for(V, 4), 8192u);
         hipLaunchKernelGGL(k_cp_fix_desc, dim3(g), dim3(64), 0, s, b.vv_off, b.vv_cols, b.rowsrc,
                            b.rowdesc, b.fixd, b.counters, b.classes);
         TG_LAUNCH_CHECK("k_cp_fix_desc");
