@@ -899,9 +899,12 @@ struct Slab {
 // and the walk collects each record's slots as a 32-bit mask.  R > 32: the
 // code is (record / 2) << 3 | 3 * (record & 1) + corner and the walk collects
 // six 5-bit slot numbers per word, so that 48 records fit the same columns.
-template <int R, bool CP>
+//
+// after_rows(d) runs once the row column holds the d neighbours, before the
+// adjacency is built: the gathers it starts are in flight meanwhile.
+template <int R, bool CP, typename F>
 __device__ __forceinline__ int sort_rows(const Slab &rec, int pos, int c, uint32_t *row,
-                                         uint32_t *adj) {
+                                         uint32_t *adj, F after_rows) {
     constexpr int N = 3 * R;
     constexpr bool MASKS = R <= 32;
     constexpr int NCOL = MASKS ? R : R / 2;  // words of collected slots
@@ -943,6 +946,7 @@ __device__ __forceinline__ int sort_rows(const Slab &rec, int pos, int c, uint32
     }
     const int d = slot + 1 - (3 * c < N);  // the padding counts once
     if (CP) {
+        after_rows(d);
         uint32_t m[NCOL];
 #pragma unroll
         for (int r = 0; r < NCOL; r++) m[r] = adj[r * 64];
@@ -1091,30 +1095,44 @@ __global__ __launch_bounds__(1 << BV_LOG, 2) void k_bkt_sort(
             w[k][0] = w[k][1] = w[k][2] = 0u;
         __syncthreads();
         const int at_ = mine ? pos : 0;
+        const int32_t v = v0 + (mine ? mv : 0);
+        constexpr int G = 16;  // scalar gathers in flight
+        // while the adjacency is built, where they fit the registers (float:
+        // 12.6 M cells 581 -> 556 us; double would spill, 66 -> 70 on 1 M)
+        constexpr int EARLY = sizeof(S) == 4 ? G : 0;
+        S sv = S(0), su[G];
+        auto gather = [&](int d) {
+            if constexpr (EARLY > 0) {
+                sv = scal[v];
+#pragma unroll
+                for (int i = 0; i < EARLY; i++) su[i] = scal[i < d ? (int32_t)row[i * 64] : v];
+                tgd::sched_fence();
+            }
+        };
         int d;
-        if (__any(cr > 40)) d = sort_rows<SK_MAXREC, CP>(sl, at_, cr, row, adj);
-        else if (__any(cr > 32)) d = sort_rows<40, CP>(sl, at_, cr, row, adj);
-        else if (__any(cr > 24)) d = sort_rows<32, CP>(sl, at_, cr, row, adj);
-        else if (__any(cr > 8)) d = sort_rows<24, CP>(sl, at_, cr, row, adj);
-        else d = sort_rows<8, CP>(sl, at_, cr, row, adj);
+        if (__any(cr > 40)) d = sort_rows<SK_MAXREC, CP>(sl, at_, cr, row, adj, gather);
+        else if (__any(cr > 32)) d = sort_rows<40, CP>(sl, at_, cr, row, adj, gather);
+        else if (__any(cr > 24)) d = sort_rows<32, CP>(sl, at_, cr, row, adj, gather);
+        else if (__any(cr > 8)) d = sort_rows<24, CP>(sl, at_, cr, row, adj, gather);
+        else d = sort_rows<8, CP>(sl, at_, cr, row, adj, gather);
         const bool hv = mine && (cnt > SK_MAXREC || d > SLOTS);
         const bool ok = mine && !hv;
         uint32_t nl = 0, nu = 0;
         if (CP && ok) {
-            const int32_t v = v0 + mv;
-            const S sv = scal[v];
             uint32_t lm = 0;
-            constexpr int G = 16;  // scalar gathers in flight
-            for (int s0 = 0; s0 < d; s0 += G) {
-                int32_t u[G];
-                S su[G];
+            if constexpr (EARLY == 0) sv = scal[v];
 #pragma unroll
-                for (int i = 0; i < G; i++) u[i] = s0 + i < d ? (int32_t)row[(s0 + i) * 64] : v;
-#pragma unroll
-                for (int i = 0; i < G; i++) su[i] = s0 + i < d ? scal[u[i]] : sv;
+            for (int i = 0; i < EARLY; i++)
+                lm |= (uint32_t)is_lower(su[i], sv, (int32_t)row[i * 64], v) << i;
+            for (int s0 = EARLY; s0 < d; s0 += G) {
+                S sr[G];
 #pragma unroll
                 for (int i = 0; i < G; i++)
-                    lm |= (uint32_t)is_lower(su[i], sv, u[i], v) << ((s0 + i) & 31);
+                    sr[i] = scal[s0 + i < d ? (int32_t)row[(s0 + i) * 64] : v];
+#pragma unroll
+                for (int i = 0; i < G; i++)
+                    lm |= (uint32_t)is_lower(sr[i], sv, (int32_t)row[(s0 + i) * 64], v)
+                          << ((s0 + i) & 31);
             }
             const uint32_t om = d >= 32 ? ~0u : (1u << d) - 1u;
             lm &= om;
@@ -1156,23 +1174,23 @@ __global__ __launch_bounds__(1 << BV_LOG, 2) void k_bkt_sort(
             base[0] = ht ? atomicAdd(counters + C_HEAVY, ht) : 0;
             base[1] = ft ? atomicAdd(counters + tg::C_FIXD, ft) : 0;
         }
-        const int32_t v = v0 + tid;
+        const int32_t vt = v0 + tid;
         if (vm) {
-            rowsrc[v] = 3 * cbeg + out + (vh ? xt + yb + yi - y : xb + xi - x);
+            rowsrc[vt] = 3 * cbeg + out + (vh ? xt + yb + yi - y : xb + xi - x);
             if (!vh) {
-                deg[v] = x;
+                deg[vt] = x;
                 if (CP) {
-                    classes[3 * (int64_t)v] = vl;
-                    classes[3 * (int64_t)v + 1] = vu;
-                    classes[3 * (int64_t)v + 2] = verdict(vl, vu);
+                    classes[3 * (int64_t)vt] = vl;
+                    classes[3 * (int64_t)vt + 1] = vu;
+                    classes[3 * (int64_t)vt + 2] = verdict(vl, vu);
                 }
             }
         }
         cur[tid] = xb + xi - x;
         __syncthreads();
         const uint64_t below = (1ull << lane) - 1ull;
-        if (vh) heavy[base[0] + hb + (int32_t)__popcll(hm & below)] = v;
-        if (fx) fixd[base[1] + fb + (int32_t)__popcll(fm & below)] = v;
+        if (vh) heavy[base[0] + hb + (int32_t)__popcll(hm & below)] = vt;
+        if (fx) fixd[base[1] + fb + (int32_t)__popcll(fm & below)] = vt;
         if (ok) {
             uint32_t *to = stage + cur[mv];
             for (int s = 0; s < d; s++) to[s] = row[s * 64];
