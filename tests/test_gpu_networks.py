@@ -81,6 +81,17 @@ def test_relations_at_network_sizes(gpu, drop):
     check_all(gpu, cells[rng.permutation(len(cells))][:T], V, expect_ft=False)
 
 
+@pytest.mark.parametrize("upper", [[1, 2, 4], [13, 14, 15], [29, 30, 31], [60, 61, 62, 63], [254, 300]])
+def test_edges_of_long_rows(gpu, upper):
+    """Every relation on centres with that many cells, so that many + 2 upper
+    neighbours; the ids of a row's edges in any order."""
+    from test_gpu_relations import check_all
+
+    cells, V = fans(upper, ring=400)
+    order = np.random.default_rng(len(upper)).permutation(len(cells))
+    check_all(gpu, np.ascontiguousarray(cells[order]), V, expect_ft=False)
+
+
 @pytest.mark.parametrize("V", [4095, 16384, 16385, 2048 * 4096, 2048 * 4096 + 1])
 def test_offsets_at_scan_forms(gpu, V):
     """A few cells spread over V vertices: the offsets come from one scan."""

@@ -193,6 +193,7 @@ __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
             o.flush();
             continue;
         }
+        for (int32_t i = 0; i < rn; i++) ef[i] = INF;
         for (int32_t k = kb; k < ke; k++) {
             const int32_t p = vtc[k];
             const int32_t t = p >> 2, jv = p & 3;
@@ -249,104 +250,24 @@ __device__ __forceinline__ int32_t rank_of(const uint2 *__restrict__ rank, int32
     return (int32_t)w.y + __popc(w.x & ((1u << (p & 31)) - 1u));
 }
 
-// Lane per vertex v: ids of v's upper edges (VV-aligned) and EV.
-__global__ void k_edge_ids(const int32_t *__restrict__ vv_off, const int32_t *__restrict__ vv,
-                           int64_t V, const int32_t *__restrict__ efirst,
-                           const uint2 *__restrict__ rank, int32_t *__restrict__ vv_eid,
-                           int32_t *__restrict__ ev) {
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t rb = vv_off[v], re = vv_off[v + 1];
-        // eight entries at a time: unconditional loads from clamped indices
-        // (the rank words of an unused lane are those of the row's first
-        // entry), then the writes of the upper entries
-        for (int32_t i0 = rb; i0 < re; i0 += 8) {
-            int32_t u[8], p[8], id[8];
+// EV in id order: a set bit's rank is its edge's id, and its position names the
+// cell and the pair.  Everything is read and written in sequence (ids written
+// from the vertices' side scatter over EV, a line each).  5 M cells: 45 us.
+__global__ void k_ev(const int4 *__restrict__ tv4, int64_t T, const uint2 *__restrict__ rank,
+                     int2 *__restrict__ ev) {
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < T;
+         t += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t p0 = (int32_t)(6 * t), w0 = p0 >> 5, w5 = (p0 + 5) >> 5;
+        const uint2 a = rank[w0], b = w5 != w0 ? rank[w5] : a;
+        const int4 q = tv4[t];
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const int32_t i = min(i0 + c, re - 1);
-                u[c] = vv[i];
-                p[c] = efirst[i];
-            }
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const int on = (int)(i0 + c < re) & (int)(u[c] > v) & (int)(p[c] != INF);
-                const int32_t q = on ? p[c] : 0;
-                const int32_t r = rank_of(rank, q);
-                id[c] = on ? r : -1;
-            }
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                if (id[c] < 0) continue;
-                vv_eid[i0 + c] = id[c];
-                ev[2 * (int64_t)id[c]] = (int32_t)v;
-                ev[2 * (int64_t)id[c] + 1] = u[c];
-            }
-        }
-    }
-}
-
-// VE rows {hi, id}: the upper entries (u > v) of v's VV row, ordered by edge
-// id.  An edge's id ranks its first position, and the reference mints the
-// ids of v's row in the order v's cells first meet its upper neighbours, so
-// ordering by id is the reference's row order.  Rows are sorted in an LDS
-// column (insertion sort) when they fit, else in place in global memory.
-constexpr int VE_THREADS = 64, VE_CAP = 64;
-
-__global__ void k_ve_count(const int32_t *__restrict__ vv_off, const int32_t *__restrict__ vv,
-                           int64_t V, int32_t *__restrict__ cnt) {
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t rb = vv_off[v], rn = vv_off[v + 1] - rb;
-        // entries > v: the row is ascending and never holds v
-        int32_t lo = 0, hi = rn;
-        while (lo < hi) {
-            const int32_t mid = (lo + hi) >> 1;
-            if (vv[rb + mid] < (int32_t)v) lo = mid + 1;
-            else hi = mid;
-        }
-        cnt[v] = rn - lo;
-    }
-}
-
-__global__ __launch_bounds__(VE_THREADS) void k_ve_fill(const int32_t *__restrict__ vv_off,
-                                                        const int32_t *__restrict__ vv,
-                                                        const int32_t *__restrict__ vv_eid,
-                                                        int64_t V, const int32_t *__restrict__ off,
-                                                        int32_t *__restrict__ out) {
-    __shared__ int64_t col[VE_CAP][VE_THREADS];  // (id << 32) | hi
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < V;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t re = vv_off[v + 1];
-        const int32_t n = off[v + 1] - off[v];
-        int32_t *row = out + 2 * (int64_t)off[v];
-        const int32_t ub = re - n;  // first upper entry
-        if (n <= VE_CAP) {
-            for (int32_t k = 0; k < n; k++) {
-                const int64_t key = ((int64_t)vv_eid[ub + k] << 32) | (uint32_t)vv[ub + k];
-                int32_t p = k;
-                while (p > 0 && col[p - 1][threadIdx.x] > key) {
-                    col[p][threadIdx.x] = col[p - 1][threadIdx.x];
-                    p--;
-                }
-                col[p][threadIdx.x] = key;
-            }
-            for (int32_t k = 0; k < n; k++) {  // (hi, id) pairs, one 8-byte store each
-                const int64_t key = col[k][threadIdx.x];
-                reinterpret_cast<int2 *>(row)[k] = make_int2((int32_t)(uint32_t)key, (int32_t)(key >> 32));
-            }
-        } else {
-            for (int32_t k = 0; k < n; k++) {
-                const int32_t id = vv_eid[ub + k], u = vv[ub + k];
-                int32_t p = k;
-                while (p > 0 && row[2 * (p - 1) + 1] > id) {
-                    row[2 * p] = row[2 * (p - 1)];
-                    row[2 * p + 1] = row[2 * (p - 1) + 1];
-                    p--;
-                }
-                row[2 * p] = u;
-                row[2 * p + 1] = id;
-            }
+        for (int k = 0; k < 6; k++) {
+            const int32_t p = p0 + k;
+            const uint2 w = (p >> 5) != w0 ? b : a;
+            if (!((w.x >> (p & 31)) & 1u)) continue;
+            const int pi[6] = {0, 0, 0, 1, 1, 2}, pj[6] = {1, 2, 3, 2, 3, 3};
+            const int32_t x = corner(q, pi[k]), y = corner(q, pj[k]);
+            ev[(int32_t)w.y + __popc(w.x & ((1u << (p & 31)) - 1u))] = make_int2(min(x, y), max(x, y));
         }
     }
 }
@@ -529,63 +450,6 @@ __global__ void k_face_ids(const int4 *__restrict__ tv4, int64_t T,
         // the first position's cell is the smallest holding the face
         ft[2 * (int64_t)id] = t;
         ft[2 * (int64_t)id + 1] = other[p];
-    }
-}
-
-// VF rows {mid, hi, id}: the row of a holds the faces whose positional low
-// vertex is a.  Lane per vertex walks its tets ascending and takes the slots
-// where a sits at the low position and which are their face's first
-// occurrence; positions ascend, so ids ascend.
-template <bool FILL>
-__global__ void k_vf(const int4 *__restrict__ tv4, const int32_t *__restrict__ vt_off,
-                     const int32_t *__restrict__ vtc, int64_t V, const int32_t *__restrict__ ffirst,
-                     const int32_t *__restrict__ tf, int32_t *__restrict__ cnt_or_off,
-                     int32_t *__restrict__ out) {
-    for (int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; a < V;
-         a += (int64_t)gridDim.x * blockDim.x) {
-        int32_t *row = FILL ? out + 3 * (int64_t)cnt_or_off[a] : nullptr;
-        int32_t n = 0;
-        const int32_t kb = vt_off[a], ke = vt_off[a + 1];
-        // eight cells at a time: their slot flags, ids and corners are
-        // loaded together, then the row is written in cell order
-        for (int32_t k0 = kb; k0 < ke; k0 += 8) {
-            int32_t pc[8], ff[8][3], id[8][3];
-            int4 q[8];
-#pragma unroll
-            for (int c = 0; c < 8; c++) pc[c] = k0 + c < ke ? vtc[k0 + c] : -1;
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const int32_t t = pc[c] >> 2, j = pc[c] & 3;
-                // position 0 is low in slots 0-2, position 1 in slot 3
-                const bool on = pc[c] >= 0 && j <= 1;
-#pragma unroll
-                for (int m = 0; m < 3; m++) {
-                    const bool use = on && (j == 0 || m == 0);
-                    const int64_t pos = 4 * (int64_t)t + (j == 0 ? m : 3);
-                    ff[c][m] = use ? ffirst[pos] : -1;
-                    id[c][m] = use && FILL ? tf[pos] : 0;
-                }
-                q[c] = on && FILL ? tv4[t] : make_int4(0, 0, 0, 0);
-            }
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const int32_t t = pc[c] >> 2, j = pc[c] & 3;
-#pragma unroll
-                for (int m = 0; m < 3; m++) {
-                    const int sl = j == 0 ? m : 3;
-                    if (ff[c][m] != 4 * t + sl || ff[c][m] < 0) continue;
-                    if (FILL) {
-                        int lo, mid, hi;
-                        face_pos(sl, lo, mid, hi);
-                        // one 12-byte store per entry
-                        const int32_t ent[3] = {corner(q[c], mid), corner(q[c], hi), id[c][m]};
-                        __builtin_memcpy(row + 3 * n, ent, sizeof ent);
-                    }
-                    n++;
-                }
-            }
-        }
-        if (!FILL) cnt_or_off[a] = n;
     }
 }
 
@@ -1005,6 +869,228 @@ __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ e
     if (e == E - 1) off[E] = base + total;
 }
 
+// VE rows {hi, id}: the upper entries (u > v) of v's VV row, ordered by edge
+// id.  An edge's id ranks its first position, and the reference mints the
+// ids of v's row in the order v's cells first meet its upper neighbours, so
+// ordering by id is the reference's row order.  Lane per vertex: the upper
+// entries are counted for the chained scan, their ids looked up (and kept
+// VV-aligned, for EE) and sorted in registers.  A row of more than 32 upper
+// entries is ordered by the whole wave, each lane counting the smaller ids.
+// Bound by the rank lookups: their words are lines of a table that one XCD's
+// L2 does not hold.  2.2 M cells: 115 us, 5 M: 274; a count, a scan, the
+// ids with EV and a fill by an LDS sort in launches of their own: 160 and 370.
+constexpr int VE_THREADS = 256;
+
+template <int N>
+__device__ __forceinline__ void ve_row(const int32_t *__restrict__ vv,
+                                       const int32_t *__restrict__ efirst,
+                                       const uint2 *__restrict__ rank, int32_t n,
+                                       int32_t *__restrict__ eid, int2 *__restrict__ row) {
+    uint64_t k[N];  // (id << 32) | hi
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        k[i] = ~0ull;
+        if (i < n) {
+            const int32_t id = rank_of(rank, efirst[i]);
+            eid[i] = id;
+            k[i] = ((uint64_t)(uint32_t)id << 32) | (uint32_t)vv[i];
+        }
+    }
+    tgn::sort_keys(k);
+#pragma unroll
+    for (int i = 0; i < N; i++)
+        if (i < n) row[i] = make_int2((int32_t)(uint32_t)k[i], (int32_t)(k[i] >> 32));
+}
+
+__global__ __launch_bounds__(VE_THREADS) void k_ve(const int32_t *__restrict__ vv_off,
+                                                   const int32_t *__restrict__ vv, int64_t V,
+                                                   const int32_t *__restrict__ efirst,
+                                                   const uint2 *__restrict__ rank,
+                                                   int32_t *ticket, uint64_t *state,
+                                                   int32_t *__restrict__ vv_eid,
+                                                   int32_t *__restrict__ off,
+                                                   int2 *__restrict__ out) {
+    __shared__ int32_t wtot[VE_THREADS / 64];
+    __shared__ int32_t shared_tile;
+    __shared__ int64_t base;
+    const int lane = __lane_id(), wid = threadIdx.x / 64;
+    const int32_t tile = take_tile(ticket, shared_tile);
+    const int64_t v = (int64_t)tile * VE_THREADS + threadIdx.x;
+    const bool act = v < V;
+    const int32_t rb = act ? vv_off[v] : 0, re = act ? vv_off[v + 1] : 0;
+    int32_t n = 0;  // entries > v: the row is ascending and never holds v
+    for (int32_t i0 = rb; i0 < re; i0 += 8) {
+        int32_t u[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) u[c] = vv[min(i0 + c, re - 1)];
+#pragma unroll
+        for (int c = 0; c < 8; c++) n += i0 + c < re && u[c] > (int32_t)v;
+    }
+    const int32_t inc = tgd::wave_inclusive_sum(n);
+    if (lane == 63) wtot[wid] = inc;
+    __syncthreads();
+    int32_t before = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < VE_THREADS / 64; i++) {
+        if (i < wid) before += wtot[i];
+        total += wtot[i];
+    }
+    if (wid == 0) {
+        if (lane == 0) tgd::store_agent(state + tile, TILE_SUM | (uint64_t)total);
+        const int64_t b = tiles_before(state, tile);
+        if (lane == 0) {
+            tgd::store_agent(state + tile, TILE_PREFIX | (uint64_t)(b + total));
+            base = b;
+        }
+    }
+    __syncthreads();
+    const int32_t at = (int32_t)base + before + inc - n, ub = re - n;  // first upper entry
+    if (act) off[v] = at;
+    if (v == V - 1) off[V] = (int32_t)base + total;
+    int2 *row = out + at;
+    const int32_t ns = n <= 32 ? n : 0;
+    if (__any(ns > 16)) ve_row<32>(vv + ub, efirst + ub, rank, ns, vv_eid + ub, row);
+    else ve_row<16>(vv + ub, efirst + ub, rank, ns, vv_eid + ub, row);
+    for (uint64_t big = __ballot(n > 32); big; big &= big - 1) {  // the wave on one row
+        const int l = __ffsll((unsigned long long)big) - 1;
+        const int32_t bn = __shfl(n, l), bu = __shfl(ub, l), ba = __shfl(at, l);
+        for (int32_t k0 = 0; k0 < bn; k0 += 64) {
+            const int32_t k = bu + min(k0 + lane, bn - 1);
+            const int32_t id = rank_of(rank, efirst[k]);
+            int32_t p = 0;  // ids below the lane's
+            for (int32_t j0 = 0; j0 < bn; j0 += 64) {
+                const int32_t o = rank_of(rank, efirst[bu + min(j0 + lane, bn - 1)]);
+                for (int32_t j = 0; j < min(64, bn - j0); j++) p += __shfl(o, j) < id;
+            }
+            if (k0 + lane < bn) {
+                vv_eid[k] = id;
+                out[ba + p] = make_int2(vv[k], id);
+            }
+        }
+    }
+}
+
+// VF rows {mid, hi, id}: the row of a holds the faces whose positional low
+// vertex is a.  Lane per vertex walks its tets ascending and takes the slots
+// where a sits at the low position (corner 0: slots 0-2, corner 1: slot 3) and
+// which are their face's first occurrence; positions ascend, so ids ascend.
+// Which slots are first occurrences, and their ids, come from the rank words
+// (8 bytes for eight cells, where the first positions and TF are a line per
+// cell).  The first walk counts and keeps three bits for each of the first 32
+// cells; after the chained scan the second one visits only cells that give a
+// face.  2.2 M cells: 0.25 ms; first positions and TF read instead, in this
+// kernel or in two with a scan between them, 0.38.
+constexpr int VF_THREADS = 256;
+__global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
+                                                   const int32_t *__restrict__ vt_off,
+                                                   const int32_t *__restrict__ vtc, int64_t V,
+                                                   const uint2 *__restrict__ rank,
+                                                   int32_t *ticket,
+                                                   uint64_t *state, int32_t *__restrict__ off,
+                                                   int32_t *__restrict__ out) {
+    __shared__ int32_t wtot[VF_THREADS / 64];
+    __shared__ int32_t shared_tile;
+    __shared__ int64_t base;
+    const int lane = __lane_id(), wid = threadIdx.x / 64;
+    const int32_t tile = take_tile(ticket, shared_tile);
+    const int64_t a = (int64_t)tile * VF_THREADS + threadIdx.x;
+    const bool act = a < V;
+    const int32_t kb = act ? vt_off[a] : 0, ke = act ? vt_off[a + 1] : 0;
+    // slots of cell code p that are first occurrences with a low: bits 0-2, out
+    // of the flags of the code's rank word
+    auto firsts = [&](int32_t p, uint32_t bits) -> uint32_t {
+        const uint32_t f = bits >> (4 * ((p >> 2) & 7));
+        return (p & 3) == 0 ? f & 7u : (p & 3) == 1 ? (f >> 3) & 1u : 0u;
+    };
+    uint32_t m0 = 0, m1 = 0, m2 = 0;  // bit k: the cell's 1st, 2nd, 3rd slot, for the first 32 cells
+    int32_t n = 0;
+    for (int32_t k0 = kb; k0 < ke; k0 += 8) {
+        int32_t p[8];
+        uint32_t ff[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) p[c] = k0 + c < ke ? vtc[k0 + c] : 2;
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+            ff[c] = (p[c] & 3) <= 1 ? rank[p[c] >> 5].x : 0u;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const uint32_t f = firsts(p[c], ff[c]);
+            n += __popc(f);
+            if (k0 + c - kb < 32) {
+                m0 |= (f & 1u) << ((k0 + c - kb) & 31);
+                m1 |= ((f >> 1) & 1u) << ((k0 + c - kb) & 31);
+                m2 |= (f >> 2) << ((k0 + c - kb) & 31);
+            }
+        }
+    }
+    const int32_t inc = tgd::wave_inclusive_sum(n);
+    if (lane == 63) wtot[wid] = inc;
+    __syncthreads();
+    int32_t before = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < VF_THREADS / 64; i++) {
+        if (i < wid) before += wtot[i];
+        total += wtot[i];
+    }
+    if (wid == 0) {
+        if (lane == 0) tgd::store_agent(state + tile, TILE_SUM | (uint64_t)total);
+        const int64_t b = tiles_before(state, tile);
+        if (lane == 0) {
+            tgd::store_agent(state + tile, TILE_PREFIX | (uint64_t)(b + total));
+            base = b;
+        }
+    }
+    __syncthreads();
+    if (!act) return;
+    const int32_t at = (int32_t)base + before + inc - n;
+    off[a] = at;
+    if (a == V - 1) off[V] = (int32_t)base + total;
+    int32_t *row = out + 3 * (int64_t)at;
+    auto write = [&](int32_t p, uint32_t f, const int4 &q, const uint2 &w) {
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            if (!((f >> m) & 1u)) continue;
+            const int sl = (p & 3) == 0 ? m : 3;
+            int lo, mid, hi;
+            face_pos(sl, lo, mid, hi);
+            // one 12-byte store per entry
+            const int bit = (4 * (p >> 2) + sl) & 31;
+            const int32_t id = (int32_t)w.y + __popc(w.x & ((1u << bit) - 1u));
+            const int32_t ent[3] = {corner(q, mid), corner(q, hi), id};
+            __builtin_memcpy(row, ent, sizeof ent);
+            row += 3;
+        }
+    };
+    uint32_t any = m0 | m1 | m2;
+    while (any) {  // eight cells at a time
+        int32_t p[8];
+        uint32_t f[8];
+        int4 q[8];
+        uint2 w[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const int k = any ? __ffs(any) - 1 : 0;
+            f[c] = any ? ((m0 >> k) & 1u) | ((m1 >> k) & 1u) << 1 | ((m2 >> k) & 1u) << 2 : 0u;
+            any &= any - 1u;
+            p[c] = vtc[kb + k];
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            q[c] = tv4[p[c] >> 2];
+            w[c] = rank[p[c] >> 5];
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) write(p[c], f[c], q[c], w[c]);
+    }
+    for (int32_t k = kb + 32; k < ke; k++) {
+        const int32_t p = vtc[k];
+        if ((p & 3) > 1) continue;
+        const uint2 w = rank[p >> 5];
+        const uint32_t f = firsts(p, w.x);
+        if (f) write(p, f, tv4[p >> 2], w);
+    }
+}
+
 // Sum of squared row lengths (VT: the lengths of all cells' four rows
 // together); one atomic per block of few.
 constexpr int SQ_THREADS = 1024, SQ_BLOCKS = 64;
@@ -1085,12 +1171,6 @@ __global__ __launch_bounds__(FF_THREADS) void k_ff(const int32_t *__restrict__ f
     for (int32_t i = tid; i < total; i += FF_THREADS) out[base + i] = rows[i];
 }
 
-__global__ void k_fill_i32v(int32_t *p, int32_t v, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
 __global__ void k_widen(const int32_t *__restrict__ in, int64_t n, int64_t *__restrict__ out) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x)
@@ -1116,10 +1196,11 @@ int read_i64(tg_mesh &m, const void *src, int64_t index, int64_t &out) {
 }
 
 // rank structure over n flags (0 or 1): rank_of(rank, p) is the number of
-// flags set before position p
-// (with, when given, two further words read in the same wait)
-int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank, int64_t &total,
-                const int32_t *two = nullptr, int32_t *two_out = nullptr) {
+// flags set before position p.  total, when asked for, is read back, with two
+// further words in the same wait.
+int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank,
+                int64_t *total = nullptr, const int32_t *two = nullptr,
+                int32_t *two_out = nullptr) {
     const int64_t nw = (n + 31) / 32;
     int rc;
     if ((rc = m.bitmap.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(nw, 1))) ||
@@ -1140,12 +1221,13 @@ int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank, i
                            rank.as<uint2>());
         TG_LAUNCH_CHECK("k_rank_words");
     }
+    if (!total) return tg::OK;
     int32_t *h = (int32_t *)m.h_pinned;
     TG_HIP(hipMemcpyAsync(h, wpre + nw, sizeof(int32_t), hipMemcpyDeviceToHost, m.stream));
     if (two)
         TG_HIP(hipMemcpyAsync(h + 2, two, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, m.stream));
     TG_HIP(hipStreamSynchronize(m.stream));
-    total = h[0];
+    *total = h[0];
     if (two) {
         two_out[0] = h[2];
         two_out[1] = h[3];
@@ -1198,9 +1280,6 @@ int ensure_edges(tg_mesh &m) {
         return rc;
     uint8_t *flags = m.tmp_a.as<uint8_t>();
     if ((rc = fill_u8(flags, 0, 6 * T, m.stream))) return rc;
-    hipLaunchKernelGGL(k_fill_i32v, dim3(grid(nnz)), dim3(256), 0, m.stream,
-                       m.edge_first.as<int32_t>(), INF, nnz);
-    TG_LAUNCH_CHECK("k_fill_i32v");
     if (V > 0) {
         hipLaunchKernelGGL(k_edge_first, dim3(grid(V, EDGE_THREADS)), dim3(EDGE_THREADS), 0, m.stream,
                            m.tv.as<const int4>(), m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(),
@@ -1208,29 +1287,29 @@ int ensure_edges(tg_mesh &m) {
                            m.edge_first.as<int32_t>(), flags, m.te.as<int32_t>());
         TG_LAUNCH_CHECK("k_edge_first");
     }
-    int64_t E = 0;
-    if ((rc = build_ranks(m, flags, 6 * T, m.edge_rank, E))) return rc;
+    const int64_t E = nnz / 2;  // every edge is in both its ends' rows
+    if ((rc = build_ranks(m, flags, 6 * T, m.edge_rank))) return rc;
     m.n_edges = E;
+    const int64_t tiles = (V + VE_THREADS - 1) / VE_THREADS;
+    Chain c;
     if ((rc = m.ev.ensure(I * 2 * (size_t)std::max<int64_t>(E, 1))) ||
-        (rc = m.ve_vals.ensure(I * 2 * (size_t)std::max<int64_t>(E, 1))))
+        (rc = m.ve_vals.ensure(I * 2 * (size_t)std::max<int64_t>(E, 1))) ||
+        (rc = chain_state(m, tiles, c)))
         return rc;
     int32_t *voff = m.ve_off.as<int32_t>();
     if (V > 0) {
-        hipLaunchKernelGGL(k_ve_count, dim3(grid(V)), dim3(256), 0, m.stream,
-                           m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V, voff);
-        TG_LAUNCH_CHECK("k_ve_count");
-    }
-    if ((rc = scan_exclusive_i32(voff, voff, V, m.scan_tmp.p, m.stream))) return rc;
-    if (V > 0) {
-        hipLaunchKernelGGL(k_edge_ids, dim3(grid(V)), dim3(256), 0, m.stream,
+        hipLaunchKernelGGL(k_ve, dim3((unsigned)tiles), dim3(VE_THREADS), 0, m.stream,
                            m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
-                           m.edge_first.as<int32_t>(), m.edge_rank.as<uint2>(),
-                           m.vv_eid.as<int32_t>(), m.ev.as<int32_t>());
-        TG_LAUNCH_CHECK("k_edge_ids");
-        hipLaunchKernelGGL(k_ve_fill, dim3(grid(V, VE_THREADS)), dim3(VE_THREADS), 0, m.stream,
-                           m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(),
-                           m.vv_eid.as<int32_t>(), V, voff, m.ve_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_ve_fill");
+                           m.edge_first.as<int32_t>(), m.edge_rank.as<uint2>(), c.ticket, c.state,
+                           m.vv_eid.as<int32_t>(), voff, m.ve_vals.as<int2>());
+        TG_LAUNCH_CHECK("k_ve");
+    } else if ((rc = fill_i32(voff, 0, 1, m.stream))) {
+        return rc;
+    }
+    if (T > 0) {
+        hipLaunchKernelGGL(k_ev, dim3(grid(T)), dim3(256), 0, m.stream, m.tv.as<const int4>(), T,
+                           m.edge_rank.as<uint2>(), m.ev.as<int2>());
+        TG_LAUNCH_CHECK("k_ev");
     }
     if (T > 0) {
         hipLaunchKernelGGL(k_te, dim3(grid(6 * T)), dim3(256), 0, m.stream, m.te.as<int32_t>(),
@@ -1295,7 +1374,7 @@ int ensure_faces(tg_mesh &m) {
     int64_t F = 0;
     int32_t errs[2] = {0, 0};  // C_FTERR, C_IDERR
     static_assert(C_IDERR == C_FTERR + 1, "read together");
-    if ((rc = build_ranks(m, flags, 4 * T, m.face_rank, F, err, errs))) return rc;
+    if ((rc = build_ranks(m, flags, 4 * T, m.face_rank, &F, err, errs))) return rc;
     if (errs[1]) return fail(ERR_STATE, "face ids: TE and ET disagree (a cell is missing from ET)");
     m.ft_ok = errs[0] == 0;
     m.n_faces = F;
@@ -1310,19 +1389,18 @@ int ensure_faces(tg_mesh &m) {
         TG_LAUNCH_CHECK("k_face_ids");
     }
     int32_t *voff = m.face_off.as<int32_t>();
-    if (V > 0) {
-        hipLaunchKernelGGL((k_vf<false>), dim3(grid(V)), dim3(256), 0, m.stream,
-                           m.tv.as<const int4>(), m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(), V,
-                           ffirst, m.tf.as<int32_t>(), voff, nullptr);
-        TG_LAUNCH_CHECK("k_vf count");
-    }
-    if ((rc = scan_exclusive_i32(voff, voff, V, m.scan_tmp.p, m.stream))) return rc;
     if ((rc = m.vf_vals.ensure(I * 3 * (size_t)std::max<int64_t>(F, 1)))) return rc;
     if (V > 0) {
-        hipLaunchKernelGGL((k_vf<true>), dim3(grid(V)), dim3(256), 0, m.stream,
+        const int64_t tiles = (V + VF_THREADS - 1) / VF_THREADS;
+        Chain c;
+        if ((rc = chain_state(m, tiles, c))) return rc;
+        hipLaunchKernelGGL(k_vf, dim3((unsigned)tiles), dim3(VF_THREADS), 0, m.stream,
                            m.tv.as<const int4>(), m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(), V,
-                           ffirst, m.tf.as<int32_t>(), voff, m.vf_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_vf fill");
+                           m.face_rank.as<uint2>(), c.ticket, c.state, voff,
+                           m.vf_vals.as<int32_t>());
+        TG_LAUNCH_CHECK("k_vf");
+    } else if ((rc = fill_i32(voff, 0, 1, m.stream))) {
+        return rc;
     }
     m.face_rank.release();
     m.faces_built = true;
