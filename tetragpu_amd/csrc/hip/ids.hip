@@ -6,9 +6,8 @@
 // (1,2) (1,3) (2,3)) among all edges' first positions.  One lane per vertex
 // v walks v's tets in ascending order and records, for every upper
 // neighbour u > v (an entry of the ascending VV row), the first position it
-// meets; first positions are flagged in a byte array, packed to a bitmap
-// whose word popcounts are scanned, and an edge's id is the rank of its
-// first position.  No atomics.
+// meets; first positions are flagged in a byte array, packed to bits with
+// scanned counts, and an edge's id is the rank of its first position.  No atomics.
 //
 // Faces (src/cpu_extraction.cpp:122-222): slot s of cell c is the positional
 // triple (cv[lo], cv[mid], cv[hi]) with (lo, mid, hi) = (0,1,2) (0,1,3)
@@ -17,10 +16,10 @@
 // key is the smallest position among those cells' slots with the same
 // positional triple, and face ids are ranks of first occurrences.
 //
-// The remaining relations are two-pass CSR builds (count, scan, fill) over
-// sorted rows, or joins with a chained scan (ET(e) = VT(lo) n VT(hi), TT, EE);
-// EF, FF by merging sorted
-// lists; FT from the face matches.
+// The other relations with rows count, scan and write in one launch each (a
+// chained scan over tiles): ET(e) = VT(lo) n VT(hi), TT and EE as joins, VE
+// and VF from a vertex's VV row and cells, EF and FF from TE and TF; FT comes
+// from the face matches.
 #include <algorithm>
 
 #include "ids.h"
@@ -212,84 +211,120 @@ __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
     }
 }
 
-// bytes (0 or 1) -> bitmap words and their popcounts.  32 bytes per lane in
-// two 16-byte loads; the multiplication gathers the low bits of four bytes
-// (bit 8 i moves to bit 28 + i; no other product bit reaches 28).
+// Rank units: 96 flags and the number of flags set before them in 16 bytes, so
+// a random lookup touches one line, and 5 bytes of table hold 30 flags, where
+// a count per 32-bit word takes 7.5 and keeps less of the table in each L2
+// (VE of 5 M cells 274 -> 202 us, EE's rows 233 -> 132, TE 152 -> 141).
+// 96 holds whole cells' flags, for edges (6) and for faces (4).
+constexpr int UNIT = 96;
+
+// bytes (0 or 1) -> a unit's flag words (y, z, w) and their number.  16-byte
+// loads; the multiplication gathers the low bits of four bytes (bit 8 i moves
+// to bit 28 + i; no other product bit reaches 28).
 __global__ void k_pack_flags(const uint8_t *__restrict__ flags, int64_t n,
-                             uint32_t *__restrict__ bits, int32_t *__restrict__ pop) {
-    const int64_t nw = (n + 31) / 32;
-    for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w < nw;
-         w += (int64_t)gridDim.x * blockDim.x) {
-        uint32_t m = 0;
-        const int64_t b = 32 * w;
-        if (b + 32 <= n) {
+                             uint4 *__restrict__ rank, int32_t *__restrict__ pop) {
+    const int64_t nu = (n + UNIT - 1) / UNIT;
+    for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < nu;
+         u += (int64_t)gridDim.x * blockDim.x) {
+        uint32_t m[3] = {0, 0, 0};
+        const int64_t b = UNIT * u;
+        if (b + UNIT <= n) {
             const uint4 *p = reinterpret_cast<const uint4 *>(flags + b);
-            const uint4 q0 = p[0], q1 = p[1];
-            const uint32_t x[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
-            for (int i = 0; i < 8; i++) m |= ((x[i] * 0x10204080u) >> 28) << (4 * i);
+            for (int w = 0; w < 3; w++) {
+                const uint4 q0 = p[2 * w], q1 = p[2 * w + 1];
+                const uint32_t x[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+                for (int i = 0; i < 8; i++) m[w] |= ((x[i] * 0x10204080u) >> 28) << (4 * i);
+            }
         } else {
-            for (int i = 0; i < 32 && b + i < n; i++) m |= (uint32_t)(flags[b + i] != 0) << i;
+#pragma unroll
+            for (int w = 0; w < 3; w++)
+                for (int i = 0; i < 32 && b + 32 * w + i < n; i++)
+                    m[w] |= (uint32_t)(flags[b + 32 * w + i] != 0) << i;
         }
-        bits[w] = m;
-        pop[w] = __popc(m);
+        rank[u] = make_uint4(0u, m[0], m[1], m[2]);
+        pop[u] = __popc(m[0]) + __popc(m[1]) + __popc(m[2]);
     }
 }
 
-// A bitmap word and the number of set bits before it, side by side: a random
-// rank lookup touches one line instead of two.
-__global__ void k_rank_words(const uint32_t *__restrict__ bits, const int32_t *__restrict__ wpre,
-                             int64_t nw, uint2 *__restrict__ rank) {
-    for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w < nw;
-         w += (int64_t)gridDim.x * blockDim.x)
-        rank[w] = make_uint2(bits[w], (uint32_t)wpre[w]);
+__global__ void k_rank_counts(const int32_t *__restrict__ before, int64_t nu,
+                              uint4 *__restrict__ rank) {
+    for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < nu;
+         u += (int64_t)gridDim.x * blockDim.x)
+        rank[u].x = (uint32_t)before[u];
 }
 
-__device__ __forceinline__ int32_t rank_of(const uint2 *__restrict__ rank, int32_t p) {
-    const uint2 w = rank[p >> 5];
-    return (int32_t)w.y + __popc(w.x & ((1u << (p & 31)) - 1u));
+// flags set before place i (0 .. 95) of a unit
+__device__ __forceinline__ int32_t rank_in(uint4 q, uint32_t i) {
+    const uint32_t a = q.y, b = q.z, c = q.w;
+    const uint32_t w = i < 32 ? a : i < 64 ? b : c;
+    return (int32_t)q.x + __popc(w & ((1u << (i & 31)) - 1u)) + (i >= 32 ? __popc(a) : 0) +
+           (i >= 64 ? __popc(b) : 0);
 }
 
-// EV in id order: a set bit's rank is its edge's id, and its position names the
-// cell and the pair.  Everything is read and written in sequence (ids written
-// from the vertices' side scatter over EV, a line each).  5 M cells: 45 us.
-__global__ void k_ev(const int4 *__restrict__ tv4, int64_t T, const uint2 *__restrict__ rank,
+__device__ __forceinline__ int32_t rank_of(const uint4 *__restrict__ rank, int32_t p) {
+    const uint32_t u = (uint32_t)p / UNIT;
+    return rank_in(rank[u], (uint32_t)p - UNIT * u);
+}
+
+// an edge's id; -1 for an entry that no cell gave a position
+__device__ __forceinline__ int32_t rank_at(const uint4 *__restrict__ rank, int32_t p) {
+    return p != INF ? rank_of(rank, p) : -1;
+}
+
+// TE: the first positions that k_edge_first recorded become edge ids.  A
+// position per lane, read and written in whole lines: 141 us at 5 M cells (a
+// cell per lane, its six lookups in flight and EV in the same launch, took 212
+// against 141 + 41).
+__global__ void k_te(int32_t *__restrict__ te, int64_t n, const uint4 *__restrict__ rank) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x)
+        te[i] = rank_at(rank, te[i]);
+}
+
+// EV in id order: a set flag's rank is its edge's id, and its place names the
+// cell and the pair, so EV is written in sequence (from the vertices' side it
+// is a line per id).  5 M cells: 41 us.
+__global__ void k_ev(const int4 *__restrict__ tv4, int64_t T, const uint4 *__restrict__ rank,
                      int2 *__restrict__ ev) {
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < T;
          t += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t p0 = (int32_t)(6 * t), w0 = p0 >> 5, w5 = (p0 + 5) >> 5;
-        const uint2 a = rank[w0], b = w5 != w0 ? rank[w5] : a;
+        const uint4 w = rank[t / (UNIT / 6)];
+        const uint32_t i = 6 * (uint32_t)(t % (UNIT / 6));  // a cell's flags are in one unit
+        const uint32_t lo = i < 32 ? w.y : i < 64 ? w.z : w.w;
+        const uint32_t hi = i < 32 ? w.z : i < 64 ? w.w : 0u;
+        const uint32_t f = (uint32_t)((((uint64_t)hi << 32) | lo) >> (i & 31)) & 63u;
         const int4 q = tv4[t];
+        const int32_t id = rank_in(w, i);
 #pragma unroll
         for (int k = 0; k < 6; k++) {
-            const int32_t p = p0 + k;
-            const uint2 w = (p >> 5) != w0 ? b : a;
-            if (!((w.x >> (p & 31)) & 1u)) continue;
+            if (!((f >> k) & 1u)) continue;
             const int pi[6] = {0, 0, 0, 1, 1, 2}, pj[6] = {1, 2, 3, 2, 3, 3};
             const int32_t x = corner(q, pi[k]), y = corner(q, pj[k]);
-            ev[(int32_t)w.y + __popc(w.x & ((1u << (p & 31)) - 1u))] = make_int2(min(x, y), max(x, y));
+            ev[id + __popc(f & ((1u << k) - 1u))] = make_int2(min(x, y), max(x, y));
         }
     }
 }
 
-// Each vertex's edge ids, ascending (for EE): the upper entries' ids are in
-// vv_eid, a lower entry's is the rank of its first position, which
-// k_edge_first noted for both ends of an edge.  (Searching v in each lower
-// neighbour's row took 0.63 ms at 5.3 M cells, and sorting the rows in memory
-// 0.28; this pass 0.19.)  Rows of up to 32 entries are sorted in registers,
-// longer ones in memory.
-__global__ __launch_bounds__(256) void k_vertex_edges(const int32_t *__restrict__ vv_off,
-                                                      const int32_t *__restrict__ vv, int64_t V,
+// Each vertex's edge ids, ascending (for EE): the upper entries' ids are VE's,
+// a lower entry's is the rank of its first position, which k_edge_first noted
+// for both ends of an edge.  (Searching v in each lower neighbour's row took
+// 0.63 ms at 5.3 M cells, and sorting the rows in memory 0.28; VE's
+// ids from a copy along VV and a count per 32-bit word 0.23; this pass 0.13.)  Rows of up to 32 entries are sorted in registers, longer ones in
+// memory.
+__global__ __launch_bounds__(256) void k_vertex_edges(const int32_t *__restrict__ vv_off, int64_t V,
                                                       const int32_t *__restrict__ efirst,
-                                                      const uint2 *__restrict__ rank,
-                                                      const int32_t *__restrict__ vv_eid,
+                                                      const uint4 *__restrict__ rank,
+                                                      const int32_t *__restrict__ ve_off,
+                                                      const int2 *__restrict__ ve,
                                                       int32_t *__restrict__ out) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V) return;
     const int32_t rb = vv_off[v], rn = vv_off[v + 1] - rb;
+    const int32_t vb = ve_off[v], lower = rn - (ve_off[v + 1] - vb);
     auto id_of = [&](int32_t i) {
-        const int32_t p = efirst[i];
-        return vv[i] > (int32_t)v ? vv_eid[i] : p != INF ? rank_of(rank, p) : -1;
+        return i < rb + lower ? rank_at(rank, efirst[i]) : ve[vb + (i - rb - lower)].y;
     };
     if (rn <= 32) {
         int32_t k[32];
@@ -306,15 +341,6 @@ __global__ __launch_bounds__(256) void k_vertex_edges(const int32_t *__restrict_
             for (; j > 0 && out[rb + j - 1] > x; j--) out[rb + j] = out[rb + j - 1];
             out[rb + j] = x;
         }
-    }
-}
-
-// TE: the first positions recorded by k_edge_first become edge ids
-__global__ void k_te(int32_t *__restrict__ te, int64_t n, const uint2 *__restrict__ rank) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t p = te[i];
-        te[i] = p != INF ? rank_of(rank, p) : -1;
     }
 }
 
@@ -431,7 +457,7 @@ __global__ void k_face_first(const int4 *__restrict__ tv4, int64_t T, const int3
 // FT (<= 2 tets, ascending, -1 pad)
 __global__ void k_face_ids(const int4 *__restrict__ tv4, int64_t T,
                            const int32_t *__restrict__ ffirst, const int32_t *__restrict__ other,
-                           const uint2 *__restrict__ rank, int32_t *__restrict__ tf,
+                           const uint4 *__restrict__ rank, int32_t *__restrict__ tf,
                            int32_t *__restrict__ fv, int32_t *__restrict__ ft) {
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < 4 * T;
          p += (int64_t)gridDim.x * blockDim.x) {
@@ -873,26 +899,26 @@ __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ e
 // id.  An edge's id ranks its first position, and the reference mints the
 // ids of v's row in the order v's cells first meet its upper neighbours, so
 // ordering by id is the reference's row order.  Lane per vertex: the upper
-// entries are counted for the chained scan, their ids looked up (and kept
-// VV-aligned, for EE) and sorted in registers.  A row of more than 32 upper
+// entries are counted for the chained scan, their ids looked up and sorted in
+// registers.  A row of more than 32 upper
 // entries is ordered by the whole wave, each lane counting the smaller ids.
 // Bound by the rank lookups: their words are lines of a table that one XCD's
-// L2 does not hold.  2.2 M cells: 115 us, 5 M: 274; a count, a scan, the
-// ids with EV and a fill by an LDS sort in launches of their own: 160 and 370.
+// L2 does not hold.  2.2 M cells: 81 us, 5 M: 202; a count, a scan, the
+// ids with EV and a fill by an LDS sort in launches of their own: 142 (with EV's
+// 16) and 340 (41).
 constexpr int VE_THREADS = 256;
 
 template <int N>
 __device__ __forceinline__ void ve_row(const int32_t *__restrict__ vv,
                                        const int32_t *__restrict__ efirst,
-                                       const uint2 *__restrict__ rank, int32_t n,
-                                       int32_t *__restrict__ eid, int2 *__restrict__ row) {
+                                       const uint4 *__restrict__ rank, int32_t n,
+                                       int2 *__restrict__ row) {
     uint64_t k[N];  // (id << 32) | hi
 #pragma unroll
     for (int i = 0; i < N; i++) {
         k[i] = ~0ull;
         if (i < n) {
-            const int32_t id = rank_of(rank, efirst[i]);
-            eid[i] = id;
+            const int32_t id = rank_at(rank, efirst[i]);
             k[i] = ((uint64_t)(uint32_t)id << 32) | (uint32_t)vv[i];
         }
     }
@@ -905,9 +931,8 @@ __device__ __forceinline__ void ve_row(const int32_t *__restrict__ vv,
 __global__ __launch_bounds__(VE_THREADS) void k_ve(const int32_t *__restrict__ vv_off,
                                                    const int32_t *__restrict__ vv, int64_t V,
                                                    const int32_t *__restrict__ efirst,
-                                                   const uint2 *__restrict__ rank,
+                                                   const uint4 *__restrict__ rank,
                                                    int32_t *ticket, uint64_t *state,
-                                                   int32_t *__restrict__ vv_eid,
                                                    int32_t *__restrict__ off,
                                                    int2 *__restrict__ out) {
     __shared__ int32_t wtot[VE_THREADS / 64];
@@ -949,23 +974,20 @@ __global__ __launch_bounds__(VE_THREADS) void k_ve(const int32_t *__restrict__ v
     if (v == V - 1) off[V] = (int32_t)base + total;
     int2 *row = out + at;
     const int32_t ns = n <= 32 ? n : 0;
-    if (__any(ns > 16)) ve_row<32>(vv + ub, efirst + ub, rank, ns, vv_eid + ub, row);
-    else ve_row<16>(vv + ub, efirst + ub, rank, ns, vv_eid + ub, row);
+    if (__any(ns > 16)) ve_row<32>(vv + ub, efirst + ub, rank, ns, row);
+    else ve_row<16>(vv + ub, efirst + ub, rank, ns, row);
     for (uint64_t big = __ballot(n > 32); big; big &= big - 1) {  // the wave on one row
         const int l = __ffsll((unsigned long long)big) - 1;
         const int32_t bn = __shfl(n, l), bu = __shfl(ub, l), ba = __shfl(at, l);
         for (int32_t k0 = 0; k0 < bn; k0 += 64) {
             const int32_t k = bu + min(k0 + lane, bn - 1);
-            const int32_t id = rank_of(rank, efirst[k]);
+            const int32_t id = rank_at(rank, efirst[k]);
             int32_t p = 0;  // ids below the lane's
             for (int32_t j0 = 0; j0 < bn; j0 += 64) {
-                const int32_t o = rank_of(rank, efirst[bu + min(j0 + lane, bn - 1)]);
+                const int32_t o = rank_at(rank, efirst[bu + min(j0 + lane, bn - 1)]);
                 for (int32_t j = 0; j < min(64, bn - j0); j++) p += __shfl(o, j) < id;
             }
-            if (k0 + lane < bn) {
-                vv_eid[k] = id;
-                out[ba + p] = make_int2(vv[k], id);
-            }
+            if (k0 + lane < bn) out[ba + p] = make_int2(vv[k], id);
         }
     }
 }
@@ -974,17 +996,17 @@ __global__ __launch_bounds__(VE_THREADS) void k_ve(const int32_t *__restrict__ v
 // vertex is a.  Lane per vertex walks its tets ascending and takes the slots
 // where a sits at the low position (corner 0: slots 0-2, corner 1: slot 3) and
 // which are their face's first occurrence; positions ascend, so ids ascend.
-// Which slots are first occurrences, and their ids, come from the rank words
-// (8 bytes for eight cells, where the first positions and TF are a line per
+// Which slots are first occurrences, and their ids, come from the rank units
+// (16 bytes for 24 cells, where the first positions and TF are a line per
 // cell).  The first walk counts and keeps three bits for each of the first 32
 // cells; after the chained scan the second one visits only cells that give a
-// face.  2.2 M cells: 0.25 ms; first positions and TF read instead, in this
+// face.  2.2 M cells: 0.23 ms; first positions and TF read instead, in this
 // kernel or in two with a scan between them, 0.38.
 constexpr int VF_THREADS = 256;
 __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
                                                    const int32_t *__restrict__ vt_off,
                                                    const int32_t *__restrict__ vtc, int64_t V,
-                                                   const uint2 *__restrict__ rank,
+                                                   const uint4 *__restrict__ rank,
                                                    int32_t *ticket,
                                                    uint64_t *state, int32_t *__restrict__ off,
                                                    int32_t *__restrict__ out) {
@@ -997,9 +1019,14 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
     const bool act = a < V;
     const int32_t kb = act ? vt_off[a] : 0, ke = act ? vt_off[a + 1] : 0;
     // slots of cell code p that are first occurrences with a low: bits 0-2, out
-    // of the flags of the code's rank word
+    // of the flags of the cell's rank unit
+    constexpr uint32_t CELLS = UNIT / 4;
+    auto word = [&](int32_t p) {  // the cell's flags are in one word
+        const uint32_t t = (uint32_t)p >> 2, u = t / CELLS;
+        return (const uint32_t *)(rank + u) + 1 + (t - CELLS * u) / 8;
+    };
     auto firsts = [&](int32_t p, uint32_t bits) -> uint32_t {
-        const uint32_t f = bits >> (4 * ((p >> 2) & 7));
+        const uint32_t t = (uint32_t)p >> 2, f = bits >> (4 * (t % CELLS % 8));
         return (p & 3) == 0 ? f & 7u : (p & 3) == 1 ? (f >> 3) & 1u : 0u;
     };
     uint32_t m0 = 0, m1 = 0, m2 = 0;  // bit k: the cell's 1st, 2nd, 3rd slot, for the first 32 cells
@@ -1011,7 +1038,7 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
         for (int c = 0; c < 8; c++) p[c] = k0 + c < ke ? vtc[k0 + c] : 2;
 #pragma unroll
         for (int c = 0; c < 8; c++)
-            ff[c] = (p[c] & 3) <= 1 ? rank[p[c] >> 5].x : 0u;
+            ff[c] = (p[c] & 3) <= 1 ? *word(p[c]) : 0u;
 #pragma unroll
         for (int c = 0; c < 8; c++) {
             const uint32_t f = firsts(p[c], ff[c]);
@@ -1046,7 +1073,7 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
     off[a] = at;
     if (a == V - 1) off[V] = (int32_t)base + total;
     int32_t *row = out + 3 * (int64_t)at;
-    auto write = [&](int32_t p, uint32_t f, const int4 &q, const uint2 &w) {
+    auto write = [&](int32_t p, uint32_t f, const int4 q, const uint4 w) {
 #pragma unroll
         for (int m = 0; m < 3; m++) {
             if (!((f >> m) & 1u)) continue;
@@ -1054,8 +1081,7 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
             int lo, mid, hi;
             face_pos(sl, lo, mid, hi);
             // one 12-byte store per entry
-            const int bit = (4 * (p >> 2) + sl) & 31;
-            const int32_t id = (int32_t)w.y + __popc(w.x & ((1u << bit) - 1u));
+            const int32_t id = rank_in(w, 4 * (((uint32_t)p >> 2) % CELLS) + sl);
             const int32_t ent[3] = {corner(q, mid), corner(q, hi), id};
             __builtin_memcpy(row, ent, sizeof ent);
             row += 3;
@@ -1066,7 +1092,7 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
         int32_t p[8];
         uint32_t f[8];
         int4 q[8];
-        uint2 w[8];
+        uint4 w[8];
 #pragma unroll
         for (int c = 0; c < 8; c++) {
             const int k = any ? __ffs(any) - 1 : 0;
@@ -1077,7 +1103,7 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
 #pragma unroll
         for (int c = 0; c < 8; c++) {
             q[c] = tv4[p[c] >> 2];
-            w[c] = rank[p[c] >> 5];
+            w[c] = rank[((uint32_t)p[c] >> 2) / CELLS];
         }
 #pragma unroll
         for (int c = 0; c < 8; c++) write(p[c], f[c], q[c], w[c]);
@@ -1085,9 +1111,8 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
     for (int32_t k = kb + 32; k < ke; k++) {
         const int32_t p = vtc[k];
         if ((p & 3) > 1) continue;
-        const uint2 w = rank[p >> 5];
-        const uint32_t f = firsts(p, w.x);
-        if (f) write(p, f, tv4[p >> 2], w);
+        const uint32_t f = firsts(p, *word(p));
+        if (f) write(p, f, tv4[p >> 2], rank[((uint32_t)p >> 2) / CELLS]);
     }
 }
 
@@ -1201,29 +1226,27 @@ int read_i64(tg_mesh &m, const void *src, int64_t index, int64_t &out) {
 int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank,
                 int64_t *total = nullptr, const int32_t *two = nullptr,
                 int32_t *two_out = nullptr) {
-    const int64_t nw = (n + 31) / 32;
+    const int64_t nu = (n + UNIT - 1) / UNIT;
     int rc;
-    if ((rc = m.bitmap.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(nw, 1))) ||
-        (rc = m.rank_tmp.ensure(sizeof(int32_t) * (size_t)(nw + 1))) ||
-        (rc = rank.ensure(sizeof(uint2) * (size_t)std::max<int64_t>(nw, 1))) ||
-        (rc = m.scan_tmp.ensure(tg::scan_tmp_bytes(nw))))
+    if ((rc = m.rank_tmp.ensure(sizeof(int32_t) * (size_t)(nu + 1))) ||
+        (rc = rank.ensure(sizeof(uint4) * (size_t)std::max<int64_t>(nu, 1))) ||
+        (rc = m.scan_tmp.ensure(tg::scan_tmp_bytes(nu))))
         return rc;
-    uint32_t *bits = m.bitmap.as<uint32_t>();
-    int32_t *wpre = m.rank_tmp.as<int32_t>();
-    if (nw > 0) {
-        hipLaunchKernelGGL(k_pack_flags, dim3(grid(nw)), dim3(256), 0, m.stream, flags, n, bits,
-                           wpre);
+    int32_t *before = m.rank_tmp.as<int32_t>();
+    if (nu > 0) {
+        hipLaunchKernelGGL(k_pack_flags, dim3(grid(nu)), dim3(256), 0, m.stream, flags, n,
+                           rank.as<uint4>(), before);
         TG_LAUNCH_CHECK("k_pack_flags");
     }
-    if ((rc = tg::scan_exclusive_i32(wpre, wpre, nw, m.scan_tmp.p, m.stream))) return rc;
-    if (nw > 0) {
-        hipLaunchKernelGGL(k_rank_words, dim3(grid(nw)), dim3(256), 0, m.stream, bits, wpre, nw,
-                           rank.as<uint2>());
-        TG_LAUNCH_CHECK("k_rank_words");
+    if ((rc = tg::scan_exclusive_i32(before, before, nu, m.scan_tmp.p, m.stream))) return rc;
+    if (nu > 0) {
+        hipLaunchKernelGGL(k_rank_counts, dim3(grid(nu)), dim3(256), 0, m.stream, before, nu,
+                           rank.as<uint4>());
+        TG_LAUNCH_CHECK("k_rank_counts");
     }
     if (!total) return tg::OK;
     int32_t *h = (int32_t *)m.h_pinned;
-    TG_HIP(hipMemcpyAsync(h, wpre + nw, sizeof(int32_t), hipMemcpyDeviceToHost, m.stream));
+    TG_HIP(hipMemcpyAsync(h, before + nu, sizeof(int32_t), hipMemcpyDeviceToHost, m.stream));
     if (two)
         TG_HIP(hipMemcpyAsync(h + 2, two, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, m.stream));
     TG_HIP(hipStreamSynchronize(m.stream));
@@ -1273,7 +1296,6 @@ int ensure_edges(tg_mesh &m) {
         return rc;
     const size_t I = sizeof(int32_t);
     if ((rc = m.edge_first.ensure(I * (size_t)std::max<int64_t>(nnz, 1))) ||
-        (rc = m.vv_eid.ensure(I * (size_t)std::max<int64_t>(nnz, 1))) ||
         (rc = m.te.ensure(I * 6 * (size_t)std::max<int64_t>(T, 1))) ||
         (rc = m.tmp_a.ensure(std::max<size_t>(6 * (size_t)T, 1))) ||  // flags
         (rc = m.ve_off.ensure(I * (size_t)(V + 1))))
@@ -1300,21 +1322,19 @@ int ensure_edges(tg_mesh &m) {
     if (V > 0) {
         hipLaunchKernelGGL(k_ve, dim3((unsigned)tiles), dim3(VE_THREADS), 0, m.stream,
                            m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
-                           m.edge_first.as<int32_t>(), m.edge_rank.as<uint2>(), c.ticket, c.state,
-                           m.vv_eid.as<int32_t>(), voff, m.ve_vals.as<int2>());
+                           m.edge_first.as<int32_t>(), m.edge_rank.as<uint4>(), c.ticket, c.state,
+                           voff, m.ve_vals.as<int2>());
         TG_LAUNCH_CHECK("k_ve");
     } else if ((rc = fill_i32(voff, 0, 1, m.stream))) {
         return rc;
     }
     if (T > 0) {
-        hipLaunchKernelGGL(k_ev, dim3(grid(T)), dim3(256), 0, m.stream, m.tv.as<const int4>(), T,
-                           m.edge_rank.as<uint2>(), m.ev.as<int2>());
-        TG_LAUNCH_CHECK("k_ev");
-    }
-    if (T > 0) {
         hipLaunchKernelGGL(k_te, dim3(grid(6 * T)), dim3(256), 0, m.stream, m.te.as<int32_t>(),
-                           6 * T, m.edge_rank.as<uint2>());
+                           6 * T, m.edge_rank.as<uint4>());
         TG_LAUNCH_CHECK("k_te");
+        hipLaunchKernelGGL(k_ev, dim3(grid(T)), dim3(256), 0, m.stream, m.tv.as<const int4>(), T,
+                           m.edge_rank.as<uint4>(), m.ev.as<int2>());
+        TG_LAUNCH_CHECK("k_ev");
     }
     m.edges_built = true;
     return OK;
@@ -1384,7 +1404,7 @@ int ensure_faces(tg_mesh &m) {
         return rc;
     if (T > 0) {
         hipLaunchKernelGGL(k_face_ids, dim3(grid(4 * T)), dim3(256), 0, m.stream,
-                           m.tv.as<const int4>(), T, ffirst, other, m.face_rank.as<uint2>(),
+                           m.tv.as<const int4>(), T, ffirst, other, m.face_rank.as<uint4>(),
                            m.tf.as<int32_t>(), m.fv.as<int32_t>(), m.ft.as<int32_t>());
         TG_LAUNCH_CHECK("k_face_ids");
     }
@@ -1396,7 +1416,7 @@ int ensure_faces(tg_mesh &m) {
         if ((rc = chain_state(m, tiles, c))) return rc;
         hipLaunchKernelGGL(k_vf, dim3((unsigned)tiles), dim3(VF_THREADS), 0, m.stream,
                            m.tv.as<const int4>(), m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(), V,
-                           m.face_rank.as<uint2>(), c.ticket, c.state, voff,
+                           m.face_rank.as<uint4>(), c.ticket, c.state, voff,
                            m.vf_vals.as<int32_t>());
         TG_LAUNCH_CHECK("k_vf");
     } else if ((rc = fill_i32(voff, 0, 1, m.stream))) {
@@ -1529,9 +1549,9 @@ int ensure_ee(tg_mesh &m) {
     int64_t nnz = 0;
     if (E > 0) {
         hipLaunchKernelGGL(k_vertex_edges, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, m.stream,
-                           m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
-                           m.edge_first.as<int32_t>(), m.edge_rank.as<uint2>(),
-                           m.vv_eid.as<int32_t>(), m.tmp_c.as<int32_t>());
+                           m.vv_off.as<int32_t>(), V, m.edge_first.as<int32_t>(),
+                           m.edge_rank.as<uint4>(), m.ve_off.as<int32_t>(), m.ve_vals.as<int2>(),
+                           m.tmp_c.as<int32_t>());
         TG_LAUNCH_CHECK("k_vertex_edges");
         // an edge's row: its ends' edges, which share only itself
         if ((rc = row_squares(m, m.vv_off.as<int32_t>(), V, c, nnz))) return rc;

@@ -59,10 +59,10 @@ struct tg_mesh {
 
     // id-assigning and derived relations
     tg::DevArr vt_vals;
-    tg::DevArr edge_first, ve_off, ve_vals, ev, te, vv_eid, et_off, et_vals;
+    tg::DevArr edge_first, ve_off, ve_vals, ev, te, et_off, et_vals;
     tg::DevArr face_off, vf_vals, fv, tf, fe, ft, ef_off, ef_vals;
     tg::DevArr tt_off, tt_vals, ff_off, ff_vals, ee_off, ee_vals;
-    tg::DevArr bitmap, rank_tmp, edge_rank, face_rank, tmp_a, tmp_b, tmp_c;
+    tg::DevArr rank_tmp, edge_rank, face_rank, tmp_a, tmp_b, tmp_c;
     bool edges_built = false, faces_built = false, vt_built = false, et_built = false,
          fe_built = false, ft_built = false, ef_built = false, tt_built = false,
          ff_built = false, ee_built = false;

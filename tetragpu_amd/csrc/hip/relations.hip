@@ -40,10 +40,10 @@ static void release_all_impl(tg_mesh *m, hipStream_t s, bool release, bool idle)
     tg::DevArr *all[] = {&me.tv,       &me.scal,     &me.vt_cnt,   &me.vt_off,   &me.vt_cur,   &me.vtc,
                          &me.scratch,  &me.deg,      &me.vv_off,   &me.vv_cols,  &me.classes,  &me.heavy,
                          &me.fix,      &me.fixbig,   &me.counters, &me.scan_tmp, &me.labels,   &me.vt_vals,
-                         &me.edge_first, &me.ve_off, &me.ve_vals,  &me.ev,       &me.te,       &me.vv_eid,
+                         &me.edge_first, &me.ve_off, &me.ve_vals,  &me.ev,       &me.te,
                          &me.et_off,   &me.et_vals,  &me.face_off, &me.vf_vals,  &me.fv,       &me.tf,
                          &me.fe,       &me.ft,       &me.ef_off,   &me.ef_vals,  &me.tt_off,   &me.tt_vals,
-                         &me.ff_off,   &me.ff_vals,  &me.ee_off,   &me.ee_vals,  &me.bitmap,   &me.rank_tmp, &me.edge_rank, &me.face_rank,
+                         &me.ff_off,   &me.ff_vals,  &me.ee_off,   &me.ee_vals,  &me.rank_tmp, &me.edge_rank, &me.face_rank,
                          &me.tmp_a,    &me.tmp_b,    &me.tmp_c,    &me.bk_h1,    &me.bk_h2,    &me.bk_rowsrc,
                          &me.bk_fixd,  &me.bk_rowdesc, &me.bk_rec};
     for (auto *a : all) {
