@@ -69,7 +69,7 @@ def valu_busy(workload: str, dom_ms: float):
     v = load_valu(workload)
     if not v or dom_ms <= 0:
         return None
-    k = next((x for n, x in v["kernels"].items() if n.startswith("k_bkt_vv_cp")), None)
+    k = next((x for n, x in v["kernels"].items() if n.startswith("k_bkt_sort")), None)
     if not k:
         return None
     return round(k["SQ_INSTS_VALU"] * 4 / (dom_ms * 1e-3 * v["clock_hz"] * v["simds"]), 3)
@@ -173,7 +173,7 @@ def summarize(d: Path, workload: str) -> int:
     runs = None
 
     def n_runs(c):
-        return max(len(v) for k, x in c.items() if k.startswith("k_bkt_vv_cp") for v in x.values())
+        return max(len(v) for k, x in c.items() if k.startswith("k_bkt_sort") for v in x.values())
 
     if all((d / f"{w}_{c}" / "run_counter_collection.csv").exists()
            for w in ("bench", "copy") for c in ("FETCH_SIZE", "WRITE_SIZE")):
@@ -186,17 +186,19 @@ def summarize(d: Path, workload: str) -> int:
             scale[c] = 1048576.0 / (sum(vals) / len(vals))
             bc = read_counters(d / f"bench_{c}" / "run_counter_collection.csv")
             runs = n_runs(bc)
-            per[c] = {k: sum(x.get(c, [])) * 1024 * scale[c] / runs for k, x in bc.items()}
+            # the path's own kernels (the run also times a plain device copy)
+            per[c] = {k: sum(x.get(c, [])) * 1024 * scale[c] / runs for k, x in bc.items()
+                      if k.startswith("k_")}
         kernels = sorted(set(per["FETCH_SIZE"]) | set(per["WRITE_SIZE"]),
                          key=lambda k: -(per["FETCH_SIZE"].get(k, 0) + per["WRITE_SIZE"].get(k, 0)))
-        dom = next(k for k in kernels if k.startswith("k_bkt_vv_cp"))
+        dom = next(k for k in kernels if k.startswith("k_bkt_sort"))
         fetch = sum(per["FETCH_SIZE"].values())
         write = sum(per["WRITE_SIZE"].values())
         j = {"workload": workload, "kernel_digest": dig, "hot_path_runs": runs,
              "bytes_per_step": round(fetch + write), "fetch_bytes_per_step": round(fetch),
              "write_bytes_per_step": round(write),
              "fetch_scale": round(scale["FETCH_SIZE"], 4),
-             "write_scale": round(scale["WRITE_SIZE"], 4), "dominant_kernel": "k_bkt_vv_cp",
+             "write_scale": round(scale["WRITE_SIZE"], 4), "dominant_kernel": "k_bkt_sort",
              "dominant_kernel_bytes": round(per["FETCH_SIZE"].get(dom, 0)
                                             + per["WRITE_SIZE"].get(dom, 0)),
              "kernels": {k: {"fetch": round(per["FETCH_SIZE"].get(k, 0)),
@@ -245,7 +247,7 @@ def summarize(d: Path, workload: str) -> int:
     if (d / "pmc_valu" / "run_counter_collection.csv").exists():
         cc = read_counters(d / "pmc_valu" / "run_counter_collection.csv")
         ks = {k: {c: sum(v) / len(v) for c, v in x.items()} for k, x in cc.items()
-              if k.startswith("k_bkt_vv_cp")}
+              if k.startswith("k_bkt_sort")}
         (prof / f"valu_{workload}.json").write_text(json.dumps(
             {"workload": workload, "kernel_digest": dig, "clock_hz": 2.4e9, "simds": 1024,
              "command": "timeout -s KILL 90 rocprofv3 --pmc SQ_INSTS_VALU SQ_INSTS_SALU "

@@ -14,13 +14,16 @@
 //   L2  k_l2_count / k_l2_scatter : slices of each coarse bin -> buckets;
 //       per-(bucket, slice) counts h2[bucket][slice], exclusive scan (which
 //       also gives each bucket's record range), LDS-atomic ranks.
-//   B   k_bkt_vv_cp : per bucket, a lock-free linear-probing hash set of 32
-//       slots per vertex (neighbour ids), a 32-bit adjacency mask per slot
-//       from the shared-tet link triangles, lower/upper masks from the
-//       scalars (ballots), link components by bit-parallel BFS, rows sorted
-//       by a 32-register sorting network and staged in LDS for coalesced
-//       stores.  Vertices with more than 32 neighbours go to k_bkt_heavy
-//       (one workgroup per vertex: LDS hash set, lock-free union-find).
+//   B   k_bkt_sort : per bucket, the records are placed vertex by vertex in
+//       LDS; a lane per vertex sorts its records' keys in registers, reads the
+//       distinct neighbours and a 32-bit adjacency mask per slot (the
+//       shared-tet link triangles) off in order, and labels the link's
+//       components from the lower/upper masks by bit-parallel BFS.  Rows are
+//       staged in LDS for coalesced stores.  Vertices with more than 32
+//       neighbours or 48 records go to k_bkt_heavy (one workgroup per vertex:
+//       LDS hash set, lock-free union-find).  k_bkt_vv_cp is the form with
+//       hash sets shared by the block, k_bkt_own the one with a set per lane.
+// Meshes in spatial order route in one level (k_s1_count, k_s1_scatter).
 // Then: scan of degrees, row compaction into the CSR, and the row-membership
 // link pass for vertices whose shared-tet link has >= 2 components in a class
 // (the shared-tet link graph is a subgraph of the reference's, so counts of 0
