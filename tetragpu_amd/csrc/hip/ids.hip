@@ -802,13 +802,23 @@ constexpr int ET_WIN = 448, EE_WIN = 1728;
 // lane per edge builds its sorted, duplicate-free row in an LDS column (in a
 // padded slot of 2|ET(e)| words of tmp while the column is too short), the
 // block's total joins the chained scan, and the row goes to its place.  Bound
-// by the gathers of two rows (TE, TF) per cell of ET.
+// by the lines that the gathers of ET's cells move: one a cell, from rows that
+// hold its corners and faces together (TE and TF, a line each: 468 us at 2.2 M
+// cells, this 303 and 25 to lay the rows out).
 constexpr int EF_THREADS = 256, EF_CAP = 32;  // 32 KB a block
+
+// Each cell's corners and faces in 32 bytes, for k_ef's gathers.
+__global__ void k_cell_faces(const int4 *__restrict__ tv4, const int4 *__restrict__ tf4, int64_t T,
+                             int4 *__restrict__ rows) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < 2 * T;
+         i += (int64_t)gridDim.x * blockDim.x)
+        rows[i] = i & 1 ? tf4[i >> 1] : tv4[i >> 1];
+}
 
 __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ et_off,
                                                    int64_t E, const int32_t *__restrict__ et,
-                                                   const int32_t *__restrict__ te,
-                                                   const int32_t *__restrict__ tf,
+                                                   const int2 *__restrict__ ev,
+                                                   const int4 *__restrict__ rows,
                                                    int32_t *ticket, uint64_t *state,
                                                    int64_t *__restrict__ off,
                                                    int32_t *__restrict__ out,
@@ -825,34 +835,33 @@ __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ e
     const bool lds = 2 * (b1 - b0) <= EF_CAP;
     int32_t *grow = tmp + 2 * b0;
     int64_t m = 0;
-    // four cells at a time: their TE and TF rows are loaded together
-    // (unconditional loads from a clamped cell index)
+    const int2 lh = act ? ev[e] : make_int2(-1, -1);
+    // four cells at a time, their rows loaded together (unconditional loads
+    // from a clamped cell index)
     for (int64_t i0 = b0; i0 < b1; i0 += 4) {
         int32_t tc[4];
-        int2 r01[4], r23[4], r45[4];
-        int4 fr[4];
+        int4 q[4], fr[4];
 #pragma unroll
         for (int c = 0; c < 4; c++) tc[c] = et[min(i0 + c, b1 - 1)];
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const int2 *tr = reinterpret_cast<const int2 *>(te + 6 * (int64_t)tc[c]);
-            r01[c] = tr[0];
-            r23[c] = tr[1];
-            r45[c] = tr[2];
-            fr[c] = reinterpret_cast<const int4 *>(tf)[tc[c]];
+            q[c] = rows[2 * (int64_t)tc[c]];
+            fr[c] = rows[2 * (int64_t)tc[c] + 1];
         }
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             if (i0 + c >= b1) break;
-            const int32_t ee = (int32_t)e;
-            const int k = r01[c].x == ee ? 0 : r01[c].y == ee ? 1 : r23[c].x == ee ? 2
-                        : r23[c].y == ee ? 3 : r45[c].x == ee ? 4 : r45[c].y == ee ? 5 : 6;
-            if (k == 6) continue;  // TE and ET disagree: no face of this cell
-            // the two face slots holding both corners of edge slot k
-            const int s0[6] = {0, 0, 1, 0, 1, 2}, s1[6] = {1, 2, 2, 3, 3, 3};
+            uint32_t apart = 0;  // corners that the edge does not have
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int32_t u = corner(q[c], j);
+                apart |= (uint32_t)(u != lh.x && u != lh.y) << j;
+            }
+            if (__popc(apart) != 2) continue;  // ET disagrees: no face of this cell
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const int s = h ? s1[k] : s0[k];
+                // face slot 3 - j leaves out corner j
+                const int s = 3 - (h ? 31 - __clz(apart) : __ffs(apart) - 1);
                 const int32_t x = s == 0 ? fr[c].x : s == 1 ? fr[c].y : s == 2 ? fr[c].z : fr[c].w;
                 if (lds) {  // insert into the ascending column unless present
                     int p = (int)m;
@@ -1458,17 +1467,23 @@ int ensure_ef(tg_mesh &m) {
     const int64_t tiles = (E + EF_THREADS - 1) / EF_THREADS;
     const int64_t et_nnz = 6 * m.n_cells, nnz = 3 * m.n_faces;  // a face holds three edges
     Chain c;
+    // tmp_c: rows too long for LDS; tmp_a: the cells' corners and faces
     if ((rc = m.ef_off.ensure(sizeof(int64_t) * (size_t)(E + 1))) ||
         (rc = m.ef_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1))) ||
         (rc = m.tmp_c.ensure(sizeof(int32_t) * 2 * (size_t)std::max<int64_t>(et_nnz, 1))) ||
+        (rc = m.tmp_a.ensure(sizeof(int4) * 2 * (size_t)std::max<int64_t>(m.n_cells, 1))) ||
         (rc = chain_state(m, tiles, c)))
         return rc;
     int64_t *off = m.ef_off.as<int64_t>();
     if (E > 0) {
+        hipLaunchKernelGGL(k_cell_faces, dim3(grid(2 * m.n_cells)), dim3(256), 0, m.stream,
+                           m.tv.as<const int4>(), m.tf.as<const int4>(), m.n_cells,
+                           m.tmp_a.as<int4>());
+        TG_LAUNCH_CHECK("k_cell_faces");
         hipLaunchKernelGGL(k_ef, dim3((unsigned)tiles), dim3(EF_THREADS), 0, m.stream,
-                           m.et_off.as<int64_t>(), E, m.et_vals.as<int32_t>(), m.te.as<int32_t>(),
-                           m.tf.as<int32_t>(), c.ticket, c.state, off, m.ef_vals.as<int32_t>(),
-                           m.tmp_c.as<int32_t>());
+                           m.et_off.as<int64_t>(), E, m.et_vals.as<int32_t>(),
+                           m.ev.as<const int2>(), m.tmp_a.as<const int4>(), c.ticket, c.state, off,
+                           m.ef_vals.as<int32_t>(), m.tmp_c.as<int32_t>());
         TG_LAUNCH_CHECK("k_ef");
     } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
         return rc;
