@@ -138,7 +138,10 @@ int tg_critpoints(tg_mesh *m);
  * resident in HBM, no host synchronisation, no allocation after the first
  * call on a mesh (graph-capturable). */
 int tg_vv_critpoints(tg_mesh *m);
-/* Wait for the mesh's stream; reports device-side capacity errors. */
+/* Wait for the mesh's stream; reports device-side capacity errors, each once.
+ * After one (a vertex with more than 4096 neighbours, whose VV row and class
+ * are missing) the other rows can be read; builds of the relations that number
+ * edges or faces return TG_ERR_CAPACITY each time. */
 int tg_sync(tg_mesh *m);
 
 /* Shape of a built relation: rows, entries, int32 words per entry, and

@@ -210,7 +210,44 @@ def case_split(seed: int = 3, n: int = 4) -> None:
             raise AssertionError(f"expected TG_ERR_ALLOC for {list(kw)}")
 
 
-CASES = {"split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
+def case_capacity(hub_first: int = 0, variant: int = 2) -> None:
+    """A vertex with more neighbours than a kernel holds (4096): the relations
+    that number edges are refused each time they are asked for, not only when
+    the error is first met; VV and VT stay readable."""
+    from oracle import binding as O
+
+    n = 4200
+    i = np.arange(n, dtype=np.int32)
+    strip = np.stack([i, i + 1, i + 2], 1) + (1 if hub_first else 0)
+    hub = np.full((n, 1), 0 if hub_first else n + 2, np.int32)
+    cells = np.ascontiguousarray(np.hstack([hub, strip] if hub_first else [strip, hub]))
+    V = n + 3
+
+    def refused(d, *names):
+        try:
+            d.build(t.flags(*names))
+        except _native.NativeError as e:
+            assert e.status == -5 and "4096" in str(e), e
+        else:
+            raise AssertionError(f"{names} built on an incomplete VV")
+
+    with t.Mesh(cells, V, np.zeros(V, np.float32)) as d:
+        d.set_config(variant=variant)
+        refused(d, "TE", "VE", "EV")
+        for names in (("TE", "VE", "EV"), ("EE",), ("TF", "VF"), ("EF",)):
+            refused(d, *names)
+        off, _ = d.relation("VV")               # every row but the hub's is there
+        assert off[hub[0, 0]] == off[hub[0, 0] + 1]
+        d.build(t.flags("VT"))
+        ref = O.vt(cells, V)
+        vt = d.relation("VT")
+        assert np.array_equal(vt[0], ref.off) and np.array_equal(vt[1], ref.val), "VT"
+        d.vv_critpoints()                       # a new run of the same mesh
+        refused(d, "TE")
+        refused(d, "TE")
+
+
+CASES = {"capacity": case_capacity, "split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
          "vv_cp": case_vv_cp, "window": case_window, "hubs": case_hubs, "soup": case_soup, "routes": case_routes}
 
 

@@ -1,0 +1,23 @@
+"""Meshes with long rows on the CPU kernel emulator (AddressSanitizer, exact
+allocations), against the oracle: the parts of the relation builds that only
+vertices with many cells or neighbours reach.  No GPU is needed.
+"""
+import subprocess
+import sys
+
+import pytest
+
+from test_emu_kernels import EMU, emu_env  # noqa: F401  (fixture)
+
+CASES = [
+    # more neighbours than a kernel holds, the hub with the highest or the
+    # lowest id, in the bucketed and the vertex-lane form
+    ("capacity", 0, 2), ("capacity", 1, 2), ("capacity", 0, 1), ("capacity", 1, 1),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+def test_long_rows(emu_env, case):  # noqa: F811
+    r = subprocess.run([sys.executable, str(EMU / "run_case.py"), *map(str, case)], env=emu_env,
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0 and "ok " in r.stdout, (r.stdout + r.stderr)[-4000:]

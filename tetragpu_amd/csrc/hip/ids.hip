@@ -1303,6 +1303,9 @@ int ensure_edges(tg_mesh &m) {
     if ((rc = ensure_vv(m)) || (rc = ensure_vt_sorted(m)) ||
         (rc = sync_check_read(m, m.vv_off.as<int32_t>() + V, nnz)))
         return rc;
+    // an edge is counted from both its ends' rows: with one missing, what
+    // follows would be sized for fewer edges than the kernels write
+    if (m.vv_short) return capacity_error();
     const size_t I = sizeof(int32_t);
     if ((rc = m.edge_first.ensure(I * (size_t)std::max<int64_t>(nnz, 1))) ||
         (rc = m.te.ensure(I * 6 * (size_t)std::max<int64_t>(T, 1))) ||

@@ -56,6 +56,7 @@ struct tg_mesh {
     bool vt_sorted = false;         // vtc rows ascending
     bool vv_built = false, cp_built = false;
     bool counters_pending = false;  // a pipeline ran since the last error check
+    bool vv_short = false;          // that check found a vertex whose row is missing in VV
 
     // id-assigning and derived relations
     tg::DevArr vt_vals;
@@ -95,7 +96,9 @@ int ensure_vt_corners(tg_mesh &m);
 int ensure_vv(tg_mesh &m);
 // Enqueue the relations selected by `flags` (reference flag bits).
 int build_relations(tg_mesh &m, uint32_t flags);
-// Synchronise the mesh stream and report device-side errors.
+// The error of a vertex with more neighbours than the kernels hold.
+int capacity_error();
+// Synchronise the mesh stream and report device-side errors, each once.
 int sync_and_check(tg_mesh &m);
 // The same, with one int32 or int64 read from device memory in the same wait.
 int sync_check_read(tg_mesh &m, const int32_t *src, int64_t &out);

@@ -231,6 +231,7 @@ static int run_vv(tg_mesh &m, bool classify) {
         }
     }
     m.vv_built = true;
+    m.vv_short = false;
     m.vv_nnz = -1;
     if (classify) m.cp_built = true;
     m.counters_pending = true;
@@ -335,8 +336,6 @@ int build_relations(tg_mesh &m, uint32_t flags) {
     return OK;
 }
 
-namespace {
-
 int capacity_error() {
     char buf[160];
     std::snprintf(buf, sizeof buf,
@@ -346,6 +345,8 @@ int capacity_error() {
     set_error(buf);
     return ERR_CAPACITY;
 }
+
+namespace {
 
 // One wait for the stream's work, the run's error bits (when a run is
 // unchecked) and up to eight bytes from src: each readback on its own leaves
@@ -360,7 +361,10 @@ int wait_check_read(tg_mesh &m, const void *src, size_t bytes, void *out) {
         TG_HIP(hipMemcpyAsync(h + 1, src, bytes, hipMemcpyDeviceToHost, m.stream));
     TG_HIP(hipStreamSynchronize(m.stream));
     m.counters_pending = false;
-    if (check && (*(const int32_t *)h & ERRBIT_CAPACITY)) return capacity_error();
+    if (check && (*(const int32_t *)h & ERRBIT_CAPACITY)) {
+        m.vv_short = true;
+        return capacity_error();
+    }
     if (bytes) std::memcpy(out, h + 1, bytes);
     return OK;
 }
