@@ -247,7 +247,14 @@ def case_capacity(hub_first: int = 0, variant: int = 2) -> None:
         refused(d, "TE")
 
 
-CASES = {"capacity": case_capacity, "split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
+def case_hub_rows(shared: int = 50, apart: int = 0, between: int = 0, order: int = 0) -> None:
+    """Every relation around two hubs (test_gpu_long_rows.hub_mesh)."""
+    from test_gpu_long_rows import check_hubs
+
+    check_hubs(t, shared, apart, between, order)
+
+
+CASES = {"hub_rows": case_hub_rows, "capacity": case_capacity, "split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
          "vv_cp": case_vv_cp, "window": case_window, "hubs": case_hubs, "soup": case_soup, "routes": case_routes}
 
 

@@ -4,6 +4,7 @@ vertices with many cells or neighbours reach.  No GPU is needed.
 """
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
@@ -13,11 +14,22 @@ CASES = [
     # more neighbours than a kernel holds, the hub with the highest or the
     # lowest id, in the bucketed and the vertex-lane form
     ("capacity", 0, 2), ("capacity", 1, 2), ("capacity", 0, 1), ("capacity", 1, 1),
+    # rows beyond the join networks, alone in a wave and beside short ones
+    ("hub_rows", 50, 0, 0, 0), ("hub_rows", 20, 33, 10, 1),
 ]
 
 
+@pytest.fixture(scope="module")
+def results(emu_env):  # noqa: F811
+    def run(case):
+        return subprocess.run([sys.executable, str(EMU / "run_case.py"), *map(str, case)],
+                              env=emu_env, capture_output=True, text=True, timeout=600)
+
+    with ThreadPoolExecutor(6) as ex:
+        return dict(zip(CASES, ex.map(run, CASES)))
+
+
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
-def test_long_rows(emu_env, case):  # noqa: F811
-    r = subprocess.run([sys.executable, str(EMU / "run_case.py"), *map(str, case)], env=emu_env,
-                       capture_output=True, text=True, timeout=600)
+def test_long_rows(results, case):
+    r = results[case]
     assert r.returncode == 0 and "ok " in r.stdout, (r.stdout + r.stderr)[-4000:]

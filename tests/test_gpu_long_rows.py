@@ -1,0 +1,77 @@
+"""GPU parity where vertices have many cells and neighbours: rows that the
+joins' networks do not take and that a whole wave orders or merges.  Everything
+is integer and compared exactly with the CPU oracle."""
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def hub_mesh(n, apart, between):
+    """`n` cells (a, b, s_i, s_i+1) around the edge of two hubs, `apart` cells
+    around each hub alone, and `between` cells of a strip that touches
+    neither; the hubs' shared cells come among the others at regular places."""
+    cells = [(0, 1, 2 + i, 3 + i) for i in range(n)]
+    v = n + 3
+    for hub in (0, 1):
+        cells += [(hub, v + i, v + i + 1, v + i + 2) for i in range(apart)]
+        v += apart + 2 if apart else 0
+    strip = [(v + i, v + i + 1, v + i + 2, v + i + 3) for i in range(between)]
+    v += between + 3 if between else 0
+    cells = cells + strip
+    order = np.argsort(np.arange(len(cells)) * 7 % max(len(cells), 1), kind="stable")
+    return np.array(cells, np.int32)[order], v
+
+
+def check_hubs(t, shared, apart, between, order):
+    """order 0: as hub_mesh gives it; else random cells and ids by that seed."""
+    from test_gpu_relations import check_all
+
+    cells, V = hub_mesh(shared, apart, between)
+    if order:
+        rng = np.random.default_rng(order)
+        ids = rng.permutation(V).astype(np.int32)
+        cells = np.ascontiguousarray(np.sort(ids[cells], axis=1)[rng.permutation(len(cells))])
+    check_all(t, cells, V, expect_ft=False)
+
+
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("shared,apart,between", [
+    (50, 0, 0), (1000, 0, 0),            # the same long row twice
+    (300, 900, 700), (1, 65, 0),         # stretches of one hub alone
+    (49, 0, 64), (46, 3, 200),           # a few long rows in a wave of short ones
+    (1, 4000, 0),                        # near the most neighbours a kernel holds
+])
+def test_hub_rows(gpu, shared, apart, between, order):
+    check_hubs(gpu, shared, apart, between, order)
+
+
+def seconds(t, cells, V, first, then):
+    """The shortest of five builds of `then` on meshes that hold `first`."""
+    best = float("inf")
+    for _ in range(5):
+        with t.Mesh(cells, V) as m:
+            m.build(t.flags(first))
+            m.shape(first)
+            t0 = time.perf_counter()
+            m.build(t.flags(then))
+            m.shape(then)
+            best = min(best, time.perf_counter() - t0)
+    return best
+
+
+@pytest.mark.parametrize("first,then,n", [("VT", "TT", 34)])
+def test_long_rows_cost_their_entries(gpu, first, then, n):
+    """4000 cells around one vertex give as many entries as a grid of n^3 cubes
+    and take no more than 20 times as long (both take about 0.1 ms; one lane's
+    merge of each row took 15 times, one that starts anew for every window of
+    a wave's output 700)."""
+    i = np.arange(4000, dtype=np.int32)
+    fan = np.ascontiguousarray(np.stack([i, i + 1, i + 2, np.full(4000, 4002, np.int32)], 1))
+    m = gpu.kuhn(n, seed=1)
+    long = seconds(gpu, fan, 4003, first, then)
+    short = seconds(gpu, m.cells, m.n_points, first, then)
+    print(f"{then}: long rows {1e6 * long:.0f} us, short rows {1e6 * short:.0f} us", flush=True)
+    assert long < 20 * short

@@ -119,6 +119,15 @@ __device__ __forceinline__ void sched_fence() {
 #endif
 }
 
+// x of one lane (the same lane number in all of them).
+__device__ __forceinline__ int32_t lane_value(int32_t x, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_readlane(x, lane);
+#else
+    return __shfl(x, lane, 64);
+#endif
+}
+
 // Words that workgroups of one launch hand to each other (one word carries
 // flag and value, so no order with other memory is needed).
 __device__ __forceinline__ uint64_t load_agent(const uint64_t *p) {

@@ -17,7 +17,7 @@
 // positional triple, and face ids are ranks of first occurrences.
 //
 // The other relations with rows count, scan and write in one launch each (a
-// chained scan over tiles): ET(e) = VT(lo) n VT(hi), TT and EE as joins, VE
+// chained scan over tiles; rows of many cells or edges in launches beside it): ET(e) = VT(lo) n VT(hi), TT and EE as joins, VE
 // and VF from a vertex's VV row and cells, EF and FF from TE and TF; FT comes
 // from the face matches.
 #include <algorithm>
@@ -533,8 +533,8 @@ __device__ __forceinline__ void insert_sorted(int32_t *row, int64_t &m, int32_t 
 // bitonic network, and what the join keeps is counted; the block's total joins
 // a chained scan over tiles of rows, which gives every row its exact place;
 // then the rows go through an LDS window per wave to contiguous 16-byte stores.
-// A wave takes the smallest network that holds its rows; a lane with a row
-// beyond the largest one merges serially from global memory.
+// A wave takes the smallest network that holds its rows; what has a row beyond
+// the largest one is left to LongRows' ways.
 //
 // What bounds it: the gathers of NR x 64 different rows per wave (TT: 4 rows of
 // 96 bytes a cell, 2.0 M cells in random order 0.65 ms) and VALU issue of the
@@ -544,6 +544,10 @@ __device__ __forceinline__ void insert_sorted(int32_t *row, int64_t &m, int32_t 
 // their lengths and packed them (TT 2.71 ms).
 constexpr int JOIN_ROW = 48;  // longest row of the largest network
 enum Join { UNION_LESS_SELF, INTERSECT };
+// Outputs with a source row beyond JOIN_ROW: there are none, or a wave each
+// joins them in launches of their own, before the main one (their lengths) and
+// after it (their values; it leaves them out).
+enum LongRows { NO_LONG, LISTED };
 
 // Tiles' totals as they become known: bits 62-63 hold 0 (nothing yet), 1 (the
 // tile's own sum) or 2 (the sum of all tiles up to it).
@@ -596,33 +600,6 @@ struct Rows {  // the lane's rows
     }
 };
 
-// Serial merge from global memory: f(i, x) for the i-th value x that the join
-// keeps, ascending; returns their number.
-template <int NR, Join J, int SH, typename F>
-__device__ __forceinline__ int32_t join_serial(const int32_t *src, const Rows<NR> &r, int32_t self,
-                                               F f) {
-    int32_t i[NR], h[NR], m = 0;
-#pragma unroll
-    for (int c = 0; c < NR; c++) {
-        i[c] = 0;
-        h[c] = r.n[c] > 0 ? src[r.p[c]] >> SH : INF;
-    }
-    while (true) {
-        int32_t x = h[0];
-#pragma unroll
-        for (int c = 1; c < NR; c++) x = min(x, h[c]);
-        if (x == INF) return m;
-        int in = 0;
-#pragma unroll
-        for (int c = 0; c < NR; c++)
-            if (h[c] == x) {
-                in++;
-                h[c] = ++i[c] < r.n[c] ? src[r.p[c] + i[c]] >> SH : INF;
-            }
-        if (J == INTERSECT ? in == NR : x != self) f(m++, x);
-    }
-}
-
 // Block of one kernel: its threads and the words of a wave's output window.
 template <int THREADS, int WIN>
 struct JoinBlock {
@@ -635,41 +612,51 @@ struct JoinBlock {
 // One wave's share of a tile with a network for rows of up to R entries.
 // Contains two workgroup barriers; every wave of the block makes one call
 // (of some R), so all waves meet at both.
-template <int NR, Join J, int SH, int R, int THREADS, int WIN>
+template <int NR, Join J, int SH, LongRows L, int R, int THREADS, int WIN>
 __device__ __forceinline__ void join_wave(JoinBlock<THREADS, WIN> &blk,
                                           const int32_t *__restrict__ src, const Rows<NR> &r,
-                                          bool act, int32_t self, int64_t row, int64_t rows,
-                                          uint64_t *state, int64_t *__restrict__ off,
-                                          int32_t *__restrict__ out) {
+                                          int64_t rows, int32_t mlong, uint64_t *state,
+                                          int64_t *__restrict__ off, int32_t *__restrict__ out) {
     static_assert(NR == 2 || NR == 4, "merge tree");
     constexpr int N = NR * R;
     const int lane = __lane_id(), wid = threadIdx.x / 64;
-    const int32_t tile = blk.tile;
+    // uniform values are made scalars: the keys take nearly all vector registers
+    const int32_t tile = tgd::lane_value(blk.tile, 0);
+    const int64_t row = (int64_t)tile * THREADS + threadIdx.x;
+    const int32_t self = (int32_t)row;
     int32_t *win = blk.win[wid];
-    int32_t k[N];
+    // outputs with a row beyond the largest network: mlong values each, left
+    // out of the window
+    const bool is_long = L != NO_LONG && r.longest() > JOIN_ROW;
+    const uint64_t longs = L != NO_LONG ? __ballot(is_long) : 0;
+    int32_t k[N], n[NR];
     int nv = 0;
 #pragma unroll
-    for (int c = 0; c < NR; c++) nv += r.n[c];
+    for (int c = 0; c < NR; c++) {
+        n[c] = is_long ? 0 : r.n[c];
+        nv += n[c];
+    }
     if constexpr (NR == 4) {
-        load_row<0, R, false, SH>(k, src + r.p[0], r.n[0]);
-        load_row<R, R, true, SH>(k, src + r.p[1], r.n[1]);
-        load_row<2 * R, R, true, SH>(k, src + r.p[2], r.n[2]);
-        load_row<3 * R, R, false, SH>(k, src + r.p[3], r.n[3]);
+        load_row<0, R, false, SH>(k, src + r.p[0], n[0]);
+        load_row<R, R, true, SH>(k, src + r.p[1], n[1]);
+        load_row<2 * R, R, true, SH>(k, src + r.p[2], n[2]);
+        load_row<3 * R, R, false, SH>(k, src + r.p[3], n[3]);
         tgn::bitonic_merge<0, 2 * R, false>(k);
         tgn::bitonic_merge<2 * R, 2 * R, true>(k);
     } else {
-        load_row<0, R, true, SH>(k, src + r.p[0], r.n[0]);
-        load_row<R, R, false, SH>(k, src + r.p[1], r.n[1]);
+        load_row<0, R, true, SH>(k, src + r.p[0], n[0]);
+        load_row<R, R, false, SH>(k, src + r.p[1], n[1]);
     }
     tgn::bitonic_merge<0, N, true>(k);
-    const bool serial = r.longest() > JOIN_ROW;
     int32_t m = 0;  // distinct values, less the lane's own and the padding; or equal pairs
 #pragma unroll
     for (int j = 1; j < N; j++) m += J == INTERSECT ? k[j] == k[j - 1] : k[j] != k[j - 1];
     m -= J == INTERSECT ? max(N - nv - 1, 0) : (int)(nv < N);
-    if (!act) m = 0;
-    if (serial) m = join_serial<NR, J, SH>(src, r, self, [](int32_t, int32_t) {});
-    const int32_t inc = tgd::wave_inclusive_sum(m);
+    if (row >= rows || is_long) m = 0;
+    // places of the lane's values in the wave's window and in the wave's output
+    if (!is_long) mlong = 0;
+    const int32_t winc = tgd::wave_inclusive_sum(m);
+    const int32_t inc = longs ? tgd::wave_inclusive_sum(m + mlong) : winc;
     if (lane == 63) blk.wtot[wid] = inc;
     __syncthreads();
     int32_t before = 0, total = 0;
@@ -678,29 +665,26 @@ __device__ __forceinline__ void join_wave(JoinBlock<THREADS, WIN> &blk,
         if (i < wid) before += blk.wtot[i];
         total += blk.wtot[i];
     }
+    before = tgd::lane_value(before, 0);
+    total = tgd::lane_value(total, 0);
     if (threadIdx.x == 0) tgd::store_agent(state + tile, TILE_SUM | (uint64_t)total);
-    const int32_t first = inc - m, wn = __shfl(inc, 63, 64);
+    const int32_t first = inc - m - mlong, wfirst = winc - m;
+    const int32_t wn = tgd::lane_value(winc, 63);
     // the wave's rows, one window after the other; the first one is filled
     // while the tile's place is being found
     for (int32_t w0 = 0;; w0 += WIN) {
-        int32_t pos = first - w0 - 1;
-        if (serial) {
-            join_serial<NR, J, SH>(src, r, self, [&](int32_t i, int32_t x) {
-                if ((uint32_t)(first - w0 + i) < (uint32_t)WIN) win[first - w0 + i] = x;
-            });
-        } else {
-            // compared afresh in every window: masks kept from the count
-            // above, one per key, would not fit the scalar registers
-            const int32_t mv = tgd::opaque(nv);
-            int32_t prev = -1;
+        int32_t pos = wfirst - w0 - 1;
+        // compared afresh in every window: masks kept from the count
+        // above, one per key, would not fit the scalar registers
+        const int32_t mv = tgd::opaque(nv);
+        int32_t prev = -1;
 #pragma unroll
-            for (int j = 0; j < N; j++) {
-                k[j] = tgd::opaque(k[j]);
-                const bool keep = (J == INTERSECT ? k[j] == prev : k[j] != prev && k[j] != self) && j < mv;
-                prev = k[j];
-                pos += keep;
-                if (keep && (uint32_t)pos < (uint32_t)WIN) win[pos] = k[j];
-            }
+        for (int j = 0; j < N; j++) {
+            k[j] = tgd::opaque(k[j]);
+            const bool keep = (J == INTERSECT ? k[j] == prev : k[j] != prev && k[j] != self) && j < mv;
+            prev = k[j];
+            pos += keep;
+            if (keep && (uint32_t)pos < (uint32_t)WIN) win[pos] = k[j];
         }
         if (w0 == 0) {
             if (wid == 0) {
@@ -711,17 +695,30 @@ __device__ __forceinline__ void join_wave(JoinBlock<THREADS, WIN> &blk,
                 }
             }
             __syncthreads();
-            if (act) off[row] = blk.base + before + first;
+            if (row < rows) off[row] = blk.base + before + first;
             if (row == rows - 1) off[rows] = blk.base + total;
         }
         tgd::wave_sync();  // the window is whole
-        int32_t *dst = out + (blk.base + before + w0);
-        const int32_t cnt = min(wn - w0, WIN);
-        for (int32_t i = 4 * lane; i + 3 < cnt; i += 256)
-            *reinterpret_cast<i32x4u *>(dst + i) = *reinterpret_cast<const i32x4u *>(win + i);
-        const int32_t tail = cnt & ~3;
-        if (cnt > 0 && tail + lane < cnt) dst[tail + lane] = win[tail + lane];
-        if (w0 + WIN >= wn) return;
+        // words [from, to) of the windows' sequence, of which the output has
+        // `shift` more before them
+        auto copy = [&](int32_t from, int32_t to, int32_t shift) {
+            const int32_t a = max(from - w0, 0), b = min(to - w0, WIN);
+            int32_t *dst = out + (blk.base + before + w0 + shift);
+            for (int32_t i = a + 4 * lane; i + 3 < b; i += 256)
+                *reinterpret_cast<i32x4u *>(dst + i) = *reinterpret_cast<const i32x4u *>(win + i);
+            const int32_t tail = a + ((b - a) & ~3);
+            if (a < b && tail + lane < b) dst[tail + lane] = win[tail + lane];
+        };
+        int32_t from = 0, shift = 0;
+        for (uint64_t b = longs; b; b &= b - 1) {  // the rows between the long ones
+            const int l = __ffsll((unsigned long long)b) - 1;
+            const int32_t to = tgd::lane_value(wfirst, l);
+            copy(from, to, tgd::lane_value(first, l) - to);
+            from = to;
+            shift = tgd::lane_value(inc, l) - to;
+        }
+        copy(from, wn, shift);
+        if (w0 + WIN >= wn) break;
         tgd::wave_sync();  // and has been read
     }
 }
@@ -733,29 +730,63 @@ __device__ __forceinline__ int32_t take_tile(int32_t *ticket, int32_t &shared) {
     return shared;
 }
 
+// The rows that an output joins.  TT: the VT rows of a cell's corners.
+struct CellRows {
+    const int4 *__restrict__ tv4;
+    const int32_t *__restrict__ vt_off;
+    __device__ __forceinline__ Rows<4> operator()(int64_t t, bool act) const {
+        Rows<4> r;
+        const int4 q = act ? tv4[t] : make_int4(0, 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const i32x2u o = *reinterpret_cast<const i32x2u *>(vt_off + corner(q, c));
+            r.p[c] = o.x;
+            r.n[c] = act ? o.y - o.x : 0;
+        }
+        return r;
+    }
+};
+// ET and EE: the rows of an edge's ends (corner codes by vt_off, or edge ids
+// by vv_off).
+struct EdgeRows {
+    const int32_t *__restrict__ ev;
+    int64_t V;
+    const int32_t *__restrict__ row_off;
+    __device__ __forceinline__ Rows<2> operator()(int64_t e, bool act) const {
+        Rows<2> r;
+        const int2 ends = act ? reinterpret_cast<const int2 *>(ev)[e] : make_int2(0, 0);
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int32_t v = c ? ends.y : ends.x;
+            const bool ok = v >= 0 && v < V;  // always, for a built EV
+            const i32x2u o = *reinterpret_cast<const i32x2u *>(row_off + (ok ? v : 0));
+            r.p[c] = o.x;
+            r.n[c] = act && ok ? o.y - o.x : 0;
+        }
+        return r;
+    }
+};
+
 // Window: what two blocks per CU (as many as the registers allow) leave of
 // the LDS; one window for 64 x 69 words (two windows of 2240: 0.76 ms at 2.0 M
 // split cells, one 0.65).
 constexpr int TT_THREADS = 256, TT_WIN = 5088;
-__global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const int4 *__restrict__ tv4, int64_t T,
-                                                      const int32_t *__restrict__ vt_off,
+template <LongRows L>
+__global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const CellRows rows_of, int64_t T,
                                                       const int32_t *__restrict__ vtc,
+                                                      const int32_t *__restrict__ long_len,
                                                       int32_t *ticket, uint64_t *state,
                                                       int64_t *__restrict__ off,
                                                       int32_t *__restrict__ out) {
     __shared__ __align__(16) JoinBlock<TT_THREADS, TT_WIN> blk;
     const int64_t t = (int64_t)take_tile(ticket, blk.tile) * TT_THREADS + threadIdx.x;
     const bool act = t < T;
-    Rows<4> r;
-    const int4 q = act ? tv4[t] : make_int4(0, 0, 0, 0);
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const i32x2u o = *reinterpret_cast<const i32x2u *>(vt_off + corner(q, c));
-        r.p[c] = o.x;
-        r.n[c] = act ? o.y - o.x : 0;
-    }
-    const int need = r.longest() > JOIN_ROW ? 0 : r.longest();  // serial lanes need no network
-#define TG_JOIN(R) join_wave<4, UNION_LESS_SELF, 2, R>(blk, vtc, r, act, (int32_t)t, t, T, state, off, out)
+    const Rows<4> r = rows_of(t, act);
+    const bool is_long = L != NO_LONG && r.longest() > JOIN_ROW;
+    const int32_t mlong = is_long ? long_len[t] : 0;
+    const int need = is_long ? 0 : r.longest();
+#define TG_JOIN(R)                                                                              \
+    join_wave<4, UNION_LESS_SELF, 2, L, R>(blk, vtc, r, T, mlong, state, off, out)
     if (__any(need > 40)) TG_JOIN(JOIN_ROW);
     else if (__any(need > 32)) TG_JOIN(40);
     else if (__any(need > 24)) TG_JOIN(32);
@@ -763,33 +794,25 @@ __global__ __launch_bounds__(TT_THREADS, 2) void k_tt(const int4 *__restrict__ t
 #undef TG_JOIN
 }
 
-// ET and EE: the rows of edge e's two ends in src (corner codes by vt_off, or
-// edge ids by vv_off).  512 edges a tile: tile numbers cost 10 ns each.
-// Windows: one for ET (64 x 5 words), one for EE (64 x 26).
+// 512 edges a tile: tile numbers cost 10 ns each.  Windows: one for ET (64 x 5
+// words), one for EE (64 x 26).
 constexpr int EJ_THREADS = 512;
-template <Join J, int SH, int WIN>
-__global__ __launch_bounds__(EJ_THREADS, 4) void k_edge_join(const int32_t *__restrict__ ev, int64_t E,
-                                                             int64_t V,
-                                                             const int32_t *__restrict__ row_off,
+template <Join J, int SH, LongRows L, int WIN>
+__global__ __launch_bounds__(EJ_THREADS, 4) void k_edge_join(const EdgeRows rows_of, int64_t E,
                                                              const int32_t *__restrict__ src,
+                                                             const int32_t *__restrict__ long_len,
                                                              int32_t *ticket, uint64_t *state,
                                                              int64_t *__restrict__ off,
                                                              int32_t *__restrict__ out) {
     __shared__ __align__(16) JoinBlock<EJ_THREADS, WIN> blk;
     const int64_t e = (int64_t)take_tile(ticket, blk.tile) * EJ_THREADS + threadIdx.x;
     const bool act = e < E;
-    Rows<2> r;
-    const int2 ends = act ? reinterpret_cast<const int2 *>(ev)[e] : make_int2(0, 0);
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-        const int32_t v = c ? ends.y : ends.x;
-        const bool ok = v >= 0 && v < V;  // always, for a built EV
-        const i32x2u o = *reinterpret_cast<const i32x2u *>(row_off + (ok ? v : 0));
-        r.p[c] = o.x;
-        r.n[c] = act && ok ? o.y - o.x : 0;
-    }
-    const int need = r.longest() > JOIN_ROW ? 0 : r.longest();  // serial lanes need no network
-#define TG_JOIN(R) join_wave<2, J, SH, R>(blk, src, r, act, (int32_t)e, e, E, state, off, out)
+    const Rows<2> r = rows_of(e, act);
+    const bool is_long = L != NO_LONG && r.longest() > JOIN_ROW;
+    // EE: the ends' rows share only the edge itself
+    const int32_t mlong = !is_long ? 0 : J == INTERSECT ? long_len[e] : r.n[0] + r.n[1] - 2;
+    const int need = is_long ? 0 : r.longest();
+#define TG_JOIN(R) join_wave<2, J, SH, L, R>(blk, src, r, E, mlong, state, off, out)
     if (__any(need > 32)) TG_JOIN(JOIN_ROW);
     else if (__any(need > 24)) TG_JOIN(32);
     else if (__any(need > 16)) TG_JOIN(24);
@@ -797,6 +820,182 @@ __global__ __launch_bounds__(EJ_THREADS, 4) void k_edge_join(const int32_t *__re
 #undef TG_JOIN
 }
 constexpr int ET_WIN = 448, EE_WIN = 1728;
+
+// Outputs with a row beyond JOIN_ROW, in any order; n has to start at 0.
+constexpr int LIST_THREADS = 256;
+template <typename RO>
+__global__ __launch_bounds__(LIST_THREADS) void k_list_long(const RO rows_of, int64_t count,
+                                                            int32_t *__restrict__ list,
+                                                            int32_t *__restrict__ n) {
+    const int lane = __lane_id();
+    const int64_t step = (int64_t)gridDim.x * LIST_THREADS;
+    for (int64_t b = (int64_t)blockIdx.x * LIST_THREADS; b < count; b += step) {
+        const int64_t i = b + threadIdx.x;
+        const bool is_long = rows_of(i, i < count).longest() > JOIN_ROW;
+        const uint64_t m = __ballot(is_long);
+        if (!m) continue;
+        int32_t at = 0;
+        if (lane == 0) at = atomicAdd(n, (int32_t)__popcll(m));
+        at = tgd::lane_value(at, 0) + (int32_t)__popcll(m & ((1ull << lane) - 1ull));
+        if (is_long) list[at] = (int32_t)i;
+    }
+}
+
+// Union of the rows at at[c] .. end[c], less `self`, which every row holds, by
+// one wave: returns the number of values and, with WRITE, leaves them at out,
+// ascending.  A step takes 64 / NR entries of each row; those up to the
+// smallest of the rows' last ones taken are sorted across the wave and
+// consumed, so equal entries meet in one step.  Where one row alone has entries
+// before the others' next ones, the stretch is found by a 64-way search and
+// copied whole.
+template <int NR, int SH, bool WRITE>
+__device__ __forceinline__ int32_t union_by_wave(const int32_t *__restrict__ src, int32_t (&at)[NR],
+                                                 const int32_t (&end)[NR], int32_t self,
+                                                 int32_t *__restrict__ out) {
+    static_assert(NR == 2 || NR == 4, "merge of halves");
+    constexpr int W = 64 / NR;
+    const int lane = __lane_id(), row = lane / W, j = lane % W;
+    int32_t m = 0;
+    while (true) {
+        int32_t i = at[0], e = end[0];
+#pragma unroll
+        for (int c = 1; c < NR; c++) {
+            i = row == c ? at[c] : i;
+            e = row == c ? end[c] : e;
+        }
+        int32_t x = j < e - i ? src[i + j] >> SH : INF;
+        int32_t head[NR], last[NR], limit = INF;
+        int a = 0;  // the row with the smallest entry
+#pragma unroll
+        for (int c = 0; c < NR; c++) {
+            head[c] = tgd::lane_value(x, W * c);
+            last[c] = tgd::lane_value(x, W * c + W - 1);
+            limit = min(limit, last[c]);
+            if (c > 0 && head[c] < head[0]) head[0] = head[c], a = c;
+        }
+        if (head[0] == INF) return m;
+        int32_t lo = 0, hi = 0, la = 0, others = INF;
+#pragma unroll
+        for (int c = 0; c < NR; c++) {
+            if (c == a) lo = at[c], hi = end[c], la = last[c];
+            else others = min(others, tgd::lane_value(x, W * c));
+        }
+        if (la < others) {  // a stretch of row a alone: [from, lo) when found
+            const int32_t from = lo;
+            lo += W;
+            if (others == INF) lo = hi;
+            while (lo < hi) {
+                const int32_t step = (hi - lo + 63) / 64, p = lo + lane * step;
+                const int32_t below = (int32_t)__popcll(__ballot(p < hi && src[p] >> SH < others));
+                if (below == 0) break;
+                hi = min(hi, lo + below * step);
+                lo += (below - 1) * step + 1;
+            }
+            if (WRITE) {
+                constexpr int U = 4;
+                const int32_t n = lo - from;
+                for (int32_t k = lane; k < n; k += 64 * U) {
+                    int32_t y[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        y[u] = k + 64 * u < n ? src[from + k + 64 * u] >> SH : 0;
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (k + 64 * u < n) out[m + k + 64 * u] = y[u];
+                }
+            }
+            m += lo - from;
+#pragma unroll
+            for (int c = 0; c < NR; c++)
+                if (c == a) at[c] = lo;
+            continue;
+        }
+        const uint64_t taken = __ballot(x <= limit && x != INF);
+        if (x > limit) x = INF;
+#pragma unroll
+        for (int w = 2 * W; w <= 64; w *= 2) {  // merge sorted halves of w lanes
+#pragma unroll
+            for (int d = w - 1; d >= 1; d = d == w - 1 ? w / 4 : d / 2) {
+                const int32_t y = __shfl_xor(x, d, 64);
+                // d = w - 1: partners are mirrored, the upper half keeps the larger
+                const bool upper = lane & (d == w - 1 ? w / 2 : d);
+                x = upper ? max(x, y) : min(x, y);
+            }
+        }
+        const int32_t y = __shfl_up(x, 1, 64);
+        const bool keep = x != INF && x != self && (lane == 0 || x != y);
+        const uint64_t kept = __ballot(keep);
+        if (WRITE && keep) out[m + (int32_t)__popcll(kept & ((1ull << lane) - 1ull))] = x;
+        m += (int32_t)__popcll(kept);
+#pragma unroll
+        for (int c = 0; c < NR; c++)
+            at[c] += (int32_t)__popcll(taken & ((W == 32 ? 0xFFFFFFFFull : 0xFFFFull) << (W * c)));
+    }
+}
+
+// Intersection of two rows by one wave, as union_by_wave: the lanes search the
+// longer row for the shorter one's entries.
+template <int SH, bool WRITE>
+__device__ __forceinline__ int32_t intersect_by_wave(const int32_t *__restrict__ src,
+                                                     const int32_t (&at)[2], const int32_t (&end)[2],
+                                                     int32_t *__restrict__ out) {
+    const int lane = __lane_id();
+    const int32_t n0 = end[0] - at[0], n1 = end[1] - at[1];
+    const int32_t *a = src + (n0 <= n1 ? at[0] : at[1]), *b = src + (n0 <= n1 ? at[1] : at[0]);
+    const int32_t na = min(n0, n1), nb = max(n0, n1);
+    int32_t m = 0;
+    for (int32_t i0 = 0; i0 < na; i0 += 64) {
+        const int32_t x = i0 + lane < na ? a[i0 + lane] >> SH : INF;
+        int32_t lo = 0, hi = nb;
+        while (lo < hi) {
+            const int32_t mid = (lo + hi) >> 1;
+            if (b[mid] >> SH < x) lo = mid + 1;
+            else hi = mid;
+        }
+        const bool keep = lo < nb && b[lo] >> SH == x;
+        const uint64_t kept = __ballot(keep);
+        if (WRITE && keep) out[m + (int32_t)__popcll(kept & ((1ull << lane) - 1ull))] = x;
+        m += (int32_t)__popcll(kept);
+    }
+    return m;
+}
+
+// The listed outputs, a wave each: their lengths, or (WRITE) their values at
+// the places that the main launch gave them.  Bound by chains of dependent
+// loads, some ten a row, of which 8192 waves keep as many in flight; a lane each
+// in the main launch walked a chain of a row's length once more for every window
+// of its wave's output.  TT of 100 k cells, 12 % with a row beyond 48: 2620 ->
+// 165 us (one lane's single merge, the rows packed afterwards: 660); of 4000
+// cells around one vertex 53 -> 0.09 ms (2.3).  ET of 293 k cells around 32
+// vertices of up to 2000: 2.96 -> 0.19 ms (1.26).  The list and the lengths are
+// an extra pass over the outputs, so meshes without long rows leave them out.
+constexpr int LONG_THREADS = 256, LONG_BLOCKS = 2048;
+template <int NR, Join J, int SH, bool WRITE, typename RO>
+__global__ __launch_bounds__(LONG_THREADS) void k_join_long(const RO rows_of,
+                                                            const int32_t *__restrict__ src,
+                                                            const int32_t *__restrict__ list,
+                                                            const int32_t *__restrict__ n,
+                                                            int32_t *__restrict__ len,
+                                                            const int64_t *__restrict__ off,
+                                                            int32_t *__restrict__ out) {
+    const int32_t count = *n, waves = (int32_t)gridDim.x * (LONG_THREADS / 64);
+    const int lane = __lane_id();
+    for (int32_t i = (int32_t)blockIdx.x * (LONG_THREADS / 64) + threadIdx.x / 64; i < count; i += waves) {
+        const int32_t id = tgd::lane_value(list[i], 0);
+        const Rows<NR> r = rows_of(id, true);
+        int32_t at[NR], end[NR];
+#pragma unroll
+        for (int c = 0; c < NR; c++) {
+            at[c] = tgd::lane_value(r.p[c], 0);
+            end[c] = at[c] + tgd::lane_value(r.n[c], 0);
+        }
+        int32_t *to = WRITE ? out + off[id] : nullptr;
+        int32_t m;
+        if constexpr (J == INTERSECT) m = intersect_by_wave<SH, WRITE>(src, at, end, to);
+        else m = union_by_wave<NR, SH, WRITE>(src, at, end, id, to);
+        if (!WRITE && lane == 0) len[id] = m;
+    }
+}
 
 // EF(e): faces holding e, from the two faces of e in each cell of ET(e).  One
 // lane per edge builds its sorted, duplicate-free row in an LDS column (in a
@@ -1126,24 +1325,37 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
 }
 
 // Sum of squared row lengths (VT: the lengths of all cells' four rows
-// together); one atomic per block of few.
+// together) and the longest row; one atomic of each per block of few.
 constexpr int SQ_THREADS = 1024, SQ_BLOCKS = 64;
 __global__ __launch_bounds__(SQ_THREADS) void k_row_squares(const int32_t *__restrict__ row_off,
                                                             int64_t rows,
-                                                            unsigned long long *__restrict__ sum) {
+                                                            unsigned long long *__restrict__ sum,
+                                                            int32_t *__restrict__ longest) {
     __shared__ int64_t ws[SQ_THREADS / 64];
+    __shared__ int32_t wm[SQ_THREADS / 64];
     int64_t s = 0;
+    int32_t m = 0;
     for (int64_t v = (int64_t)blockIdx.x * SQ_THREADS + threadIdx.x; v < rows;
          v += (int64_t)gridDim.x * SQ_THREADS) {
         const int64_t n = row_off[v + 1] - row_off[v];
         s += n * n;
+        m = max(m, (int32_t)n);
     }
     s = tgd::wave_sum(s);
-    if (__lane_id() == 0) ws[threadIdx.x / 64] = s;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) m = max(m, __shfl_xor(m, d, 64));
+    if (__lane_id() == 0) {
+        ws[threadIdx.x / 64] = s;
+        wm[threadIdx.x / 64] = m;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < SQ_THREADS / 64; w++) s += ws[w];
+        for (int w = 1; w < SQ_THREADS / 64; w++) {
+            s += ws[w];
+            m = max(m, wm[w]);
+        }
         if (s) atomicAdd(sum, (unsigned long long)s);
+        if (m) atomicMax(longest, m);
     }
 }
 
@@ -1220,15 +1432,6 @@ int fail(int code, const char *msg) {
     return code;
 }
 
-int read_i64(tg_mesh &m, const void *src, int64_t index, int64_t &out) {
-    int64_t *h = (int64_t *)m.h_pinned;
-    TG_HIP(hipMemcpyAsync(h, (const int64_t *)src + index, sizeof(int64_t),
-                          hipMemcpyDeviceToHost, m.stream));
-    TG_HIP(hipStreamSynchronize(m.stream));
-    out = *h;
-    return tg::OK;
-}
-
 // rank structure over n flags (0 or 1): rank_of(rank, p) is the number of
 // flags set before position p.  total, when asked for, is read back, with two
 // further words in the same wait.
@@ -1267,28 +1470,46 @@ int build_ranks(tg_mesh &m, const uint8_t *flags, int64_t n, tg::DevArr &rank,
     return tg::OK;
 }
 
-// Zeroed state of a chained scan over `tiles` tiles, in tmp_b: a sum, the tile
-// counter, the tiles' sums.
+// Zeroed state of a chained scan over `tiles` tiles, in tmp_b: a sum, the
+// longest row, the number of listed outputs, the tile counter, the tiles' sums.
 struct Chain {
     int64_t *sum;
-    int32_t *ticket;
+    int32_t *longest, *listed, *ticket;
     uint64_t *state;
 };
 int chain_state(tg_mesh &m, int64_t tiles, Chain &c) {
-    int rc = m.tmp_b.ensure(sizeof(int64_t) * (size_t)(tiles + 2));
+    int rc = m.tmp_b.ensure(sizeof(int64_t) * (size_t)(tiles + 3));
     if (rc) return rc;
     c.sum = m.tmp_b.as<int64_t>();
-    c.ticket = reinterpret_cast<int32_t *>(c.sum + 1);
-    c.state = reinterpret_cast<uint64_t *>(c.sum + 2);
-    return tg::fill_i32((int32_t *)c.sum, 0, 2 * (tiles + 2), m.stream);
+    c.longest = reinterpret_cast<int32_t *>(c.sum + 1);
+    c.listed = c.longest + 1;
+    c.ticket = reinterpret_cast<int32_t *>(c.sum + 2);
+    c.state = reinterpret_cast<uint64_t *>(c.sum + 3);
+    return tg::fill_i32((int32_t *)c.sum, 0, 2 * (tiles + 3), m.stream);
 }
 
-// Sum of squared row lengths, read back (synchronises).
-int row_squares(tg_mesh &m, const int32_t *row_off, int64_t rows, const Chain &c, int64_t &sum) {
+// Sum of squared row lengths and the longest row, read back (synchronises).
+int row_squares(tg_mesh &m, const int32_t *row_off, int64_t rows, const Chain &c, int64_t &sum,
+                int32_t &longest) {
     hipLaunchKernelGGL(k_row_squares, dim3(std::min(grid(rows, SQ_THREADS), (unsigned)SQ_BLOCKS)),
-                       dim3(SQ_THREADS), 0, m.stream, row_off, rows, (unsigned long long *)c.sum);
+                       dim3(SQ_THREADS), 0, m.stream, row_off, rows, (unsigned long long *)c.sum,
+                       c.longest);
     TG_LAUNCH_CHECK("k_row_squares");
-    return read_i64(m, c.sum, 0, sum);
+    int64_t *h = (int64_t *)m.h_pinned;
+    TG_HIP(hipMemcpyAsync(h, c.sum, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, m.stream));
+    TG_HIP(hipStreamSynchronize(m.stream));
+    sum = h[0];
+    longest = *(const int32_t *)(h + 1);
+    return tg::OK;
+}
+
+// The outputs with a row beyond JOIN_ROW into list (room for `count`).
+template <typename RO>
+int list_long(tg_mesh &m, const RO &rows_of, int64_t count, const Chain &c, int32_t *list) {
+    hipLaunchKernelGGL((k_list_long<RO>), dim3(std::min(grid(count, LIST_THREADS), 8192u)),
+                       dim3(LIST_THREADS), 0, m.stream, rows_of, count, list, c.listed);
+    TG_LAUNCH_CHECK("k_list_long");
+    return tg::OK;
 }
 
 }  // namespace
@@ -1366,14 +1587,33 @@ int ensure_et(tg_mesh &m) {
         (rc = chain_state(m, tiles, c)))
         return rc;
     int64_t *off = m.et_off.as<int64_t>();
-    if (E > 0) {
-        hipLaunchKernelGGL((k_edge_join<INTERSECT, 2, ET_WIN>), dim3((unsigned)tiles),
-                           dim3(EJ_THREADS), 0, m.stream, m.ev.as<int32_t>(), E, m.n_points,
-                           m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(), c.ticket, c.state, off,
-                           m.et_vals.as<int32_t>());
+    static_assert(JOIN_ROW >= LANE_CELLS, "few_cells: no row beyond the networks");
+    const bool listed = !m.few_cells;  // tmp_a: the edges with long rows, and their lengths by edge
+    if (listed && (rc = m.tmp_a.ensure(sizeof(int32_t) * 2 * (size_t)std::max<int64_t>(E, 1)))) return rc;
+    const EdgeRows rows_of{m.ev.as<int32_t>(), m.n_points, m.vt_off.as<int32_t>()};
+    const int32_t *vtc = m.vtc.as<int32_t>();
+    int32_t *list = m.tmp_a.as<int32_t>(), *len = list + E, *out = m.et_vals.as<int32_t>();
+    if (E == 0) {
+        if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) return rc;
+    } else if (!listed) {
+        hipLaunchKernelGGL((k_edge_join<INTERSECT, 2, NO_LONG, ET_WIN>), dim3((unsigned)tiles),
+                           dim3(EJ_THREADS), 0, m.stream, rows_of, E, vtc, nullptr, c.ticket, c.state,
+                           off, out);
         TG_LAUNCH_CHECK("k_edge_join<ET>");
-    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
-        return rc;
+    } else {
+        if ((rc = list_long(m, rows_of, E, c, list))) return rc;
+        hipLaunchKernelGGL((k_join_long<2, INTERSECT, 2, false, EdgeRows>), dim3(LONG_BLOCKS),
+                           dim3(LONG_THREADS), 0, m.stream, rows_of, vtc, list, c.listed, len, nullptr,
+                           nullptr);
+        TG_LAUNCH_CHECK("k_join_long<ET>");
+        hipLaunchKernelGGL((k_edge_join<INTERSECT, 2, LISTED, ET_WIN>), dim3((unsigned)tiles),
+                           dim3(EJ_THREADS), 0, m.stream, rows_of, E, vtc, len, c.ticket, c.state, off,
+                           out);
+        TG_LAUNCH_CHECK("k_edge_join<ET>");
+        hipLaunchKernelGGL((k_join_long<2, INTERSECT, 2, true, EdgeRows>), dim3(LONG_BLOCKS),
+                           dim3(LONG_THREADS), 0, m.stream, rows_of, vtc, list, c.listed, nullptr, off,
+                           out);
+        TG_LAUNCH_CHECK("k_join_long<ET>");
     }
     m.et_built = true;
     return OK;
@@ -1507,18 +1747,37 @@ int ensure_tt(tg_mesh &m) {
         return rc;
     int64_t *off = m.tt_off.as<int64_t>();
     int64_t rows = 0;
+    int32_t longest = 0;
     // the cells' rows together: every vertex's row once per entry
-    if (T > 0 && (rc = row_squares(m, m.vt_off.as<int32_t>(), V, c, rows))) return rc;
-    // a cell's four rows hold the cell itself four times
-    if ((rc = m.tt_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(rows - 4 * T, 1))))
+    if (T > 0 && (rc = row_squares(m, m.vt_off.as<int32_t>(), V, c, rows, longest))) return rc;
+    const bool listed = longest > JOIN_ROW;
+    // a cell's four rows hold the cell itself four times; tmp_a: the cells
+    // with long rows, and their lengths by cell
+    if ((rc = m.tt_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(rows - 4 * T, 1))) ||
+        (listed && (rc = m.tmp_a.ensure(sizeof(int32_t) * 2 * (size_t)T))))
         return rc;
-    if (T > 0) {
-        hipLaunchKernelGGL(k_tt, dim3((unsigned)tiles), dim3(TT_THREADS), 0, m.stream,
-                           m.tv.as<const int4>(), T, m.vt_off.as<int32_t>(), m.vtc.as<int32_t>(),
-                           c.ticket, c.state, off, m.tt_vals.as<int32_t>());
+    const CellRows rows_of{m.tv.as<const int4>(), m.vt_off.as<int32_t>()};
+    const int32_t *vtc = m.vtc.as<int32_t>();
+    int32_t *list = m.tmp_a.as<int32_t>(), *len = list + T, *out = m.tt_vals.as<int32_t>();
+    if (T == 0) {
+        if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) return rc;
+    } else if (!listed) {
+        hipLaunchKernelGGL((k_tt<NO_LONG>), dim3((unsigned)tiles), dim3(TT_THREADS), 0, m.stream,
+                           rows_of, T, vtc, nullptr, c.ticket, c.state, off, out);
         TG_LAUNCH_CHECK("k_tt");
-    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
-        return rc;
+    } else {
+        if ((rc = list_long(m, rows_of, T, c, list))) return rc;
+        hipLaunchKernelGGL((k_join_long<4, UNION_LESS_SELF, 2, false, CellRows>), dim3(LONG_BLOCKS),
+                           dim3(LONG_THREADS), 0, m.stream, rows_of, vtc, list, c.listed, len, nullptr,
+                           nullptr);
+        TG_LAUNCH_CHECK("k_join_long<TT>");
+        hipLaunchKernelGGL((k_tt<LISTED>), dim3((unsigned)tiles), dim3(TT_THREADS), 0, m.stream,
+                           rows_of, T, vtc, len, c.ticket, c.state, off, out);
+        TG_LAUNCH_CHECK("k_tt");
+        hipLaunchKernelGGL((k_join_long<4, UNION_LESS_SELF, 2, true, CellRows>), dim3(LONG_BLOCKS),
+                           dim3(LONG_THREADS), 0, m.stream, rows_of, vtc, list, c.listed, nullptr, off,
+                           out);
+        TG_LAUNCH_CHECK("k_join_long<TT>");
     }
     m.tt_nnz = T > 0 ? -1 : 0;
     m.tt_built = true;
@@ -1565,6 +1824,7 @@ int ensure_ee(tg_mesh &m) {
         return rc;
     int64_t *off = m.ee_off.as<int64_t>();
     int64_t nnz = 0;
+    int32_t longest = 0;
     if (E > 0) {
         hipLaunchKernelGGL(k_vertex_edges, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, m.stream,
                            m.vv_off.as<int32_t>(), V, m.edge_first.as<int32_t>(),
@@ -1572,18 +1832,32 @@ int ensure_ee(tg_mesh &m) {
                            m.tmp_c.as<int32_t>());
         TG_LAUNCH_CHECK("k_vertex_edges");
         // an edge's row: its ends' edges, which share only itself
-        if ((rc = row_squares(m, m.vv_off.as<int32_t>(), V, c, nnz))) return rc;
+        if ((rc = row_squares(m, m.vv_off.as<int32_t>(), V, c, nnz, longest))) return rc;
         nnz -= n2;
     }
-    if ((rc = m.ee_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1)))) return rc;
-    if (E > 0) {
-        hipLaunchKernelGGL((k_edge_join<UNION_LESS_SELF, 0, EE_WIN>), dim3((unsigned)tiles),
-                           dim3(EJ_THREADS), 0, m.stream, m.ev.as<int32_t>(), E, V,
-                           m.vv_off.as<int32_t>(), m.tmp_c.as<int32_t>(), c.ticket, c.state, off,
-                           m.ee_vals.as<int32_t>());
-        TG_LAUNCH_CHECK("k_edge_join<EE>");
-    } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
+    const bool listed = longest > JOIN_ROW;  // tmp_a: the edges with long rows
+    if ((rc = m.ee_vals.ensure(sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1))) ||
+        (listed && (rc = m.tmp_a.ensure(sizeof(int32_t) * (size_t)E))))
         return rc;
+    const EdgeRows rows_of{m.ev.as<int32_t>(), V, m.vv_off.as<int32_t>()};
+    const int32_t *ids = m.tmp_c.as<int32_t>();
+    int32_t *list = m.tmp_a.as<int32_t>(), *out = m.ee_vals.as<int32_t>();
+    if (E == 0) {
+        if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) return rc;
+    } else if (!listed) {
+        hipLaunchKernelGGL((k_edge_join<UNION_LESS_SELF, 0, NO_LONG, EE_WIN>), dim3((unsigned)tiles),
+                           dim3(EJ_THREADS), 0, m.stream, rows_of, E, ids, nullptr, c.ticket, c.state,
+                           off, out);
+        TG_LAUNCH_CHECK("k_edge_join<EE>");
+    } else {
+        hipLaunchKernelGGL((k_edge_join<UNION_LESS_SELF, 0, LISTED, EE_WIN>), dim3((unsigned)tiles),
+                           dim3(EJ_THREADS), 0, m.stream, rows_of, E, ids, nullptr, c.ticket, c.state,
+                           off, out);
+        TG_LAUNCH_CHECK("k_edge_join<EE>");
+        if ((rc = list_long(m, rows_of, E, c, list))) return rc;
+        hipLaunchKernelGGL((k_join_long<2, UNION_LESS_SELF, 0, true, EdgeRows>), dim3(LONG_BLOCKS), dim3(LONG_THREADS),
+                           0, m.stream, rows_of, ids, list, c.listed, nullptr, off, out);
+        TG_LAUNCH_CHECK("k_join_long<EE>");
     }
     m.ee_nnz = nnz;
     m.ee_built = true;

@@ -26,6 +26,9 @@ enum Counter : int {
 };
 enum ErrBit : int { ERRBIT_CAPACITY = 1 };
 
+// Cells of a vertex that one lane of the default bucket kernel takes; it counts
+// vertices with more (or with over 32 neighbours) in C_HEAVY.
+constexpr int LANE_CELLS = 48;
 // Largest vertex degree the serial per-vertex kernels hold in LDS.
 constexpr int HEAVY_CAP = 4096;
 

@@ -56,7 +56,9 @@ struct tg_mesh {
     bool vt_sorted = false;         // vtc rows ascending
     bool vv_built = false, cp_built = false;
     bool counters_pending = false;  // a pipeline ran since the last error check
-    bool vv_short = false;          // that check found a vertex whose row is missing in VV
+    bool heavy_counted = false;     // its C_HEAVY counts vertices of more than LANE_CELLS cells
+    bool few_cells = false;         // known from that: no vertex has more
+    bool vv_short = false;          // the last check found a vertex whose row is missing in VV
 
     // id-assigning and derived relations
     tg::DevArr vt_vals;

@@ -232,6 +232,7 @@ static int run_vv(tg_mesh &m, bool classify) {
     }
     m.vv_built = true;
     m.vv_short = false;
+    m.heavy_counted = hot_variant(m) == 2;
     m.vv_nnz = -1;
     if (classify) m.cp_built = true;
     m.counters_pending = true;
@@ -348,24 +349,26 @@ int capacity_error() {
 
 namespace {
 
-// One wait for the stream's work, the run's error bits (when a run is
+// One wait for the stream's work, the run's counters (when a run is
 // unchecked) and up to eight bytes from src: each readback on its own leaves
 // the device idle for about 30 us.
 int wait_check_read(tg_mesh &m, const void *src, size_t bytes, void *out) {
     int64_t *h = (int64_t *)m.h_pinned;
     const bool check = m.counters_pending;
     if (check)
-        TG_HIP(hipMemcpyAsync(h, m.counters.as<int32_t>() + C_ERR, sizeof(int32_t),
+        TG_HIP(hipMemcpyAsync(h + 1, m.counters.p, sizeof(int32_t) * N_COUNTERS,
                               hipMemcpyDeviceToHost, m.stream));
     if (bytes)
-        TG_HIP(hipMemcpyAsync(h + 1, src, bytes, hipMemcpyDeviceToHost, m.stream));
+        TG_HIP(hipMemcpyAsync(h, src, bytes, hipMemcpyDeviceToHost, m.stream));
     TG_HIP(hipStreamSynchronize(m.stream));
     m.counters_pending = false;
-    if (check && (*(const int32_t *)h & ERRBIT_CAPACITY)) {
+    const int32_t *counters = (const int32_t *)(h + 1);
+    if (check && m.heavy_counted && counters[C_HEAVY] == 0) m.few_cells = true;
+    if (check && (counters[C_ERR] & ERRBIT_CAPACITY)) {
         m.vv_short = true;
         return capacity_error();
     }
-    if (bytes) std::memcpy(out, h + 1, bytes);
+    if (bytes) std::memcpy(out, h, bytes);
     return OK;
 }
 

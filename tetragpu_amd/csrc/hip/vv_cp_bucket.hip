@@ -854,7 +854,7 @@ __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_vv_cp(
 // tables it replaced waited on chains of dependent LDS round trips.  LDS is
 // what limits the waves: 20 KB a wave, records of nine bytes, for 64 vertices
 // of 33 records each.
-constexpr int SK_MAXREC = 48;       // records per vertex; more go to the heavy kernel
+constexpr int SK_MAXREC = tg::LANE_CELLS;  // records per vertex; more go to the heavy kernel
 constexpr int SK_PRE = 24;          // records per thread held in registers while counting
 constexpr int SK_ROWS = SLOTS + 1;  // row slots per vertex, the last one for what does not fit
 template <int BV>
