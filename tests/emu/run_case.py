@@ -254,7 +254,24 @@ def case_hub_rows(shared: int = 50, apart: int = 0, between: int = 0, order: int
     check_hubs(t, shared, apart, between, order)
 
 
-CASES = {"hub_rows": case_hub_rows, "capacity": case_capacity, "split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
+def case_vertex_rows(n: int = 140, hub_first: int = 1) -> None:
+    """Edge relations where a vertex's row is ordered by the whole block."""
+    from test_gpu_relations import oracle_all, same_csr, same_fixed
+
+    i = np.random.default_rng(n).permutation(n).astype(np.int32)
+    strip = np.stack([i, i + 1, i + 2], 1) + (1 if hub_first else 0)
+    hub = np.full((n, 1), 0 if hub_first else n + 2, np.int32)
+    cells = np.ascontiguousarray(np.hstack([hub, strip] if hub_first else [strip, hub]))
+    ref = oracle_all(cells, n + 3)
+    with t.Mesh(cells, n + 3) as d:
+        d.build(t.flags("TE", "EV", "VE", "EE"))
+        same_fixed(d.relation("TE"), ref["TE"], "TE")
+        same_fixed(d.relation("EV"), ref["EV"], "EV")
+        same_csr(d.relation("VE"), ref["VE"], "VE")
+        same_csr(d.relation("EE"), ref["EE"], "EE")
+
+
+CASES = {"hub_rows": case_hub_rows, "vertex_rows": case_vertex_rows, "capacity": case_capacity, "split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
          "vv_cp": case_vv_cp, "window": case_window, "hubs": case_hubs, "soup": case_soup, "routes": case_routes}
 
 

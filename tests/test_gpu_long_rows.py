@@ -62,13 +62,13 @@ def seconds(t, cells, V, first, then):
     return best
 
 
-@pytest.mark.parametrize("first,then,n", [("VT", "TT", 34)])
+@pytest.mark.parametrize("first,then,n", [("VT", "TT", 34), ("TE", "EE", 44)])
 def test_long_rows_cost_their_entries(gpu, first, then, n):
-    """4000 cells around one vertex give as many entries as a grid of n^3 cubes
-    and take no more than 20 times as long (both take about 0.1 ms; one lane's
-    merge of each row took 15 times, one that starts anew for every window of
-    a wave's output 700)."""
-    i = np.arange(4000, dtype=np.int32)
+    """4000 cells around one vertex in random order give about as many entries as
+    a grid of n^3 cubes and take no more than 20 times as long (both take 0.1 to
+    0.2 ms; a row's merge that starts anew for every window of a wave's output
+    takes hundreds of times as long, one lane's sort by insertion thousands)."""
+    i = np.random.default_rng(4).permutation(4000).astype(np.int32)
     fan = np.ascontiguousarray(np.stack([i, i + 1, i + 2, np.full(4000, 4002, np.int32)], 1))
     m = gpu.kuhn(n, seed=1)
     long = seconds(gpu, fan, 4003, first, then)

@@ -307,41 +307,117 @@ __global__ void k_ev(const int4 *__restrict__ tv4, int64_t T, const uint4 *__res
     }
 }
 
+// Long rows of keys, all different, in order.  Up to WAVE_ROW keys by one wave:
+// every lane's key is compared with every key of the row, 64 a load; more, up
+// to as many as a VV row holds, by the block's bitonic sort in LDS.  EE after
+// TE on the 100 k-cell fan mesh (rows of up to 313): 0.32 ms, with one lane's
+// insertion in memory 7.3, with its heapsort 0.92; on 4000 cells around one
+// vertex 0.16 ms, 4.1 if one wave compares there too.
+constexpr int WAVE_ROW = 128;
+
+// f(place, key) for each key of a row, place being the number of smaller ones.
+template <typename F>
+__device__ __forceinline__ void rank_by_wave(const int32_t *__restrict__ key, int32_t n, F f) {
+    const int lane = __lane_id();
+    for (int32_t i0 = 0; i0 < n; i0 += 64) {
+        const int32_t x = key[min(i0 + lane, n - 1)];
+        int32_t place = 0;
+        for (int32_t j0 = 0; j0 < n; j0 += 64) {
+            const int32_t y = j0 + lane < n ? key[j0 + lane] : INF;
+#pragma unroll 16
+            for (int j = 0; j < 64; j++) place += tgd::lane_value(y, j) < x;
+        }
+        if (i0 + lane < n) f(place, x);
+    }
+}
+
+template <int THREADS>
+struct LongRow {
+    int32_t key[tg::HEAVY_CAP];
+    int32_t row[THREADS], n;
+};
+
+// The row of n keys at key + at of each lane that has more than 32:
+// f(to, place, key) for all of its keys.  Every thread of the block calls it.
+template <int THREADS, typename F>
+__device__ __forceinline__ void order_long_rows(LongRow<THREADS> &st, const int32_t *__restrict__ key,
+                                                int32_t at, int32_t n, int32_t to, F f) {
+    const int tid = threadIdx.x;
+    for (uint64_t b = __ballot(n > 32 && n <= WAVE_ROW); b; b &= b - 1) {
+        const int l = __ffsll((unsigned long long)b) - 1;
+        const int32_t lto = tgd::lane_value(to, l);
+        rank_by_wave(key + tgd::lane_value(at, l), tgd::lane_value(n, l),
+                     [&](int32_t place, int32_t x) { f(lto, place, x); });
+    }
+    if (__syncthreads_and(n <= WAVE_ROW)) return;
+    if (tid == 0) st.n = 0;
+    __syncthreads();
+    if (n > WAVE_ROW) st.row[atomicAdd(&st.n, 1)] = tid;
+    __syncthreads();
+    for (int r = 0; r < st.n; r++) {
+        if (tid == st.row[r]) {  // handed over by way of the staging
+            st.key[0] = at;
+            st.key[1] = n;
+            st.key[2] = to;
+        }
+        __syncthreads();
+        const int32_t rat = st.key[0], rn = min(st.key[1], (int32_t)tg::HEAVY_CAP), rto = st.key[2];
+        __syncthreads();
+        int32_t size = 2 * WAVE_ROW;
+        while (size < rn) size *= 2;
+        for (int32_t i = tid; i < size; i += THREADS) st.key[i] = i < rn ? key[rat + i] : INF;
+        __syncthreads();
+        for (int32_t k = 2; k <= size; k *= 2)
+            for (int32_t j = k / 2; j > 0; j /= 2) {
+                for (int32_t i = tid; i < size / 2; i += THREADS) {
+                    const int32_t lo = 2 * i - (i & (j - 1)), hi = lo + j;
+                    const int32_t x = st.key[lo], y = st.key[hi];
+                    if ((x > y) == ((lo & k) == 0)) {
+                        st.key[lo] = y;
+                        st.key[hi] = x;
+                    }
+                }
+                __syncthreads();
+            }
+        for (int32_t i = tid; i < rn; i += THREADS) f(rto, i, st.key[i]);
+        __syncthreads();
+    }
+}
+
 // Each vertex's edge ids, ascending (for EE): the upper entries' ids are VE's,
 // a lower entry's is the rank of its first position, which k_edge_first noted
 // for both ends of an edge.  (Searching v in each lower neighbour's row took
 // 0.63 ms at 5.3 M cells, and sorting the rows in memory 0.28; VE's
-// ids from a copy along VV and a count per 32-bit word 0.23; this pass 0.13.)  Rows of up to 32 entries are sorted in registers, longer ones in
-// memory.
-__global__ __launch_bounds__(256) void k_vertex_edges(const int32_t *__restrict__ vv_off, int64_t V,
-                                                      const int32_t *__restrict__ efirst,
-                                                      const uint4 *__restrict__ rank,
-                                                      const int32_t *__restrict__ ve_off,
-                                                      const int2 *__restrict__ ve,
-                                                      int32_t *__restrict__ out) {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
-    const int32_t rb = vv_off[v], rn = vv_off[v + 1] - rb;
-    const int32_t vb = ve_off[v], lower = rn - (ve_off[v + 1] - vb);
-    auto id_of = [&](int32_t i) {
-        return i < rb + lower ? rank_at(rank, efirst[i]) : ve[vb + (i - rb - lower)].y;
-    };
+// ids from a copy along VV and a count per 32-bit word 0.23; this pass 0.13.)
+// Rows of up to 32 entries are sorted in registers.  In longer ones the first
+// positions are ordered, as which the ids ascend, and each is looked up once.
+constexpr int VX_THREADS = 256;
+__global__ __launch_bounds__(VX_THREADS) void k_vertex_edges(const int32_t *__restrict__ vv_off,
+                                                             int64_t V,
+                                                             const int32_t *__restrict__ efirst,
+                                                             const uint4 *__restrict__ rank,
+                                                             const int32_t *__restrict__ ve_off,
+                                                             const int2 *__restrict__ ve,
+                                                             int32_t *__restrict__ out) {
+    __shared__ LongRow<VX_THREADS> lng;
+    const int64_t v = (int64_t)blockIdx.x * VX_THREADS + threadIdx.x;
+    const int32_t rb = v < V ? vv_off[v] : 0, rn = v < V ? vv_off[v + 1] - rb : 0;
     if (rn <= 32) {
+        const int32_t vb = v < V ? ve_off[v] : 0, lower = v < V ? rn - (ve_off[v + 1] - vb) : 0;
         int32_t k[32];
 #pragma unroll
-        for (int i = 0; i < 32; i++) k[i] = i < rn ? id_of(rb + i) : INF;
+        for (int i = 0; i < 32; i++) {
+            k[i] = INF;
+            if (i < rn) k[i] = i < lower ? rank_at(rank, efirst[rb + i]) : ve[vb + (i - lower)].y;
+        }
         tgn::sort_keys(k);
 #pragma unroll
         for (int i = 0; i < 32; i++)
             if (i < rn) out[rb + i] = k[i];
-    } else {
-        for (int32_t i = 0; i < rn; i++) {
-            const int32_t x = id_of(rb + i);
-            int32_t j = i;
-            for (; j > 0 && out[rb + j - 1] > x; j--) out[rb + j] = out[rb + j - 1];
-            out[rb + j] = x;
-        }
     }
+    order_long_rows(lng, efirst, rb, rn, rb, [&](int32_t to, int32_t place, int32_t p) {
+        out[to + place] = rank_at(rank, p);
+    });
 }
 
 // ---- faces ----------------------------------------------------------------------
@@ -1108,8 +1184,7 @@ __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ e
 // ids of v's row in the order v's cells first meet its upper neighbours, so
 // ordering by id is the reference's row order.  Lane per vertex: the upper
 // entries are counted for the chained scan, their ids looked up and sorted in
-// registers.  A row of more than 32 upper
-// entries is ordered by the whole wave, each lane counting the smaller ids.
+// registers, longer rows of them ordered as k_vertex_edges orders its own.
 // Bound by the rank lookups: their words are lines of a table that one XCD's
 // L2 does not hold.  2.2 M cells: 81 us, 5 M: 202; a count, a scan, the
 // ids with EV and a fill by an LDS sort in launches of their own: 142 (with EV's
@@ -1136,13 +1211,15 @@ __device__ __forceinline__ void ve_row(const int32_t *__restrict__ vv,
         if (i < n) row[i] = make_int2((int32_t)(uint32_t)k[i], (int32_t)(k[i] >> 32));
 }
 
-__global__ __launch_bounds__(VE_THREADS) void k_ve(const int32_t *__restrict__ vv_off,
+__global__ __launch_bounds__(VE_THREADS) void k_ve(const int4 *__restrict__ tv4,
+                                                   const int32_t *__restrict__ vv_off,
                                                    const int32_t *__restrict__ vv, int64_t V,
                                                    const int32_t *__restrict__ efirst,
                                                    const uint4 *__restrict__ rank,
                                                    int32_t *ticket, uint64_t *state,
                                                    int32_t *__restrict__ off,
                                                    int2 *__restrict__ out) {
+    __shared__ LongRow<VE_THREADS> lng;
     __shared__ int32_t wtot[VE_THREADS / 64];
     __shared__ int32_t shared_tile;
     __shared__ int64_t base;
@@ -1184,20 +1261,12 @@ __global__ __launch_bounds__(VE_THREADS) void k_ve(const int32_t *__restrict__ v
     const int32_t ns = n <= 32 ? n : 0;
     if (__any(ns > 16)) ve_row<32>(vv + ub, efirst + ub, rank, ns, row);
     else ve_row<16>(vv + ub, efirst + ub, rank, ns, row);
-    for (uint64_t big = __ballot(n > 32); big; big &= big - 1) {  // the wave on one row
-        const int l = __ffsll((unsigned long long)big) - 1;
-        const int32_t bn = __shfl(n, l), bu = __shfl(ub, l), ba = __shfl(at, l);
-        for (int32_t k0 = 0; k0 < bn; k0 += 64) {
-            const int32_t k = bu + min(k0 + lane, bn - 1);
-            const int32_t id = rank_at(rank, efirst[k]);
-            int32_t p = 0;  // ids below the lane's
-            for (int32_t j0 = 0; j0 < bn; j0 += 64) {
-                const int32_t o = rank_at(rank, efirst[bu + min(j0 + lane, bn - 1)]);
-                for (int32_t j = 0; j < min(64, bn - j0); j++) p += __shfl(o, j) < id;
-            }
-            if (k0 + lane < bn) out[ba + p] = make_int2(vv[k], id);
-        }
-    }
+    // longer rows: ids ascend as first positions do; a position names its edge
+    order_long_rows(lng, efirst, ub, n, at, [&](int32_t to, int32_t place, int32_t p) {
+        const int4 q = tv4[p / 6];
+        const int k = p % 6, i = k < 3 ? 0 : k < 5 ? 1 : 2, j = k < 3 ? k + 1 : k < 5 ? k - 1 : 3;
+        out[to + place] = make_int2(max(corner(q, i), corner(q, j)), rank_at(rank, p));
+    });
 }
 
 // VF rows {mid, hi, id}: the row of a holds the faces whose positional low
@@ -1554,7 +1623,7 @@ int ensure_edges(tg_mesh &m) {
     int32_t *voff = m.ve_off.as<int32_t>();
     if (V > 0) {
         hipLaunchKernelGGL(k_ve, dim3((unsigned)tiles), dim3(VE_THREADS), 0, m.stream,
-                           m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
+                           m.tv.as<const int4>(), m.vv_off.as<int32_t>(), m.vv_cols.as<int32_t>(), V,
                            m.edge_first.as<int32_t>(), m.edge_rank.as<uint4>(), c.ticket, c.state,
                            voff, m.ve_vals.as<int2>());
         TG_LAUNCH_CHECK("k_ve");
@@ -1826,7 +1895,8 @@ int ensure_ee(tg_mesh &m) {
     int64_t nnz = 0;
     int32_t longest = 0;
     if (E > 0) {
-        hipLaunchKernelGGL(k_vertex_edges, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, m.stream,
+        hipLaunchKernelGGL(k_vertex_edges, dim3((unsigned)((V + VX_THREADS - 1) / VX_THREADS)),
+                           dim3(VX_THREADS), 0, m.stream,
                            m.vv_off.as<int32_t>(), V, m.edge_first.as<int32_t>(),
                            m.edge_rank.as<uint4>(), m.ve_off.as<int32_t>(), m.ve_vals.as<int2>(),
                            m.tmp_c.as<int32_t>());
