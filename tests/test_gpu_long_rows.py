@@ -53,8 +53,8 @@ def seconds(t, cells, V, first, then):
     best = float("inf")
     for _ in range(5):
         with t.Mesh(cells, V) as m:
-            m.build(t.flags(first))
-            m.shape(first)
+            m.build(t.flags(*first.split(",")))
+            m.shape(first.split(",")[0])
             t0 = time.perf_counter()
             m.build(t.flags(then))
             m.shape(then)
@@ -62,12 +62,14 @@ def seconds(t, cells, V, first, then):
     return best
 
 
-@pytest.mark.parametrize("first,then,n", [("VT", "TT", 34), ("TE", "EE", 44)])
+@pytest.mark.parametrize("first,then,n", [("VT", "TT", 34), ("TE", "EE", 44), ("VV,VT", "TE", 44)])
 def test_long_rows_cost_their_entries(gpu, first, then, n):
     """4000 cells around one vertex in random order give about as many entries as
     a grid of n^3 cubes and take no more than 20 times as long (both take 0.1 to
     0.2 ms; a row's merge that starts anew for every window of a wave's output
-    takes hundreds of times as long, one lane's sort by insertion thousands)."""
+    takes hundreds of times as long, one lane's sort by insertion thousands).  The
+    fan's TE is small, 0.5 ms; one lane that searches the vertex's row for each
+    of its cells takes 16."""
     i = np.random.default_rng(4).permutation(4000).astype(np.int32)
     fan = np.ascontiguousarray(np.stack([i, i + 1, i + 2, np.full(4000, 4002, np.int32)], 1))
     m = gpu.kuhn(n, seed=1)

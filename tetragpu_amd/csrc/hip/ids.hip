@@ -73,25 +73,20 @@ __device__ __forceinline__ int32_t bsearch_i32(const int32_t *a, int32_t n, int3
 typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef int32_t i32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// k_edge_first stages its row in LDS: one column per thread (consecutive threads in consecutive banks),
-// filled by independent 16-byte loads, so a row costs one memory latency
-// instead of one per element; the merge then reads LDS.  Whole quads are
-// read, up to three words past the row (the source array carries that
-// slack), and all four words go to the column: the words past the row land
-// where the next row is staged, or in the column's three spare slots after
-// the last row.  A thread whose rows exceed the column merges from global
-// memory.
+// A thread's row of n words in its LDS column (consecutive threads in
+// consecutive banks), by independent 16-byte loads, so that it costs one memory
+// latency instead of one per element.  Whole quads are read, up to three words
+// past the row (the source array carries that slack).
 template <int W>
-__device__ __forceinline__ void stage_quads(int32_t (*buf)[W], int at,
-                                            const int32_t *__restrict__ src, int32_t n,
-                                            int shift) {
+__device__ __forceinline__ void stage_quads(int32_t (*buf)[W], const int32_t *__restrict__ src,
+                                            int32_t n) {
 #pragma unroll 4
     for (int32_t k = 0; k < n; k += 4) {
         const i32x4u v = *reinterpret_cast<const i32x4u *>(src + k);
-        buf[at + k][threadIdx.x] = v.x >> shift;
-        buf[at + k + 1][threadIdx.x] = v.y >> shift;
-        buf[at + k + 2][threadIdx.x] = v.z >> shift;
-        buf[at + k + 3][threadIdx.x] = v.w >> shift;
+        buf[k][threadIdx.x] = v.x;
+        buf[k + 1][threadIdx.x] = v.y;
+        buf[k + 2][threadIdx.x] = v.z;
+        buf[k + 3][threadIdx.x] = v.w;
     }
 }
 
@@ -128,29 +123,35 @@ struct QuadOutExact {
 // Every pair of v's cells whose low vertex is v also records its edge's first
 // position in te (replaced by the edge id, its rank, once ranks exist): the
 // row search is done here, on v's own row, instead of once per cell on random
-// rows, and the ranks (8 bytes per 32 positions) are a sixth of the VV-aligned
-// ids that te could index instead.
+// rows, and the ranks (16 bytes per 96 positions) are a fraction of the
+// VV-aligned ids that te could index instead.
 // Rows up to EDGE_CAP entries are staged in LDS (one column per thread: the
 // VV row and the first positions), and the vertex's cells are fetched eight
-// at a time with independent loads; longer rows work in global memory.
-constexpr int EDGE_THREADS = 64, EDGE_CAP = 32;  // 17 KB a wave: nine waves per CU
+// at a time with independent loads.  A longer row is the whole wave's: its
+// first positions fill the LDS, the lanes go over the vertex's cells.  (TE, EV
+// and VE of 4000 cells around one vertex 0.5 ms, by one lane in global memory
+// 16 with the highest id and 19 with the lowest; of a 470 k-cell Delaunay
+// mesh 0.23 ms, 0.51.)
+constexpr int EDGE_THREADS = 64, EDGE_CAP = 32;  // 16 KB a wave: ten waves per CU
 
 __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
     const int4 *__restrict__ tv4, const int32_t *__restrict__ vt_off,
     const int32_t *__restrict__ vtc, const int32_t *__restrict__ vv_off,
     const int32_t *__restrict__ vv, int64_t V, int32_t *__restrict__ efirst,
     uint8_t *__restrict__ flags, int32_t *__restrict__ te_first) {
-    __shared__ int32_t srow[EDGE_CAP + 3][EDGE_THREADS];  // three spare slots for stage_quads
-    __shared__ int32_t sef[EDGE_CAP][EDGE_THREADS];
+    static_assert(EDGE_CAP % 4 == 0, "rows are staged by whole quads");
+    static_assert(2 * EDGE_CAP * EDGE_THREADS >= tg::HEAVY_CAP, "one row's first positions");
+    __shared__ int32_t lds[2 * EDGE_CAP * EDGE_THREADS];
+    int32_t(*srow)[EDGE_THREADS] = reinterpret_cast<int32_t(*)[EDGE_THREADS]>(lds);
+    int32_t(*sef)[EDGE_THREADS] = srow + EDGE_CAP;
     const int tid = threadIdx.x;
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + tid; v < V;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t rb = vv_off[v], rn = vv_off[v + 1] - rb;
-        const int32_t *row = vv + rb;
-        int32_t *ef = efirst + rb;
-        const int32_t kb = vt_off[v], ke = vt_off[v + 1];
-        if (rn <= EDGE_CAP) {
-            stage_quads(srow, 0, row, rn, 0);
+    for (int64_t v0 = (int64_t)blockIdx.x * EDGE_THREADS; v0 < V; v0 += (int64_t)gridDim.x * EDGE_THREADS) {
+        const int64_t v = v0 + tid;
+        const bool act = v < V;
+        const int32_t rb = act ? vv_off[v] : 0, rn = act ? vv_off[v + 1] - rb : 0;
+        const int32_t kb = act ? vt_off[v] : 0, ke = act ? vt_off[v + 1] : 0;
+        if (act && rn <= EDGE_CAP) {
+            stage_quads(srow, vv + rb, rn);
             for (int32_t i = 0; i < rn; i++) sef[i][tid] = INF;
             for (int32_t k0 = kb; k0 < ke; k0 += 8) {
                 int32_t pc[8];
@@ -183,31 +184,50 @@ __global__ __launch_bounds__(EDGE_THREADS) void k_edge_first(
                 }
             }
             QuadOutExact o;
-            o.row = ef;
+            o.row = efirst + rb;
             for (int32_t i = 0; i < rn; i++) {
                 const int32_t e = sef[i][tid];
                 o.put(e);
                 if (srow[i][tid] > v && e != INF) flags[e] = 1;
             }
             o.flush();
-            continue;
         }
-        for (int32_t i = 0; i < rn; i++) ef[i] = INF;
-        for (int32_t k = kb; k < ke; k++) {
-            const int32_t p = vtc[k];
-            const int32_t t = p >> 2, jv = p & 3;
-            const int4 q = tv4[t];
-            for (int j = 0; j < 4; j++) {
-                if (j == jv) continue;
-                const int32_t u = corner(q, j);
-                const int32_t idx = bsearch_i32(row, rn, u);
-                const int32_t pos = 6 * t + pair_index(min(j, jv), max(j, jv));
-                if (idx >= 0 && ef[idx] == INF) ef[idx] = pos;
-                if (u > v) te_first[pos] = idx >= 0 ? ef[idx] : INF;
+        for (uint64_t b = __ballot(rn > EDGE_CAP); b; b &= b - 1) {
+            const int l = __ffsll((unsigned long long)b) - 1;
+            const int32_t w = (int32_t)v0 + l, wrb = tgd::lane_value(rb, l), wrn = tgd::lane_value(rn, l);
+            const int32_t wkb = tgd::lane_value(kb, l), wke = tgd::lane_value(ke, l);
+            const int32_t *row = vv + wrb;
+            tgd::wave_sync();  // what was in the LDS has been read
+            for (int32_t i = tid; i < wrn; i += EDGE_THREADS) lds[i] = INF;
+            tgd::wave_sync();
+            // f(position, u) for the lane's share of the vertex's cells' edges
+            auto each = [&](auto f) {
+                for (int32_t k = wkb + tid; k < wke; k += EDGE_THREADS) {
+                    const int32_t p = vtc[k], t = p >> 2, jv = p & 3;
+                    const int4 q = tv4[t];
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (j != jv) f(6 * t + pair_index(min(j, (int)jv), max(j, (int)jv)), corner(q, j));
+                }
+            };
+            each([&](int32_t pos, int32_t u) {
+                const int32_t idx = bsearch_i32(row, wrn, u);
+                if (idx >= 0) atomicMin(&lds[idx], pos);
+                if (u > w) te_first[pos] = idx;
+            });
+            tgd::wave_sync();
+            each([&](int32_t pos, int32_t u) {
+                if (u <= w) return;
+                const int32_t idx = te_first[pos];
+                te_first[pos] = idx >= 0 ? lds[idx] : INF;
+            });
+            for (int32_t i = tid; i < wrn; i += EDGE_THREADS) {
+                const int32_t e = lds[i];
+                efirst[wrb + i] = e;
+                if (row[i] > w && e != INF) flags[e] = 1;
             }
         }
-        for (int32_t i = 0; i < rn; i++)
-            if (row[i] > v && ef[i] != INF) flags[ef[i]] = 1;
+        tgd::wave_sync();
     }
 }
 
