@@ -1298,8 +1298,10 @@ __global__ __launch_bounds__(VE_THREADS) void k_ve(const int4 *__restrict__ tv4,
 // cell).  The first walk counts and keeps three bits for each of the first 32
 // cells; after the chained scan the second one visits only cells that give a
 // face.  2.2 M cells: 0.23 ms; first positions and TF read instead, in this
-// kernel or in two with a scan between them, 0.38.
-constexpr int VF_THREADS = 256;
+// kernel or in two with a scan between them, 0.38.  The cells of a vertex with
+// more than VF_ROW are the wave's, a lane each (4000 cells around the vertex of
+// the lowest id: TF, FV and VF after ET 2.3 -> 0.16 ms).
+constexpr int VF_THREADS = 256, VF_ROW = 96;
 __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
                                                    const int32_t *__restrict__ vt_off,
                                                    const int32_t *__restrict__ vtc, int64_t V,
@@ -1328,11 +1330,13 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
     };
     uint32_t m0 = 0, m1 = 0, m2 = 0;  // bit k: the cell's 1st, 2nd, 3rd slot, for the first 32 cells
     int32_t n = 0;
-    for (int32_t k0 = kb; k0 < ke; k0 += 8) {
+    const bool by_wave = ke - kb > VF_ROW;
+    const int32_t le = by_wave ? kb : ke;  // end of the cells that the lane takes
+    for (int32_t k0 = kb; k0 < le; k0 += 8) {
         int32_t p[8];
         uint32_t ff[8];
 #pragma unroll
-        for (int c = 0; c < 8; c++) p[c] = k0 + c < ke ? vtc[k0 + c] : 2;
+        for (int c = 0; c < 8; c++) p[c] = k0 + c < le ? vtc[k0 + c] : 2;
 #pragma unroll
         for (int c = 0; c < 8; c++)
             ff[c] = (p[c] & 3) <= 1 ? *word(p[c]) : 0u;
@@ -1346,6 +1350,17 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
                 m2 |= (f >> 2) << ((k0 + c - kb) & 31);
             }
         }
+    }
+    for (uint64_t b = __ballot(by_wave); b; b &= b - 1) {
+        const int l = __ffsll((unsigned long long)b) - 1;
+        const int32_t end = tgd::lane_value(ke, l);
+        int32_t c = 0;
+        for (int32_t k = tgd::lane_value(kb, l) + lane; k < end; k += 64) {
+            const int32_t p = vtc[k];
+            if ((p & 3) <= 1) c += __popc(firsts(p, *word(p)));
+        }
+        c = tgd::wave_sum(c);
+        if (lane == l) n = c;
     }
     const int32_t inc = tgd::wave_inclusive_sum(n);
     if (lane == 63) wtot[wid] = inc;
@@ -1365,12 +1380,10 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
         }
     }
     __syncthreads();
-    if (!act) return;
     const int32_t at = (int32_t)base + before + inc - n;
-    off[a] = at;
+    if (act) off[a] = at;
     if (a == V - 1) off[V] = (int32_t)base + total;
-    int32_t *row = out + 3 * (int64_t)at;
-    auto write = [&](int32_t p, uint32_t f, const int4 q, const uint4 w) {
+    auto write = [&](int32_t *&row, int32_t p, uint32_t f, const int4 q, const uint4 w) {
 #pragma unroll
         for (int m = 0; m < 3; m++) {
             if (!((f >> m) & 1u)) continue;
@@ -1384,6 +1397,7 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
             row += 3;
         }
     };
+    int32_t *row = out + 3 * (int64_t)at;
     uint32_t any = m0 | m1 | m2;
     while (any) {  // eight cells at a time
         int32_t p[8];
@@ -1403,13 +1417,26 @@ __global__ __launch_bounds__(VF_THREADS) void k_vf(const int4 *__restrict__ tv4,
             w[c] = rank[((uint32_t)p[c] >> 2) / CELLS];
         }
 #pragma unroll
-        for (int c = 0; c < 8; c++) write(p[c], f[c], q[c], w[c]);
+        for (int c = 0; c < 8; c++) write(row, p[c], f[c], q[c], w[c]);
     }
-    for (int32_t k = kb + 32; k < ke; k++) {
+    for (int32_t k = kb + 32; k < le; k++) {
         const int32_t p = vtc[k];
         if ((p & 3) > 1) continue;
         const uint32_t f = firsts(p, *word(p));
-        if (f) write(p, f, tv4[p >> 2], rank[((uint32_t)p >> 2) / CELLS]);
+        if (f) write(row, p, f, tv4[p >> 2], rank[((uint32_t)p >> 2) / CELLS]);
+    }
+    for (uint64_t b = __ballot(by_wave); b; b &= b - 1) {
+        const int l = __ffsll((unsigned long long)b) - 1;
+        const int32_t end = tgd::lane_value(ke, l);
+        int32_t done = tgd::lane_value(at, l);
+        for (int32_t k0 = tgd::lane_value(kb, l); k0 < end; k0 += 64) {
+            const int32_t p = k0 + lane < end ? vtc[k0 + lane] : 2;
+            const uint32_t f = (p & 3) <= 1 ? firsts(p, *word(p)) : 0u;
+            const int32_t c = tgd::wave_inclusive_sum((int32_t)__popc(f));
+            int32_t *to = out + 3 * (int64_t)(done + c - (int32_t)__popc(f));
+            if (f) write(to, p, f, tv4[p >> 2], rank[((uint32_t)p >> 2) / CELLS]);
+            done += tgd::lane_value(c, 63);
+        }
     }
 }
 
