@@ -351,6 +351,24 @@ __device__ __forceinline__ void rank_by_wave(const int32_t *__restrict__ key, in
     }
 }
 
+// size keys in LDS, a power of two, ascending; by a whole block, which has
+// written them before a barrier.  Ends with one.
+template <int THREADS>
+__device__ __forceinline__ void sort_by_block(int32_t *key, int32_t size) {
+    for (int32_t k = 2; k <= size; k *= 2)
+        for (int32_t j = k / 2; j > 0; j /= 2) {
+            for (int32_t i = threadIdx.x; i < size / 2; i += THREADS) {
+                const int32_t lo = 2 * i - (i & (j - 1)), hi = lo + j;
+                const int32_t x = key[lo], y = key[hi];
+                if ((x > y) == ((lo & k) == 0)) {
+                    key[lo] = y;
+                    key[hi] = x;
+                }
+            }
+            __syncthreads();
+        }
+}
+
 template <int THREADS>
 struct LongRow {
     int32_t key[tg::HEAVY_CAP];
@@ -387,18 +405,7 @@ __device__ __forceinline__ void order_long_rows(LongRow<THREADS> &st, const int3
         while (size < rn) size *= 2;
         for (int32_t i = tid; i < size; i += THREADS) st.key[i] = i < rn ? key[rat + i] : INF;
         __syncthreads();
-        for (int32_t k = 2; k <= size; k *= 2)
-            for (int32_t j = k / 2; j > 0; j /= 2) {
-                for (int32_t i = tid; i < size / 2; i += THREADS) {
-                    const int32_t lo = 2 * i - (i & (j - 1)), hi = lo + j;
-                    const int32_t x = st.key[lo], y = st.key[hi];
-                    if ((x > y) == ((lo & k) == 0)) {
-                        st.key[lo] = y;
-                        st.key[hi] = x;
-                    }
-                }
-                __syncthreads();
-            }
+        sort_by_block<THREADS>(st.key, size);
         for (int32_t i = tid; i < rn; i += THREADS) f(rto, i, st.key[i]);
         __syncthreads();
     }
@@ -1095,8 +1102,8 @@ __global__ __launch_bounds__(LONG_THREADS) void k_join_long(const RO rows_of,
 
 // EF(e): faces holding e, from the two faces of e in each cell of ET(e).  One
 // lane per edge builds its sorted, duplicate-free row in an LDS column (in a
-// padded slot of 2|ET(e)| words of tmp while the column is too short), the
-// block's total joins the chained scan, and the row goes to its place.  Bound
+// padded slot of 2|ET(e)| words of tmp where the column is too short: by the
+// wave up to 64 cells, then by the block), the block's total joins the chained scan, and the row goes to its place.  Bound
 // by the lines that the gathers of ET's cells move: one a cell, from rows that
 // hold its corners and faces together (TE and TF, a line each: 468 us at 2.2 M
 // cells, this 303 and 25 to lay the rows out).
@@ -1120,20 +1127,87 @@ __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ e
                                                    int32_t *__restrict__ tmp) {
     __shared__ int32_t col[EF_CAP][EF_THREADS];
     __shared__ int32_t wtot[EF_THREADS / 64];
-    __shared__ int32_t shared_tile;
+    __shared__ int32_t shared_tile, nlong, lng[EF_THREADS];
     __shared__ int64_t base;
+    __shared__ struct { int64_t first; int32_t n, lo, hi; } one;
     const int tid = threadIdx.x, lane = __lane_id(), wid = tid / 64;
     const int32_t tile = take_tile(ticket, shared_tile);
     const int64_t e = (int64_t)tile * EF_THREADS + tid;
     const bool act = e < E;
     const int64_t b0 = act ? et_off[e] : 0, b1 = act ? et_off[e + 1] : 0;
-    const bool lds = 2 * (b1 - b0) <= EF_CAP;
+    const bool lds = 2 * (b1 - b0) <= EF_CAP, by_wave = !lds && b1 - b0 <= 64;
     int32_t *grow = tmp + 2 * b0;
     int64_t m = 0;
     const int2 lh = act ? ev[e] : make_int2(-1, -1);
+    // the two faces of a cell that hold the edge (lo, hi), from its row; false:
+    // ET disagrees, no face of this cell
+    auto faces = [](const int4 q, const int4 fr, int32_t lo, int32_t hi, int32_t (&x)[2]) {
+        uint32_t apart = 0;  // corners that the edge does not have
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int32_t u = corner(q, j);
+            apart |= (uint32_t)(u != lo && u != hi) << j;
+        }
+        if (__popc(apart) != 2) return false;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            // face slot 3 - j leaves out corner j
+            const int s = 3 - (h ? 31 - __clz(apart) : __ffs(apart) - 1);
+            x[h] = s == 0 ? fr.x : s == 1 ? fr.y : s == 2 ? fr.z : fr.w;
+        }
+        return true;
+    };
+    // the longest rows: sorted by the block in the columns' LDS
+    const bool by_block = b1 - b0 > 64 && 2 * (b1 - b0) <= EF_CAP * EF_THREADS;
+    if (!__syncthreads_and(!by_block)) {
+        if (tid == 0) nlong = 0;
+        __syncthreads();
+        if (by_block) lng[atomicAdd(&nlong, 1)] = tid;
+        __syncthreads();
+        int32_t *key = &col[0][0];
+        for (int r = 0; r < nlong; r++) {
+            if (tid == lng[r]) {
+                one.first = b0;
+                one.n = (int32_t)(b1 - b0);
+                one.lo = lh.x;
+                one.hi = lh.y;
+            }
+            __syncthreads();
+            int32_t size = 256;
+            while (size < 2 * one.n) size *= 2;
+            for (int32_t i = tid; i < size / 2; i += EF_THREADS) {
+                int32_t x[2] = {INF, INF};
+                if (i < one.n) {
+                    const int64_t t = et[one.first + i];
+                    if (!faces(rows[2 * t], rows[2 * t + 1], one.lo, one.hi, x)) x[0] = x[1] = INF;
+                }
+                key[2 * i] = x[0];
+                key[2 * i + 1] = x[1];
+            }
+            __syncthreads();
+            sort_by_block<EF_THREADS>(key, size);
+            int32_t kept = 0;  // each face once
+            for (int32_t i0 = 0; i0 < size; i0 += EF_THREADS) {
+                const int32_t i = i0 + tid, x = key[i];
+                const bool keep = x != INF && (i == 0 || key[i - 1] != x);
+                const uint64_t mask = __ballot(keep);
+                if (lane == 0) wtot[wid] = (int32_t)__popcll(mask);
+                __syncthreads();
+                int32_t place = kept + (int32_t)__popcll(mask & ((1ull << lane) - 1ull));
+#pragma unroll
+                for (int w = 0; w < EF_THREADS / 64; w++) {
+                    if (w < wid) place += wtot[w];
+                    kept += wtot[w];
+                }
+                if (keep) tmp[2 * one.first + place] = x;
+                __syncthreads();
+            }
+            if (tid == lng[r]) m = kept;
+        }
+    }
     // four cells at a time, their rows loaded together (unconditional loads
     // from a clamped cell index)
-    for (int64_t i0 = b0; i0 < b1; i0 += 4) {
+    for (int64_t i0 = b0; i0 < (by_wave || by_block ? b0 : b1); i0 += 4) {
         int32_t tc[4];
         int4 q[4], fr[4];
 #pragma unroll
@@ -1146,18 +1220,11 @@ __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ e
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             if (i0 + c >= b1) break;
-            uint32_t apart = 0;  // corners that the edge does not have
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int32_t u = corner(q[c], j);
-                apart |= (uint32_t)(u != lh.x && u != lh.y) << j;
-            }
-            if (__popc(apart) != 2) continue;  // ET disagrees: no face of this cell
+            int32_t two[2];
+            if (!faces(q[c], fr[c], lh.x, lh.y, two)) continue;
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                // face slot 3 - j leaves out corner j
-                const int s = 3 - (h ? 31 - __clz(apart) : __ffs(apart) - 1);
-                const int32_t x = s == 0 ? fr[c].x : s == 1 ? fr[c].y : s == 2 ? fr[c].z : fr[c].w;
+                const int32_t x = two[h];
                 if (lds) {  // insert into the ascending column unless present
                     int p = (int)m;
                     while (p > 0 && col[p - 1][tid] > x) p--;
@@ -1170,6 +1237,41 @@ __global__ __launch_bounds__(EF_THREADS) void k_ef(const int64_t *__restrict__ e
                 }
             }
         }
+    }
+    // rows beyond the column, of up to 64 cells: a lane per cell, the faces
+    // without the repeated ones placed by comparing all pairs
+    for (uint64_t b = __ballot(by_wave); b; b &= b - 1) {
+        const int l = __ffsll((unsigned long long)b) - 1;
+        const int64_t first = __shfl(b0, l, 64);
+        const int32_t n = tgd::lane_value((int32_t)(b1 - b0), l);
+        const int32_t lo = tgd::lane_value(lh.x, l), hi = tgd::lane_value(lh.y, l);
+        int32_t x[2] = {INF, INF};
+        if (lane < n) {
+            const int64_t t = et[first + lane];
+            if (!faces(rows[2 * t], rows[2 * t + 1], lo, hi, x)) x[0] = x[1] = INF;
+        }
+        bool again[2] = {false, false};  // an earlier cell has the face
+        for (int j = 0; j < n; j++) {
+            const int32_t y0 = tgd::lane_value(x[0], j), y1 = tgd::lane_value(x[1], j);
+#pragma unroll
+            for (int h = 0; h < 2; h++) again[h] |= j < lane && (x[h] == y0 || x[h] == y1);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (again[h]) x[h] = INF;
+        int32_t place[2] = {0, 0};
+        for (int j = 0; j < n; j++) {
+            const int32_t y0 = tgd::lane_value(x[0], j), y1 = tgd::lane_value(x[1], j);
+#pragma unroll
+            for (int h = 0; h < 2; h++) place[h] += (y0 < x[h]) + (y1 < x[h]);
+        }
+        int32_t kept = 0;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (x[h] != INF) tmp[2 * first + place[h]] = x[h];
+            kept += (int32_t)__popcll(__ballot(x[h] != INF));
+        }
+        if (lane == l) m = kept;
     }
     const int32_t inc = tgd::wave_inclusive_sum((int32_t)m);
     if (lane == 63) wtot[wid] = inc;
