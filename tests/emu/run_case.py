@@ -247,11 +247,12 @@ def case_capacity(hub_first: int = 0, variant: int = 2) -> None:
         refused(d, "TE")
 
 
-def case_hub_rows(shared: int = 50, apart: int = 0, between: int = 0, order: int = 0) -> None:
+def case_hub_rows(shared: int = 50, apart: int = 0, between: int = 0, order: int = 0,
+                  variant: int = 0) -> None:
     """Every relation around two hubs (test_gpu_long_rows.hub_mesh)."""
     from test_gpu_long_rows import check_hubs
 
-    check_hubs(t, shared, apart, between, order)
+    check_hubs(t, shared, apart, between, order, variant)
 
 
 def case_vertex_rows(n: int = 140, hub_first: int = 1) -> None:

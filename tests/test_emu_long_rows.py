@@ -15,7 +15,7 @@ CASES = [
     # lowest id, in the bucketed and the vertex-lane form
     ("capacity", 0, 2), ("capacity", 1, 2), ("capacity", 0, 1), ("capacity", 1, 1),
     # rows beyond the join networks, alone in a wave and beside short ones
-    ("hub_rows", 50, 0, 0, 0), ("hub_rows", 20, 33, 10, 1),
+    ("hub_rows", 50, 0, 0, 0), ("hub_rows", 20, 33, 10, 1), ("hub_rows", 30, 20, 0, 1, 1),
     # a vertex's faces by the wave, an edge's by the wave and by the block
     ("hub_rows", 1, 100, 0, 1), ("hub_rows", 70, 1, 0, 1),
     # a vertex's edges ordered by the whole block

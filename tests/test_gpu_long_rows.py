@@ -25,7 +25,7 @@ def hub_mesh(n, apart, between):
     return np.array(cells, np.int32)[order], v
 
 
-def check_hubs(t, shared, apart, between, order):
+def check_hubs(t, shared, apart, between, order, variant=0):
     """order 0: as hub_mesh gives it; else random cells and ids by that seed."""
     from test_gpu_relations import check_all
 
@@ -34,7 +34,13 @@ def check_hubs(t, shared, apart, between, order):
         rng = np.random.default_rng(order)
         ids = rng.permutation(V).astype(np.int32)
         cells = np.ascontiguousarray(np.sort(ids[cells], axis=1)[rng.permutation(len(cells))])
-    check_all(t, cells, V, expect_ft=False)
+    check_all(t, cells, V, variant, expect_ft=False)
+
+
+def test_hub_rows_vertex_lane(gpu):
+    """VV from the form that does not count the vertices of many cells."""
+    check_hubs(gpu, 46, 30, 200, 1, variant=1)
+    check_hubs(gpu, 5, 20, 200, 1, variant=1)
 
 
 @pytest.mark.parametrize("order", [0, 1])

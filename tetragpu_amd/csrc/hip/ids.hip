@@ -1806,7 +1806,13 @@ int ensure_et(tg_mesh &m) {
         return rc;
     int64_t *off = m.et_off.as<int64_t>();
     static_assert(JOIN_ROW >= LANE_CELLS, "few_cells: no row beyond the networks");
-    const bool listed = !m.few_cells;  // tmp_a: the edges with long rows, and their lengths by edge
+    bool listed = !m.few_cells;  // tmp_a: the edges with long rows, and their lengths by edge
+    if (listed && !m.heavy_counted && E > 0) {  // VV came from a form that does not tell
+        int64_t squares;
+        int32_t longest;
+        if ((rc = row_squares(m, m.vt_off.as<int32_t>(), m.n_points, c, squares, longest))) return rc;
+        listed = longest > JOIN_ROW;
+    }
     if (listed && (rc = m.tmp_a.ensure(sizeof(int32_t) * 2 * (size_t)std::max<int64_t>(E, 1)))) return rc;
     const EdgeRows rows_of{m.ev.as<int32_t>(), m.n_points, m.vt_off.as<int32_t>()};
     const int32_t *vtc = m.vtc.as<int32_t>();
