@@ -272,7 +272,15 @@ def case_vertex_rows(n: int = 140, hub_first: int = 1) -> None:
         same_csr(d.relation("EE"), ref["EE"], "EE")
 
 
-CASES = {"hub_rows": case_hub_rows, "vertex_rows": case_vertex_rows, "capacity": case_capacity, "split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
+def case_heavy(which: int = 0) -> None:
+    """VV and classes of vertices that the row kernel leaves to the heavy one."""
+    from test_gpu_long_rows import HEAVY, check_heavy
+
+    sizes, ring = HEAVY[which]
+    check_heavy(t, sizes, ring, np.float32)
+
+
+CASES = {"heavy": case_heavy, "hub_rows": case_hub_rows, "vertex_rows": case_vertex_rows, "capacity": case_capacity, "split": case_split, "noalloc": case_noalloc, "after_hot_path": case_after_hot_path, "all_relations": case_all_relations,
          "vv_cp": case_vv_cp, "window": case_window, "hubs": case_hubs, "soup": case_soup, "routes": case_routes}
 
 

@@ -18,6 +18,8 @@ CASES = [
     ("hub_rows", 50, 0, 0, 0), ("hub_rows", 20, 33, 10, 1), ("hub_rows", 30, 20, 0, 1, 1),
     # a vertex's faces by the wave, an edge's by the wave and by the block
     ("hub_rows", 1, 100, 0, 1), ("hub_rows", 70, 1, 0, 1),
+    # VV and classes of vertices with many cells
+    ("heavy", 0), ("heavy", 1), ("heavy", 2),
     # a vertex's edges ordered by the whole block
     ("vertex_rows", 127, 1), ("vertex_rows", 140, 0),
 ]

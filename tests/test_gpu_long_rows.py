@@ -83,3 +83,43 @@ def test_long_rows_cost_their_entries(gpu, first, then, n):
     short = seconds(gpu, m.cells, m.n_points, first, then)
     print(f"{then}: long rows {1e6 * long:.0f} us, short rows {1e6 * short:.0f} us", flush=True)
     assert long < 20 * short
+
+
+HEAVY = [([46, 47, 48, 49, 50, 59, 60, 61], 20),   # cells around the row kernel's limit
+         ([29, 30, 31, 48, 61, 62, 63, 64], 80),   # 31 to 33 and 63 to 66 neighbours
+         ([126, 127, 128, 129, 130, 300], 30)]     # records that one wave takes, and more
+
+
+def check_heavy(t, sizes, ring, dtype, seed=3):
+    from test_gpu_networks import check_vv_cp, fans
+
+    cells, V = fans(sizes, ring)
+    rng = np.random.default_rng(seed)
+    check_vv_cp(t, cells, V, rng.random(V).astype(dtype), 7)
+    check_vv_cp(t, cells, V, rng.integers(0, 3, V).astype(dtype), 8)  # ties
+
+
+@pytest.mark.parametrize("sizes,ring", HEAVY)
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_vertices_of_many_cells(gpu, sizes, ring, dtype):
+    """VV and classes of the vertices that the row kernel leaves to the heavy one."""
+    check_heavy(gpu, sizes, ring, dtype)
+
+
+def test_many_vertices_of_many_cells_cost(gpu):
+    """With every second cell of a grid split, a tenth of the vertices have 49 to
+    60 cells and 27 to 32 neighbours: 2.5 times the cells, 3.6 times the time
+    (41 times with a workgroup for each of them)."""
+    def run(m):
+        with gpu.Mesh(m.cells, m.n_points, m.scalars) as d:
+            best = float("inf")
+            for _ in range(6):
+                t0 = time.perf_counter()
+                d.vv_critpoints()
+                d.shape("VV")
+                best = min(best, time.perf_counter() - t0)
+        return best
+
+    plain, split = run(gpu.kuhn(48, seed=3)), run(gpu.kuhn(48, seed=3, split_fraction=0.5))
+    print(f"split {1e6 * split:.0f} us, plain {1e6 * plain:.0f} us", flush=True)
+    assert split < 10 * plain

@@ -1435,13 +1435,13 @@ __global__ __launch_bounds__(2 << BV_LOG) void k_bkt_own(
     }
 }
 
-// Vertices with more than 32 neighbours (or whose bucket table overflowed):
-// one workgroup per vertex scans its bucket's corner records.  Neighbours go
-// to an LDS open-addressing set of 2 * HEAVY_CAP slots (CAS inserts), the
+// Vertices with more than 32 neighbours or 48 records (or whose bucket table
+// overflowed): a wave each up to 64 neighbours and 128 records, else a
+// workgroup scans the bucket's corner records.  Neighbours go to an LDS open-addressing set of 2 * HEAVY_CAP slots (CAS inserts), the
 // shared-tet link edges between same-class slots to a lock-free union-find
 // (a root is only ever linked under a smaller root, by CAS), and the row is
 // sorted by a bitonic network in LDS.
-constexpr int HV_THREADS = 256;
+constexpr int HV_THREADS = 1024;  // the LDS leaves one block per CU
 constexpr int HV_SLOTS = 2 * HEAVY_CAP;
 constexpr int HV_BITS = 13;  // log2(HV_SLOTS)
 static_assert((1 << HV_BITS) == HV_SLOTS, "heavy set size");
@@ -1516,103 +1516,293 @@ __device__ __forceinline__ void block_bitonic(int32_t *list, int P) {
         }
 }
 
+// A heavy vertex of up to 128 records and 64 neighbours, by one wave: an
+// interior vertex of 27 to 64 neighbours has 50 to 124 cells.  Bound by the scan
+// of the bucket's records and the chains after it.  A workgroup each spent 40
+// us on the full set's slots: a Kuhn mesh with every second cell split 1 -> 4,
+// 1.7 M cells, 44 k vertices of 49 to 60 cells, took 7.0 ms where it takes 0.61.
+// (A network for 60 records beside the others in k_bkt_sort: 0.58, but its
+// registers cost 12.6 M cells without such vertices 1.47 -> 1.64.)
+constexpr int HW_REC = 128, HW_NB = 64, HW_SLOTS = 128;
+struct HeavyWave {
+    int32_t rec[HW_REC];    // places of the records
+    int32_t set[HW_SLOTS];  // neighbours by hash, then the places of their keys in the row
+    int32_t key[HW_NB], slot[HW_NB], row[HW_NB];
+    uint32_t adj[2 * HW_NB];
+    int32_t bad;
+};
+
+// Components of `mask` under the lanes' adjacency rows, numbered in order of
+// their lowest lanes; own: that of the lane.
+__device__ __forceinline__ uint32_t wave_components(uint64_t adj, uint64_t mask, uint32_t &own) {
+    const int lane = __lane_id();
+    uint32_t n = 0;
+    for (uint64_t rem = mask; rem; n++) {
+        uint64_t comp = rem & (0ull - rem);
+        while (true) {
+            const uint64_t more = (__ballot((adj & comp) != 0 && ((mask >> lane) & 1u)) | comp);
+            if (more == comp) break;
+            comp = more;
+        }
+        if ((comp >> lane) & 1u) own = n;
+        rem &= ~comp;
+    }
+    return n;
+}
+
+// What a wave made of a heavy vertex: more records or neighbours than that
+// (nothing has been written); its row and, but for the link pass without or
+// with row descriptors, its classes.
+enum HeavyEnd { HEAVY_LEFT, HEAVY_DONE, HEAVY_FIX, HEAVY_FIXD };
+template <typename S>
+__device__ __forceinline__ HeavyEnd heavy_by_wave(const Rec &rec, int32_t cbeg, int32_t cend,
+                                                  int32_t v, const S *__restrict__ scal, int classify,
+                                                  HeavyWave &st, int32_t *__restrict__ dst,
+                                                  uint8_t *__restrict__ ddst,
+                                                  int32_t *__restrict__ deg,
+                                                  uint32_t *__restrict__ classes) {
+    const int lane = __lane_id();
+    const uint64_t below = (1ull << lane) - 1ull;
+    int c = 0;  // the bucket's records of v
+    constexpr int U = 8;
+    for (int32_t i0 = cbeg; i0 < cend && c <= HW_REC; i0 += 64 * U) {
+        uint32_t w[U];
+#pragma unroll
+        for (int k = 0; k < U; k++) w[k] = rec.w0[min(i0 + 64 * k + lane, cend - 1)];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const int32_t i = i0 + 64 * k + lane;
+            const bool mine = i < cend && (int32_t)(w[k] & M24) == v;
+            const uint64_t m = __ballot(mine);
+            const int at = c + (int)__popcll(m & below);
+            if (mine && at < HW_REC) st.rec[at] = i;
+            c += (int)__popcll(m);
+        }
+    }
+    if (c > HW_REC) return HEAVY_LEFT;
+    for (int s = lane; s < HW_SLOTS; s += 64) {
+        st.set[s] = -1;
+        st.adj[s] = 0u;
+    }
+    if (lane == 0) st.bad = 0;
+    tgd::wave_sync();
+    int sl[2][3];  // the slots of the lane's records' neighbours
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int r = lane + 64 * k;
+        if (r >= c) continue;
+        const int32_t i = st.rec[r];
+        uint32_t rv, u[3];
+        rec_unpack(rec.w0[i], rec.w1[i], rec.w2[i], rv, u[0], u[1], u[2]);
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            uint32_t s = (u[q] * 2654435769u) >> 25;
+            sl[k][q] = -1;
+            for (int probe = 0; probe < HW_SLOTS; probe++, s = (s + 1) & (HW_SLOTS - 1)) {
+                const int32_t old = atomicCAS(&st.set[s], -1, (int32_t)u[q]);
+                if (old != -1 && old != (int32_t)u[q]) continue;
+                sl[k][q] = (int)s;
+                break;
+            }
+            if (sl[k][q] < 0) st.bad = 1;  // full: more than HW_NB
+        }
+    }
+    tgd::wave_sync();
+    int m = 0;
+    bool over = st.bad != 0;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int32_t u = st.set[lane + 64 * k];
+        const uint64_t there = __ballot(u >= 0);
+        const int at = m + (int)__popcll(there & below);
+        if (u >= 0 && at < HW_NB) {
+            st.key[at] = u;
+            st.slot[at] = lane + 64 * k;
+        }
+        m += (int)__popcll(there);
+    }
+    over = over || m > HW_NB;
+    if (__any(over)) return HEAVY_LEFT;
+    tgd::wave_sync();
+    const bool on = lane < m;
+    const int32_t mine = on ? st.key[lane] : INT32_MAX;
+    int place = 0;
+    for (int j = 0; j < m; j++) place += tgd::lane_value(mine, j) < mine;
+    if (on) {
+        st.row[place] = mine;
+        st.set[st.slot[lane]] = place;
+    }
+    tgd::wave_sync();
+    const int32_t u = on ? st.row[lane] : v;
+    if (on) dst[lane] = u;
+    if (lane == 0) deg[v] = m;
+    HeavyEnd end = HEAVY_DONE;
+    if (classify) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            if (lane + 64 * k >= c) continue;
+            const int a = st.set[sl[k][0]], b = st.set[sl[k][1]], d = st.set[sl[k][2]];
+            const uint64_t bits = 1ull << a | 1ull << b | 1ull << d;
+            const uint32_t lo = (uint32_t)bits, hi = (uint32_t)(bits >> 32);
+            for (int q = 0; q < 3; q++) {
+                const int x = q == 0 ? a : q == 1 ? b : d;
+                if (lo) atomicOr(&st.adj[2 * x], lo);
+                if (hi) atomicOr(&st.adj[2 * x + 1], hi);
+            }
+        }
+        tgd::wave_sync();
+        const uint64_t adj = on ? (uint64_t)st.adj[2 * lane + 1] << 32 | st.adj[2 * lane] : 0ull;
+        const S sv = scal[v];
+        const uint64_t all = __ballot(on), low = __ballot(on && is_lower(scal[u], sv, u, v));
+        uint32_t own = 0;
+        const uint32_t nl = wave_components(adj, low, own), nu = wave_components(adj, all & ~low, own);
+        if (lane == 0) {
+            classes[3 * (int64_t)v] = nl;
+            classes[3 * (int64_t)v + 1] = nu;
+            classes[3 * (int64_t)v + 2] = verdict(nl, nu);
+        }
+        if (nl >= 2 || nu >= 2) end = m <= SLOTS ? HEAVY_FIXD : HEAVY_FIX;
+        if (end == HEAVY_FIXD && on) ddst[lane] = (uint8_t)(((low >> lane) & 1u) << 5 | own);
+    }
+    tgd::wave_sync();  // the staging is reused
+    return end;
+}
+
 template <int BV_LOG, typename S>
 __global__ __launch_bounds__(HV_THREADS) void k_bkt_heavy(
     const Rec rec, const int32_t *__restrict__ h2s, int32_t nslice,
     const S *__restrict__ scal, int classify, int32_t *__restrict__ scratch,
     int32_t *__restrict__ deg, const int32_t *__restrict__ rowsrc,
     uint32_t *__restrict__ classes, const int32_t *__restrict__ heavy,
-    int32_t *__restrict__ fix, int32_t *__restrict__ fixbig, int32_t *__restrict__ counters) {
-    __shared__ int32_t set[HV_SLOTS];
-    __shared__ int32_t par[HV_SLOTS];
+    int32_t *__restrict__ fix, int32_t *__restrict__ fixbig, int32_t *__restrict__ fixd,
+    uint8_t *__restrict__ rowdesc, int32_t *__restrict__ counters) {
+    __shared__ int32_t set_par[2 * HV_SLOTS];
+    int32_t *set = set_par, *par = set_par + HV_SLOTS;
     __shared__ uint8_t lowf[HV_SLOTS];
     __shared__ int32_t list[HEAVY_CAP];
     __shared__ int32_t misc[5];  // distinct neighbours, full flag, lower roots, upper roots, fill
-    const int tid = threadIdx.x;
+    constexpr int NW = HV_THREADS / 64;
+    __shared__ int32_t taken[NW], end[NW];  // the waves' vertices and what became of them
+    static_assert(sizeof(HeavyWave) * NW <= sizeof set_par, "the waves' staging is in the set and the parents");
+    const int tid = threadIdx.x, wid = tid / 64;
     const int32_t n = counters[C_HEAVY];
-    for (int32_t h = blockIdx.x; h < n; h += gridDim.x) {
-        const int32_t v = heavy[h];
-        const int32_t bkt = v >> BV_LOG;
-        const int32_t cbeg = h2s[(int64_t)bkt * nslice], cend = h2s[(int64_t)(bkt + 1) * nslice];
-        const S sv = classify ? scal[v] : S(0);
-        for (int i = tid; i < HV_SLOTS; i += HV_THREADS) {
-            set[i] = -1;
-            par[i] = i;
-        }
-        if (tid < 5) misc[tid] = 0;
-        __syncthreads();
-        // neighbour set
-        for (int32_t i = cbeg + tid; i < cend; i += HV_THREADS) {
-            uint32_t rv, x, y, z;
-            rec_unpack(rec.w0[i], rec.w1[i], rec.w2[i], rv, x, y, z);
-            if ((int32_t)rv != v) continue;
-            if ((hv_insert(set, (int32_t)x, &misc[0]) | hv_insert(set, (int32_t)y, &misc[0]) |
-                 hv_insert(set, (int32_t)z, &misc[0])) < 0)
-                misc[1] = 1;
-        }
-        __syncthreads();
-        const int m = misc[0];
-        if (misc[1] || m > HEAVY_CAP) {  // block-uniform
-            if (tid == 0) {
-                atomicOr(counters + C_ERR, tg::ERRBIT_CAPACITY);
-                deg[v] = 0;
-                if (classify) {
-                    classes[3 * (int64_t)v] = 0;
-                    classes[3 * (int64_t)v + 1] = 0;
-                    classes[3 * (int64_t)v + 2] = 0;
-                }
+    // a vertex per wave, then the block on those that were too much for one
+    for (int32_t h0 = blockIdx.x; h0 < n; h0 += NW * gridDim.x) {
+        {
+            const int32_t h = h0 + wid * (int32_t)gridDim.x, v = h < n ? heavy[h] : -1;
+            HeavyEnd e = HEAVY_DONE;
+            if (h < n) {
+                const int32_t bkt = v >> BV_LOG, rs = rowsrc[v];
+                e = heavy_by_wave(rec, h2s[(int64_t)bkt * nslice], h2s[(int64_t)(bkt + 1) * nslice], v,
+                                  scal, classify, reinterpret_cast<HeavyWave *>(set_par)[wid],
+                                  scratch + rs, rowdesc + rs, deg, classes);
             }
-            __syncthreads();
-            continue;
+            if (__lane_id() == 0) {
+                taken[wid] = v;
+                end[wid] = e;
+            }
         }
-        if (classify) {
+        __syncthreads();
+        if (wid == 0) {  // one list atomic per round, not one per vertex
+            const int lane = __lane_id(), e = lane < NW ? end[lane] : HEAVY_DONE;
+            const uint64_t fm = __ballot(e == HEAVY_FIX), dm = __ballot(e == HEAVY_FIXD);
+            const uint64_t below = (1ull << lane) - 1ull;
+            int32_t fb = 0, db = 0;
+            if (lane == 0) {
+                fb = fm ? atomicAdd(counters + C_FIX, (int32_t)__popcll(fm)) : 0;
+                db = dm ? atomicAdd(counters + tg::C_FIXD, (int32_t)__popcll(dm)) : 0;
+            }
+            fb = tgd::lane_value(fb, 0) + (int32_t)__popcll(fm & below);
+            db = tgd::lane_value(db, 0) + (int32_t)__popcll(dm & below);
+            if (e == HEAVY_FIX) fix[fb] = taken[lane];
+            if (e == HEAVY_FIXD) fixd[db] = taken[lane];
+        }
+        for (int w = 0; w < NW; w++) {
+            if (end[w] != HEAVY_LEFT) continue;
+            const int32_t v = taken[w];
+            const int32_t bkt = v >> BV_LOG;
+            const int32_t cbeg = h2s[(int64_t)bkt * nslice], cend = h2s[(int64_t)(bkt + 1) * nslice];
+            const S sv = classify ? scal[v] : S(0);
             for (int i = tid; i < HV_SLOTS; i += HV_THREADS) {
-                const int32_t u = set[i];
-                lowf[i] = u >= 0 ? (uint8_t)is_lower(scal[u], sv, u, v) : (uint8_t)0;
+                set[i] = -1;
+                par[i] = i;
             }
+            if (tid < 5) misc[tid] = 0;
             __syncthreads();
-            // shared-tet link edges between neighbours of one class
+            // neighbour set
             for (int32_t i = cbeg + tid; i < cend; i += HV_THREADS) {
                 uint32_t rv, x, y, z;
                 rec_unpack(rec.w0[i], rec.w1[i], rec.w2[i], rv, x, y, z);
                 if ((int32_t)rv != v) continue;
-                const int a = hv_find(set, (int32_t)x), b = hv_find(set, (int32_t)y),
-                          c = hv_find(set, (int32_t)z);
-                if ((a | b | c) < 0) continue;  // not reached: every key was inserted above
-                if (lowf[a] == lowf[b]) uf_unite(par, a, b);
-                if (lowf[a] == lowf[c]) uf_unite(par, a, c);
-                if (lowf[b] == lowf[c]) uf_unite(par, b, c);
+                if ((hv_insert(set, (int32_t)x, &misc[0]) | hv_insert(set, (int32_t)y, &misc[0]) |
+                     hv_insert(set, (int32_t)z, &misc[0])) < 0)
+                    misc[1] = 1;
             }
             __syncthreads();
-        }
-        // row (compacted) and component roots per class
-        for (int i = tid; i < HV_SLOTS; i += HV_THREADS) {
-            const int32_t u = set[i];
-            if (u < 0) continue;
-            list[atomicAdd(&misc[4], 1)] = u;
-            if (classify && par[i] == i) atomicAdd(&misc[lowf[i] ? 2 : 3], 1);
-        }
-        int P = 1;
-        while (P < m) P <<= 1;
-        for (int i = m + tid; i < P; i += HV_THREADS) list[i] = INT32_MAX;
-        __syncthreads();
-        block_bitonic(list, P);
-        int32_t *dst = scratch + rowsrc[v];
-        for (int i = tid; i < m; i += HV_THREADS) dst[i] = list[i];
-        if (tid == 0) {
-            const uint32_t nl = (uint32_t)misc[2], nu = (uint32_t)misc[3];
-            deg[v] = m;
+            const int m = misc[0];
+            if (misc[1] || m > HEAVY_CAP) {  // block-uniform
+                if (tid == 0) {
+                    atomicOr(counters + C_ERR, tg::ERRBIT_CAPACITY);
+                    deg[v] = 0;
+                    if (classify) {
+                        classes[3 * (int64_t)v] = 0;
+                        classes[3 * (int64_t)v + 1] = 0;
+                        classes[3 * (int64_t)v + 2] = 0;
+                    }
+                }
+                __syncthreads();
+                continue;
+            }
             if (classify) {
-                classes[3 * (int64_t)v] = nl;
-                classes[3 * (int64_t)v + 1] = nu;
-                classes[3 * (int64_t)v + 2] = verdict(nl, nu);
-                if (nl >= 2 || nu >= 2) {
-                    if (m <= 64) fix[atomicAdd(counters + C_FIX, 1)] = v;
-                    else fixbig[atomicAdd(counters + C_FIXBIG, 1)] = v;
+                for (int i = tid; i < HV_SLOTS; i += HV_THREADS) {
+                    const int32_t u = set[i];
+                    lowf[i] = u >= 0 ? (uint8_t)is_lower(scal[u], sv, u, v) : (uint8_t)0;
+                }
+                __syncthreads();
+                // shared-tet link edges between neighbours of one class
+                for (int32_t i = cbeg + tid; i < cend; i += HV_THREADS) {
+                    uint32_t rv, x, y, z;
+                    rec_unpack(rec.w0[i], rec.w1[i], rec.w2[i], rv, x, y, z);
+                    if ((int32_t)rv != v) continue;
+                    const int a = hv_find(set, (int32_t)x), b = hv_find(set, (int32_t)y),
+                              c = hv_find(set, (int32_t)z);
+                    if ((a | b | c) < 0) continue;  // not reached: every key was inserted above
+                    if (lowf[a] == lowf[b]) uf_unite(par, a, b);
+                    if (lowf[a] == lowf[c]) uf_unite(par, a, c);
+                    if (lowf[b] == lowf[c]) uf_unite(par, b, c);
+                }
+                __syncthreads();
+            }
+            // row (compacted) and component roots per class
+            for (int i = tid; i < HV_SLOTS; i += HV_THREADS) {
+                const int32_t u = set[i];
+                if (u < 0) continue;
+                list[atomicAdd(&misc[4], 1)] = u;
+                if (classify && par[i] == i) atomicAdd(&misc[lowf[i] ? 2 : 3], 1);
+            }
+            int P = 1;
+            while (P < m) P <<= 1;
+            for (int i = m + tid; i < P; i += HV_THREADS) list[i] = INT32_MAX;
+            __syncthreads();
+            block_bitonic(list, P);
+            int32_t *dst = scratch + rowsrc[v];
+            for (int i = tid; i < m; i += HV_THREADS) dst[i] = list[i];
+            if (tid == 0) {
+                const uint32_t nl = (uint32_t)misc[2], nu = (uint32_t)misc[3];
+                deg[v] = m;
+                if (classify) {
+                    classes[3 * (int64_t)v] = nl;
+                    classes[3 * (int64_t)v + 1] = nu;
+                    classes[3 * (int64_t)v + 2] = verdict(nl, nu);
+                    if (nl >= 2 || nu >= 2) {
+                        if (m <= 64) fix[atomicAdd(counters + C_FIX, 1)] = v;
+                        else fixbig[atomicAdd(counters + C_FIXBIG, 1)] = v;
+                    }
                 }
             }
+            __syncthreads();  // the set, list and counters are reused by the next vertex
         }
-        __syncthreads();  // the set, list and counters are reused by the next vertex
+        __syncthreads();
     }
 }
 
@@ -1902,11 +2092,11 @@ int launch_bucketed_typed(tg::BucketBuffers &k, bool classify, hipStream_t s) {
     if (p.bv_log == 7)
         hipLaunchKernelGGL((k_bkt_heavy<7, S>), dim3(256), dim3(HV_THREADS), 0, s, r2, ranges, nsl,
                            scal, cls, b.scratch, b.deg, k.rowsrc, b.classes, b.heavy, b.fix,
-                           b.fixbig, b.counters);
+                           b.fixbig, b.fixd, b.rowdesc, b.counters);
     else
         hipLaunchKernelGGL((k_bkt_heavy<8, S>), dim3(256), dim3(HV_THREADS), 0, s, r2, ranges, nsl,
                            scal, cls, b.scratch, b.deg, k.rowsrc, b.classes, b.heavy, b.fix,
-                           b.fixbig, b.counters);
+                           b.fixbig, b.fixd, b.rowdesc, b.counters);
     TG_LAUNCH_CHECK("k_bkt_heavy");
     if (mk) mk->mark("bkt_heavy", s);
     return tg::OK;
