@@ -52,11 +52,6 @@ inline unsigned grid_for(int64_t n, int block) {
 size_t scan_tmp_bytes(int64_t n);
 int scan_exclusive_i32(const int32_t *in, int32_t *out, int64_t n, void *tmp,
                        hipStream_t s);
-int scan_exclusive_i64(const int64_t *in, int64_t *out, int64_t n, void *tmp,
-                       hipStream_t s);
-// Widening scan: 32-bit counts into 64-bit offsets.
-int scan_exclusive_i32_to_i64(const int32_t *in, int64_t *out, int64_t n,
-                              void *tmp, hipStream_t s);
 
 // Stream-ordered caching allocator (pool.hip): a freed block is reused only
 // after `stream` has passed the free.  pool_alloc returns nullptr on failure

@@ -714,7 +714,9 @@ struct JoinBlock {
 
 // One wave's share of a tile with a network for rows of up to R entries.
 // Contains two workgroup barriers; every wave of the block makes one call
-// (of some R), so all waves meet at both.
+// (of some R), so all waves meet at both.  (The waves may be at calls in
+// different branches: gfx950's barrier counts arrivals, whatever instruction
+// they come from.)
 template <int NR, Join J, int SH, LongRows L, int R, int THREADS, int WIN>
 __device__ __forceinline__ void join_wave(JoinBlock<THREADS, WIN> &blk,
                                           const int32_t *__restrict__ src, const Rows<NR> &r,
@@ -1635,12 +1637,6 @@ __global__ __launch_bounds__(FF_THREADS) void k_ff(const int32_t *__restrict__ f
     for (int32_t i = tid; i < total; i += FF_THREADS) out[base + i] = rows[i];
 }
 
-__global__ void k_widen(const int32_t *__restrict__ in, int64_t n, int64_t *__restrict__ out) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = in[i];
-}
-
 unsigned grid(int64_t n, int block = 256) {
     return std::min<unsigned>(tg::grid_for(n, block), 65536u);
 }
@@ -1952,6 +1948,7 @@ int ensure_ef(tg_mesh &m) {
                            m.ev.as<const int2>(), m.tmp_a.as<const int4>(), c.ticket, c.state, off,
                            m.ef_vals.as<int32_t>(), m.tmp_c.as<int32_t>());
         TG_LAUNCH_CHECK("k_ef");
+        m.tmp_a.release();  // 32 bytes a cell, which nothing else needs
     } else if ((rc = fill_i32((int32_t *)off, 0, 2, m.stream))) {
         return rc;
     }

@@ -12,17 +12,16 @@ namespace tg {
 
 // Device counters shared by one pipeline run.
 enum Counter : int {
-    C_HEAVY = 0,   // vertices routed to the serial VV kernel
+    C_HEAVY = 0,   // vertices left to the heavy kernel
     C_FIX = 1,     // vertices needing the row-membership link pass (deg<=64)
     C_FIXBIG = 2,  // same, deg > 64
     C_ERR = 3,     // error bits (ERRBIT_*)
-    C_MAXDEG = 4,  // largest VV degree seen
-    C_FIXD = 5,    // bucketed vertices needing the link pass (row descriptors)
-    C_FTERR = 6,   // a face held by more than two cells
-    C_IDERR = 7,   // face ids: a relation read back inconsistent
-    C_WIDE = 8,    // one-level routing: tiles whose corners span too many buckets
-    C_SCRATCH = 9, // one-off reductions of the host API
-    N_COUNTERS = 10
+    C_FIXD = 4,    // bucketed vertices needing the link pass (row descriptors)
+    C_FTERR = 5,   // a face held by more than two cells
+    C_IDERR = 6,   // face ids: a relation read back inconsistent
+    C_WIDE = 7,    // one-level routing: tiles whose corners span too many buckets
+    C_SCRATCH = 8, // one-off reductions of the host API
+    N_COUNTERS = 9
 };
 enum ErrBit : int { ERRBIT_CAPACITY = 1 };
 

@@ -67,7 +67,7 @@ struct tg_mesh {
     tg::DevArr tt_off, tt_vals, ff_off, ff_vals, ee_off, ee_vals;
     tg::DevArr rank_tmp, edge_rank, face_rank, tmp_a, tmp_b, tmp_c;
     bool edges_built = false, faces_built = false, vt_built = false, et_built = false,
-         fe_built = false, ft_built = false, ef_built = false, tt_built = false,
+         fe_built = false, ef_built = false, tt_built = false,
          ff_built = false, ee_built = false;
     bool ft_ok = true;  // every face is held by at most two cells
     // entry counts of built relations; -1: known to the device only, read when asked for

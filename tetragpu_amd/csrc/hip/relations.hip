@@ -251,7 +251,8 @@ static int vt_bucketed(tg_mesh &m, bool &done) {
     if (rc) return rc;
     if (!m.bplan.ok || 4 * m.n_cells > (int64_t)INT32_MAX) return OK;
     if ((rc = prepare_buckets(m))) return rc;
-    if ((rc = m.bk_rec.ensure(12 * sizeof(int32_t) * (size_t)std::max<int64_t>(m.n_cells, 1))))
+    // four records of two words a cell
+    if ((rc = m.bk_rec.ensure(8 * sizeof(int32_t) * (size_t)std::max<int64_t>(m.n_cells, 1))))
         return rc;
     BucketBuffers k = bucket_buffers(m);
     k.rec2 = m.bk_rec.as<uint32_t>();

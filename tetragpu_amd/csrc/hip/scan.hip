@@ -185,14 +185,6 @@ int scan_exclusive_i32(const int32_t *in, int32_t *out, int64_t n, void *tmp,
                        hipStream_t s) {
     return scan_impl<int32_t, int32_t, int32_t>(in, out, n, tmp, s);
 }
-int scan_exclusive_i64(const int64_t *in, int64_t *out, int64_t n, void *tmp,
-                       hipStream_t s) {
-    return scan_impl<int64_t, int64_t, int64_t>(in, out, n, tmp, s);
-}
-int scan_exclusive_i32_to_i64(const int32_t *in, int64_t *out, int64_t n,
-                              void *tmp, hipStream_t s) {
-    return scan_impl<int32_t, int64_t, int64_t>(in, out, n, tmp, s);
-}
 
 int fill_i32(int32_t *p, int32_t value, int64_t n, hipStream_t s) {
     if (n <= 0) return OK;

@@ -764,9 +764,9 @@ __global__ __launch_bounds__(FB_THREADS) void k_cp_fix_big(
 }
 
 // Both passes in one launch, for the bucketed form, whose lists hold only what
-// the heavy kernel queued (rows over 32 entries by their length, so neither
-// pass adds to the other's list): most meshes have none, and an empty launch
-// costs 4 us.
+// the heavy kernel queued (by the row's length: up to 64 entries in the first,
+// more in the second, so neither pass adds to the other's list): most meshes
+// have none, and an empty launch costs 4 us.
 constexpr int REST_WAVES = 1024, REST_BIG = 256;  // blocks of each
 template <typename S>
 __global__ __launch_bounds__(FB_THREADS) void k_cp_fix_rest(

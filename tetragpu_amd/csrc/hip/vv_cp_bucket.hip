@@ -896,7 +896,9 @@ struct Slab {
 // adjacency column.  Returns their number (over SLOTS: the columns are not
 // usable).  Contains one workgroup barrier, between the reads of the records
 // and the columns that overlay them; every wave of the block makes one call
-// (of some R), so all waves meet at it.
+// (of some R), so all waves meet at it.  (The waves may be at calls in different
+// branches: gfx950's barrier counts arrivals, whatever instruction they come
+// from.)
 //
 // A key is neighbour << 8 | code.  R <= 32: the code is the record's number
 // and the walk collects each record's slots as a 32-bit mask.  R > 32: the
@@ -2069,7 +2071,7 @@ int launch_bucketed_typed(tg::BucketBuffers &k, bool classify, hipStream_t s) {
     if (p.owner) {
         if (p.bv_log == 7) TG_BKT((k_bkt_own<7, S>), 256);
         else TG_BKT((k_bkt_own<8, S>), 512);
-    } else if (p.ins == 1 || V > (int32_t)M24) {  // the sorting form keeps key 2^24 - 1 for padding
+    } else if (p.ins == 1) {
         if (p.bv_log == 7) TG_BKT((k_bkt_vv_cp<7, S>), 256);
         else TG_BKT((k_bkt_vv_cp<8, S>), 512);
     } else {
@@ -2120,6 +2122,7 @@ BucketPlan plan_buckets(int64_t n_cells, int64_t n_points, int bv_log, int64_t t
     p.nb = (int32_t)nb;
     p.fs = std::max(0, ceil_log2(nb) - 8);  // coarse bins <= 256
     p.nc = (int32_t)((nb + (1 << p.fs) - 1) >> p.fs);
+    // ids below 2^24 - 1: the sorting form keeps that key for padding
     p.ok = V > 0 && V <= (int64_t)M24 && (1 << p.fs) <= MAX_FINE && p.nc <= MAX_COARSE;
     p.tpc = std::max<int64_t>(1024, tpc);
     p.nchunks = (int32_t)std::max<int64_t>(1, (T + p.tpc - 1) / p.tpc);
