@@ -4,7 +4,6 @@
 // allocation is its own heap block, freed at once, so AddressSanitizer
 // reports out-of-bounds and use-after-free accesses at the faulting line.
 #include <hip/hip_runtime.h>
-#include <ucontext.h>
 
 #include <sys/mman.h>
 
@@ -18,9 +17,38 @@
 #if defined(__has_feature)
 #if __has_feature(address_sanitizer)
 #define EMU_ASAN 1
+#include <sanitizer/asan_interface.h>
 #include <sanitizer/common_interface_defs.h>
 #endif
 #endif
+
+// Saves the callee-saved registers and the stack, goes on where `to` was saved.
+// (swapcontext takes a system call, and AddressSanitizer's wrapper of it clears
+// the shadow of the whole stack: 1 us a switch, of which a cross-lane operation
+// takes two for each of its lanes.)
+extern "C" void emu_switch(void **from, void *to);
+asm(R"(
+.text
+.globl emu_switch
+.hidden emu_switch
+.type emu_switch, @function
+emu_switch:
+    pushq %rbp
+    pushq %rbx
+    pushq %r12
+    pushq %r13
+    pushq %r14
+    pushq %r15
+    movq %rsp, (%rdi)
+    movq %rsi, %rsp
+    popq %r15
+    popq %r14
+    popq %r13
+    popq %r12
+    popq %rbx
+    popq %rbp
+    ret
+)");
 
 namespace emu {
 
@@ -34,7 +62,7 @@ constexpr size_t STACK = 256 << 10;
 constexpr int MAX_ITEMS = 1024;
 
 struct Fiber {
-    ucontext_t ctx;
+    void *sp = nullptr;
     char *stack = nullptr;
     State st = DONE;
     uint64_t slot = 0;
@@ -50,7 +78,7 @@ struct Fibers {
 };
 thread_local Fibers g_fibers;
 thread_local Fiber *const g_f = g_fibers.f;
-thread_local ucontext_t g_sched;
+thread_local void *g_sched = nullptr;
 thread_local int g_cur = -1, g_n = 0;
 thread_local uint64_t g_part[MAX_ITEMS / 64];  // lanes released together by the last wave barrier
 thread_local const std::function<void()> *g_body = nullptr;
@@ -79,7 +107,7 @@ void to_sched(State st) {
     void *fake = nullptr;
     __sanitizer_start_switch_fiber(&fake, g_main_bottom, g_main_size);
 #endif
-    swapcontext(&g_f[g_cur].ctx, &g_sched);
+    emu_switch(&g_f[g_cur].sp, g_sched);
 #ifdef EMU_ASAN
     __sanitizer_finish_switch_fiber(fake, &g_main_bottom, &g_main_size);
 #endif
@@ -94,7 +122,8 @@ void entry() {
 #ifdef EMU_ASAN
     __sanitizer_start_switch_fiber(nullptr, g_main_bottom, g_main_size);
 #endif
-    setcontext(&g_sched);
+    emu_switch(&g_f[g_cur].sp, g_sched);
+    std::abort();  // a finished work-item is not resumed
 }
 
 void run_block() {
@@ -106,11 +135,13 @@ void run_block() {
                                    MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
             if (f.stack == MAP_FAILED) die("fiber stack allocation failed");
         }
-        getcontext(&f.ctx);
-        f.ctx.uc_stack.ss_sp = f.stack;
-        f.ctx.uc_stack.ss_size = STACK;
-        f.ctx.uc_link = nullptr;
-        makecontext(&f.ctx, entry, 0);
+        void **top = (void **)(f.stack + STACK);
+#ifdef EMU_ASAN
+        __asan_unpoison_memory_region(f.stack + STACK - 4096, 4096);  // entry's frame did not return
+#endif
+        top[-2] = (void *)entry;
+        for (int r = 3; r <= 8; r++) top[-r] = nullptr;
+        f.sp = top - 8;
         f.st = RUN;
         f.slot = 0;
     }
@@ -122,7 +153,7 @@ void run_block() {
 #ifdef EMU_ASAN
             __sanitizer_start_switch_fiber(&g_fake, g_f[i].stack, STACK);
 #endif
-            swapcontext(&g_sched, &g_f[i].ctx);
+            emu_switch(&g_sched, g_f[i].sp);
 #ifdef EMU_ASAN
             __sanitizer_finish_switch_fiber(g_fake, nullptr, nullptr);
 #endif
